@@ -150,6 +150,9 @@ struct tm_mesh {
     // fewer than three neighbours (flips preserve this set on valid meshes)
     DevBuf<int> generic;
     int n_generic = 0;
+    // the sweeps' rows (FlipRows), allocated by the first sweep and rebuilt by each
+    DevBuf<int> flip_nb;
+    DevBuf<int2> flip_er;
     // Internal vertex order (Morton order of the creation-time positions):
     // perm[i] = user id of internal vertex i, iperm[u] = internal id of user
     // vertex u.  Topology and device arrays use internal ids; every id or
@@ -165,6 +168,13 @@ struct tm_mesh {
     FlipMeshView flip_view()
     {
         return FlipMeshView{x.p, d_to.p, d_next.p, d_prev.p, d_face.p, d_vhe.p, d_fhe.p, nv, nh, nf};
+    }
+    FlipRows flip_rows(bool edges)
+    {
+        const size_t n = (size_t)kMaxValence * nv;
+        flip_nb.alloc(n);
+        if (edges) flip_er.alloc(n);
+        return FlipRows{flip_nb.p, edges ? flip_er.p : nullptr};
     }
     ~tm_mesh()
     {
@@ -633,14 +643,14 @@ struct tm_energy {
     DevBuf<double> rep_v, rep_g;
     DevBuf<double> theta;    // pass 1's dihedral angles for pass 2 (kRingPad per vertex, float or double)
     DevBuf<Globals> globals;
-    DevBuf<int> flip_result, proposals, pf_status;
-    DevBuf<double> uniforms, pf_dprops, pf_state;
+    DevBuf<int> flip_result, proposals, pf_rec, pf_lost;
+    DevBuf<double> uniforms, pf_state;
+    DevBuf<unsigned> pf_count;
     double pf_last[8] = {};    // pf_state at the end of the last parallel sweep (tm_energy_pflip_state)
     DevBuf<unsigned long long> pf_owner;
     DevBuf<SerialState> sf_state;
-    DevBuf<int> sf_int;
-    DevBuf<double> sf_dbl;
-    DevBuf<unsigned long long> sf_vstamp, sf_estamp, sf_fstamp;
+    DevBuf<int> sf_rec;
+    DevBuf<unsigned long long> sf_fstamp;
     Tuning tune;
     tm_nlist* spare = nullptr;    // the previous list, rebuilt in place by update_repulsion
     // bumped whenever something a replica group copies into its device
@@ -1264,6 +1274,18 @@ int tm_nlist_point_distances(tm_nlist* nl, tm_mesh* mesh, int pid, double dmax, 
 }
 
 // ---- flips ----
+// Arguments of one parallel sweep, its buffers allocated.
+static PflipArgs pflip_args(tm_energy& E, tm_mesh& M, const EParams& ep, uint64_t seed, int nflips, int batch)
+{
+    E.pf_owner.alloc(M.nh / 2);
+    E.pf_rec.alloc((size_t)kFlipRecord * batch);
+    E.pf_lost.alloc(batch);
+    E.pf_state.alloc(8);
+    E.pf_count.alloc(1);
+    return PflipArgs{M.flip_view(), E.nlist->view(), ep, M.flip_rows(true), seed, nflips, batch, E.globals.p,
+                     E.pf_owner.p, E.pf_rec.p, E.pf_lost.p, E.pf_state.p, E.pf_count.p};
+}
+
 // The serial sweep in windows of W proposals (launch_serial_windows).  The
 // number of windows a sweep needs depends on how many proposals each
 // commits, so they are launched in batches sized from the rate so far, with
@@ -1273,31 +1295,17 @@ static void serial_windows(tm_energy& E, tm_mesh& M, int nflips, const int* prop
 {
     const size_t w = (size_t)W;
     E.sf_state.alloc(1);
-    E.sf_int.alloc(w * (2 + 2 + 4 + 4 + 4 * kMaxValence));
-    E.sf_dbl.alloc(w * 12);
-    E.sf_vstamp.alloc(M.nv);
-    E.sf_estamp.alloc(M.nh / 2);
-    HIPCHECK(hipMemsetAsync(E.sf_vstamp.p, 0, sizeof(unsigned long long) * M.nv, g_rt.stream));
-    HIPCHECK(hipMemsetAsync(E.sf_estamp.p, 0, sizeof(unsigned long long) * (M.nh / 2), g_rt.stream));
+    E.sf_rec.alloc(w * kFlipRecord);
     E.sf_fstamp.alloc(M.nf);
-    HIPCHECK(hipMemsetAsync(E.sf_fstamp.p, 0, sizeof(unsigned long long) * M.nf, g_rt.stream));
-    SerialWindow sw;
-    sw.e = E.sf_int.p;
-    sw.valid = sw.e + w;
-    sw.pv = sw.valid + w;
-    sw.fc = sw.pv + 4 * w;
-    sw.nbn = sw.fc + 2 * w;
-    sw.nb = sw.nbn + 4 * w;
-    sw.dO = E.sf_dbl.p;
-    sw.dN = sw.dO + 6 * w;
+    const FlipRows rows = M.flip_rows(false);
     const EParams p = eparams_of(E);
     const NListView nl = E.nlist->view();
-    launch_serial_init(E.globals.p, p, nflips, E.sf_state.p, g_rt.stream);
+    launch_serial_begin(M.flip_view(), rows, E.globals.p, p, nflips, E.sf_state.p, E.sf_fstamp.p, g_rt.stream);
     int batch = std::max(1, std::min(1024, nflips / W + 1));
     SerialState h{};
     for (;;) {
-        launch_serial_windows(M.flip_view(), nl, p, nflips, proposals, uniforms, n_uniforms, seed, injected, W,
-                              E.sf_state.p, sw, E.sf_vstamp.p, E.sf_estamp.p, E.sf_fstamp.p, batch, g_rt.stream);
+        launch_serial_windows(M.flip_view(), rows, nl, p, nflips, proposals, uniforms, n_uniforms, seed, injected, W,
+                              E.sf_state.p, E.sf_rec.p, E.sf_fstamp.p, batch, g_rt.stream);
         check_launch();
         d2h(&h, E.sf_state.p, sizeof(SerialState));
         sync();
@@ -1314,7 +1322,6 @@ static int flip_impl(tm_energy* em, tm_mesh* mesh, int nflips, const int* propos
 {
     API_BEGIN
     upload_points(*mesh);
-    refresh_host_topology(*mesh);
     // initial properties and energy (flips.cpp:30-31), FP64
     run_pass1(*em, *mesh, 0, nullptr);
     if (injected && nflips > 0) {
@@ -1363,19 +1370,8 @@ int tm_flip_parallel(tm_energy* em, tm_mesh* mesh, double flip_ratio, uint64_t s
     if (batch <= 0) batch = std::max(1, ne / 1024);
     upload_points(*mesh);
     run_pass1(*em, *mesh, 0, nullptr);
-    if (!em->pf_owner.p || em->pf_owner.n < (size_t)ne) {
-        em->pf_owner.alloc(ne);
-        HIPCHECK(hipMemsetAsync(em->pf_owner.p, 0, sizeof(unsigned long long) * ne, g_rt.stream));
-    } else {
-        HIPCHECK(hipMemsetAsync(em->pf_owner.p, 0, sizeof(unsigned long long) * ne, g_rt.stream));
-    }
-    em->pf_status.alloc(batch);
-    em->pf_dprops.alloc((size_t)12 * batch);    // -old, then new
-    em->pf_state.alloc(8);
     if (nflips > 0)
-        launch_flip_parallel(mesh->flip_view(), em->nlist->view(), eparams_of(*em), nflips, batch,
-                             em->tune.pflip_window, seed,
-                             em->globals.p, em->pf_owner.p, em->pf_status.p, em->pf_dprops.p, em->pf_state.p,
+        launch_flip_parallel(pflip_args(*em, *mesh, eparams_of(*em), seed, nflips, batch), em->tune.pflip_window,
                              g_rt.stream);
     check_launch();
     HIPCHECK(hipMemsetAsync(mesh->flag.p, 0, sizeof(int), g_rt.stream));
@@ -1563,7 +1559,7 @@ struct tm_replicas {
     // parallel flip sweeps of the group: per-replica arguments and block
     // prefix tables (rebuilt by every sweep)
     DevBuf<PflipArgs> pf_args;
-    DevBuf<int> pf_claim0, pf_eval0, pf_apply0;
+    DevBuf<int> pf_block0;
     std::vector<int> h_ones;
     int total_disp = 0, total_rc = 0;    // displacement partials, cached-query blocks
     std::vector<unsigned> gens;    // each member's tm_energy::gen when the table was built
@@ -1789,8 +1785,8 @@ int tm_replicas_pflip(tm_replicas* rs, double flip_ratio, const uint64_t* seeds,
         for (int s = 0; s < S.R; s++) slot_of[owner[s]] = s;
     }
     std::vector<PflipArgs> h(S.R);
-    std::vector<int> c0(S.R + 1, 0), e0(S.R + 1, 0), a0(S.R + 1, 0);
-    int rounds = 0;
+    std::vector<int> b0(S.R + 1, 0);
+    int rounds = 0, max_nv = 0, max_nh = 0, max_batch = 0;
     for (int r = 0; r < S.R; r++) {
         tm_mesh& M = *S.meshes[r];
         tm_energy& E = *S.ems[r];
@@ -1799,30 +1795,21 @@ int tm_replicas_pflip(tm_replicas* rs, double flip_ratio, const uint64_t* seeds,
         upload_points(M);
         run_pass1(E, M, 0, nullptr);
         const int ne = M.nh / 2, nflips = (int)(ne * flip_ratio), batch = std::max(1, ne / 1024);
-        if (!E.pf_owner.p || E.pf_owner.n < (size_t)ne) E.pf_owner.alloc(ne);
-        HIPCHECK(hipMemsetAsync(E.pf_owner.p, 0, sizeof(unsigned long long) * ne, g_rt.stream));
-        E.pf_status.alloc(batch);
-        E.pf_dprops.alloc((size_t)12 * batch);
-        E.pf_state.alloc(8);
         EParams ep = eparams_of(E);
         if (S.has_ladder) ep.kappa_b = S.h_ladder[slot_of[r]];
-        h[r] = PflipArgs{M.flip_view(), E.nlist->view(), ep, seeds[r], nflips, batch, E.globals.p, E.pf_owner.p,
-                         E.pf_status.p, E.pf_dprops.p, E.pf_dprops.p + 6 * (size_t)batch, E.pf_state.p};
+        h[r] = pflip_args(E, M, ep, seeds[r], nflips, batch);
         if (nflips > 0) rounds = std::max(rounds, (nflips + batch - 1) / batch);
-        c0[r + 1] = c0[r] + (batch + kClaimPerBlock - 1) / kClaimPerBlock;
-        e0[r + 1] = e0[r] + batch;
-        a0[r + 1] = a0[r] + (batch + 127) / 128;
+        b0[r + 1] = b0[r] + pflip_round_blocks(batch);
+        max_nv = std::max(max_nv, M.nv);
+        max_nh = std::max(max_nh, M.nh);
+        max_batch = std::max(max_batch, batch);
     }
     S.pf_args.alloc(S.R);
-    S.pf_claim0.alloc(S.R + 1);
-    S.pf_eval0.alloc(S.R + 1);
-    S.pf_apply0.alloc(S.R + 1);
+    S.pf_block0.alloc(S.R + 1);
     h2d(S.pf_args.p, h.data(), sizeof(PflipArgs) * S.R);
-    h2d(S.pf_claim0.p, c0.data(), sizeof(int) * (S.R + 1));
-    h2d(S.pf_eval0.p, e0.data(), sizeof(int) * (S.R + 1));
-    h2d(S.pf_apply0.p, a0.data(), sizeof(int) * (S.R + 1));
-    PflipGroup g{S.pf_args.p, S.R, rounds, S.ems[0]->tune.pflip_window, S.pf_claim0.p, c0[S.R],
-                 S.pf_eval0.p, e0[S.R], S.pf_apply0.p, a0[S.R]};
+    h2d(S.pf_block0.p, b0.data(), sizeof(int) * (S.R + 1));
+    const PflipGroup g{S.pf_args.p, S.R, rounds, S.ems[0]->tune.pflip_window, S.pf_block0.p, b0[S.R],
+                       max_nv, max_nh, max_batch};
     launch_flip_parallel_grouped(g, g_rt.stream);
     check_launch();
     std::vector<double> st(8 * (size_t)S.R, 0.0);

@@ -30,6 +30,7 @@
 #include <hip/hip_ext.h>
 #include "tm_internal.h"
 #include "tm_om.h"
+#include "tm_wave.h"
 
 #include <algorithm>
 
@@ -215,39 +216,6 @@ __device__ __forceinline__ Globals globals_of_sums(double v[6], const EParams& p
 constexpr int kGroup = 8;
 static_assert(kGroup == kRingPad, "exclusion tests read kGroup ring columns without the valence");
 static_assert(kGroup == kPairLanes && kPairCap <= 15, "pair-cache counts are 4 bits per lane");
-
-// Sums over the 8 lanes of a group with DPP lane moves (no LDS traffic):
-// xor 1 and xor 2 within quads, then each lane i of the group pairs with lane
-// 7 - i (row_half_mirror), which joins the two quads.  Every lane ends with
-// the same bits (the last step adds the same two quad sums, a + b == b + a).
-constexpr int kDppXor1 = 0xB1;        // quad_perm [1,0,3,2]
-constexpr int kDppXor2 = 0x4E;        // quad_perm [2,3,0,1]
-constexpr int kDppHalfMirror = 0x141; // row_half_mirror
-template <int CTRL>
-__device__ __forceinline__ int dpp_i(int v)
-{
-    return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xF, 0xF, false);
-}
-template <int CTRL>
-__device__ __forceinline__ double dpp_d(double v)
-{
-    int lo = __double2loint(v), hi = __double2hiint(v);
-    return __hiloint2double(dpp_i<CTRL>(hi), dpp_i<CTRL>(lo));
-}
-__device__ __forceinline__ double group_sum(double x)
-{
-    x += dpp_d<kDppXor1>(x);
-    x += dpp_d<kDppXor2>(x);
-    x += dpp_d<kDppHalfMirror>(x);
-    return x;
-}
-__device__ __forceinline__ int group_sum(int x)
-{
-    x += dpp_i<kDppXor1>(x);
-    x += dpp_i<kDppXor2>(x);
-    x += dpp_i<kDppHalfMirror>(x);
-    return x;
-}
 
 // Exclusion test of the cell list (cell_list.h:170-202) on the ring table:
 // j is excluded at level 1 if it is in ring(v), and at level 2 also if ring(j)

@@ -1,6 +1,7 @@
 // tm_flips.hip -- ring-table rebuild and the edge-flip sweeps: the serial
 // sweep (one workgroup, k_flip_serial, or windows of proposals evaluated at
-// once and committed in order, k_sf_*) and the parallel sweep (k_pflip_*).
+// once and committed in order, k_sf_window) and the parallel sweep
+// (k_pflip_round).
 //
 // flip_serial (src/flips.cpp:22-80) is a Metropolis loop in which every
 // proposal depends on the topology left by the previous one.  The
@@ -18,6 +19,7 @@
 #include "tm_internal.h"
 #include "tm_om.h"
 #include "tm_rng.h"
+#include "tm_wave.h"
 
 #include <algorithm>
 
@@ -110,122 +112,84 @@ __device__ __forceinline__ bool flip_ok(const Topo& t, int e)
     return !adjacent && na + 1 < kMaxValence && nb + 1 < kMaxValence;
 }
 
-__device__ __forceinline__ void do_flip(const FlipMeshView& fm, int e)
-{
-    // OpenMesh TriConnectivity::flip
-    int a0 = 2 * e, b0 = 2 * e + 1;
-    int a1 = fm.he_next[a0], a2 = fm.he_next[a1];
-    int b1 = fm.he_next[b0], b2 = fm.he_next[b1];
-    int va0 = fm.he_to[a0], va1 = fm.he_to[a1];
-    int vb0 = fm.he_to[b0], vb1 = fm.he_to[b1];
-    int fa = fm.he_face[a0], fb = fm.he_face[b0];
-    fm.he_to[a0] = va1;
-    fm.he_to[b0] = vb1;
-    fm.he_next[a0] = a2; fm.he_prev[a2] = a0;
-    fm.he_next[a2] = b1; fm.he_prev[b1] = a2;
-    fm.he_next[b1] = a0; fm.he_prev[a0] = b1;
-    fm.he_next[b0] = b2; fm.he_prev[b2] = b0;
-    fm.he_next[b2] = a1; fm.he_prev[a1] = b2;
-    fm.he_next[a1] = b0; fm.he_prev[b0] = a1;
-    fm.he_face[a1] = fb;
-    fm.he_face[b1] = fa;
-    fm.f_he[fa] = a0;
-    fm.f_he[fb] = b0;
-    if (fm.v_he[va0] == b0) fm.v_he[va0] = a1;
-    if (fm.v_he[vb0] == a0) fm.v_he[vb0] = b1;
-}
-
-// The topology after flipping interior edge e, without writing it: every
-// accessor returns what do_flip stores, so a workgroup can evaluate the
-// flipped patch while others read the unflipped mesh.
-struct FlippedTopo {
-    Topo t;
-    const double* x;
-    int a0, a1, a2, b0, b1, b2;
-    int va1, vb1, va0, vb0, fa, fb;
-    int vhe_a, vhe_b;    // v_he of va0 and vb0 after the flip
-
-    __device__ FlippedTopo(const Topo& base, int e) : t(base), x(base.x)
-    {
-        a0 = 2 * e;
-        b0 = 2 * e + 1;
-        a1 = t.next(a0);
-        a2 = t.next(a1);
-        b1 = t.next(b0);
-        b2 = t.next(b1);
-        va0 = t.to(a0);
-        va1 = t.to(a1);
-        vb0 = t.to(b0);
-        vb1 = t.to(b1);
-        fa = t.face(a0);
-        fb = t.face(b0);
-        const int ha = t.vhe(va0), hb = t.vhe(vb0);
-        vhe_a = ha == b0 ? a1 : ha;
-        vhe_b = hb == a0 ? b1 : hb;
-    }
-    __device__ __forceinline__ d3 P(int v) const { return t.P(v); }
-    __device__ __forceinline__ int to(int h) const { return h == a0 ? va1 : (h == b0 ? vb1 : t.to(h)); }
-    __device__ __forceinline__ int from(int h) const { return to(h ^ 1); }
-    __device__ __forceinline__ int next(int h) const
-    {
-        if (h == a0) return a2;
-        if (h == a2) return b1;
-        if (h == b1) return a0;
-        if (h == b0) return b2;
-        if (h == b2) return a1;
-        if (h == a1) return b0;
-        return t.next(h);
-    }
-    __device__ __forceinline__ int prev(int h) const
-    {
-        if (h == a2) return a0;
-        if (h == b1) return a2;
-        if (h == a0) return b1;
-        if (h == b2) return b0;
-        if (h == a1) return b2;
-        if (h == b0) return a1;
-        return t.prev(h);
-    }
-    __device__ __forceinline__ int face(int h) const { return h == a1 ? fb : (h == b1 ? fa : t.face(h)); }
-    __device__ __forceinline__ bool he_boundary(int h) const { return face(h) < 0; }
-    __device__ __forceinline__ bool edge_boundary(int e) const { return face(2 * e) < 0 || face(2 * e + 1) < 0; }
-    __device__ __forceinline__ int cw(int h) const { return next(h ^ 1); }
-    __device__ __forceinline__ int vhe(int v) const { return v == va0 ? vhe_a : (v == vb0 ? vhe_b : t.vhe(v)); }
-    __device__ __forceinline__ int fhe(int f) const { return f == fa ? a0 : (f == fb ? b0 : t.fhe(f)); }
+// An interior edge's two triangles: what a flip reads.  a0 = 2e, b0 = 2e + 1.
+struct FlipEdge {
+    int e;
+    int pv[4];             // to(a0), to(a1), to(b0), to(b1)
+    int a1, a2, b1, b2;    // the halfedges that follow a0 and b0
+    int fa, fb;            // faces of a0 and b0 (-1 on a boundary, the rest then unset)
+    int ha, hb;            // v_he of to(a0) and to(b0)
 };
-
-// do_flip(fm, e) twice (a rejected proposal), stored in one pass.  The
-// second flip undoes the connectivity but not the ids: the edge's two
-// halfedges swap direction, the two faces swap triangles, and the v_he of
-// the edge's endpoints move off the swapped halfedges exactly as the first
-// flip moved them (the second flip's v_he tests cannot hold, since its
-// endpoints' outgoing halfedges are not the edge's).
-__device__ __forceinline__ void do_flip_twice(const FlipMeshView& fm, int e)
+__device__ __forceinline__ FlipEdge load_flip_edge(const FlipMeshView& fm, int e)
 {
-    int a0 = 2 * e, b0 = 2 * e + 1;
-    int a1 = fm.he_next[a0], a2 = fm.he_next[a1];
-    int b1 = fm.he_next[b0], b2 = fm.he_next[b1];
-    int va0 = fm.he_to[a0], vb0 = fm.he_to[b0];
-    int ta2 = fm.he_to[a2], tb2 = fm.he_to[b2];
-    int fa = fm.he_face[a0], fb = fm.he_face[b0];
-    int ha = fm.v_he[va0], hb = fm.v_he[vb0];
-    fm.he_to[a0] = ta2;
-    fm.he_to[b0] = tb2;
-    fm.he_next[a0] = b1; fm.he_prev[b1] = a0;
-    fm.he_next[b1] = b2; fm.he_prev[b2] = b1;
-    fm.he_next[b2] = a0; fm.he_prev[a0] = b2;
-    fm.he_next[b0] = a1; fm.he_prev[a1] = b0;
-    fm.he_next[a1] = a2; fm.he_prev[a2] = a1;
-    fm.he_next[a2] = b0; fm.he_prev[b0] = a2;
-    fm.he_face[a1] = fb;
-    fm.he_face[a2] = fb;
-    fm.he_face[b1] = fa;
-    fm.he_face[b2] = fa;
-    fm.f_he[fa] = a0;
-    fm.f_he[fb] = b0;
-    if (ha == b0) fm.v_he[va0] = a1;
-    if (hb == a0) fm.v_he[vb0] = b1;
+    FlipEdge f{};
+    f.e = e;
+    const int2 nx = reinterpret_cast<const int2*>(fm.he_next)[e], to = reinterpret_cast<const int2*>(fm.he_to)[e];
+    const int2 fc = reinterpret_cast<const int2*>(fm.he_face)[e];
+    f.fa = fc.x;
+    f.fb = fc.y;
+    if (f.fa < 0 || f.fb < 0) return f;
+    f.a1 = nx.x;
+    f.b1 = nx.y;
+    f.pv[0] = to.x;
+    f.pv[2] = to.y;
+    f.pv[1] = fm.he_to[f.a1];
+    f.pv[3] = fm.he_to[f.b1];
+    f.a2 = fm.he_next[f.a1];
+    f.b2 = fm.he_next[f.b1];
+    f.ha = fm.v_he[f.pv[0]];
+    f.hb = fm.v_he[f.pv[2]];
+    return f;
 }
+
+// OpenMesh TriConnectivity::flip of f.e
+__device__ __forceinline__ void store_flip(const FlipMeshView& fm, const FlipEdge& f)
+{
+    const int a0 = 2 * f.e, b0 = a0 + 1;
+    fm.he_to[a0] = f.pv[1];
+    fm.he_to[b0] = f.pv[3];
+    fm.he_next[a0] = f.a2; fm.he_prev[f.a2] = a0;
+    fm.he_next[f.a2] = f.b1; fm.he_prev[f.b1] = f.a2;
+    fm.he_next[f.b1] = a0; fm.he_prev[a0] = f.b1;
+    fm.he_next[b0] = f.b2; fm.he_prev[f.b2] = b0;
+    fm.he_next[f.b2] = f.a1; fm.he_prev[f.a1] = f.b2;
+    fm.he_next[f.a1] = b0; fm.he_prev[b0] = f.a1;
+    fm.he_face[f.a1] = f.fb;
+    fm.he_face[f.b1] = f.fa;
+    fm.f_he[f.fa] = a0;
+    fm.f_he[f.fb] = b0;
+    if (f.ha == b0) fm.v_he[f.pv[0]] = f.a1;
+    if (f.hb == a0) fm.v_he[f.pv[2]] = f.b1;
+}
+
+// store_flip twice (a rejected proposal) in one pass.  The second flip
+// undoes the connectivity but not the ids: the edge's two halfedges swap
+// direction, the two faces swap triangles, and the v_he of the edge's
+// endpoints move off the swapped halfedges exactly as the first flip moved
+// them (the second flip's v_he tests cannot hold, since its endpoints'
+// outgoing halfedges are not the edge's).
+__device__ __forceinline__ void store_flip_twice(const FlipMeshView& fm, const FlipEdge& f)
+{
+    const int a0 = 2 * f.e, b0 = a0 + 1;
+    fm.he_to[a0] = f.pv[2];
+    fm.he_to[b0] = f.pv[0];
+    fm.he_next[a0] = f.b1; fm.he_prev[f.b1] = a0;
+    fm.he_next[f.b1] = f.b2; fm.he_prev[f.b2] = f.b1;
+    fm.he_next[f.b2] = a0; fm.he_prev[a0] = f.b2;
+    fm.he_next[b0] = f.a1; fm.he_prev[f.a1] = b0;
+    fm.he_next[f.a1] = f.a2; fm.he_prev[f.a2] = f.a1;
+    fm.he_next[f.a2] = b0; fm.he_prev[b0] = f.a2;
+    fm.he_face[f.a1] = f.fb;
+    fm.he_face[f.a2] = f.fb;
+    fm.he_face[f.b1] = f.fa;
+    fm.he_face[f.b2] = f.fa;
+    fm.f_he[f.fa] = a0;
+    fm.f_he[f.fb] = b0;
+    if (f.ha == b0) fm.v_he[f.pv[0]] = f.a1;
+    if (f.hb == a0) fm.v_he[f.pv[2]] = f.b1;
+}
+
+__device__ __forceinline__ void do_flip(const FlipMeshView& fm, int e) { store_flip(fm, load_flip_edge(fm, e)); }
 
 __device__ __forceinline__ double energy_of(const double pr[6], const EParams& p)
 {
@@ -260,12 +224,6 @@ __device__ __forceinline__ double energy_of(const double pr[6], const EParams& p
 // A vertex whose valence exceeds kMaxValence is evaluated by its lane 0
 // with om_vertex_properties.
 constexpr int kCoopLanes = 16;
-// The parallel sweep's patch kernels keep to 128 registers (four waves per
-// SIMD, 16 workgroups per CU): a sweep over a replica group has far more
-// patches than the GPU holds at once, and occupancy, not one patch's
-// latency, then bounds it (at 153 registers, 12 workgroups per CU, a round
-// over 32 meshes of 491520 edges took 21% longer).
-#define TM_COOP_OCCUPANCY __attribute__((amdgpu_waves_per_eu(4)))
 constexpr int kCoopChunk = 4 * kCoopLanes;
 
 struct CoopShared {
@@ -277,9 +235,6 @@ struct CoopShared {
     double slot[4][kMaxValence][4];     // area, volume, edge curvature, tether
     int run_s[4][9], run_len[4][9];     // candidate runs (CandRuns) of the repulsion query
     double pos[4][3];                   // the patch vertex's position
-    int ve[4];                          // the patch vertices
-    int flip_ok;                        // flip_ok(e), when coop_patch tests it
-    int lost[4];                        // a patch edge of the vertex is owned by another proposal
     double rep[4][kCoopChunk];
     double vp[4][6];
     double sum[6];
@@ -375,18 +330,9 @@ __device__ __forceinline__ bool coop_excluded(const TP& t, const CoopShared& S, 
 }
 
 // Called by all 64 threads of the workgroup; S.vp and S.sum hold the result
-// on return.  test_flip (on the topology before the flip, e interior): S.flip_ok
-// = flip_ok(t, e) from the one-rings of phase 1, which include those of the
-// two vertices opposite the edge (patch vertices 1 and 3), and nothing more
-// is evaluated when it is false.  owner (same topology): S.lost = some edge
-// of the parallel sweep's patch, the spokes h >> 1 and rims next(h) >> 1 of
-// every outgoing halfedge h of the four vertices (the flip patch), is
-// owned by another key, tested on phase 2's halfedges; nothing more is
-// evaluated then.
+// on return.
 template <class TP>
-__device__ void coop_patch(const TP& t, const NListView& nl, const EParams& p, int e, CoopShared& S,
-                           bool test_flip = false, const unsigned long long* __restrict__ owner = nullptr,
-                           unsigned long long key = 0)
+__device__ void coop_patch(const TP& t, const NListView& nl, const EParams& p, int e, CoopShared& S)
 {
     const int g = threadIdx.x / kCoopLanes, l = threadIdx.x % kCoopLanes;
     const int ve = patch_vertex(t, e, g);
@@ -422,32 +368,9 @@ __device__ void coop_patch(const TP& t, const NListView& nl, const EParams& p, i
             } while (h != h0);
         }
         S.n[g] = n;
-        S.ve[g] = ve;
         if (n < 0) S.total[g] = 0;
-        // a ring too long for LDS: its patch edges by a walk of their own
-        bool lost = false;
-        if (owner && n < 0 && h0 >= 0) {
-            int h = h0, guard = 0;
-            do {
-                lost = lost || owner[h >> 1] != key || owner[t.next(h) >> 1] != key;
-                h = t.cw(h);
-            } while (h != h0 && ++guard < 4 * kMaxValence);
-        }
-        S.lost[g] = lost;
     }
     __syncthreads();
-    if (test_flip) {
-        // flip_ok's walks: the opposite vertices differ, are not adjacent
-        // and have valence below kMaxValence (n is -1 above it)
-        if (threadIdx.x == 0) {
-            const int a = S.ve[1], b = S.ve[3], na = S.n[1], nb = S.n[3];
-            bool ok = a != b && na >= 0 && na < kMaxValence && nb >= 0 && nb < kMaxValence;
-            for (int k = 0; ok && k < na; k++) ok = S.nb[1][k] != b;
-            S.flip_ok = ok;
-        }
-        __syncthreads();
-        if (!S.flip_ok) return;
-    }
     const int n = S.n[g];
 
     // phase 2
@@ -463,10 +386,8 @@ __device__ void coop_patch(const TP& t, const NListView& nl, const EParams& p, i
             S.slot[g][s][2] = 0.5 * el * da;
             S.slot[g][s][3] = p.bond_type == 0 ? bond_edge_value(el, p) : bond_area_value(mu_face_area(t, h), p);
         }
-        if (owner && (owner[h >> 1] != key || owner[t.next(h) >> 1] != key)) S.lost[g] = 1;
     }
     __syncthreads();
-    if (owner && (S.lost[0] | S.lost[1] | S.lost[2] | S.lost[3])) return;
 
     // phase 3
     const d3 pi{S.pos[g][0], S.pos[g][1], S.pos[g][2]};
@@ -648,505 +569,853 @@ void launch_flip_serial(const FlipMeshView& fm, const NListView& nl, const EPara
                        seed, injected, g0, result);
 }
 
+// ==================================================== rows of the one-rings ==
+// The sweeps below read every vertex's one-ring from a row of its own instead
+// of walking the halfedges: nb[kRowW v + k] is the k-th neighbour in the
+// circulator's (clockwise) order, with kNoFace set when the halfedge to it has
+// no face, and the row ends with -1 when it is shorter than kRowW.  er holds
+// each slot's spoke edge and rim edge (the edge of the next halfedge in its
+// face), the edges the parallel sweep claims.  A walk around a ring is a chain
+// of about twelve dependent loads; a row is one, and a patch's four rows, the
+// positions of their entries and the candidates of its repulsion query are
+// five levels in all.  Rows are built at the start of a sweep and rewritten
+// for the four vertices of every accepted flip; a rejected flip (do_flip
+// twice) leaves every vertex's neighbours and their cyclic order.
+constexpr int kRowW = kMaxValence;
+constexpr int kRowPair = 8;    // slots read or written in one round of vector operations
+constexpr int kNoFace = 1 << 30;
+
+__device__ __forceinline__ void build_rows(const FlipMeshView& fm, const FlipRows& rows, int v)
+{
+    const int h0 = fm.v_he[v];
+    int* nb = rows.nb + (size_t)kRowW * v;
+    int2* er = rows.er ? rows.er + (size_t)kRowW * v : nullptr;
+    // the leading kRowPair slots in registers, stored as vectors
+    int id[kRowPair], sp[kRowPair], rm[kRowPair];
+#pragma unroll
+    for (int k = 0; k < kRowPair; k++) {
+        id[k] = -1;
+        sp[k] = rm[k] = 0;
+    }
+    int n = 0, h = h0;
+    if (h0 >= 0) {
+#pragma unroll
+        for (int k = 0; k < kRowPair; k++) {
+            if (k > 0 && h == h0) break;
+            id[k] = fm.he_to[h] | (fm.he_face[h] < 0 ? kNoFace : 0);
+            sp[k] = h >> 1;
+            rm[k] = er ? fm.he_next[h] >> 1 : 0;
+            n++;
+            h = fm.he_next[h ^ 1];
+        }
+        if (h != h0)
+            do {
+                nb[n] = fm.he_to[h] | (fm.he_face[h] < 0 ? kNoFace : 0);
+                if (er) er[n] = make_int2(h >> 1, fm.he_next[h] >> 1);
+                n++;
+                h = fm.he_next[h ^ 1];
+            } while (h != h0 && n < kRowW);
+    }
+#pragma unroll
+    for (int k = 0; k < kRowPair; k += 4) {
+        reinterpret_cast<int4*>(nb)[k / 4] = make_int4(id[k], id[k + 1], id[k + 2], id[k + 3]);
+        if (er) {
+            reinterpret_cast<int4*>(er)[k / 2] = make_int4(sp[k], rm[k], sp[k + 1], rm[k + 1]);
+            reinterpret_cast<int4*>(er)[k / 2 + 1] = make_int4(sp[k + 2], rm[k + 2], sp[k + 3], rm[k + 3]);
+        }
+    }
+    if (n >= kRowPair && n < kRowW) nb[n] = -1;
+}
+
+
+// The row of patch vertex g after the flip of e.  With the edge's triangles
+// (B, A, C) and (A, B, D), A = to(2e) (g 0) and B = to(2e + 1) (g 2) lose
+// each other: the slot that follows takes the new edge, e again, as its rim.
+// C = to(next(2e)) (g 1) and D (g 3) gain each other before their slot of B
+// and of A, with rims ed[0] (of the new slot) and ed[1] (of the slot after).
+// One thread per vertex; rows of at most kRowPair slots are read in one
+// round of loads, longer ones are shifted in memory.
+__device__ __forceinline__ void flip_row(const FlipRows& rows, int ve, int g, int partner, int opposite, int e,
+                                         int2 ed)
+{
+    int* nb = rows.nb + (size_t)kRowW * ve;
+    int2* er = rows.er ? rows.er + (size_t)kRowW * ve : nullptr;
+    int id[kRowPair + 1];
+    int2 ee[kRowPair + 1];
+#pragma unroll
+    for (int k = 0; k <= kRowPair; k++) {
+        id[k] = nb[k];
+        ee[k] = er ? er[k] : make_int2(0, 0);
+    }
+    int n = kRowPair + 1;
+#pragma unroll
+    for (int k = kRowPair; k >= 0; k--)
+        if (id[k] < 0) n = k;
+    if (n <= kRowPair) {
+        int r = -1;
+#pragma unroll
+        for (int k = 0; k < kRowPair; k++)
+            if (k < n && (id[k] & ~kNoFace) == partner) r = k;
+        if (g & 1) {
+            // slots r .. n-1 move up by one
+#pragma unroll
+            for (int k = kRowPair; k > 0; k--)
+                if (k > r && k <= n) {
+                    nb[k] = id[k - 1];
+                    if (er) er[k] = make_int2(ee[k - 1].x, k == r + 1 ? ed.y : ee[k - 1].y);
+                }
+            nb[r] = opposite;
+            if (er) er[r] = make_int2(e, ed.x);
+            if (n + 1 < kRowW) nb[n + 1] = -1;
+        } else {
+#pragma unroll
+            for (int k = 0; k < kRowPair; k++)
+                if (k >= r && k + 1 < n) {
+                    nb[k] = id[k + 1];
+                    if (er) er[k] = make_int2(ee[k + 1].x, k == r ? e : ee[k + 1].y);
+                }
+            nb[n - 1] = -1;
+            if (er && r == n - 1) er[0].y = e;    // the slot that follows the last is the first
+        }
+        return;
+    }
+    n = 0;
+    int r = -1;
+    while (n < kRowW && nb[n] >= 0) {
+        if ((nb[n] & ~kNoFace) == partner) r = n;
+        n++;
+    }
+    if (g & 1) {
+        if (er) er[r].y = ed.y;
+        for (int k = n; k > r; k--) {
+            nb[k] = nb[k - 1];
+            if (er) er[k] = er[k - 1];
+        }
+        nb[r] = opposite;
+        if (er) er[r] = make_int2(e, ed.x);
+        if (n + 1 < kRowW) nb[n + 1] = -1;
+    } else {
+        if (er) er[r + 1 < n ? r + 1 : 0].y = e;
+        for (int k = r; k + 1 < n; k++) {
+            nb[k] = nb[k + 1];
+            if (er) er[k] = er[k + 1];
+        }
+        nb[n - 1] = -1;
+    }
+}
+
+// ------------------------------------------------------- patch evaluation --
+// Order between a wave's own LDS writes and reads (the LDS serves one wave's
+// operations in order, so only the compiler must keep them).
+__device__ __forceinline__ void wave_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+constexpr int kPatchWaves = 4;    // proposals per 256-thread workgroup, one wave each
+
+constexpr int kCandBatch = 4;                 // candidates in flight per lane
+constexpr int kListMax = 16 * kCandBatch;     // of one step of a vertex's 16 lanes
+struct PatchShared {
+    double pos[4][kRowW][3];    // positions of the one-rings
+    double pv[4][3];            // positions of the patch vertices
+    alignas(16) int nb[4][kRowW];    // the one-rings (kNoFace bits kept)
+    int pre[4][9], st[4][9];    // candidate runs: inclusive prefix of their lengths, starts
+    int list[4][kListMax];      // candidates inside the cutoff that a ring test has not excluded
+};
+
+struct NoClaim {
+    __device__ __forceinline__ void load(int, int) {}
+    __device__ __forceinline__ void issue(bool) {}
+    __device__ __forceinline__ void more(int, int, bool) {}
+};
+
+struct PatchResult {
+    bool ok;          // is_flip_ok and the valence cap (flip_ok)
+    double val[6];    // lanes 0-7: sums before the flip, lanes 8-15: after it
+    __device__ __forceinline__ void difference(double (&d)[6]) const
+    {
+#pragma unroll
+        for (int c = 0; c < 6; c++) d[c] = __shfl(val[c], 8, 64) - __shfl(val[c], 0, 64);
+    }
+};
+
+// vertex_properties (mesh_properties.cpp:12-49) summed over the four vertices
+// of interior edge e's flip patch (flip_utils.cpp:19-41), before and after the
+// flip, by one wave.  Lanes 16 g .. 16 g + 15 serve patch vertex g (ve[g]: to(2e),
+// to(next(2e)), to(2e+1), to(next(2e+1))): first its row, one slot per lane,
+// and the ring positions, into LDS; then lanes 0-7 of the group take the
+// slots of the ring before the flip and lanes 8-15 those after it, which is
+// the same ring without the edge's other end (g 0, 2) or with the other
+// opposite vertex (g 1, 3) in front of the slot of `partner`; then all 16
+// test the repulsion candidates once, each against both rings.  Every
+// sum is a fixed butterfly, so the bits depend on the rows alone.  What bounds
+// it is the chain of dependent loads: rows, positions and cell ranges,
+// candidate ids, candidate positions.  claim: PatchClaim claims every edge of
+// the patch meanwhile, NoClaim nothing.
+template <class Claim>
+__device__ __forceinline__ PatchResult patch_eval(const FlipMeshView& fm, const NListView& nl, const EParams& p,
+                                                  const FlipRows& rows, const int (&pv)[4], PatchShared& S,
+                                                  Claim& claim)
+{
+    const int lane = threadIdx.x & 63, g = lane >> 4, q = lane & 15;
+    const int side = (lane >> 3) & 1, k8 = lane & 7;
+    const int ve = g == 0 ? pv[0] : (g == 1 ? pv[1] : (g == 2 ? pv[2] : pv[3]));
+    const int partner = g < 2 ? pv[2] : pv[0];
+    const int opp = g == 1 ? pv[3] : pv[1];    // of C: D, of D: C (g odd only)
+    const bool rep_on = p.rep_lc1 > 0 && nl.kind >= 0;
+
+    // rows (a second chunk of 16 slots only where the first is full), the
+    // vertices' own positions
+    const int* row = rows.nb + (size_t)kRowW * ve;
+    int id = row[q];
+    claim.load(ve, q);
+    const d3 xv{fm.x[3 * ve], fm.x[3 * ve + 1], fm.x[3 * ve + 2]};
+    unsigned full = (unsigned)(__ballot(id >= 0) >> (16 * g)) & 0xffffu;
+    int n0 = __ffs(~full) - 1;    // slots before the end mark
+    int id2 = -1, n2 = 0;
+    if (__ballot(n0 == 16)) {
+        if (n0 == 16) id2 = row[16 + q];
+        const unsigned f2 = (unsigned)(__ballot(id2 >= 0) >> (16 * g)) & 0xffffu;
+        n2 = n0 == 16 ? __ffs(~f2) - 1 : 0;
+    }
+    const bool has = q < n0, has2 = q < n2;
+    // cell ranges of the repulsion query: lane q < 9 takes row q of the stencil
+    int rs = 0, rl = 0;
+    if (rep_on && q < 9) {
+        if (nl.kind == 0) {
+            int c[3];
+            cell_coords(nl, xv, c);
+            const int kk = c[2] + q / 3 - 1, jj = c[1] + q % 3 - 1;
+            const int i0 = max(c[0] - 1, 0), i1 = min(c[0] + 1, nl.shape[0] - 1);
+            if (kk >= 0 && kk < nl.shape[2] && jj >= 0 && jj < nl.shape[1] && i0 <= i1) {
+                const int base = jj * nl.strides[1] + kk * nl.strides[2];
+                rs = nl.cell_start[base + i0];
+                rl = nl.cell_start[base + i1 + 1] - rs;
+            }
+        } else if (q == 0) {
+            rs = nl.adj_start[ve];
+            rl = nl.adj_start[ve + 1] - rs;
+        }
+    }
+    const int j0 = id & ~kNoFace, j2 = id2 & ~kNoFace;
+    d3 xj{0, 0, 0};
+    if (has) xj = d3{fm.x[3 * j0], fm.x[3 * j0 + 1], fm.x[3 * j0 + 2]};
+    claim.issue(has);
+    if (__ballot(has2)) claim.more(ve, 16 + q, has2);
+    if (has) {
+        S.nb[g][q] = id;
+        S.pos[g][q][0] = xj.x;
+        S.pos[g][q][1] = xj.y;
+        S.pos[g][q][2] = xj.z;
+    }
+    if (has2) {
+        S.nb[g][16 + q] = id2;
+        for (int c = 0; c < 3; c++) S.pos[g][16 + q][c] = fm.x[3 * j2 + c];
+    }
+    if (q == 0) {
+        S.pv[g][0] = xv.x;
+        S.pv[g][1] = xv.y;
+        S.pv[g][2] = xv.z;
+    }
+    n0 += n2;
+    // the partner's slot, and flip_ok: opposite vertices distinct, not
+    // adjacent, both below the valence cap
+    const unsigned at = (unsigned)(__ballot(has && j0 == partner) >> (16 * g)) & 0xffffu;
+    const unsigned at2 = (unsigned)(__ballot(has2 && j2 == partner) >> (16 * g)) & 0xffffu;
+    const int r = at ? __ffs(at) - 1 : (at2 ? 16 + __ffs(at2) - 1 : -1);
+    const bool bad = r < 0 || ((g & 1) && (n0 >= kMaxValence || ve == opp || (has && j0 == opp) || (has2 && j2 == opp)));
+    PatchResult res;
+    res.ok = __ballot(bad) == 0ull;
+    if (!res.ok) return res;
+    // inclusive prefix of the run lengths over lanes 0-8
+    int pre = rl;
+#pragma unroll
+    for (int o = 1; o < 16; o <<= 1) {
+        const int y = __shfl_up(pre, o, 16);
+        if (q >= o) pre += y;
+    }
+    const int total = __shfl(pre, 8, 16);
+    if (q < 9) {
+        S.pre[g][q] = pre;
+        S.st[g][q] = rs - (pre - rl);
+    }
+    wave_sync();
+
+    // the first candidates' ids, in flight during the ring terms
+    int cand[kCandBatch];
+    auto load_candidates = [&](int t0) {
+        const int* ids = nl.kind == 0 ? nl.cell_verts : nl.adj;
+#pragma unroll
+        for (int u = 0; u < kCandBatch; u++) {
+            const int t = t0 + 16 * u + q;
+            cand[u] = -1;
+            if (t < total) {
+                int w = 0;
+#pragma unroll
+                for (int i = 0; i < 8; i++) w += t >= S.pre[g][i] ? 1 : 0;
+                cand[u] = ids[S.st[g][w] + t];
+            }
+        }
+    };
+    load_candidates(0);
+
+    // ring terms
+    const int nS = side ? ((g & 1) ? n0 + 1 : n0 - 1) : n0;
+    auto slot_of = [&](int s) {    // slot of the stored ring, or -1 for the vertex the flip adds
+        if (!side) return s;
+        if (g & 1) return s < r ? s : (s == r ? -1 : s - 1);
+        return s < r ? s : s + 1;
+    };
+    auto at_slot = [&](int i) {
+        const double* a = i < 0 ? S.pv[4 - g] : S.pos[g][i];    // g odd: 4 - g is the other opposite vertex
+        return d3{a[0], a[1], a[2]};
+    };
+    double area = 0, vol = 0, curv = 0, teth = 0;
+    for (int c0 = 0; __ballot(c0 + k8 < nS); c0 += 8) {
+        const int s = c0 + k8;
+        const int i1 = s < nS ? slot_of(s) : 0, i2 = slot_of(s + 1 < nS ? s + 1 : 0);
+        const bool nof = i1 >= 0 && (S.nb[g][i1] & kNoFace), nofn = i2 >= 0 && (S.nb[g][i2] & kNoFace);
+        // a halfedge without a face contributes nothing
+        if (s < nS && !nof) {
+        const d3 ec = at_slot(i1) - xv, ep = at_slot(slot_of(s > 0 ? s - 1 : nS - 1)) - xv, en = at_slot(i2) - xv;
+        const d3 nc = cross(ec, ep), nn = cross(en, ec);
+        const double nl0 = norm(nc), el = norm(ec);
+        double da = 0.0;
+        if (!nofn) {
+            const double denom = nl0 * norm(nn);
+            if (denom != 0) da = om_angle(dot(nc, nn) / denom, dot(cross(nc, nn), ec));
+        }
+        const double fa = nl0 / 2;
+        curv += 0.5 * el * da;
+        area += fa;
+        vol += dot(xv, nc) / 6;
+        teth += p.bond_type == 0 ? bond_edge_value(el, p) : bond_area_value(fa, p);
+        }
+    }
+    area = group_sum(area) / 3;
+    vol = group_sum(vol) / 3;
+    curv = group_sum(curv) / 2;
+    teth = group_sum(teth) / (p.bond_type == 0 ? 2 : 3);
+
+    // repulsion: each candidate inside the cutoff against the ring before the
+    // flip and the one after it (mesh_repulsion.h:28-54; exclusion as in
+    // ring_excluded of the energy passes: at level 2, when the candidate's own
+    // ring, as it is on that side, meets the vertex's)
+    double rep0 = 0.0, rep1 = 0.0;
+    if (rep_on) {
+        const double dmax = p.rep_lc1, dmax2 = dmax * dmax * (1.0 + 1e-15);
+        const double dsure2 = dmax * dmax * (1.0 - 1e-15);    // surely inside: no root needed
+        const int excl = nl.kind == 0 ? nl.exclusion : 0;
+        const int lost = (g & 1) ? -1 : partner, gained = (g & 1) ? opp : -1;
+        // the ring in registers, -2 past its end (rings above kRowPair: the
+        // rest from LDS)
+        int rg[kRowPair];
+        const bool wide = __ballot(n0 > kRowPair) != 0ull;
+#pragma unroll
+        for (int i = 0; i < kRowPair; i++) rg[i] = S.nb[g][i];
+#pragma unroll
+        for (int i = 0; i < kRowPair; i++) rg[i] = i < n0 ? rg[i] & ~kNoFace : -2;
+        auto in_ring = [&](int w) {
+            bool hit = false;
+#pragma unroll
+            for (int i = 0; i < kRowPair; i++) hit |= rg[i] == w;
+            if (wide)
+                for (int i = kRowPair; i < n0; i++) hit |= (S.nb[g][i] & ~kNoFace) == w;
+            return hit;
+        };
+        for (int t0 = 0;;) {
+            d3 d[kCandBatch];
+#pragma unroll
+            for (int u = 0; u < kCandBatch; u++)
+                if (cand[u] >= 0) d[u] = xv - d3{fm.x[3 * cand[u]], fm.x[3 * cand[u] + 1], fm.x[3 * cand[u] + 2]};
+            // within the cutoff, excluded before (bit 30) and after (bit 31).
+            // At level 2 the ring before the flip counts on both sides: the two
+            // ends of the edge still share C and D after it, and C and D share
+            // A and B before it.  Few candidates are left, if any: they are
+            // collected, so that one step of the lanes deals with them
+            int listed = 0;
+#pragma unroll
+            for (int u = 0; u < kCandBatch; u++) {
+                const int c = cand[u];
+                bool e0 = true, e1 = true;
+                const double sq = c >= 0 ? sqnorm(d[u]) : 0.0;
+                if (c >= 0 && sq <= dmax2 && (sq < dsure2 || sqrt(sq) < dmax)) {
+                    e0 = e1 = nl.kind == 0 && c == ve;
+                    if (excl >= 1 && !e0) {
+                        e0 = in_ring(c);
+                        e1 = (e0 && c != lost) || c == gained;
+                        if (excl > 1) e0 = e1 = e0 || e1;
+                    }
+                }
+                const bool left = !(e0 && e1);
+                const unsigned b = (unsigned)(__ballot(left) >> (16 * g)) & 0xffffu;
+                if (left) S.list[g][listed + __popc(b & ((1u << q) - 1u))] = c | (e0 ? 1 << 30 : 0) | (e1 ? 1 << 31 : 0);
+                listed += __popc(b);
+            }
+            wave_sync();
+            for (int i0 = 0; __ballot(i0 < listed); i0 += 16) {
+                if (i0 + q < listed) {
+                    const int w = S.list[g][i0 + q], c = w & ~(3 << 30);
+                    bool e0 = w & (1 << 30), e1 = w < 0;
+                    const d3 dc = xv - d3{fm.x[3 * c], fm.x[3 * c + 1], fm.x[3 * c + 2]};
+                    if (excl > 1) {
+                        // the candidate's neighbours, as stored and on the flipped side
+                        const int* cr = rows.nb + (size_t)kRowW * c;
+                        const int4 w0 = reinterpret_cast<const int4*>(cr)[0], w1 = reinterpret_cast<const int4*>(cr)[1];
+                        const int cw[kRowPair] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
+                        const int cl = c == pv[0] ? pv[2] : (c == pv[2] ? pv[0] : -1);
+                        const int cg = c == pv[1] ? pv[3] : (c == pv[3] ? pv[1] : -1);
+                        auto meet = [&](int x) {
+                            const bool in0 = in_ring(x);
+                            e0 |= in0;
+                            e1 |= x != cl && ((in0 && x != lost) || x == gained);
+                        };
+                        int n = 0;
+                        for (; n < kRowPair; n++) {
+                            int x = cw[0];
+    #pragma unroll
+                            for (int i = 1; i < kRowPair; i++) x = n == i ? cw[i] : x;
+                            if (x < 0) break;
+                            meet(x & ~kNoFace);
+                        }
+                        if (n == kRowPair)
+                            for (; n < kRowW && cr[n] >= 0; n++) meet(cr[n] & ~kNoFace);
+                        if (cg >= 0) e1 |= (in_ring(cg) && cg != lost) || cg == gained;
+                    }
+                    if (!(e0 && e1)) {
+                        const double v = rep_value(norm(dc), p.rep_lc1, p.rep_r);
+                        if (!e0) rep0 += v;
+                        if (!e1) rep1 += v;
+                    }
+                }
+            }
+            t0 += kListMax;
+            if (!__ballot(t0 < total)) break;
+            load_candidates(t0);
+        }
+        rep0 = row_sum(rep0);
+        rep1 = row_sum(rep1);
+    }
+    res.val[0] = area;
+    res.val[1] = vol;
+    res.val[2] = curv;
+    res.val[3] = 2 * curv * curv / area;
+    res.val[4] = teth;
+    res.val[5] = side ? rep1 : rep0;
+#pragma unroll
+    for (int k = 0; k < 6; k++) {
+        res.val[k] += __shfl_xor(res.val[k], 16, 64);
+        res.val[k] += __shfl_xor(res.val[k], 32, 64);
+    }
+    return res;
+}
+
+// ---------------------------------------------- the last workgroup's turn --
+// One launch evaluates many proposals and then decides on all of them: every
+// workgroup hands its results over and counts itself, and the one that counts
+// last decides.  The hand-over uses no fence: on this part a device-scope
+// fence writes back and invalidates the whole L2 of the workgroup's XCD.
+// Results are stored and read with relaxed device-scope atomics, which pass
+// by the caches that are not coherent between XCDs; each workgroup waits for
+// its own stores to complete (s_waitcnt) before it counts, and the last one
+// reads after its count has returned.  Nothing waits for another workgroup.
+template <class T>
+__device__ __forceinline__ void put(T* a, T v)
+{
+    __hip_atomic_store(a, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <class T>
+__device__ __forceinline__ T get(const T* a)
+{
+    return __hip_atomic_load(a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// A proposal's record, one 128-byte line that its wave stores in one go: words
+// 0-11 the patch differences (after minus before), 12 its validity (1
+// flippable, 0 not, -1 index out of range), 13-25 the FlipEdge.  The readers
+// take lines with several lanes each: read by one thread each, a record would
+// be thirteen requests for the same line.
+__device__ __forceinline__ void put_record(int* rec, int lane, int valid, const double (&d)[6], const FlipEdge& f)
+{
+    int w = 0;
+#pragma unroll
+    for (int c = 0; c < 6; c++)
+        if ((lane >> 1) == c) w = (lane & 1) ? __double2hiint(d[c]) : __double2loint(d[c]);
+    const int rest[14] = {valid, f.e, f.pv[0], f.pv[1], f.pv[2], f.pv[3], f.a1, f.a2, f.b1, f.b2, f.fa, f.fb, f.ha,
+                          f.hb};
+#pragma unroll
+    for (int c = 0; c < 14; c++)
+        if (lane == 12 + c) w = rest[c];
+    if (lane < 26) put(rec + lane, w);
+}
+__device__ __forceinline__ FlipEdge flip_edge_of(const int* m)    // words 13 .. 25 of a record
+{
+    return FlipEdge{m[13], {m[14], m[15], m[16], m[17]}, m[18], m[19], m[20], m[21], m[22], m[23], m[24], m[25]};
+}
+
+// true for every thread of the last of `blocks` workgroups; the counter is
+// left at zero for the next launch
+__device__ __forceinline__ bool last_block(unsigned* counter, unsigned blocks)
+{
+    __shared__ int s_last;
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");    // this wave's stores have completed
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const unsigned c = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        s_last = c + 1 == blocks;
+        if (s_last) put(counter, 0u);
+    }
+    __syncthreads();
+    return s_last != 0;
+}
+
+// The Metropolis test (flips.cpp:57-64) u <= min(1, exp(-de)) as de <= -log(u):
+// the logarithm is taken once per proposal, not in every step of a walk.
+// u = 0 always passes (-log(0) is infinite), a NaN never.
+__device__ __forceinline__ double minus_log(double u) { return -log(u); }
+
 // ================================================ windowed serial sweep ==
-// The serial sweep's decisions and topology, bit for bit, from windows of W
-// proposals evaluated at once.  Per window:
-//   k_sf_eval    one workgroup per proposal and side: is_flip_ok and the
-//                patch properties before the flip (side 0) and after it on
-//                FlippedTopo (side 1), on the topology at the window start.
-//   k_sf_commit  one workgroup commits the window in order up to the first
-//                proposal whose evaluation an earlier one may have changed.
+// The serial sweep's decisions and topology from windows of W proposals
+// evaluated at once.  One launch per window: a wave per proposal evaluates
+// is_flip_ok and its patch before and after the flip on the topology at the
+// window start, and the last workgroup commits the window in order up to the
+// first proposal whose evaluation an earlier one has changed.
 // What an earlier proposal j of the window changes for a later one k:
 //   * accepted: the one-rings of j's four patch vertices V(j).  k read the
-//     one-rings of its patch vertices P_k (in circulator order) and, for
-//     exclusion level 2, the neighbour sets of their one-ring vertices
-//     N(P_k); so V(j) meeting P_k (or N(P_k)) makes k stale.
-//   * rejected (do_flip twice): every vertex keeps its neighbours in the
-//     same cyclic order, and each halfedge a walk reaches leads to the same
-//     vertex; only ids move.  The edge's two halfedges swap direction (a
-//     later proposal of the same edge sees its patch in another order), and
-//     an endpoint whose v_he was one of them starts its circulator
-//     elsewhere (a later proposal with that vertex in P_k sums its ring in
-//     another order).  The faces' f_he move too; only boundary sector
-//     angles read them, and no flip evaluation does.
-// Valid proposals stamp their edge and those endpoints with their window
-// position (atomicMax of a window-keyed 64-bit key keeps the smallest);
-// accepted ones are checked against the later proposals' P_k and N(P_k) as
-// they are found.  A rejected proposal can still share a triangle with a
-// later committed one, so flips whose faces an earlier valid proposal of the
-// window touched (stamped like the edges) are applied after the others, in
-// order, by one lane.  Up to the first stale proposal, lanes 0-5 run the serial
-// sweep's rounding path (props -= old, += new; on rejection -= new, += old)
-// through the rejected branch, one component each; the lanes then take the
-// Metropolis decisions at once, and the first acceptance ends the segment:
-// its state is the serial one, and the walk continues after it.
+//     one-rings of its patch vertices P_k and, for exclusion level 2, the
+//     neighbour sets of their one-ring vertices N(P_k); so V(j) meeting P_k (or
+//     N(P_k)) makes k stale.
+//   * rejected (do_flip twice): nothing that an evaluation reads.  Every
+//     vertex keeps its neighbours in the same cyclic order; only ids move.
+// The commit tests all proposals up to the first stale one against the
+// current state at once and takes the first acceptance: a rejection leaves the
+// state, so every decision is that of the sequential walk.  The halfedge
+// arrays are then rewritten (do_flip or do_flip twice) by one thread per
+// committed proposal.  Proposals that share a face must follow each other (a
+// stamp per face holds the window's first valid proposal on it): those
+// connected through shared faces get ascending ranks, and the ranks are
+// applied one after the other.
 // A window commits at least its first proposal, which cannot be stale.
-__device__ __forceinline__ unsigned long long sf_key(int window, int W, int k)
+// At level 7 (491520 edges) a window of 256 takes 38 us; evaluating by ring
+// walks (30 us) and committing along the serial rounding path (51 us) were two
+// launches.
+__global__ void __launch_bounds__(256) k_sf_begin(FlipMeshView fm, FlipRows rows, const Globals* __restrict__ g0,
+                                                  EParams p, int nflips, SerialState* __restrict__ st,
+                                                  unsigned long long* __restrict__ fstamp)
 {
-    return ((unsigned long long)(unsigned)(window + 1) << 32) | (unsigned)(W - k);
-}
-
-// bitmap position (12 bits) of a vertex in the commit's staleness filter
-__device__ __forceinline__ unsigned sf_hash(int u) { return ((unsigned)u * 2654435761u) >> 20; }
-
-// window position recorded in a stamp, or W if the stamp is older
-__device__ __forceinline__ int sf_pos(unsigned long long key, unsigned wid, int W)
-{
-    return (unsigned)(key >> 32) == wid ? W - (int)(unsigned)(key & 0xffffffffu) : W;
-}
-
-__global__ void __launch_bounds__(64) k_sf_init(const Globals* __restrict__ g0, EParams p, int nflips,
-                                                SerialState* __restrict__ st)
-{
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t < fm.nv) build_rows(fm, rows, t);
+    if (t < fm.nf) fstamp[t] = 0ull;
+    if (t != 0) return;
     double props[6];
     for (int k = 0; k < 6; k++) props[k] = st->props[k] = g0->props[k];
     st->e0 = energy_of(props, p);
     st->pos = 0;
     st->done = nflips <= 0;
     st->used = st->acc = st->err = st->window = 0;
+    st->count = 0u;
 }
 
-__global__ void __launch_bounds__(64) k_sf_eval(FlipMeshView fm, NListView nl, EParams p, int nflips,
-                                                const int* __restrict__ proposals, uint64_t seed, int injected,
-                                                int W, int need_nb, const SerialState* __restrict__ st,
-                                                SerialWindow w, unsigned long long* __restrict__ vstamp,
-                                                unsigned long long* __restrict__ estamp,
-                                                unsigned long long* __restrict__ fstamp)
-{
-    __shared__ CoopShared S;
-    __shared__ int s_ok;
-    if (st->done) return;
-    const int k = blockIdx.x, side = blockIdx.y, tid = threadIdx.x;
-    const int i = st->pos + k;
-    if (i >= nflips) return;
-    const Topo t{fm.x, fm.he_to, fm.he_next, fm.he_prev, fm.he_face, fm.v_he, fm.f_he};
-    const int ne = fm.nh / 2;
-    const int e = injected ? proposals[i] : rng_edge(seed, (uint64_t)i, ne);
-    if (e < 0 || e >= ne) {
-        if (side == 0 && tid == 0) w.valid[k] = -1;
-        return;
-    }
-    // the vertices whose one-rings decide validity and the patch terms (for
-    // a boundary edge, is_flip_ok reads only the edge's own halfedges)
-    if (side == 0 && tid < 4)
-        w.pv[4 * k + tid] = t.edge_boundary(e) ? t.to(2 * e + (tid & 1)) : patch_vertex(t, e, tid);
-    if (side == 0 && tid == 0) w.e[k] = e;
-    if (tid == 0) s_ok = !t.edge_boundary(e);
-    __syncthreads();
-    if (!s_ok) {
-        if (side == 0 && tid == 0) w.valid[k] = 0;
-        return;
-    }
-    // side 0 decides flip_ok from its one-rings; side 1 evaluates the
-    // flipped patch without waiting for it (FlippedTopo is a valid view of
-    // any interior edge; its values are read only for valid proposals)
-    if (side == 0) {
-        coop_patch(t, nl, p, e, S, true);
-        if (!S.flip_ok) {
-            if (tid == 0) w.valid[k] = 0;
-            return;
-        }
-        const unsigned long long key = sf_key(st->window, W, k);
-        if (tid == 0) {
-            for (int c = 0; c < 6; c++) w.dO[6 * k + c] = S.sum[c];
-            w.valid[k] = 1;
-            atomicMax(&estamp[e], key);
-        } else if (tid >= 3 && tid < 5) {
-            const int f = t.face(2 * e + tid - 3);
-            w.fc[2 * k + tid - 3] = f;
-            atomicMax(&fstamp[f], key);
-        } else if (tid < 3) {
-            // an endpoint whose v_he is one of the edge's halfedges
-            const int h = 2 * e + tid - 1;
-            const int v = t.to(h);
-            if (t.vhe(v) == (h ^ 1)) atomicMax(&vstamp[v], key);
-        }
-        if (need_nb) {
-            const int g = tid / kCoopLanes, l = tid % kCoopLanes;
-            const int n = S.n[g];
-            if (l == 0) w.nbn[4 * k + g] = n;
-            for (int s = l; s < n; s += kCoopLanes) w.nb[(size_t)(4 * k + g) * kMaxValence + s] = S.nb[g][s];
-        }
-    } else {
-        const FlippedTopo ft(t, e);
-        coop_patch(ft, nl, p, e, S);
-        if (tid == 0)
-            for (int c = 0; c < 6; c++) w.dN[6 * k + c] = S.sum[c];
-    }
-}
+constexpr int kRecInts = 26;    // the used words of a record
+struct SerialShared {
+    alignas(16) int rec[kSerialWindowMax * kRecInts];
+    // one-rings of every proposal's patch, kRowPair slots each and -1 past the
+    // end, as int4 chunks rotated by the proposal's number (bank conflicts)
+    int4 ring[kSerialWindowMax][kRowPair];
+    alignas(16) int label[kSerialWindowMax];
+    int slots[2][kPatchWaves];
+    int wsum[kPatchWaves];
+    unsigned long long wide[kPatchWaves];    // proposals with a ring longer than kRowPair
+    int maxrank;
+    int nflip, flip[kSerialWindowMax];
+};
 
-// The reads of do_flip for up to kPer edges, then the writes: the edges'
-// halfedges are disjoint, so the loads of all of them overlap.
-template <int N>
-__device__ __forceinline__ void flip_batch(const FlipMeshView& fm, const int (&e)[N], const int (&mode)[N])
+__device__ __forceinline__ void sf_commit(const FlipMeshView& fm, const FlipRows& rows, const EParams& p, int nflips,
+                                          const double* __restrict__ uniforms, int n_uniforms, uint64_t seed,
+                                          int injected, int W, int need_nb, SerialState* __restrict__ st,
+                                          const int* rec, const unsigned long long* fstamp, SerialShared& S)
 {
-    // mode: 0 none, 1 do_flip, 2 do_flip twice
-    int a1[N], a2[N], b1[N], b2[N], va0[N], vb0[N], va1[N], vb1[N], ta2[N], tb2[N], fa[N], fb[N], ha[N], hb[N];
-#pragma unroll
-    for (int r = 0; r < N; r++) {
-        if (!mode[r]) continue;
-        const int a0 = 2 * e[r], b0 = a0 + 1;
-        a1[r] = fm.he_next[a0];
-        b1[r] = fm.he_next[b0];
-        va0[r] = fm.he_to[a0];
-        vb0[r] = fm.he_to[b0];
-        fa[r] = fm.he_face[a0];
-        fb[r] = fm.he_face[b0];
-    }
-#pragma unroll
-    for (int r = 0; r < N; r++) {
-        if (!mode[r]) continue;
-        a2[r] = fm.he_next[a1[r]];
-        b2[r] = fm.he_next[b1[r]];
-        va1[r] = fm.he_to[a1[r]];
-        vb1[r] = fm.he_to[b1[r]];
-        ha[r] = fm.v_he[va0[r]];
-        hb[r] = fm.v_he[vb0[r]];
-    }
-#pragma unroll
-    for (int r = 0; r < N; r++) {
-        if (!mode[r]) continue;
-        ta2[r] = fm.he_to[a2[r]];
-        tb2[r] = fm.he_to[b2[r]];
-    }
-#pragma unroll
-    for (int r = 0; r < N; r++) {
-        if (!mode[r]) continue;
-        const int a0 = 2 * e[r], b0 = a0 + 1;
-        if (mode[r] == 1) {
-            // do_flip
-            fm.he_to[a0] = va1[r];
-            fm.he_to[b0] = vb1[r];
-            fm.he_next[a0] = a2[r]; fm.he_prev[a2[r]] = a0;
-            fm.he_next[a2[r]] = b1[r]; fm.he_prev[b1[r]] = a2[r];
-            fm.he_next[b1[r]] = a0; fm.he_prev[a0] = b1[r];
-            fm.he_next[b0] = b2[r]; fm.he_prev[b2[r]] = b0;
-            fm.he_next[b2[r]] = a1[r]; fm.he_prev[a1[r]] = b2[r];
-            fm.he_next[a1[r]] = b0; fm.he_prev[b0] = a1[r];
-            fm.he_face[a1[r]] = fb[r];
-            fm.he_face[b1[r]] = fa[r];
-        } else {
-            // do_flip_twice
-            fm.he_to[a0] = ta2[r];
-            fm.he_to[b0] = tb2[r];
-            fm.he_next[a0] = b1[r]; fm.he_prev[b1[r]] = a0;
-            fm.he_next[b1[r]] = b2[r]; fm.he_prev[b2[r]] = b1[r];
-            fm.he_next[b2[r]] = a0; fm.he_prev[a0] = b2[r];
-            fm.he_next[b0] = a1[r]; fm.he_prev[a1[r]] = b0;
-            fm.he_next[a1[r]] = a2[r]; fm.he_prev[a2[r]] = a1[r];
-            fm.he_next[a2[r]] = b0; fm.he_prev[b0] = a2[r];
-            fm.he_face[a1[r]] = fb[r];
-            fm.he_face[a2[r]] = fb[r];
-            fm.he_face[b1[r]] = fa[r];
-            fm.he_face[b2[r]] = fa[r];
-        }
-        fm.f_he[fa[r]] = a0;
-        fm.f_he[fb[r]] = b0;
-        if (ha[r] == b0) fm.v_he[va0[r]] = a1[r];
-        if (hb[r] == a0) fm.v_he[vb0[r]] = b1[r];
-    }
-}
-
-__global__ void __launch_bounds__(64) k_sf_commit(FlipMeshView fm, EParams p, int nflips,
-                                                  const double* __restrict__ uniforms, int n_uniforms,
-                                                  uint64_t seed, int injected, int W, int need_nb,
-                                                  SerialState* __restrict__ st, SerialWindow w,
-                                                  const unsigned long long* __restrict__ vstamp,
-                                                  const unsigned long long* __restrict__ estamp,
-                                                  const unsigned long long* __restrict__ fstamp)
-{
-    constexpr int kPer = kSerialWindowMax / 64;
-    constexpr int kChunk = 64;                  // valid proposals per decision round
-    __shared__ int s_valid[kSerialWindowMax];
-    __shared__ int s_stale[kSerialWindowMax];
-    __shared__ int s_defer[kSerialWindowMax];   // an earlier valid proposal has one of its faces
-    __shared__ int s_accf[kSerialWindowMax];    // accepted
-    __shared__ int s_vk[kSerialWindowMax];      // window position of the m-th valid proposal
-    __shared__ int s_rank[kSerialWindowMax + 1];    // valid proposals before position k
-    __shared__ int s_pv[4 * kSerialWindowMax];
-    __shared__ int s_nbn[4 * kSerialWindowMax];
-    __shared__ int s_ring[4 * kMaxValence];     // one-rings of an accepted proposal's patch
-    __shared__ int s_dlist[kSerialWindowMax];   // positions of the deferred flips, ascending
-    __shared__ unsigned s_bits[128];            // hash bitmap of s_ring and the accepted patch
-    // per proposal: the bitmap positions of its patch vertices (12 bits each)
-    // and, in bit 63, whether one of its one-rings was too long to record
-    __shared__ unsigned long long s_ph[kSerialWindowMax];
-    // by rank among the valid proposals: uniforms, the rounding path's
-    // states and the patch properties before and after the flip
-    __shared__ double s_u[kSerialWindowMax];
-    __shared__ double s_q[6 * kSerialWindowMax];
-    __shared__ double s_o[6 * kSerialWindowMax];
-    __shared__ double s_n[6 * kSerialWindowMax];
-    __shared__ double s_P[6], s_Prej[6];
-    __shared__ double s_e0;
-    __shared__ int s_acc, s_err, s_end, s_first, s_ovf, s_ndef;
-    const int tid = threadIdx.x;
-    if (st->done) return;
-    const int pos0 = st->pos;
+    const int tid = threadIdx.x, wave = tid >> 6;
+    const int pos0 = st->pos, used0 = st->used, wid = st->window + 1;
     const int cnt = min(W, nflips - pos0);
-    const unsigned wid = (unsigned)st->window + 1u;
-    const int used0 = st->used;
-
-    // ---- stage; position k = 64 r + tid
-    int v[kPer], e[kPer];
-#pragma unroll
-    for (int r = 0; r < kPer; r++) {
-        const int k = 64 * r + tid;
-        v[r] = k < cnt ? w.valid[k] : -2;
-        e[r] = v[r] >= 0 ? w.e[k] : 0;
-    }
-    int pv[kPer][4], fc[kPer][2];
-#pragma unroll
-    for (int r = 0; r < kPer; r++) {
-        const int k = 64 * r + tid;
-        for (int g = 0; g < 4; g++) pv[r][g] = v[r] >= 0 ? w.pv[4 * k + g] : 0;
-        for (int g = 0; g < 2; g++) fc[r][g] = v[r] == 1 ? w.fc[2 * k + g] : 0;
-    }
-#pragma unroll
-    for (int r = 0; r < kPer; r++) {
-        const int k = 64 * r + tid;
-        int stale = 0, defer = 0;
-        if (v[r] >= 0) {
-            for (int g = 0; g < 4; g++) stale |= sf_pos(vstamp[pv[r][g]], wid, W) < k;
-            stale |= sf_pos(estamp[e[r]], wid, W) < k;
-            for (int g = 0; g < 4; g++) s_pv[4 * k + g] = pv[r][g];
-        }
-        unsigned long long ph = 0ull;
-        if (v[r] >= 0)
-            for (int g = 0; g < 4; g++) ph |= (unsigned long long)sf_hash(pv[r][g]) << (12 * g);
-        if (v[r] == 1) {
-            defer = sf_pos(fstamp[fc[r][0]], wid, W) < k || sf_pos(fstamp[fc[r][1]], wid, W) < k;
-            if (need_nb)
-                for (int g = 0; g < 4; g++) {
-                    const int nn = w.nbn[4 * k + g];
-                    s_nbn[4 * k + g] = nn;
-                    if (nn < 0) ph |= 1ull << 63;
-                }
-        }
-        s_ph[k] = ph;
-        s_valid[k] = v[r];
-        s_stale[k] = stale;
-        s_defer[k] = defer;
-        s_accf[k] = 0;
-    }
-    // the patch properties of the valid proposals, all rows in flight at once
-    // (one workgroup: registers are not the limit)
-    double po[kPer][6], pn[kPer][6];
-#pragma unroll
-    for (int r = 0; r < kPer; r++) {
-        const int k = 64 * r + tid;
-#pragma unroll
-        for (int c = 0; c < 6; c++) {
-            po[r][c] = v[r] == 1 ? w.dO[6 * k + c] : 0.0;
-            pn[r][c] = v[r] == 1 ? w.dN[6 * k + c] : 0.0;
-        }
-    }
-    // ranks among the valid proposals (their uniform index is used0 + rank)
-    // and the list of deferred flips
-    int base = 0, dbase = 0;
-#pragma unroll
-    for (int r = 0; r < kPer; r++) {
-        const int k = 64 * r + tid;
-        const unsigned long long below = (1ull << tid) - 1ull;
-        const unsigned long long bd = __ballot(s_defer[k] != 0);
-        if (s_defer[k]) s_dlist[dbase + __popcll(bd & below)] = k;
-        dbase += __popcll(bd);
-        const unsigned long long b = __ballot(v[r] == 1);
-        const int m = base + __popcll(b & ((1ull << tid) - 1ull));
-        s_rank[k] = m;
-        if (v[r] == 1) {
-            const int u = used0 + m;
-            s_vk[m] = k;
-            s_u[m] = injected ? (u < n_uniforms ? uniforms[u] : 2.0) : rng_uniform(seed, (uint64_t)u);
-            for (int c = 0; c < 6; c++) {
-                s_o[6 * m + c] = po[r][c];
-                s_n[6 * m + c] = pn[r][c];
-            }
-        }
-        base += __popcll(b);
-    }
-    if (tid == 0) {
-        s_rank[kSerialWindowMax] = base;
-        s_ndef = dbase;
-        for (int c = 0; c < 6; c++) s_P[c] = st->props[c];
-        s_e0 = st->e0;
-        s_acc = st->acc;
-        s_err = 0;
-        // an injected stream too short: the proposal that finds it empty is
-        // rejected (u = 2) and the sweep stops after it
-        s_ovf = (injected && base > n_uniforms - used0) ? max(n_uniforms - used0, 0) : kSerialWindowMax;
-    }
-    __syncthreads();
-    const int movf = s_ovf;    // rank of that proposal
-    const int ovf = movf < base ? s_vk[movf] : cnt;
-
-    // ---- decide, chunk by chunk, up to the first stale proposal
-    int pos = 0;
-    while (pos < cnt) {
-        if (tid == 0) s_end = cnt;
-        __syncthreads();
-        for (int k = pos + tid; k < cnt; k += 64)
-            if (s_stale[k] || s_valid[k] < 0) atomicMin(&s_end, k);
-        __syncthreads();
-        int end = s_end;
-        if (end == pos) break;
-        if (ovf < end) end = ovf + 1;
-        const int m0 = s_rank[pos], mend = s_rank[end];
-        const int m1 = min(mend, m0 + kChunk);
-        const int cend = m1 < mend ? s_vk[m1] : end;    // positions [pos, cend) hold valid m0 .. m1-1
-        if (tid < 6) {
-            // the serial rounding path through the rejected branch, one lane
-            // per component
-            const int c = tid;
-            double P = s_P[c];
-#pragma unroll 4
-            for (int m = m0; m < m1; m++) {
-                const double o = s_o[6 * m + c], nw = s_n[6 * m + c];
-                double q = P - o;
-                q += nw;
-                s_q[6 * m + c] = q;
-                P = q - nw;
-                P += o;
-            }
-            s_Prej[c] = P;
-        }
-        if (tid == 0) s_first = cend;
-        __syncthreads();
-        const double e0 = s_e0;
-        for (int m = m0 + tid; m < m1; m += 64) {
-            const int k = s_vk[m];
-            if (k == ovf) continue;
-            const double en = energy_of(s_q + 6 * m, p);
-            const double de = en - e0;
-            const double alpha = de < 0.0 ? 1.0 : exp(-de);
-            if (s_u[m] <= alpha) atomicMin(&s_first, k);
-        }
-        __syncthreads();
-        const int kf = s_first;
-        if (kf < cend) {
-            if (tid == 0) {
-                const int mf = s_rank[kf];
-                for (int c = 0; c < 6; c++) s_P[c] = s_q[6 * mf + c];
-                s_e0 = energy_of(s_q + 6 * mf, p);
-                s_acc += 1;
-                s_accf[kf] = 1;
-            }
-            // later proposals whose patch meets the accepted patch are stale;
-            // for exclusion level 2 also those with a patch vertex adjacent
-            // to it (adjacency is symmetric: the accepted patch meets their
-            // patch's one-rings), found in the accepted patch's one-rings
-            const int f0 = s_pv[4 * kf], f1 = s_pv[4 * kf + 1], f2 = s_pv[4 * kf + 2], f3 = s_pv[4 * kf + 3];
-            auto in_v = [&](int u) { return u == f0 || u == f1 || u == f2 || u == f3; };
-            int rn[4] = {0, 0, 0, 0};
-            bool all = false;
-            for (int t = tid; t < 128; t += 64) s_bits[t] = 0u;
-            if (need_nb) {
-                for (int g = 0; g < 4; g++) {
-                    rn[g] = s_nbn[4 * kf + g];
-                    all = all || rn[g] < 0;
-                }
-                for (int t = tid; t < 4 * kMaxValence; t += 64) {
-                    const int g = t / kMaxValence, s = t % kMaxValence;
-                    if (s < rn[g]) s_ring[t] = w.nb[(size_t)(4 * kf + g) * kMaxValence + s];
-                }
-            }
-            __syncthreads();
-            if (tid < 4) {
-                const unsigned h = sf_hash(s_pv[4 * kf + tid]);
-                atomicOr(&s_bits[h >> 5], 1u << (h & 31));
-            }
-            for (int t = tid; t < 4 * kMaxValence; t += 64) {
-                const int g = t / kMaxValence, s = t % kMaxValence;
-                if (s < rn[g]) {
-                    const unsigned h = sf_hash(s_ring[t]);
-                    atomicOr(&s_bits[h >> 5], 1u << (h & 31));
-                }
-            }
-            __syncthreads();
-            auto maybe = [&](unsigned long long ph, int g) {
-                const unsigned h = (unsigned)(ph >> (12 * g)) & 0xfffu;
-                return (s_bits[h >> 5] >> (h & 31)) & 1u;
-            };
-            for (int k = kf + 1 + tid; k < cnt; k += 64) {
-                if (s_valid[k] < 0) continue;
-                const unsigned long long ph = s_ph[k];
-                const bool own = need_nb && s_valid[k] == 1 && (all || (ph >> 63));
-                if (!own && !(maybe(ph, 0) | maybe(ph, 1) | maybe(ph, 2) | maybe(ph, 3))) continue;
-                const int q0 = s_pv[4 * k], q1 = s_pv[4 * k + 1], q2 = s_pv[4 * k + 2], q3 = s_pv[4 * k + 3];
-                bool hit = own || in_v(q0) || in_v(q1) || in_v(q2) || in_v(q3);
-                if (!hit && need_nb && s_valid[k] == 1) {
-                    for (int g = 0; g < 4 && !hit; g++)
-                        for (int s = 0; s < rn[g] && !hit; s++) {
-                            const int u = s_ring[g * kMaxValence + s];
-                            hit = u == q0 || u == q1 || u == q2 || u == q3;
-                        }
-                }
-                if (hit) s_stale[k] = 1;
-            }
-            pos = kf + 1;
-        } else {
-            if (tid == 0) {
-                for (int c = 0; c < 6; c++) s_P[c] = s_Prej[c];
-                if (ovf < cend) s_err = 2;
-            }
-            pos = cend;
-        }
-        __syncthreads();
-        if (s_err) break;
-    }
-
-    // ---- the committed flips: proposals whose faces no earlier one touched
-    // are disjoint from every earlier flip; the others follow, in order
     {
-        int fe[kPer], mode[kPer];
+        // sixteen lanes per record
+        const unsigned long long* src = reinterpret_cast<const unsigned long long*>(rec);
+        const int c = tid & 15, r0 = tid >> 4;
+        unsigned long long w[16];
 #pragma unroll
-        for (int r = 0; r < kPer; r++) {
-            const int k = 64 * r + tid;
-            fe[r] = e[r];
-            mode[r] = (k < pos && s_valid[k] == 1 && !s_defer[k]) ? (s_accf[k] ? 1 : 2) : 0;
+        for (int i = 0; i < 16; i++) {
+            const int r = r0 + 16 * i;
+            w[i] = r < cnt && c < kRecInts / 2 ? get(src + (size_t)(kFlipRecord / 2) * r + c) : 0ull;
         }
-        flip_batch(fm, fe, mode);
+#pragma unroll
+        for (int i = 0; i < 16; i++)
+            if (c < kRecInts / 2)
+                *reinterpret_cast<unsigned long long*>(S.rec + kRecInts * (r0 + 16 * i) + 2 * c) = w[i];
+    }
+    double P[6], e0 = st->e0;
+#pragma unroll
+    for (int c = 0; c < 6; c++) P[c] = st->props[c];
+    if (tid == 0) S.maxrank = S.nflip = 0;
+    S.label[tid] = tid;
+    __syncthreads();
+    // thread k holds proposal k of the window
+    const int k = tid;
+    const int* m = S.rec + kRecInts * k;
+    const int v = k < cnt ? m[12] : -2;
+    const int pv0 = m[14], pv1 = m[15], pv2 = m[16], pv3 = m[17];
+    const bool inner = v >= 0 && m[22] >= 0 && m[23] >= 0;
+    double dp[6];
+#pragma unroll
+    for (int c = 0; c < 6; c++) dp[c] = __hiloint2double(m[2 * c + 1], m[2 * c]);
+    // window positions of the first valid proposals on its faces, and the
+    // rings that acceptances are checked against
+    int l0 = k, l1 = k;
+    bool wide = false;
+    if (v == 1) {
+        const unsigned long long s0 = get(fstamp + m[22]), s1 = get(fstamp + m[23]);
+        if (need_nb) {
+            int4 w[8];
+#pragma unroll
+            for (int g = 0; g < 4; g++) {
+                const int4* row = reinterpret_cast<const int4*>(rows.nb + (size_t)kRowW * m[14 + g]);
+                w[2 * g] = row[0];
+                w[2 * g + 1] = row[1];
+            }
+#pragma unroll
+            for (int g = 0; g < 4; g++) {
+                int x[kRowPair] = {w[2 * g].x, w[2 * g].y, w[2 * g].z, w[2 * g].w,
+                                   w[2 * g + 1].x, w[2 * g + 1].y, w[2 * g + 1].z, w[2 * g + 1].w};
+                bool more = true;
+#pragma unroll
+                for (int i = 0; i < kRowPair; i++) {
+                    more = more && x[i] >= 0;
+                    x[i] = more ? x[i] & ~kNoFace : -1;
+                }
+                wide = wide || more;
+                S.ring[k][(2 * g + k) & 7] = make_int4(x[0], x[1], x[2], x[3]);
+                S.ring[k][(2 * g + 1 + k) & 7] = make_int4(x[4], x[5], x[6], x[7]);
+            }
+        }
+        l0 = W - (int)(unsigned)s0;
+        l1 = W - (int)(unsigned)s1;
+    }
+    // rank among the valid proposals: the uniform's index
+    const unsigned long long vb = __ballot(v == 1), wb = __ballot(wide);
+    if ((tid & 63) == 0) {
+        S.wsum[wave] = __popcll(vb);
+        S.wide[wave] = wb;
     }
     __syncthreads();
-    if (tid == 0)
-        for (int d = 0; d < s_ndef; d++) {
-            const int k = s_dlist[d];
-            if (k >= pos) break;
-            if (s_accf[k]) do_flip(fm, w.e[k]);
-            else do_flip_twice(fm, w.e[k]);
+    int mr = __popcll(vb & ((1ull << (tid & 63)) - 1ull)), nvalid = 0;
+    for (int i = 0; i < kPatchWaves; i++) {
+        if (i < wave) mr += S.wsum[i];
+        nvalid += S.wsum[i];
+    }
+    // an injected stream too short: the proposal that finds it empty is
+    // rejected and the sweep stops after it
+    const int movf = injected ? max(n_uniforms - used0, 0) : INT_MAX;
+    const bool ovf = v == 1 && mr == movf, can = v == 1 && mr < movf;
+    double nlu = 0.0;
+    if (can) nlu = minus_log(injected ? uniforms[used0 + mr] : rng_uniform(seed, (uint64_t)(used0 + mr)));
+
+    // every thread carries the state; one barrier per step
+    bool stale = false, accepted = false;
+    int pos = 0, err = 0, it = 0, nacc = 0;
+    while (pos < cnt) {
+        // the first proposal that is not to be decided now (1), finds the
+        // uniform stream empty (2) or is accepted (3)
+        int what = 0;
+        if (k >= pos && k < cnt) {
+            if (stale || v < 0) what = 1;
+            else if (ovf) what = 2;
+            else if (can) {
+                double q[6];
+#pragma unroll
+                for (int c = 0; c < 6; c++) q[c] = P[c] + dp[c];
+                what = energy_of(q, p) - e0 <= nlu ? 3 : 0;
+            }
         }
-    if (tid == 0) {
-        int err = s_err;
-        if (!err && pos < cnt && s_valid[pos] == -1) err = 1;
-        for (int c = 0; c < 6; c++) st->props[c] = s_P[c];
-        st->e0 = s_e0;
-        st->used = used0 + s_rank[pos];
-        st->acc = s_acc;
+        const unsigned long long b = __ballot(what != 0);
+        const int lane1 = b ? __ffsll((long long)b) - 1 : 0;
+        const int what1 = __builtin_amdgcn_readlane(what, lane1);
+        int* slots = S.slots[it++ & 1];
+        if ((tid & 63) == 0) slots[wave] = b ? (64 * wave + lane1) * 4 + what1 : INT_MAX;
+        __syncthreads();
+        int s = INT_MAX;
+#pragma unroll
+        for (int i = 0; i < kPatchWaves; i++) s = min(s, slots[i]);
+        if (s == INT_MAX) {
+            pos = cnt;
+            break;
+        }
+        const int first = s >> 2;
+        what = s & 3;
+        pos = what == 1 ? first : first + 1;
+        if (what == 2) err = 2;
+        if (what != 3) break;
+        const int* f = S.rec + kRecInts * first;
+#pragma unroll
+        for (int c = 0; c < 6; c++) P[c] += __hiloint2double(f[2 * c + 1], f[2 * c]);
+        e0 = energy_of(P, p);
+        nacc++;
+        if (k == first) accepted = true;
+        // later proposals whose patch meets the accepted patch are stale; at
+        // exclusion level 2 its one-rings count too (adjacency is symmetric:
+        // they meet P_k exactly when V(j) meets N(P_k))
+        bool hit = false;
+        auto check = [&](int x) { hit |= (x == pv0) | (x == pv1) | (x == pv2) | (x == pv3); };
+        if (need_nb) {
+            int4 x[kRowPair];
+#pragma unroll
+            for (int i = 0; i < kRowPair; i++) x[i] = S.ring[first][i];
+#pragma unroll
+            for (int i = 0; i < kRowPair; i++) {
+                check(x[i].x);
+                check(x[i].y);
+                check(x[i].z);
+                check(x[i].w);
+            }
+            if ((S.wide[first >> 6] >> (first & 63)) & 1ull)
+                for (int g = 0; g < 4; g++) {
+                    const int* row = rows.nb + (size_t)kRowW * f[14 + g];
+                    for (int i = 0; i < kRowW && row[i] >= 0; i++) check(row[i] & ~kNoFace);
+                }
+        }
+#pragma unroll
+        for (int g = 0; g < 4; g++) check(f[14 + g]);
+        stale = stale || (hit && inner);
+    }
+
+    // ranks of the committed flips along shared faces: the labels become the
+    // least position of each connected set
+    const bool commit = k < pos && v == 1;
+    int rank = 0;
+    if (!commit) l0 = l1 = k;
+    if (__syncthreads_or(l0 != k || l1 != k)) {
+        for (;;) {
+            const int a = min(S.label[k], min(S.label[l0], S.label[l1]));
+            const bool low = a < S.label[k] || a < S.label[l0] || a < S.label[l1];
+            if (!__syncthreads_or(low)) break;
+            if (low) {
+                atomicMin(&S.label[k], a);
+                atomicMin(&S.label[l0], a);
+                atomicMin(&S.label[l1], a);
+            }
+            __syncthreads();
+        }
+        if (commit) {
+            const int a = S.label[k];
+            const int4* lab = reinterpret_cast<const int4*>(S.label);
+#pragma unroll 8
+            for (int i = 0; i < kSerialWindowMax / 4; i++) {
+                const int4 x = lab[i];
+                rank += (x.x == a && 4 * i < k) + (x.y == a && 4 * i + 1 < k) + (x.z == a && 4 * i + 2 < k) +
+                        (x.w == a && 4 * i + 3 < k);
+            }
+            if (rank) atomicMax(&S.maxrank, rank);
+        }
+        __syncthreads();
+    }
+    if (accepted) S.flip[atomicAdd(&S.nflip, 1)] = k;
+    // rank 0 from the records, later ranks from what the earlier ones left
+    const int maxrank = S.maxrank;
+    for (int i = 0; i <= maxrank; i++) {
+        if (commit && rank == i) {
+            const FlipEdge f = i == 0 ? flip_edge_of(m) : load_flip_edge(fm, m[13]);
+            if (accepted) store_flip(fm, f);
+            else store_flip_twice(fm, f);
+        }
+        __threadfence_block();
+        __syncthreads();
+    }
+    // the rows of the accepted patches, one thread per vertex (accepted
+    // proposals of a window have disjoint patches, which earlier flips left
+    // as the records have them)
+    for (int t = tid; t < 4 * S.nflip; t += 256) {
+        const int g = t & 3;
+        const int* f = S.rec + kRecInts * S.flip[t >> 2];
+        flip_row(rows, f[14 + g], g, g < 2 ? f[16] : f[14], g == 1 ? f[17] : f[15], f[13], make_int2(0, 0));
+    }
+    // state; the uniforms used are the valid proposals before pos
+    if (pos < cnt ? k == pos : tid == 0) {
+        st->used = used0 + (pos < cnt ? mr : nvalid);
+        if (!err && pos < cnt && v == -1) err = 1;
         st->err = err;
         st->pos = pos0 + pos;
-        st->window += 1;
-        if (err || pos0 + pos >= nflips) st->done = 1;
+        st->done = (err || pos0 + pos >= nflips) ? 1 : 0;
+    }
+    if (tid == 0) {
+#pragma unroll
+        for (int c = 0; c < 6; c++) st->props[c] = P[c];
+        st->e0 = e0;
+        st->acc += nacc;
+        st->window = wid;
     }
 }
 
-void launch_serial_init(const Globals* g0, const EParams& p, int nflips, SerialState* st, hipStream_t s)
+__global__ void __launch_bounds__(256) k_sf_window(FlipMeshView fm, FlipRows rows, NListView nl, EParams p,
+                                                   int nflips, const int* __restrict__ proposals,
+                                                   const double* __restrict__ uniforms, int n_uniforms, uint64_t seed,
+                                                   int injected, int W, int need_nb, SerialState* __restrict__ st,
+                                                   int* rec, unsigned long long* fstamp)
 {
-    hipLaunchKernelGGL(k_sf_init, dim3(1), dim3(64), 0, s, g0, p, nflips, st);
+    __shared__ union Shared {
+        PatchShared patch[kPatchWaves];
+        SerialShared serial;
+        __device__ Shared() {}
+    } S;
+    if (st->done) return;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int k = blockIdx.x * kPatchWaves + wave;
+    const int cnt = min(W, nflips - st->pos);
+    const int blocks = (cnt + kPatchWaves - 1) / kPatchWaves;
+    if ((int)blockIdx.x >= blocks) return;
+    if (k < cnt) {
+        const int i = st->pos + k, ne = fm.nh / 2;
+        const int e = injected ? proposals[i] : rng_edge(seed, (uint64_t)i, ne);
+        int valid = -1;
+        FlipEdge f{};
+        double d[6] = {0, 0, 0, 0, 0, 0};
+        if (e >= 0 && e < ne) {
+            f = load_flip_edge(fm, e);
+            valid = 0;
+            if (f.fa >= 0 && f.fb >= 0) {
+                NoClaim none;
+                const PatchResult r = patch_eval(fm, nl, p, rows, f.pv, S.patch[wave], none);
+                if (r.ok) {
+                    valid = 1;
+                    const unsigned long long key =
+                        ((unsigned long long)(unsigned)(st->window + 1) << 32) | (unsigned)(W - k);
+                    if (lane < 2) atomicMax(&fstamp[lane ? f.fb : f.fa], key);
+                    r.difference(d);
+                }
+            }
+        }
+        put_record(rec + (size_t)kFlipRecord * k, lane, valid, d, f);
+    }
+    if (!last_block(&st->count, (unsigned)blocks)) return;
+    sf_commit(fm, rows, p, nflips, uniforms, n_uniforms, seed, injected, W, need_nb, st, rec, fstamp, S.serial);
 }
 
-void launch_serial_windows(const FlipMeshView& fm, const NListView& nl, const EParams& p, int nflips,
-                           const int* proposals, const double* uniforms, int n_uniforms, uint64_t seed, int injected,
-                           int W, SerialState* st, const SerialWindow& w, unsigned long long* vstamp,
-                           unsigned long long* estamp, unsigned long long* fstamp, int n_windows, hipStream_t s)
+void launch_serial_begin(const FlipMeshView& fm, const FlipRows& rows, const Globals* g0, const EParams& p, int nflips,
+                         SerialState* st, unsigned long long* fstamp, hipStream_t s)
+{
+    const int n = std::max(std::max(fm.nv, fm.nf), 1);
+    hipLaunchKernelGGL(k_sf_begin, dim3((n + 255) / 256), dim3(256), 0, s, fm, rows, g0, p, nflips, st, fstamp);
+}
+
+void launch_serial_windows(const FlipMeshView& fm, const FlipRows& rows, const NListView& nl, const EParams& p,
+                           int nflips, const int* proposals, const double* uniforms, int n_uniforms, uint64_t seed,
+                           int injected, int W, SerialState* st, int* rec, unsigned long long* fstamp,
+                           int n_windows, hipStream_t s)
 {
     const int need_nb = nl.kind == 0 && nl.exclusion > 1 && p.rep_lc1 > 0;
-    for (int r = 0; r < n_windows; r++) {
-        hipLaunchKernelGGL(k_sf_eval, dim3(W, 2), dim3(64), 0, s, fm, nl, p, nflips, proposals, seed, injected, W,
-                           need_nb, st, w, vstamp, estamp, fstamp);
-        hipLaunchKernelGGL(k_sf_commit, dim3(1), dim3(64), 0, s, fm, p, nflips, uniforms, n_uniforms, seed, injected,
-                           W, need_nb, st, w, vstamp, estamp, fstamp);
-    }
+    for (int r = 0; r < n_windows; r++)
+        hipLaunchKernelGGL(k_sf_window, dim3((W + kPatchWaves - 1) / kPatchWaves), dim3(256), 0, s, fm, rows, nl, p,
+                           nflips, proposals, uniforms, n_uniforms, seed, injected, W, need_nb, st, rec, fstamp);
 }
 
 // ============================================ conflict-free parallel sweep ==
@@ -1154,27 +1423,34 @@ void launch_serial_windows(const FlipMeshView& fm, const NListView& nl, const EP
 // the edge patch of their proposal (flip_patch, flip_utils.cpp:43-68), skip
 // proposals whose patch is taken, flip and evaluate in parallel and apply the
 // Metropolis test one flip at a time.  Here a round of B proposals is one
-// batch:
+// launch:
 //   claim   every proposal writes its priority key into all edges of its
 //           patch with a 64-bit atomicMax (later rounds have larger keys, so
-//           the owner array never needs clearing);
-//   eval    a proposal whose key survived on its whole patch is a winner;
-//           winners have pairwise disjoint patches.  Winners that pass
-//           is_flip_ok evaluate the patch properties before the flip and,
-//           on FlippedTopo, after it: delta = new - old.  The evaluation
-//           after the flip sees the proposal's own flip only (the
+//           the owner array never needs clearing).  What the maximum replaced
+//           tells the loser: a larger key of the same round is the winner's, a
+//           smaller one belongs to a proposal that has just lost the edge.  Of
+//           all proposals that claim an edge, every one but the largest is
+//           told so by its own claim or by a later one;
+//   eval    the same wave evaluates the patch before and after the flip
+//           (patch_eval) without waiting for the outcome of its claims: the
+//           evaluation after the flip sees the proposal's own flip only (the
 //           reference's threads see whichever other flips have happened);
-//   scan    the FP64 Metropolis test in proposal order on the running
-//           global properties;
-//   apply   accepted winners flip.
-// Proposals that lose the claim are skipped, like the reference's failed
-// locks.  Every phase is its own kernel, so no phase reads topology that
-// another thread is rewriting; the result depends only on the seed.
+//   scan    the last workgroup of the mesh runs the FP64 Metropolis test in
+//           proposal order on the running global properties, over the
+//           proposals that lost no edge and pass is_flip_ok: their patches
+//           are pairwise disjoint;
+//   apply   the same workgroup flips the accepted ones.
+// Proposals that lose a claim are skipped, like the reference's failed locks.
+// No workgroup reads topology that another rewrites within a launch (the last
+// one applies when all others have read); the result depends only on the seed.
+// At level 7 (491520 edges, 480 proposals) a round takes 23 us, and 37 us for 8
+// such meshes at once; claim, evaluation by ring walks, scan and application as
+// launches of their own took 7.3 + 32.5 + 11.2 + 4.6 us and 9.8 + 64.8 + 14.0 +
+// 4.7 us.
 
 // The flip patch of edge e (flip_utils.cpp:43-68) is the set of edges of h
-// and of next(h) over the outgoing halfedges h of its four vertices (the two
-// endpoints and the two opposite vertices, patch_vertex(t, e, 0..3)); the
-// claim phase and coop_patch's ownership test visit exactly these.
+// and of next(h) over the outgoing halfedges h of its four vertices: the spoke
+// and rim edges of their rows.
 
 __device__ __forceinline__ int pflip_edge(uint64_t seed, int round, int B, int i, int ne)
 {
@@ -1186,281 +1462,274 @@ __device__ __forceinline__ unsigned long long pflip_key(int round, int B, int i)
     return ((unsigned long long)(round + 1) << 32) | (unsigned)(B - i);
 }
 
-// Eight lanes per proposal, two per patch vertex, walking the vertex's
-// outgoing halfedges: lane 0 of the pair clockwise from v_he, lane 1
-// counter-clockwise (the inverse of cw, prev(h) ^ 1), each claiming its
-// halfedges' edges and next edges until they meet, so the chain of
-// dependent loads is half as long.  The patch's edges get the same
-// atomicMax as in a one-lane walk, and the maximum does not depend on the
-// order of the atomics.
-__device__ __forceinline__ void pflip_claim_body(const FlipMeshView& fm, uint64_t seed, int round, int B, int nprop,
-                                                 unsigned long long* __restrict__ owner, int lb)
-{
-    const int i = lb * kClaimPerBlock + threadIdx.x / 8;
-    if (i >= nprop) return;
-    const Topo t{fm.x, fm.he_to, fm.he_next, fm.he_prev, fm.he_face, fm.v_he, fm.f_he};
-    const int e = pflip_edge(seed, round, B, i, fm.nh / 2);
-    if (t.edge_boundary(e)) return;    // both lanes of every pair leave together
-    const unsigned long long key = pflip_key(round, B, i);
-    const int w = (threadIdx.x / 2) & 3, back = threadIdx.x & 1;
-    const int h0 = t.vhe(patch_vertex(t, e, w));
-    if (h0 < 0) return;
-    // a: the clockwise walker's next halfedge, b: the counter-clockwise
-    // walker's; both lanes hold both, so they leave the loop together
-    int a = h0, b = t.prev(h0) ^ 1, pb = -1;
-#pragma unroll 1
-    for (int it = 0; it < 2 * kMaxValence && a != pb; it++) {
-        const int h = back ? b : a;
-        if (!back || a != b) {
-            atomicMax(&owner[h >> 1], key);
-            atomicMax(&owner[t.next(h) >> 1], key);
-        }
-        if (a == b) break;
-        const int nxt = back ? (t.prev(b) ^ 1) : t.cw(a);
-        const int oth = __shfl_xor(nxt, 1, 64);
-        pb = b;
-        a = back ? oth : nxt;
-        b = back ? nxt : oth;
-    }
-}
-
-__global__ void __launch_bounds__(64) k_pflip_claim(FlipMeshView fm, uint64_t seed, int round, int B, int nprop,
-                                                    unsigned long long* __restrict__ owner)
-{
-    pflip_claim_body(fm, seed, round, B, nprop, owner, blockIdx.x);
-}
-
-// status: 0 skipped, 1 winner pending, 2 accepted, 3 rejected.
-// One workgroup per proposal and side.  Side 0 evaluates the patch before
-// the flip (dold = -old) and decides: the proposal's key survived on every
-// patch edge and is_flip_ok holds, both read off the one-rings coop_patch
-// walks anyway.  Side 1 evaluates the patch after the flip on FlippedTopo
-// (dnew = new) without waiting for the decision: FlippedTopo is a valid view
-// of any interior edge, every walk on it is bounded, and dnew is read only
-// for the proposals side 0 marks pending (a loser's evaluation is wasted,
-// a few percent of them at E / 1024 proposals per round).
-__device__ __forceinline__ void pflip_eval_body(const FlipMeshView& fm, const NListView& nl, const EParams& p,
-                                                uint64_t seed, int round, int B, int nprop,
-                                                const unsigned long long* __restrict__ owner,
-                                                int* __restrict__ status, double* __restrict__ dold,
-                                                double* __restrict__ dnew, int i)
-{
-    __shared__ CoopShared S;
-    const int side = blockIdx.y;
-    const Topo t{fm.x, fm.he_to, fm.he_next, fm.he_prev, fm.he_face, fm.v_he, fm.f_he};
-    const int e = pflip_edge(seed, round, B, i, fm.nh / 2);
-    if (threadIdx.x == 0 && side == 0) status[i] = 0;
-    if (t.edge_boundary(e)) return;
-    if (side == 0) {
-        coop_patch(t, nl, p, e, S, true, owner, pflip_key(round, B, i));
-        if (!S.flip_ok || (S.lost[0] | S.lost[1] | S.lost[2] | S.lost[3])) return;
-        if (threadIdx.x == 0) {
-            for (int k = 0; k < 6; k++) dold[6 * i + k] = -S.sum[k];
-            status[i] = 1;
-        }
-    } else {
-        const FlippedTopo ft(t, e);
-        coop_patch(ft, nl, p, e, S);
-        if (threadIdx.x == 0)
-            for (int k = 0; k < 6; k++) dnew[6 * i + k] = S.sum[k];
-    }
-}
-
-__global__ void __launch_bounds__(64) TM_COOP_OCCUPANCY
-k_pflip_eval(FlipMeshView fm, NListView nl, EParams p, uint64_t seed, int round, int B, int nprop,
-             const unsigned long long* __restrict__ owner, int* __restrict__ status, double* __restrict__ dold,
-             double* __restrict__ dnew)
-{
-    pflip_eval_body(fm, nl, p, seed, round, B, nprop, owner, status, dold, dnew, blockIdx.x);
-}
-
-__global__ void k_pflip_apply(FlipMeshView fm, uint64_t seed, int round, int B, int nprop,
-                              const int* __restrict__ status, int want)
-{
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nprop || status[i] != want) return;
-    do_flip(fm, pflip_edge(seed, round, B, i, fm.nh / 2));
-}
-
-// state: props[6], e0, accepted count (as double).  The Metropolis test
-// walks the winners in proposal order on the running properties
-// (flips.cpp:146-163), with a rejected flip restoring the running
-// properties exactly.  Most winners are rejected and a rejection leaves the
-// state unchanged, so the workgroup tests the next `window` proposals
-// against the current state at once, takes the first acceptance in
-// proposal order (an LDS atomicMin), applies it and continues after it:
-// every decision is the one the sequential walk makes, and the walk takes
-// one parallel step per acceptance instead of one dependent FP64 chain per
-// winner.  Statuses, deltas and uniforms are staged in LDS per chunk.
-constexpr int kScanThreads = 256;
-constexpr int kScanChunk = 1024;
-
-__device__ __forceinline__ void pflip_scan_body(const EParams& p, uint64_t seed, int round, int B, int nprop,
-                                                int window, int* __restrict__ status, const double* __restrict__ dold,
-                                                const double* __restrict__ dnew, double* __restrict__ state)
-{
-    __shared__ int s_st[kScanChunk];
-    __shared__ double s_dp[6 * kScanChunk];
-    __shared__ double s_u[kScanChunk];
-    __shared__ double s_state[8];
-    __shared__ int s_first[2];
-    const int tid = threadIdx.x;
-    if (tid < 8) s_state[tid] = state[tid];
-    for (int base = 0; base < nprop; base += kScanChunk) {
-        const int cnt = min(kScanChunk, nprop - base);
-        for (int k = tid; k < cnt; k += kScanThreads) {
-            const int st = status[base + k];
-            s_st[k] = st;
-            if (st == 1)
-                s_u[k] = rng_uniform(seed ^ 0x5bd1e9955bd1e995ull,
-                                     (uint64_t)round * (uint64_t)B + (uint64_t)(base + k));
-        }
-        for (int k = tid; k < 6 * cnt; k += kScanThreads) {
-            double d = dold[6 * (size_t)base + k];
-            d += dnew[6 * (size_t)base + k];
-            s_dp[k] = d;
-        }
-        if (tid == 0) s_first[0] = s_first[1] = cnt;
-        __syncthreads();
-        // s_first[it & 1] collects iteration it's first acceptance; thread 0
-        // resets the other slot, whose readers finished before the last
-        // barrier and whose writers start after the next one
-        int it = 0;
-        for (int pos = 0; pos < cnt; it++) {
-            const int k = pos + tid;
-            double q[6], en = 0.0;
-            if (tid < window && k < cnt && s_st[k] == 1) {
-                for (int c = 0; c < 6; c++) q[c] = s_state[c] + s_dp[6 * k + c];
-                en = energy_of(q, p);
-                const double de = en - s_state[6];
-                const double alpha = de < 0.0 ? 1.0 : exp(-de);
-                if (s_u[k] <= alpha) atomicMin(&s_first[it & 1], k);
-            }
-            if (tid == 0) s_first[(it + 1) & 1] = cnt;
-            __syncthreads();
-            const int kf = s_first[it & 1];
-            if (kf < cnt && k == kf) {
-                for (int c = 0; c < 6; c++) s_state[c] = q[c];
-                s_state[6] = en;
-                s_state[7] += 1.0;
-                s_st[k] = 2;
-            }
-            pos = kf < cnt ? kf + 1 : pos + window;
-            __syncthreads();
-        }
-        for (int k = tid; k < cnt; k += kScanThreads)
-            if (s_st[k] >= 1) status[base + k] = s_st[k] == 2 ? 2 : 3;
-        __syncthreads();
-    }
-    if (tid < 8) state[tid] = s_state[tid];
-}
-
-__global__ void __launch_bounds__(kScanThreads) k_pflip_scan(EParams p, uint64_t seed, int round, int B, int nprop,
-                                                             int window, int* __restrict__ status,
-                                                             const double* __restrict__ dold,
-                                                             const double* __restrict__ dnew,
-                                                             double* __restrict__ state)
-{
-    pflip_scan_body(p, seed, round, B, nprop, window, status, dold, dnew, state);
-}
-
-__device__ __forceinline__ void pflip_init_body(const Globals* __restrict__ g0, const EParams& p,
-                                                double* __restrict__ state)
-{
-    double props[6];
-    for (int k = 0; k < 6; k++) props[k] = state[k] = g0->props[k];
-    state[6] = energy_of(props, p);
-    state[7] = 0.0;
-}
-
-__global__ void k_pflip_init(const Globals* __restrict__ g0, EParams p, double* __restrict__ state)
-{
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    pflip_init_body(g0, p, state);
-}
-
-// ---- many meshes: round r of every replica per launch ----
 // proposals of replica a in round r (<= 0 once its sweep is done)
 __device__ __forceinline__ int pflip_nprop(const PflipArgs& a, int round)
 {
     return min(a.batch, a.nflips - round * a.batch);
 }
 
-__global__ void k_pflip_init_grouped(const PflipArgs* __restrict__ A)
+// One wave's claims: lane 16 g + slot claims the spoke and the rim edge of that
+// slot of patch vertex g's row.  The edges are loaded beside the row, the
+// atomics go out behind the position loads, and what they replaced is looked
+// at after the evaluation.
+struct PatchClaim {
+    const PflipArgs& a;
+    const unsigned long long key;
+    const int round;
+    int2 er = make_int2(0, 0);
+    unsigned long long o0 = 0ull, o1 = 0ull;
+    bool lost = false;
+    __device__ __forceinline__ void load(int v, int slot) { er = a.rows.er[(size_t)kRowW * v + slot]; }
+    __device__ __forceinline__ void issue(bool has)
+    {
+        if (!has) return;
+        o0 = atomicMax(&a.owner[er.x], key);
+        o1 = atomicMax(&a.owner[er.y], key);
+    }
+    __device__ __forceinline__ void more(int v, int slot, bool has)
+    {
+        if (!has) return;
+        const int2 e2 = a.rows.er[(size_t)kRowW * v + slot];
+        told(atomicMax(&a.owner[e2.x], key));
+        told(atomicMax(&a.owner[e2.y], key));
+    }
+    __device__ __forceinline__ void told(unsigned long long old)
+    {
+        if ((old >> 32) != (key >> 32) || old == key) return;
+        if (old > key) lost = true;
+        else put(a.lost + (a.batch - (int)(unsigned)old), round + 1);
+    }
+    __device__ __forceinline__ bool beaten()
+    {
+        told(o0);
+        told(o1);
+        return __ballot(lost) != 0ull;
+    }
+};
+
+constexpr int kScanPer = 2;    // proposals per thread
+struct ScanShared {
+    double dp[256 * kScanPer][7];    // patch differences and (as an integer) the validity
+    int slots[2][kPatchWaves];
+    int acc[256 * kScanPer];
+};
+
+// state: props[6], e0, accepted count (as double).  The Metropolis test
+// walks the winners in proposal order on the running properties
+// (flips.cpp:146-163), with a rejected flip restoring the running properties
+// exactly.  Most winners are rejected and a rejection leaves the state
+// unchanged, so the workgroup tests the next `window` proposals of each half
+// of a chunk of 512 (thread t holds proposals t and t + 256) against the
+// current state at once, takes the first acceptance in proposal order, applies
+// it and continues after it: every decision is the one the sequential walk
+// makes, and the walk takes one parallel step, of one barrier, per acceptance
+// instead of one dependent FP64 chain per winner.  Every thread carries the
+// state and adds the accepted difference itself.
+__device__ __forceinline__ void pflip_decide(const PflipArgs& a, int round, int nprop, int window, ScanShared& S)
 {
-    if (threadIdx.x == 0) pflip_init_body(A[blockIdx.x].g0, A[blockIdx.x].p, A[blockIdx.x].state);
+    const int tid = threadIdx.x, wave = tid >> 6;
+    const uint64_t useed = a.seed ^ 0x5bd1e9955bd1e995ull;
+    double P[6], e0 = a.state[6], nacc = a.state[7];
+#pragma unroll
+    for (int c = 0; c < 6; c++) P[c] = a.state[c];
+    constexpr int kChunk = 256 * kScanPer;
+    int it = 0;
+    for (int base = 0; base < nprop; base += kChunk) {
+        const int cnt = min(kChunk, nprop - base);
+        // eight lanes per record, its first seven pairs of words
+        unsigned long long w[8 * kScanPer];
+        int lost[kScanPer];
+        const int c8 = tid & 7, r0 = tid >> 3;
+#pragma unroll
+        for (int i = 0; i < 8 * kScanPer; i++) {
+            const int r = r0 + 32 * i;
+            w[i] = r < cnt && c8 < 7 ? get(reinterpret_cast<const unsigned long long*>(a.rec) +
+                                           (size_t)(kFlipRecord / 2) * (base + r) + c8)
+                                     : 0ull;
+        }
+#pragma unroll
+        for (int h = 0; h < kScanPer; h++) lost[h] = 256 * h + tid < cnt ? get(a.lost + base + 256 * h + tid) : 0;
+        double nlu[kScanPer];
+#pragma unroll
+        for (int h = 0; h < kScanPer; h++)
+            nlu[h] = minus_log(rng_uniform(
+                useed, (uint64_t)round * (uint64_t)a.batch + (uint64_t)(base + 256 * h + tid)));
+#pragma unroll
+        for (int i = 0; i < 8 * kScanPer; i++)
+            if (c8 < 7) S.dp[r0 + 32 * i][c8] = __longlong_as_double((long long)w[i]);
+        __syncthreads();
+        double dp[kScanPer][6];
+        bool win[kScanPer];
+#pragma unroll
+        for (int h = 0; h < kScanPer; h++) {
+            const double* d = S.dp[256 * h + tid];
+#pragma unroll
+            for (int c = 0; c < 6; c++) dp[h][c] = d[c];
+            win[h] = 256 * h + tid < cnt && __double2loint(d[6]) == 1 && lost[h] != round + 1;
+        }
+        const int reach = window * kScanPer;
+        int n = 0;
+        for (int pos = 0; pos < cnt;) {
+            bool take[kScanPer];
+#pragma unroll
+            for (int h = 0; h < kScanPer; h++) {
+                const int i = 256 * h + tid;
+                take[h] = false;
+                if (win[h] && i >= pos && i < pos + reach) {
+                    double q[6];
+#pragma unroll
+                    for (int c = 0; c < 6; c++) q[c] = P[c] + dp[h][c];
+                    take[h] = energy_of(q, a.p) - e0 <= nlu[h];
+                }
+            }
+            // the first acceptance: of the lower half, else of the upper
+            static_assert(kScanPer == 2, "halves in order");
+            const unsigned long long b0 = __ballot(take[0]), b1 = __ballot(take[1]);
+            int* slots = S.slots[it++ & 1];
+            if ((tid & 63) == 0)
+                slots[wave] = b0 ? 64 * wave + __ffsll((long long)b0) - 1
+                                 : (b1 ? 256 + 64 * wave + __ffsll((long long)b1) - 1 : INT_MAX);
+            __syncthreads();
+            int first = INT_MAX;
+#pragma unroll
+            for (int i = 0; i < kPatchWaves; i++) first = min(first, slots[i]);
+            if (first == INT_MAX) {
+                pos += reach;
+                continue;
+            }
+#pragma unroll
+            for (int c = 0; c < 6; c++) P[c] += S.dp[first][c];
+            e0 = energy_of(P, a.p);
+            nacc += 1.0;
+            if (tid == 0) S.acc[n] = base + first;
+            n++;
+            pos = first + 1;
+        }
+        __syncthreads();
+        // apply: four threads per accepted flip, one per patch vertex; their
+        // patches are disjoint, and the records hold what do_flip reads
+        for (int t = tid; t < 4 * n; t += 256) {
+            const unsigned long long* r = reinterpret_cast<const unsigned long long*>(a.rec) +
+                                          (size_t)(kFlipRecord / 2) * S.acc[t >> 2];
+            int m[26];
+#pragma unroll
+            for (int c = 6; c < 13; c++) {
+                const unsigned long long x = get(r + c);
+                m[2 * c] = (int)(unsigned)x;
+                m[2 * c + 1] = (int)(unsigned)(x >> 32);
+            }
+            const FlipEdge f = flip_edge_of(m);
+            const int g = t & 3;
+            const int2 ed = g == 1 ? make_int2(f.b2 >> 1, f.b1 >> 1) : make_int2(f.a2 >> 1, f.a1 >> 1);
+            const int me = g == 0 ? f.pv[0] : (g == 1 ? f.pv[1] : (g == 2 ? f.pv[2] : f.pv[3]));
+            if (g == 0) store_flip(a.fm, f);
+            flip_row(a.rows, me, g, g < 2 ? f.pv[2] : f.pv[0], g == 1 ? f.pv[3] : f.pv[1], f.e, ed);
+        }
+        __syncthreads();
+    }
+    if (tid == 0) {
+#pragma unroll
+        for (int c = 0; c < 6; c++) a.state[c] = P[c];
+        a.state[6] = e0;
+        a.state[7] = nacc;
+    }
 }
 
-__global__ void __launch_bounds__(64) k_pflip_claim_grouped(const PflipArgs* __restrict__ A,
-                                                            const int* __restrict__ block0, int R, int round)
+__device__ __forceinline__ void pflip_round_body(const PflipArgs& a, int round, int window, int lb)
 {
-    const int r = find_replica(block0, R, blockIdx.x);
-    const PflipArgs& a = A[r];
+    __shared__ union Shared {
+        PatchShared patch[kPatchWaves];
+        ScanShared scan;
+        __device__ Shared() {}
+    } S;
     const int nprop = pflip_nprop(a, round);
-    if (nprop <= 0) return;
-    pflip_claim_body(a.fm, a.seed, round, a.batch, nprop, a.owner, blockIdx.x - block0[r]);
+    const int blocks = nprop > 0 ? (nprop + kPatchWaves - 1) / kPatchWaves : 0;
+    if (lb >= blocks) return;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int i = lb * kPatchWaves + wave;
+    if (i < nprop) {
+        const int e = pflip_edge(a.seed, round, a.batch, i, a.fm.nh / 2);
+        const FlipEdge f = load_flip_edge(a.fm, e);
+        int valid = 0;
+        double d[6] = {0, 0, 0, 0, 0, 0};
+        if (f.fa >= 0 && f.fb >= 0) {
+            PatchClaim claim{a, pflip_key(round, a.batch, i), round};
+            const PatchResult r = patch_eval(a.fm, a.nl, a.p, a.rows, f.pv, S.patch[wave], claim);
+            valid = !claim.beaten() && r.ok ? 1 : 0;
+            if (valid) r.difference(d);
+        }
+        put_record(a.rec + (size_t)kFlipRecord * i, lane, valid, d, f);
+    }
+    if (!last_block(a.count, (unsigned)blocks)) return;
+    pflip_decide(a, round, nprop, window, S.scan);
 }
 
-__global__ void __launch_bounds__(64) TM_COOP_OCCUPANCY
-k_pflip_eval_grouped(const PflipArgs* __restrict__ A, const int* __restrict__ block0, int R, int round)
+__global__ void __launch_bounds__(256) k_pflip_round(PflipArgs a, int round, int window)
+{
+    pflip_round_body(a, round, window, blockIdx.x);
+}
+
+// rows, running state, claims and counters at the start of a sweep
+__device__ __forceinline__ void pflip_begin_body(const PflipArgs& a, int t)
+{
+    if (t < a.fm.nv) build_rows(a.fm, a.rows, t);
+    if (t < a.fm.nh / 2) a.owner[t] = 0ull;
+    if (t < a.batch) a.lost[t] = 0;
+    if (t == 0) {
+        double props[6];
+        for (int k = 0; k < 6; k++) props[k] = a.state[k] = a.g0->props[k];
+        a.state[6] = energy_of(props, a.p);
+        a.state[7] = 0.0;
+        *a.count = 0u;
+    }
+}
+
+__global__ void __launch_bounds__(256) k_pflip_begin(PflipArgs a)
+{
+    pflip_begin_body(a, blockIdx.x * blockDim.x + threadIdx.x);
+}
+
+// ---- many meshes: round r of every replica per launch ----
+__global__ void __launch_bounds__(256) k_pflip_begin_grouped(const PflipArgs* __restrict__ A)
+{
+    pflip_begin_body(A[blockIdx.y], blockIdx.x * blockDim.x + threadIdx.x);
+}
+
+__global__ void __launch_bounds__(256) k_pflip_round_grouped(const PflipArgs* __restrict__ A,
+                                                             const int* __restrict__ block0, int R, int round,
+                                                             int window)
 {
     const int r = find_replica(block0, R, blockIdx.x);
-    const PflipArgs& a = A[r];
-    const int nprop = pflip_nprop(a, round), i = blockIdx.x - block0[r];
-    if (i >= nprop) return;
-    pflip_eval_body(a.fm, a.nl, a.p, a.seed, round, a.batch, nprop, a.owner, a.status, a.dold, a.dnew, i);
+    pflip_round_body(A[r], round, window, blockIdx.x - block0[r]);
 }
 
-__global__ void __launch_bounds__(kScanThreads) k_pflip_scan_grouped(const PflipArgs* __restrict__ A, int round,
-                                                                     int window)
+static inline int pflip_begin_blocks(int nv, int nh, int batch)
 {
-    const PflipArgs& a = A[blockIdx.x];
-    const int nprop = pflip_nprop(a, round);
-    if (nprop <= 0) return;
-    pflip_scan_body(a.p, a.seed, round, a.batch, nprop, window, a.status, a.dold, a.dnew, a.state);
+    return (std::max(std::max(nv, nh / 2), std::max(batch, 1)) + 255) / 256;
 }
 
-__global__ void k_pflip_apply_grouped(const PflipArgs* __restrict__ A, const int* __restrict__ block0, int R,
-                                      int round)
-{
-    const int r = find_replica(block0, R, blockIdx.x);
-    const PflipArgs& a = A[r];
-    const int i = (blockIdx.x - block0[r]) * blockDim.x + threadIdx.x;
-    if (i >= pflip_nprop(a, round) || a.status[i] != 2) return;
-    do_flip(a.fm, pflip_edge(a.seed, round, a.batch, i, a.fm.nh / 2));
-}
+int pflip_round_blocks(int batch) { return (batch + kPatchWaves - 1) / kPatchWaves; }
 
-void launch_flip_parallel(const FlipMeshView& fm, const NListView& nl, const EParams& p, int nflips, int batch,
-                          int window, uint64_t seed, const Globals* g0, unsigned long long* owner, int* status,
-                          double* dprops, double* state, hipStream_t s)
+void launch_flip_parallel(const PflipArgs& a, int window, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_pflip_init, dim3(1), dim3(64), 0, s, g0, p, state);
-    const int rounds = (nflips + batch - 1) / batch;
+    hipLaunchKernelGGL(k_pflip_begin, dim3(pflip_begin_blocks(a.fm.nv, a.fm.nh, a.batch)), dim3(256), 0, s, a);
+    const int rounds = (a.nflips + a.batch - 1) / a.batch;
+    window = std::min(std::max(window, 1), 256);
     for (int r = 0; r < rounds; r++) {
-        int nprop = std::min(batch, nflips - r * batch);
-        dim3 grid((nprop + 127) / 128), block(128);
-        const dim3 claim_grid((nprop + kClaimPerBlock - 1) / kClaimPerBlock);
-        hipLaunchKernelGGL(k_pflip_claim, claim_grid, dim3(64), 0, s, fm, seed, r, batch, nprop, owner);
-        hipLaunchKernelGGL(k_pflip_eval, dim3(nprop, 2), dim3(64), 0, s, fm, nl, p, seed, r, batch, nprop, owner,
-                           status, dprops, dprops + 6 * (size_t)batch);
-        hipLaunchKernelGGL(k_pflip_scan, dim3(1), dim3(kScanThreads), 0, s, p, seed, r, batch, nprop,
-                           std::min(std::max(window, 1), kScanThreads), status, dprops, dprops + 6 * (size_t)batch,
-                           state);
-        hipLaunchKernelGGL(k_pflip_apply, grid, block, 0, s, fm, seed, r, batch, nprop, status, 2);
+        const int nprop = std::min(a.batch, a.nflips - r * a.batch);
+        hipLaunchKernelGGL(k_pflip_round, dim3(pflip_round_blocks(nprop)), dim3(256), 0, s, a, r, window);
     }
 }
 
 void launch_flip_parallel_grouped(const PflipGroup& g, hipStream_t s)
 {
     if (g.R <= 0) return;
-    hipLaunchKernelGGL(k_pflip_init_grouped, dim3(g.R), dim3(64), 0, s, g.d_args);
-    const int window = std::min(std::max(g.window, 1), kScanThreads);
-    for (int r = 0; r < g.rounds; r++) {
-        hipLaunchKernelGGL(k_pflip_claim_grouped, dim3(g.total_claim), dim3(64), 0, s, g.d_args, g.d_claim0, g.R, r);
-        hipLaunchKernelGGL(k_pflip_eval_grouped, dim3(g.total_eval, 2), dim3(64), 0, s, g.d_args, g.d_eval0, g.R, r);
-        hipLaunchKernelGGL(k_pflip_scan_grouped, dim3(g.R), dim3(kScanThreads), 0, s, g.d_args, r, window);
-        hipLaunchKernelGGL(k_pflip_apply_grouped, dim3(g.total_apply), dim3(128), 0, s, g.d_args, g.d_apply0, g.R, r);
-    }
+    hipLaunchKernelGGL(k_pflip_begin_grouped, dim3(pflip_begin_blocks(g.max_nv, g.max_nh, g.max_batch), g.R),
+                       dim3(256), 0, s, g.d_args);
+    const int window = std::min(std::max(g.window, 1), 256);
+    for (int r = 0; r < g.rounds; r++)
+        hipLaunchKernelGGL(k_pflip_round_grouped, dim3(g.total_blocks), dim3(256), 0, s, g.d_args, g.d_block0, g.R,
+                           r, window);
 }
 
 }    // namespace tmh

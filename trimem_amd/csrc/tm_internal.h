@@ -196,6 +196,13 @@ void launch_flip_serial(const FlipMeshView& fm, const NListView& nl, const EPara
                         const int* proposals, const double* uniforms, int n_uniforms, uint64_t seed, int injected,
                         const Globals* g0, int* result /* [accepted, used, error] */, hipStream_t s);
 
+// Rows of the one-rings (tm_flips.hip), kMaxValence slots per vertex; er null
+// where no sweep claims edges.
+struct FlipRows {
+    int* nb;     // [kMaxValence N] neighbours, ended by -1
+    int2* er;    // [kMaxValence N] spoke and rim edge of each slot
+};
+
 // windowed serial sweep: the serial sweep's decisions and topology from
 // windows of up to kSerialWindowMax proposals evaluated in parallel
 constexpr int kSerialWindowMax = 256;
@@ -203,63 +210,49 @@ struct SerialState {
     int pos, done, used, acc, err, window;
     double props[6];
     double e0;
+    unsigned count;    // workgroups of the window that have finished
 };
-struct SerialWindow {
-    int* e;        // [W] proposed edge
-    int* valid;    // [W] 1 flippable, 0 not, -1 index out of range
-    int* pv;       // [4W] vertices whose one-rings the evaluation read (the patch)
-    int* fc;       // [2W] the edge's two faces
-    double* dO;    // [6W] patch properties before the flip
-    double* dN;    // [6W] after the flip
-    int* nbn;      // [4W] one-ring sizes of the patch vertices (-1: above kMaxValence)
-    int* nb;       // [4 kMaxValence W] their one-rings (exclusion level 2 only)
-};
-void launch_serial_init(const Globals* g0, const EParams& p, int nflips, SerialState* st, hipStream_t s);
-void launch_serial_windows(const FlipMeshView& fm, const NListView& nl, const EParams& p, int nflips,
-                           const int* proposals, const double* uniforms, int n_uniforms, uint64_t seed, int injected,
-                           int W, SerialState* st, const SerialWindow& w, unsigned long long* vstamp,
-                           unsigned long long* estamp, unsigned long long* fstamp, int n_windows, hipStream_t s);
+constexpr int kFlipRecord = 32;    // ints per proposal record
+// rows, face stamps and the starting state
+void launch_serial_begin(const FlipMeshView& fm, const FlipRows& rows, const Globals* g0, const EParams& p, int nflips,
+                         SerialState* st, unsigned long long* fstamp, hipStream_t s);
+// rec: [kFlipRecord W], fstamp: [faces]
+void launch_serial_windows(const FlipMeshView& fm, const FlipRows& rows, const NListView& nl, const EParams& p,
+                           int nflips, const int* proposals, const double* uniforms, int n_uniforms, uint64_t seed,
+                           int injected, int W, SerialState* st, int* rec, unsigned long long* fstamp,
+                           int n_windows, hipStream_t s);
 
-// graph-coloured (claim-based) parallel sweep; state receives props[6], the
-// final energy and the number of accepted flips
-void launch_flip_parallel(const FlipMeshView& fm, const NListView& nl, const EParams& p, int nflips, int batch,
-                          int window, uint64_t seed, const Globals* g0, unsigned long long* owner, int* status,
-                          double* dprops, double* state, hipStream_t s);
-
-// Proposals per 64-lane block of the parallel sweep's claim phase (two lanes
-// per patch vertex).
-constexpr int kClaimPerBlock = 8;
-
-// The parallel sweep of many meshes at once: round r of every replica in one
-// launch per phase.  Each replica's kernels run the single-mesh sweep's
-// device functions on its own arguments, so its flips, decisions and state
-// are those of launch_flip_parallel with the same arguments.
+// The claim-based parallel sweep of one mesh; state receives props[6], the
+// final energy and the number of accepted flips.
 struct PflipArgs {
     FlipMeshView fm;
     NListView nl;
     EParams p;
+    FlipRows rows;
     uint64_t seed;
     int nflips, batch;
     const Globals* g0;
-    unsigned long long* owner;
-    int* status;
-    double* dold;    // [6 batch]
-    double* dnew;    // [6 batch]
-    double* state;   // [8]
+    unsigned long long* owner;    // [E] largest claim key
+    int* rec;                     // [kFlipRecord batch] the proposals' records
+    int* lost;                    // [batch] the last round + 1 in which a later claim beat one of its claims
+    double* state;                // [8]
+    unsigned* count;              // workgroups of the round that have finished
 };
+int pflip_round_blocks(int batch);    // workgroups of a round of `batch` proposals
+void launch_flip_parallel(const PflipArgs& a, int window, hipStream_t s);
+
+// The parallel sweep of many meshes at once: round r of every replica in one
+// launch.  Each replica's workgroups run the single-mesh sweep's device
+// functions on its own arguments, so its flips, decisions and state are those
+// of launch_flip_parallel with the same arguments.
 struct PflipGroup {
     const PflipArgs* d_args;
     int R;
     int rounds;            // the most rounds of any replica
     int window;
-    // prefix tables of blocks per replica: claims (16 proposals per block),
-    // evaluations (one proposal per block), applications (128 per block)
-    const int* d_claim0;
-    int total_claim;
-    const int* d_eval0;
-    int total_eval;
-    const int* d_apply0;
-    int total_apply;
+    const int* d_block0;   // prefix table of pflip_round_blocks per replica
+    int total_blocks;
+    int max_nv, max_nh, max_batch;
 };
 void launch_flip_parallel_grouped(const PflipGroup& g, hipStream_t s);
 
