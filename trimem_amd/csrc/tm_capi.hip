@@ -159,6 +159,7 @@ struct tm_mesh {
     // per-vertex row that crosses the API is mapped back to user ids.
     std::vector<int> perm, iperm;
     DevBuf<int> d_perm, d_iperm;
+    DevBuf<int> faces;       // fv_indices after flips
     DevBuf<double> stage;    // user-order rows for uploads and downloads
 
     MeshView view() const
@@ -890,7 +891,16 @@ double* tm_mesh_points(tm_mesh* mesh) { return mesh->points; }
 int tm_mesh_fv_indices(tm_mesh* mesh, int* out)
 {
     API_BEGIN
-    refresh_host_topology(*mesh);
+    if (mesh->host_stale) {
+        // flips have changed the device topology: the faces from there, instead
+        // of all six halfedge arrays and a walk over them here
+        mesh->faces.alloc((size_t)3 * mesh->nf);
+        launch_faces(mesh->view(), mesh->d_perm.p, mesh->faces.p, g_rt.stream);
+        check_launch();
+        d2h(out, mesh->faces.p, sizeof(int) * 3 * mesh->nf);
+        sync();
+        return TM_OK;
+    }
     for (int f = 0; f < mesh->nf; f++) {
         int h = mesh->f_he[f];
         out[3 * f] = mesh->perm[mesh->he_to[h]];

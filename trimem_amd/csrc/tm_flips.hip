@@ -73,6 +73,23 @@ void launch_gather_rows(const double* src, const int* idx, double* dst, int n, i
     hipLaunchKernelGGL(k_gather_rows, dim3((n * w + 255) / 256), dim3(256), 0, s, src, idx, dst, n, w);
 }
 
+// The faces as user vertex ids (fv_indices): to(h), to(next h), to(next next h)
+// of each face's halfedge, one thread per face.
+__global__ void __launch_bounds__(256) k_faces(MeshView m, const int* __restrict__ perm, int* __restrict__ out)
+{
+    const int f = blockIdx.x * blockDim.x + threadIdx.x;
+    if (f >= m.nf) return;
+    const int h0 = m.f_he[f], h1 = m.he_next[h0], h2 = m.he_next[h1];
+    out[3 * f] = perm[m.he_to[h0]];
+    out[3 * f + 1] = perm[m.he_to[h1]];
+    out[3 * f + 2] = perm[m.he_to[h2]];
+}
+
+void launch_faces(const MeshView& m, const int* perm, int* out, hipStream_t s)
+{
+    if (m.nf > 0) hipLaunchKernelGGL(k_faces, dim3((m.nf + 255) / 256), dim3(256), 0, s, m, perm, out);
+}
+
 // ---------------------------------------------------------------- RNG -----
 __device__ __forceinline__ double rng_uniform(uint64_t seed, uint64_t i) { return rng_unit(rng_draw(seed, 1, i)); }
 __device__ __forceinline__ int rng_edge(uint64_t seed, uint64_t i, int ne)

@@ -146,6 +146,8 @@ void launch_sum_geometry(const MeshView& m, int what, double* partials, unsigned
 void launch_gather_rows(const double* src, const int* idx, double* dst, int n, int w, hipStream_t s);
 
 // topology helpers (tm_flips.hip)
+// out[3 nf]: the faces' vertices as user ids (perm: internal -> user)
+void launch_faces(const MeshView& m, const int* perm, int* out, hipStream_t s);
 // Rebuild ring table and meta from the halfedge arrays; sets *overflow to 1
 // if a vertex has more than kMaxValence neighbours.
 void launch_build_ring(const MeshView& m, int* ring, int* meta, int* overflow, hipStream_t s);
