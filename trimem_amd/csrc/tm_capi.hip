@@ -7,6 +7,7 @@
 // parameter arithmetic, and copying inputs and results.
 #include "../../include/trimem_hip.h"
 #include "tm_internal.h"
+#include "tm_last.h"
 #include "tm_surrogate.h"
 
 #include <cfloat>
@@ -642,6 +643,7 @@ struct tm_energy {
     DevBuf<double> q, partials, grad, vprops, gprops;
     DevBuf<int> pair_cnt;
     DevBuf<double> rep_v, rep_g;
+    DevBuf<unsigned> pass_count;
     DevBuf<double> theta;    // pass 1's dihedral angles for pass 2 (kRingPad per vertex, float or double)
     DevBuf<Globals> globals;
     DevBuf<int> flip_result, proposals, pf_rec, pf_lost;
@@ -683,6 +685,14 @@ EParams eparams_of(const tm_energy& E)
     return p;
 }
 
+// the counters of a properties pass, zero between launches
+void alloc_pass_count(DevBuf<unsigned>& c)
+{
+    c.alloc(kLastCounters);
+    launch_fill_ints(reinterpret_cast<int*>(c.p), kLastCounters, 0, nullptr, 0, 0, nullptr, 0, 0, g_rt.stream);
+    check_launch();
+}
+
 void ensure_energy_buffers(tm_energy& E, const tm_mesh& M)
 {
     if (E.nv == M.nv && E.q.p) return;
@@ -697,6 +707,7 @@ void ensure_energy_buffers(tm_energy& E, const tm_mesh& M)
     E.grad.alloc((size_t)M.nv * 3);
     E.theta.alloc((size_t)kRingPad * M.nv);
     E.globals.alloc(1);
+    alloc_pass_count(E.pass_count);
     E.flip_result.alloc(4);
 }
 
@@ -745,6 +756,7 @@ PassBuffers buffers(tm_energy& E, tm_mesh& M)
     b.rep_v = E.rep_v.p;
     b.rep_g = E.rep_g.p;
     b.partials = E.partials.p;
+    b.count = E.pass_count.p;
     b.globals = E.globals.p;
     b.theta = E.theta.p;
     b.list = M.generic.p;
@@ -2252,6 +2264,7 @@ struct tm_surrogate {
     DevBuf<int> twin, err;
     // the feature pass: properties without repulsion, in buffers of its own
     DevBuf<double> q, gprops, vprops, partials, rep_v;
+    DevBuf<unsigned> pass_count;
     DevBuf<int> pair_cnt;
     DevBuf<Globals> globals;
     DevBuf<double> neg_force, xsave;
@@ -2321,6 +2334,7 @@ void sg_alloc(tm_surrogate& S)
     S.q.alloc(N);
     S.gprops.alloc(6 * N);
     S.vprops.alloc(6 * N);
+    alloc_pass_count(S.pass_count);
     S.partials.alloc((size_t)pass1_blocks(S.nv) * 6);
     S.rep_v.alloc(N);
     S.pair_cnt.alloc(N);
@@ -2347,6 +2361,7 @@ void sg_feature_pass(tm_surrogate& S)
     pb.rep_v = S.rep_v.p;
     pb.partials = S.partials.p;
     pb.globals = S.globals.p;
+    pb.count = S.pass_count.p;
     pb.list = M.generic.p;
     pb.nlist = 0;
     launch_pass1(M.view(), E.nlist->view(), ep, 1, pb, S.vprops.p, g_rt.stream);

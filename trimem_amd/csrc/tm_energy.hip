@@ -29,6 +29,7 @@
 // branches of calc_sector_angle / calc_dihedral_angle.
 #include <hip/hip_ext.h>
 #include "tm_internal.h"
+#include "tm_last.h"
 #include "tm_om.h"
 #include "tm_wave.h"
 
@@ -176,17 +177,10 @@ __device__ __forceinline__ void block_sum6(double v[6], double* s_red /* [nwaves
     __syncthreads();
 }
 
-__device__ __forceinline__ Globals globals_of_sums(double v[6], const EParams& p);
-
-// The end of finalize_block: the butterfly over the wave's lanes, then the
-// energy (kernel.h:110-122) and the penalty factors 2 kappa / ref (X / ref -
-// 1) (kernel.h:27-71).
-__device__ __forceinline__ Globals globals_of_sums(double v[6], const EParams& p)
+// The energy (kernel.h:110-122) and the penalty factors 2 kappa / ref (X / ref -
+// 1) (kernel.h:27-71) of the six global sums.
+__device__ __forceinline__ Globals globals_of_sums(const double v[6], const EParams& p)
 {
-#pragma unroll
-    for (int k = 0; k < 6; k++)
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) v[k] += __shfl_xor(v[k], off, 64);
     Globals g;
     const double A = v[0], V = v[1], C = v[2], B = v[3], T = v[4], R = v[5];
     for (int k = 0; k < 6; k++) g.props[k] = v[k];
@@ -206,6 +200,53 @@ __device__ __forceinline__ Globals globals_of_sums(double v[6], const EParams& p
     e += p.kappa_b * B;
     g.energy = e;
     return g;
+}
+
+// The end of a properties pass, by the workgroup of 256 threads that finishes
+// last: the six globals from the block partials (stored column by column,
+// partials[k * nblocks + b]) in a fixed order that depends on nothing but the
+// number of rows -- lane i of a wave adds rows i, i + 64, ... of its column,
+// then a butterfly joins the 64 lanes -- so every launch gets the same bits.
+// Waves 0 and 1 take two columns each, waves 2 and 3 one.  A chain of two
+// loads and a few barriers, run by the pass itself up to kTailBlocks rows.
+__device__ __forceinline__ void finalize_tail(const PassArgs& A)
+{
+    __shared__ double s_sum[6];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const bool two = wave < 2;
+    const double* c0 = A.partials + (size_t)wave * A.nblocks;
+    const double* c1 = A.partials + (size_t)(wave + 4) * A.nblocks;
+    double v0 = 0.0, v1 = 0.0;
+    constexpr int kBatch = 12;    // rows in flight per lane
+    for (int b0 = lane; b0 < A.nblocks; b0 += 64 * kBatch) {
+        double r0[kBatch], r1[kBatch];
+#pragma unroll
+        for (int u = 0; u < kBatch; u++) {
+            const int b = b0 + 64 * u;
+            r0[u] = b < A.nblocks ? get(c0 + b) : 0.0;
+            r1[u] = two && b < A.nblocks ? get(c1 + b) : 0.0;
+        }
+#pragma unroll
+        for (int u = 0; u < kBatch; u++)
+            if (b0 + 64 * u < A.nblocks) {
+                v0 += r0[u];
+                v1 += r1[u];
+            }
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        v0 += __shfl_xor(v0, off, 64);
+        v1 += __shfl_xor(v1, off, 64);
+    }
+    if (lane == 0) {
+        s_sum[wave] = v0;
+        if (two) s_sum[wave + 4] = v1;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        *A.globals = globals_of_sums(s_sum, A.p);
+        if (A.pc.dforce) *A.pc.dforce = 0;    // replica groups: the query of this evaluation recorded
+    }
 }
 
 // ------------------------------------------------------- lane groups -----
@@ -751,8 +792,9 @@ __device__ __forceinline__ bool is_generic(int meta)
 // the same 256-vertex blocks itself, in the same order; this kernel then
 // measures how far every vertex has moved since the cache's recording (the
 // largest squared displacement of the block, NaN counting as infinite), the
-// query's replay condition.
-template <class T, bool kApart = false>
+// query's replay condition.  kFinal: nothing of the pass follows, and the last
+// workgroup sums the partials (finalize_tail).
+template <class T, bool kApart = false, bool kFinal = !kApart>
 __device__ __forceinline__ void pass1_body(const PassArgs& A, int lb)
 {
     const MeshView& m = A.m;
@@ -818,10 +860,12 @@ __device__ __forceinline__ void pass1_body(const PassArgs& A, int lb)
     if (threadIdx.x < (kApart ? 5 : 6)) {
         double a = 0;
         for (int w = 0; w < kWaves; w++) a += s_red[w * 6 + threadIdx.x];
-        A.partials[threadIdx.x * A.nblocks + lb] = a;
+        put(A.partials + (size_t)threadIdx.x * A.nblocks + lb, a);
     }
     if (kApart && A.pc.x_snap && threadIdx.x == 63)
         A.pc.disp_part[lb] = fmax(fmax(s_disp[0], s_disp[1]), fmax(s_disp[2], s_disp[3]));
+    if constexpr (kFinal)
+        if (A.tail && last_block_of_many(A.count, lb, A.nblocks)) finalize_tail(A);
 }
 
 template <class T>
@@ -847,7 +891,7 @@ __global__ void __launch_bounds__(kPass1Verts) k_pass1_grouped(const PassArgs* _
 }
 
 // replica groups with the cached query: every replica with repulsion leaves
-// column 5 to it
+// column 5 to it, and every replica its globals
 template <class T>
 __global__ void __launch_bounds__(kPass1Verts) k_pass1_apart_grouped(const PassArgs* __restrict__ A,
                                                                      const int* __restrict__ block0, int R)
@@ -855,7 +899,7 @@ __global__ void __launch_bounds__(kPass1Verts) k_pass1_apart_grouped(const PassA
     const int lb = logical_block();
     const int r = find_replica(block0, R, lb);
     if (A[r].rep_v) pass1_body<T, true>(A[r], lb - block0[r]);
-    else pass1_body<T, false>(A[r], lb - block0[r]);
+    else pass1_body<T, false, false>(A[r], lb - block0[r]);
 }
 
 // Repulsion property of every ring vertex (mesh_repulsion.h:28-54):
@@ -1057,7 +1101,11 @@ __device__ __forceinline__ void wide_record(const MeshView& m, const NListView& 
 template <int kBatch>
 __device__ __forceinline__ void rep_cached_body(const PassArgs& A, int lb)
 {
-    if (!A.rep_v) return;
+    if (lb >= A.nblocks) return;    // padding of a grouped launch
+    if (!A.rep_v) {
+        if (A.tail && lb == 0) finalize_tail(A);    // no query: pass 1's partials are complete
+        return;
+    }
     const MeshView& m = A.m;
     const EParams& p = A.p;
     const PairCache& pc = A.pc;
@@ -1193,7 +1241,8 @@ __device__ __forceinline__ void rep_cached_body(const PassArgs& A, int lb)
     if (A.vprops && vi < m.nv) A.vprops[6 * vi + 5] = s_val[threadIdx.x];
     __shared__ double s_red[kPass1Verts / 64];
     const double col5 = block_sum1(s_val[threadIdx.x], s_red);
-    if (threadIdx.x == 0 && lb < A.nblocks) A.partials[5 * A.nblocks + lb] = col5;
+    if (threadIdx.x == 0) put(A.partials + 5 * (size_t)A.nblocks + lb, col5);
+    if (A.tail && last_block_of_many(A.count, lb, A.nblocks)) finalize_tail(A);
 }
 
 template <int kBatch>
@@ -1268,64 +1317,12 @@ __global__ void __launch_bounds__(kThreads) k_rep_grouped(const PassArgs* __rest
     rep_body<kThreads, kBatch>(A[r], lb - block0[r]);
 }
 
-// Fixed-order FP64 sum of the block partials of pass 1, energy and penalty
-// factors (one wave; kernel boundaries order it after pass 1).
-// The six globals from the block partials (stored column by column,
-// partials[k * nblocks + b]) in a fixed order: lane i of wave 0 adds rows
-// i, i + 64, ... of each column in turn, then a butterfly joins the 64
-// lanes.  The order depends on nothing but the number of rows, so every
-// launch that calls this gets the same bits.  The whole block stages up to
-// kFinRows rows in LDS with one round of loads (17 values per thread in
-// flight) before wave 0 adds them; kFinRows is a multiple of 64, so chunks
-// keep each lane's rows in order.  Valid in wave 0.
-constexpr int kFinThreads = 256;
-constexpr int kFinRows = 704;
-__device__ __forceinline__ Globals finalize_block(const double* __restrict__ partials, int nblocks, const EParams& p)
+// the sums of the meshes of more than kTailBlocks rows, whose pass leaves them
+// to a launch of its own
+__global__ void __launch_bounds__(256) k_finalize(PassArgs A) { finalize_tail(A); }
+__global__ void __launch_bounds__(256) k_finalize_grouped(const PassArgs* __restrict__ A)
 {
-    static_assert(kFinRows % 64 == 0, "chunks of whole lane sweeps");
-    constexpr int kBatch = (6 * kFinRows + kFinThreads - 1) / kFinThreads;
-    __shared__ double s_rows[6 * kFinRows];
-    double v[6] = {0, 0, 0, 0, 0, 0};
-    for (int c0 = 0; c0 < nblocks; c0 += kFinRows) {
-        const int rows = min(kFinRows, nblocks - c0);
-        double r[kBatch];
-#pragma unroll
-        for (int u = 0; u < kBatch; u++) {
-            const int i = threadIdx.x + u * kFinThreads, k = i / kFinRows, b = i - k * kFinRows;
-            r[u] = i < 6 * kFinRows && b < rows ? partials[k * nblocks + c0 + b] : 0.0;
-        }
-#pragma unroll
-        for (int u = 0; u < kBatch; u++) {
-            const int i = threadIdx.x + u * kFinThreads;
-            if (i < 6 * kFinRows) s_rows[i] = r[u];
-        }
-        __syncthreads();
-        if (threadIdx.x < 64)
-            for (int b = threadIdx.x; b < rows; b += 64)
-#pragma unroll
-                for (int k = 0; k < 6; k++) v[k] += s_rows[k * kFinRows + b];
-        __syncthreads();
-    }
-    return globals_of_sums(v, p);
-}
-
-// Fixed-order FP64 sum of the block partials of pass 1, energy and penalty
-// factors (kernel boundaries order it after pass 1).
-__global__ void __launch_bounds__(kFinThreads) k_finalize(PassArgs A)
-{
-    const Globals g = finalize_block(A.partials, A.nblocks, A.p);
-    if (threadIdx.x == 0) *A.globals = g;
-}
-
-// one block per replica
-__global__ void __launch_bounds__(kFinThreads) k_finalize_grouped(const PassArgs* __restrict__ A)
-{
-    const PassArgs& a = A[blockIdx.x];
-    const Globals g = finalize_block(a.partials, a.nblocks, a.p);
-    if (threadIdx.x == 0) {
-        *a.globals = g;
-        if (a.pc.dforce) *a.pc.dforce = 0;    // the query of this evaluation recorded
-    }
+    if (!A[blockIdx.x].tail) finalize_tail(A[blockIdx.x]);
 }
 
 // OpenMesh-semantics properties of the listed vertices (boundary and
@@ -1599,6 +1596,8 @@ PassArgs pass_args(const MeshView& m, const NListView& nl, const EParams& p, con
     a.list = b.list;
     a.nlist = b.nlist;
     a.nblocks = pass1_blocks(m.nv);
+    a.count = b.count;
+    a.tail = a.nblocks <= kTailBlocks;
     a.pc = a.rep_v ? b.pc : PairCache{};
     a.theta = b.theta;
     return a;
@@ -1742,7 +1741,7 @@ void launch_pass1(const MeshView& m, const NListView& nl, const EParams& p, int 
         hipLaunchKernelGGL(k_generic_props, dim3(nblocks(b.nlist, 128)), dim3(128), 0, s, m, nl, p, b.list, b.nlist,
                            b.gprops);
     launch_pass1_body(a, mixed, t, s, marks);
-    hipLaunchKernelGGL(k_finalize, dim3(1), dim3(kFinThreads), 0, s, a);
+    if (!a.tail) hipLaunchKernelGGL(k_finalize, dim3(1), dim3(256), 0, s, a);
 }
 
 void launch_pass2(const MeshView& m, const NListView& nl, const EParams& p, int mixed, const PassBuffers& b,
@@ -1755,11 +1754,16 @@ void launch_pass2(const MeshView& m, const NListView& nl, const EParams& p, int 
                            b.list, b.nlist, grad);
 }
 
+static bool group_repels(const GroupLaunch& g)
+{
+    for (int r = 0; r < g.R; r++)
+        if (g.h_args[r].rep_v) return true;
+    return false;
+}
+
 void launch_rep_grouped(const GroupLaunch& g, hipStream_t s)
 {
-    bool rep = false;
-    for (int r = 0; r < g.R; r++) rep = rep || g.h_args[r].rep_v;
-    if (!rep) return;
+    if (!group_repels(g)) return;
     if (g.total_rc > 0) {
         const dim3 grid(g.total_rc), block(256);
         switch (g.tune.rep_batch) {
@@ -1780,7 +1784,7 @@ void launch_pass1_grouped(const GroupLaunch& g, hipStream_t s, const hipEvent_t*
             hipLaunchKernelGGL(k_generic_props_at, dim3(nblocks(g.h_args[r].nlist, 128)), dim3(128), 0, s, g.d_args,
                                r);
     const dim3 grid(g.total_p1), block(kPass1Verts);
-    if (g.total_rc > 0) {
+    if (g.total_rc > 0 && group_repels(g)) {
         // the cached query after pass 1, as for single meshes
         if (g.mixed) launch_marked(k_pass1_apart_grouped<float>, grid, block, s, marks, g.d_args, g.d_block0_p1, g.R);
         else launch_marked(k_pass1_apart_grouped<double>, grid, block, s, marks, g.d_args, g.d_block0_p1, g.R);
@@ -1790,7 +1794,9 @@ void launch_pass1_grouped(const GroupLaunch& g, hipStream_t s, const hipEvent_t*
         if (g.mixed) launch_marked(k_pass1_grouped<float>, grid, block, s, marks, g.d_args, g.d_block0_p1, g.R);
         else launch_marked(k_pass1_grouped<double>, grid, block, s, marks, g.d_args, g.d_block0_p1, g.R);
     }
-    hipLaunchKernelGGL(k_finalize_grouped, dim3(g.R), dim3(kFinThreads), 0, s, g.d_args);
+    bool tail = true;
+    for (int r = 0; r < g.R; r++) tail = tail && g.h_args[r].tail;
+    if (!tail) hipLaunchKernelGGL(k_finalize_grouped, dim3(g.R), dim3(256), 0, s, g.d_args);
 }
 
 void launch_pass2_grouped(const GroupLaunch& g, hipStream_t s)

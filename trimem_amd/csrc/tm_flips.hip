@@ -19,6 +19,7 @@
 #include "tm_internal.h"
 #include "tm_om.h"
 #include "tm_rng.h"
+#include "tm_last.h"
 #include "tm_wave.h"
 
 #include <algorithm>
@@ -1029,26 +1030,6 @@ __device__ __forceinline__ PatchResult patch_eval(const FlipMeshView& fm, const 
     return res;
 }
 
-// ---------------------------------------------- the last workgroup's turn --
-// One launch evaluates many proposals and then decides on all of them: every
-// workgroup hands its results over and counts itself, and the one that counts
-// last decides.  The hand-over uses no fence: on this part a device-scope
-// fence writes back and invalidates the whole L2 of the workgroup's XCD.
-// Results are stored and read with relaxed device-scope atomics, which pass
-// by the caches that are not coherent between XCDs; each workgroup waits for
-// its own stores to complete (s_waitcnt) before it counts, and the last one
-// reads after its count has returned.  Nothing waits for another workgroup.
-template <class T>
-__device__ __forceinline__ void put(T* a, T v)
-{
-    __hip_atomic_store(a, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-template <class T>
-__device__ __forceinline__ T get(const T* a)
-{
-    return __hip_atomic_load(a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
 // A proposal's record, one 128-byte line that its wave stores in one go: words
 // 0-11 the patch differences (after minus before), 12 its validity (1
 // flippable, 0 not, -1 index out of range), 13-25 the FlipEdge.  The readers
@@ -1070,22 +1051,6 @@ __device__ __forceinline__ void put_record(int* rec, int lane, int valid, const 
 __device__ __forceinline__ FlipEdge flip_edge_of(const int* m)    // words 13 .. 25 of a record
 {
     return FlipEdge{m[13], {m[14], m[15], m[16], m[17]}, m[18], m[19], m[20], m[21], m[22], m[23], m[24], m[25]};
-}
-
-// true for every thread of the last of `blocks` workgroups; the counter is
-// left at zero for the next launch
-__device__ __forceinline__ bool last_block(unsigned* counter, unsigned blocks)
-{
-    __shared__ int s_last;
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");    // this wave's stores have completed
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        const unsigned c = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        s_last = c + 1 == blocks;
-        if (s_last) put(counter, 0u);
-    }
-    __syncthreads();
-    return s_last != 0;
 }
 
 // The Metropolis test (flips.cpp:57-64) u <= min(1, exp(-de)) as de <= -log(u):

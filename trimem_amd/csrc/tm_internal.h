@@ -49,6 +49,7 @@ struct PassBuffers {
     double* rep_v;      // [N] repulsion property per vertex (k_rep)
     double* rep_g;      // [3N] repulsion gradient, rows of vertices with pairs (k_rep)
     double* partials;   // [6 * pass1 blocks]
+    unsigned* count;    // [kLastCounters] zeros (tm_last.h)
     Globals* globals;
     const int* list;    // boundary / degenerate vertices
     int nlist;
@@ -59,6 +60,13 @@ struct PassBuffers {
     void* theta;
 };
 int pass1_blocks(int nv);
+// Up to this many rows of partials the pass's last workgroup sums them, above
+// it a launch of its own does.  Counting the workgroups costs the pass about
+// what the launch does where they are many: an evaluation (properties and
+// gradient, mixed) takes 31.6 us with the tail and 33.3 with the launch at 642
+// vertices (8 rows), 31.1 and 33.4 at 10242 (48), 36.5 and 36.7 at 23042 (96),
+// 42.6 and 42.4 at 92162 (368), 51.9 and 51.8 at 163842 (648).
+constexpr int kTailBlocks = 128;
 
 // Everything the pass kernels read and write for one mesh.  A grouped launch
 // takes a device array of these, one per replica, and a prefix table of
@@ -75,6 +83,8 @@ struct PassArgs {
     int* pair_cnt;
     double* rep_g;       // null: rows not stored (pass 1 only)
     double* partials;
+    unsigned* count;
+    int tail;            // the pass's last workgroup sums the partials (see kTailBlocks)
     Globals* globals;
     double* grad;
     double* vprops;      // optional per-vertex properties of pass 1
@@ -105,7 +115,7 @@ int tuned_blocks(int nv, int threads);    // blocks of 8-lane groups (the query)
 int pass2_blocks(int nv, int threads);    // blocks of one lane per vertex (pass 2), a multiple of 8
 // the repulsion query and the pass-2 kernel alone (for timing)
 void launch_rep(const PassArgs& a, const Tuning& t, hipStream_t s);
-// the repulsion query and the pass-1 kernel (fused or apart), no finalize;
+// the repulsion query and the pass-1 kernel, the later of which finalizes;
 // marks (optional): HIP events stamped at the pass-1 kernel's start and end
 // (either may be null)
 void launch_pass1_body(const PassArgs& a, int mixed, const Tuning& t, hipStream_t s,
