@@ -2310,19 +2310,18 @@ void sg_alloc(tm_surrogate& S)
         S.pk.v_n[l] = pp; pp += kSgW * kSgW;
     }
     // activations
-    const size_t nact = N * kSgFeatPad + (2 * (kSgLayers + 1) + 2 * kSgLayers + 4) * NW + 3 * N + (N + 3) / 4 + 1 +
-                        sg_partial_floats(S.nv);
+    const size_t nact = N * kSgFeatPad + (2 * (kSgLayers + 1) + 2 * kSgLayers + 3) * NW + 3 * N + sg_loss_rows(S.nv) +
+                        1 + sg_partial_floats(S.nv);
     S.act.alloc(nact);
     float* a = S.act.p;
     S.b.f0 = a; a += N * kSgFeatPad;
     for (int l = 0; l <= kSgLayers; l++) { S.b.Z[l] = a; a += NW; S.b.H[l] = a; a += NW; }
     for (int l = 0; l < kSgLayers; l++) { S.b.P[l] = a; a += NW; S.b.M[l] = a; a += NW; }
     S.b.dH = a; a += NW;
-    S.b.dZ = a; a += NW;
     S.b.dP = a; a += NW;
     S.b.dM = a; a += NW;
     S.b.ghat = a; a += 3 * N;
-    S.b.loss_partial = a; a += (N + 3) / 4;
+    S.b.loss_partial = a; a += sg_loss_rows(S.nv);
     S.b.loss = a; a += 1;
     S.b.partial = a;
     S.geo_buf.alloc((size_t)kSgSlots * N * 5 + 3 * N);
@@ -2334,8 +2333,8 @@ void sg_alloc(tm_surrogate& S)
     S.q.alloc(N);
     S.gprops.alloc(6 * N);
     S.vprops.alloc(6 * N);
-    alloc_pass_count(S.pass_count);
     S.partials.alloc((size_t)pass1_blocks(S.nv) * 6);
+    alloc_pass_count(S.pass_count);
     S.rep_v.alloc(N);
     S.pair_cnt.alloc(N);
     S.globals.alloc(1);
@@ -2345,7 +2344,9 @@ void sg_alloc(tm_surrogate& S)
 
 // properties without repulsion at the current positions into the
 // surrogate's own buffers, then the input features
-void sg_feature_pass(tm_surrogate& S)
+// exact_pass1: the energy manager's properties pass at these positions has just
+// written S.vprops in the mixed precision, the same values
+void sg_feature_pass(tm_surrogate& S, bool exact_pass1 = false)
 {
     tm_mesh& M = *S.mesh;
     tm_energy& E = *S.em;
@@ -2360,12 +2361,14 @@ void sg_feature_pass(tm_surrogate& S)
     pb.pair_cnt = S.pair_cnt.p;
     pb.rep_v = S.rep_v.p;
     pb.partials = S.partials.p;
-    pb.globals = S.globals.p;
     pb.count = S.pass_count.p;
+    pb.globals = S.globals.p;
     pb.list = M.generic.p;
     pb.nlist = 0;
-    launch_pass1(M.view(), E.nlist->view(), ep, 1, pb, S.vprops.p, g_rt.stream);
-    sg_features(M.view(), S.vprops.p, S.globals.p, S.norm, S.geo, S.b.f0, S.err.p, g_rt.stream);
+    const Globals* globals = S.globals.p;
+    if (exact_pass1) globals = E.globals.p;
+    else launch_pass1(M.view(), E.nlist->view(), ep, 1, pb, S.vprops.p, g_rt.stream);
+    sg_features(M.view(), S.vprops.p, globals, S.norm, S.geo, S.b.f0, S.err.p, g_rt.stream);
     check_launch();
 }
 
@@ -2381,9 +2384,9 @@ void sg_check_err(tm_surrogate& S)
 }
 
 // the exact gradient at the current positions (energy manager buffers)
-void sg_exact_gradient(tm_surrogate& S)
+void sg_exact_gradient(tm_surrogate& S, double* vprops = nullptr)
 {
-    run_pass1(*S.em, *S.mesh, S.em->precision, nullptr);
+    run_pass1(*S.em, *S.mesh, S.em->precision, vprops);
     run_pass2(*S.em, *S.mesh, S.em->precision);
 }
 
@@ -2544,16 +2547,16 @@ int tm_surrogate_loss_grad(tm_surrogate* sg, double* loss, float* grad)
     API_BEGIN
     tm_surrogate& S = *sg;
     upload_points(*S.mesh);
-    sg_exact_gradient(S);
-    sg_feature_pass(S);
+    const bool mixed = S.em->precision == TM_PREC_MIXED;
+    sg_exact_gradient(S, mixed ? S.vprops.p : nullptr);
+    sg_feature_pass(S, mixed);
     sg_forward(S.mesh->view(), S.b, S.geo, S.theta.p, S.pk, S.sigma_F, S.em->grad.p, nullptr, g_rt.stream);
     sg_backward(S.mesh->view(), S.b, S.geo, S.theta.p, S.pk, S.twin.p, S.grad.p, g_rt.stream);
     check_launch();
-    sg_check_err(S);
     float l = 0.0f;
     d2h(&l, S.b.loss, sizeof(float));
     if (grad) d2h(grad, S.grad.p, sizeof(float) * kSgParams);
-    sync();
+    sg_check_err(S);    // waits
     if (loss) *loss = l;
     API_END
 }

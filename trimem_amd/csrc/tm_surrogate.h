@@ -11,7 +11,6 @@ constexpr int kSgLayers = 3;      // message-passing layers
 constexpr int kSgFeat = 8;        // vertex input features
 constexpr int kSgFeatPad = 16;    // padded to one MFMA k-step
 constexpr int kSgSlots = 10;      // largest valence handled
-constexpr int kSgRowsPerBlock = 256;
 
 // Parameter vector (FP32): W_in [16][64], b_in [64], per layer U [64][64],
 // W [64][64], V [64][64] (W and V adjacent: [W; V] is one [128][64] block),
@@ -67,15 +66,15 @@ struct SgBuffers {
     float* P[kSgLayers];
     float* M[kSgLayers];
     float* dH;
-    float* dZ;
     float* dP;
     float* dM;
     float* ghat;                  // [N][3]
-    float* loss_partial;          // [ceil(N/4)]
+    float* loss_partial;          // [sg_loss_rows]
     float* loss;                  // [1]
     float* partial;               // reduction scratch
 };
 size_t sg_partial_floats(int nv);
+size_t sg_loss_rows(int nv);
 
 void sg_pack(const float* theta, const SgPacked& pk, hipStream_t s);
 void sg_features(const MeshView& m, const double* vprops, const Globals* g, const SgNorm& nrm, const SgGeom& geo,
