@@ -20,6 +20,7 @@
 #include <cstring>
 #include <deque>
 #include <memory>
+#include <mutex>
 #include <numeric>
 #include <random>
 #include <stdexcept>
@@ -130,6 +131,66 @@ void d2h(void* h, const void* d, size_t bytes)
 void sync() { HIPCHECK(hipStreamSynchronize(g_rt.stream)); }
 void check_launch() { HIPCHECK(hipGetLastError()); }
 
+// Pinned memory that kernels read and write (coherent: neither side caches it).
+template <class T>
+struct HostBuf {
+    T* p = nullptr;
+    void alloc(size_t count)
+    {
+        if (!p) HIPCHECK(hipHostMalloc((void**)&p, std::max<size_t>(count, 1) * sizeof(T), hipHostMallocCoherent));
+    }
+    ~HostBuf()
+    {
+        if (p) (void)hipHostFree(p);
+    }
+};
+
+// Rows of a device result into the caller's memory.  Kernels write pieces into
+// a small pinned ring, and the host copies a piece on while the next ones
+// arrive: the link and the host's copy overlap, and no result needs a device
+// buffer in its own order or a pinned one of its size.  One ring for the
+// process, its pieces written in stream order; the lock is held until the last
+// piece has been copied.  A gradient of 163842 vertices takes 250 us with 8 pieces
+// of 512 KB, 266 with 4, 283 and 304 with 8 and 4 of 256 KB (a wait per piece),
+// 299 with 2 of 2 MB (no overlap); one copy into pageable memory took 404.
+constexpr size_t kRingPiece = 512 << 10;
+constexpr int kRingPieces = 8;
+struct HostRing {
+    std::mutex lock;
+    HostBuf<char> buf;
+    hipEvent_t arrived[kRingPieces] = {};
+};
+HostRing& host_ring()
+{
+    static HostRing* ring = new HostRing;    // for the life of the process
+    return *ring;
+}
+// piece(p, first, n): enqueue the kernel that writes rows first .. first + n - 1 to p
+template <class F>
+void to_host(void* dst, size_t rows, size_t row_bytes, F&& piece)
+{
+    if (rows == 0) return;
+    HostRing& R = host_ring();
+    std::lock_guard<std::mutex> guard(R.lock);
+    R.buf.alloc(kRingPiece * kRingPieces);
+    for (hipEvent_t& e : R.arrived)
+        if (!e) HIPCHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    const size_t per = kRingPiece / row_bytes, pieces = (rows + per - 1) / per;
+    auto slot = [&](size_t k) { return R.buf.p + (k % kRingPieces) * kRingPiece; };
+    auto start = [&](size_t k) {
+        piece(slot(k), (int)(k * per), (int)std::min(per, rows - k * per));
+        check_launch();
+        if (pieces > 1) HIPCHECK(hipEventRecord(R.arrived[k % kRingPieces], g_rt.stream));
+    };
+    for (size_t k = 0; k < std::min<size_t>(pieces, kRingPieces); k++) start(k);
+    for (size_t k = 0; k < pieces; k++) {
+        if (pieces > 1) HIPCHECK(hipEventSynchronize(R.arrived[k % kRingPieces]));
+        else sync();
+        std::memcpy((char*)dst + k * per * row_bytes, slot(k), std::min(per, rows - k * per) * row_bytes);
+        if (k + kRingPieces < pieces) start(k + kRingPieces);
+    }
+}
+
 }    // namespace
 
 // --------------------------------------------------------------- mesh -----
@@ -160,8 +221,7 @@ struct tm_mesh {
     // per-vertex row that crosses the API is mapped back to user ids.
     std::vector<int> perm, iperm;
     DevBuf<int> d_perm, d_iperm;
-    DevBuf<int> faces;       // fv_indices after flips
-    DevBuf<double> stage;    // user-order rows for uploads and downloads
+    DevBuf<double> stage;    // user-order rows on their way into internal order
 
     MeshView view() const
     {
@@ -332,7 +392,6 @@ void ensure_device(tm_mesh& M)
     M.meta.alloc(M.nv);
     M.d_perm.alloc(M.nv);
     M.d_iperm.alloc(M.nv);
-    M.stage.alloc((size_t)M.nv * 6);
     h2d(M.d_perm.p, M.perm.data(), sizeof(int) * M.nv);
     h2d(M.d_iperm.p, M.iperm.data(), sizeof(int) * M.nv);
     M.flag.alloc(4);
@@ -369,13 +428,28 @@ void ensure_device(tm_mesh& M)
     M.dev = true;
 }
 
+// Below this many vertices a kernel reads the pinned positions itself, above it
+// the copy engine, which starts later and needs a kernel to reorder after it, is
+// ahead (49 GB/s over the link, the kernel 41): an upload takes 12.7 us by the
+// kernel and 14.7 by the engine at 642 vertices, 34.9 and 37.5 at 40962, 58.1 and
+// 54.8 at 81002, 105 and 91 at 163842.
+constexpr int kTakeVerts = 65536;
+
+// three doubles per vertex from host memory, in internal order
+void upload_rows(tm_mesh& M, const double* host, double* dst)
+{
+    M.stage.alloc((size_t)3 * M.nv);
+    h2d(M.stage.p, host, sizeof(double) * 3 * M.nv);
+    launch_gather_rows(M.stage.p, M.d_perm.p, dst, M.nv, 3, g_rt.stream);
+}
+
 void push_points(tm_mesh& M)
 {
     ensure_device(M);
     M.device_ahead = false;
     if (M.nv == 0) return;
-    h2d(M.stage.p, M.points, sizeof(double) * 3 * M.nv);
-    launch_gather_rows(M.stage.p, M.d_perm.p, M.x.p, M.nv, 3, g_rt.stream);
+    if (M.pinned && M.nv < kTakeVerts) launch_take_points(M.points, M.d_iperm.p, M.x.p, M.nv, g_rt.stream);
+    else upload_rows(M, M.points, M.x.p);
     check_launch();
 }
 
@@ -389,20 +463,24 @@ void upload_points(tm_mesh& M)
     if (!M.device_ahead) push_points(M);
 }
 
-// rows of an internal-order device array -> user order in the stage buffer
-// -> host
+// rows of an internal-order device array -> user order on the host, there when
+// this returns
 void download_rows(tm_mesh& M, const double* d_src, int width, double* host)
 {
-    if (M.nv == 0) return;
-    launch_gather_rows(d_src, M.d_iperm.p, M.stage.p, M.nv, width, g_rt.stream);
-    check_launch();
-    d2h(host, M.stage.p, sizeof(double) * width * M.nv);
+    to_host(host, M.nv, sizeof(double) * width, [&](void* p, int first, int n) {
+        launch_give_rows(d_src, M.d_iperm.p, (double*)p, first, n, width, g_rt.stream);
+    });
 }
 
 void pull_points(tm_mesh& M)
 {
-    download_rows(M, M.x.p, 3, M.points);
-    sync();
+    if (M.pinned) {
+        launch_give_rows(M.x.p, M.d_iperm.p, M.points, 0, M.nv, 3, g_rt.stream);
+        check_launch();
+        sync();
+    } else {
+        download_rows(M, M.x.p, 3, M.points);
+    }
     M.device_ahead = false;
 }
 
@@ -646,6 +724,7 @@ struct tm_energy {
     DevBuf<unsigned> pass_count;
     DevBuf<double> theta;    // pass 1's dihedral angles for pass 2 (kRingPad per vertex, float or double)
     DevBuf<Globals> globals;
+    HostBuf<Globals> host_globals;    // written by the passes whose sums the host waits for
     DevBuf<int> flip_result, proposals, pf_rec, pf_lost;
     DevBuf<double> uniforms, pf_state;
     DevBuf<unsigned> pf_count;
@@ -707,6 +786,7 @@ void ensure_energy_buffers(tm_energy& E, const tm_mesh& M)
     E.grad.alloc((size_t)M.nv * 3);
     E.theta.alloc((size_t)kRingPad * M.nv);
     E.globals.alloc(1);
+    E.host_globals.alloc(1);
     alloc_pass_count(E.pass_count);
     E.flip_result.alloc(4);
 }
@@ -773,16 +853,19 @@ PassBuffers buffers(tm_energy& E, tm_mesh& M)
     return b;
 }
 
-void run_pass1(tm_energy& E, tm_mesh& M, int mixed, double* vprops)
+// to_host: the sums also go to E.host_globals (read_globals)
+void run_pass1(tm_energy& E, tm_mesh& M, int mixed, double* vprops, bool to_host = false)
 {
     ensure_energy_buffers(E, M);
     if (E.nlist->nv != M.nv) throw TmError(TM_E_INVALID, "mesh does not match the energy manager");
     if (M.nv == 0) {
         HIPCHECK(hipMemsetAsync(E.globals.p, 0, sizeof(Globals), g_rt.stream));
+        if (to_host) *E.host_globals.p = Globals{};
         return;
     }
     ensure_masks(*E.nlist, M);
-    const PassBuffers b = buffers(E, M);
+    PassBuffers b = buffers(E, M);
+    if (to_host) b.host = E.host_globals.p;
     hipEvent_t marks[2] = {g_rt.pass1_marks[0], g_rt.pass1_marks[1]};
     g_rt.pass1_marks[0] = g_rt.pass1_marks[1] = nullptr;
     launch_pass1(M.view(), E.nlist->view(), eparams_of(E), mixed, b, vprops, g_rt.stream, E.tune, marks);
@@ -798,12 +881,11 @@ void run_pass2(tm_energy& E, tm_mesh& M, int mixed)
     check_launch();
 }
 
+// the sums of a pass that was told to hand them over
 Globals read_globals(tm_energy& E)
 {
-    Globals g;
-    d2h(&g, E.globals.p, sizeof(Globals));
     sync();
-    return g;
+    return *E.host_globals.p;
 }
 
 tm_props props_of(const Globals& g)
@@ -869,7 +951,7 @@ int tm_mesh_create(const double* points, int n_points, const int* faces, int n_f
     // memory otherwise so that meshes can be built on a host without a GPU
     int ndev = 0;
     if (hipGetDeviceCount(&ndev) == hipSuccess && ndev > 0 &&
-        hipHostMalloc((void**)&M->points, bytes, hipHostMallocDefault) == hipSuccess) {
+        hipHostMalloc((void**)&M->points, bytes, hipHostMallocCoherent) == hipSuccess) {
         M->pinned = true;
     } else {
         (void)hipGetLastError();
@@ -906,11 +988,9 @@ int tm_mesh_fv_indices(tm_mesh* mesh, int* out)
     if (mesh->host_stale) {
         // flips have changed the device topology: the faces from there, instead
         // of all six halfedge arrays and a walk over them here
-        mesh->faces.alloc((size_t)3 * mesh->nf);
-        launch_faces(mesh->view(), mesh->d_perm.p, mesh->faces.p, g_rt.stream);
-        check_launch();
-        d2h(out, mesh->faces.p, sizeof(int) * 3 * mesh->nf);
-        sync();
+        to_host(out, mesh->nf, 3 * sizeof(int), [&](void* p, int first, int n) {
+            launch_faces(mesh->view(), mesh->d_perm.p, (int*)p, first, n, g_rt.stream);
+        });
         return TM_OK;
     }
     for (int f = 0; f < mesh->nf; f++) {
@@ -1057,7 +1137,7 @@ int tm_energy_create(tm_mesh* mesh, const tm_params* params, tm_energy** out)
     // initial_props = properties(mesh) (energy.cpp:27); reference values
     // are not needed for the sums, unit placeholders keep the factors finite
     E->initial = tm_props{1, 1, 1, 0, 0, 0};
-    run_pass1(*E, *mesh, 0, nullptr);
+    run_pass1(*E, *mesh, 0, nullptr, true);
     E->initial = props_of(read_globals(*E));
     *out = E.release();
     API_END
@@ -1100,7 +1180,7 @@ int tm_energy_properties(tm_energy* em, tm_mesh* mesh, tm_props* out)
 {
     API_BEGIN
     upload_points(*mesh);
-    run_pass1(*em, *mesh, em->precision, nullptr);
+    run_pass1(*em, *mesh, em->precision, nullptr, true);
     *out = props_of(read_globals(*em));
     API_END
 }
@@ -1112,7 +1192,6 @@ int tm_energy_vertex_properties(tm_energy* em, tm_mesh* mesh, double* out)
     em->vprops.alloc((size_t)mesh->nv * 6);
     run_pass1(*em, *mesh, em->precision, em->vprops.p);
     download_rows(*mesh, em->vprops.p, 6, out);
-    sync();
     API_END
 }
 
@@ -1120,7 +1199,7 @@ int tm_energy_energy(tm_energy* em, tm_mesh* mesh, double* out)
 {
     API_BEGIN
     upload_points(*mesh);
-    run_pass1(*em, *mesh, em->precision, nullptr);
+    run_pass1(*em, *mesh, em->precision, nullptr, true);
     *out = read_globals(*em).energy;
     API_END
 }
@@ -1138,7 +1217,6 @@ int tm_energy_gradient(tm_energy* em, tm_mesh* mesh, double* out)
     run_pass1(*em, *mesh, em->precision, nullptr);
     run_pass2(*em, *mesh, em->precision);
     download_rows(*mesh, em->grad.p, 3, out);
-    sync();
     API_END
 }
 
@@ -1146,13 +1224,10 @@ int tm_energy_energy_gradient(tm_energy* em, tm_mesh* mesh, double* energy, doub
 {
     API_BEGIN
     upload_points(*mesh);
-    run_pass1(*em, *mesh, em->precision, nullptr);
+    run_pass1(*em, *mesh, em->precision, nullptr, true);
     run_pass2(*em, *mesh, em->precision);
-    Globals g;
-    d2h(&g, em->globals.p, sizeof(Globals));
     download_rows(*mesh, em->grad.p, 3, grad);
-    sync();
-    *energy = g.energy;
+    *energy = read_globals(*em).energy;
     API_END
 }
 
@@ -1497,8 +1572,7 @@ int tm_hmc_step(tm_hmc* hmc, const tm_hmc_params* prm, double temperature, const
     const int L = prm->num_integration_steps;
     const int harmonic = hmc->model == TM_HMC_HARMONIC;
     if (momenta && M.nv > 0) {
-        h2d(M.stage.p, momenta, sizeof(double) * n3);
-        launch_gather_rows(M.stage.p, M.d_perm.p, hmc->p.p, M.nv, 3, g_rt.stream);
+        upload_rows(M, momenta, hmc->p.p);
         check_launch();
         sync();    // the caller's array may be reused on return
     }
@@ -1890,7 +1964,6 @@ int tm_replicas_gradient(tm_replicas* rs, int r, double* out)
     API_BEGIN
     require(r >= 0 && r < rs->R, "replica index out of range");
     download_rows(*rs->meshes[r], rs->ems[r]->grad.p, 3, out);
-    sync();
     API_END
 }
 
@@ -2536,7 +2609,6 @@ int tm_surrogate_forces(tm_surrogate* sg, double* forces)
     if (forces) {
         std::vector<double> g((size_t)3 * S.nv);
         download_rows(*S.mesh, S.neg_force.p, 3, g.data());
-        sync();
         for (size_t i = 0; i < g.size(); i++) forces[i] = -g[i];
     }
     API_END
@@ -2670,8 +2742,7 @@ int tm_hmc_step_surrogate(tm_hmc* hmc, tm_surrogate* sg, const tm_hmc_params* pr
     const double dt2 = prm->time_step_sq != 0.0 ? prm->time_step_sq : dt * dt;
     const int L = prm->num_integration_steps;
     if (momenta) {
-        h2d(M.stage.p, momenta, sizeof(double) * n3);
-        launch_gather_rows(M.stage.p, M.d_perm.p, hmc->p.p, M.nv, 3, g_rt.stream);
+        upload_rows(M, momenta, hmc->p.p);
         check_launch();
         sync();
     }

@@ -244,7 +244,9 @@ __device__ __forceinline__ void finalize_tail(const PassArgs& A)
     }
     __syncthreads();
     if (threadIdx.x == 0) {
-        *A.globals = globals_of_sums(s_sum, A.p);
+        const Globals g = globals_of_sums(s_sum, A.p);
+        *A.globals = g;
+        if (A.host) *A.host = g;
         if (A.pc.dforce) *A.pc.dforce = 0;    // replica groups: the query of this evaluation recorded
     }
 }
@@ -1591,6 +1593,7 @@ PassArgs pass_args(const MeshView& m, const NListView& nl, const EParams& p, con
     a.rep_g = b.rep_g;
     a.partials = b.partials;
     a.globals = b.globals;
+    a.host = b.host;
     a.grad = grad;
     a.vprops = vprops;
     a.list = b.list;

@@ -51,6 +51,7 @@ struct PassBuffers {
     double* partials;   // [6 * pass1 blocks]
     unsigned* count;    // [kLastCounters] zeros (tm_last.h)
     Globals* globals;
+    Globals* host;      // pinned copy of globals the pass also writes; null: none
     const int* list;    // boundary / degenerate vertices
     int nlist;
     PairCache pc;       // x_snap null: the query runs in full every time
@@ -86,6 +87,7 @@ struct PassArgs {
     unsigned* count;
     int tail;            // the pass's last workgroup sums the partials (see kTailBlocks)
     Globals* globals;
+    Globals* host;       // PassBuffers::host
     double* grad;
     double* vprops;      // optional per-vertex properties of pass 1
     void* theta;         // PassBuffers::theta
@@ -156,8 +158,13 @@ void launch_sum_geometry(const MeshView& m, int what, double* partials, unsigned
 void launch_gather_rows(const double* src, const int* idx, double* dst, int n, int w, hipStream_t s);
 
 // topology helpers (tm_flips.hip)
-// out[3 nf]: the faces' vertices as user ids (perm: internal -> user)
-void launch_faces(const MeshView& m, const int* perm, int* out, hipStream_t s);
+// out[3 n]: the vertices of faces first .. first + n - 1 as user ids (perm:
+// internal -> user)
+void launch_faces(const MeshView& m, const int* perm, int* out, int first, int n, hipStream_t s);
+// x[at[i]] = host[i] (n rows of 3) and host[i] = src[idx[first + i]] (n rows of
+// w); host: pinned, 16-byte aligned
+void launch_take_points(const double* host, const int* at, double* x, int n, hipStream_t s);
+void launch_give_rows(const double* src, const int* idx, double* host, int first, int n, int w, hipStream_t s);
 // Rebuild ring table and meta from the halfedge arrays; sets *overflow to 1
 // if a vertex has more than kMaxValence neighbours.
 void launch_build_ring(const MeshView& m, int* ring, int* meta, int* overflow, hipStream_t s);
