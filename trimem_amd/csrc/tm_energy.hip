@@ -476,15 +476,24 @@ __device__ __forceinline__ void store_rep_g(const PassArgs& A, int v, const RepT
 }
 
 // ------------------------------------------------------------ pair cache ---
-// (PairCache in tm_internal.h.)  Cell of v at position pi, or -1 outside the
-// grid.
+// (PairCache in tm_internal.h.)  The cell of position pi, as an id that no other
+// cell has: the flat id inside the grid, -2 and below outside it, where a
+// sphere's outermost vertices move and their stencils still reach into the
+// grid.  (-1, no replay, only where the ids would not fit.)  While those
+// vertices had no cell and took the full query on every evaluation, the launch
+// waited for them: an evaluation of a sphere moved by 0.5% of an edge since the
+// list was built took 31.8 us at 642 vertices, now 27.6; 36.5 and 32.7 at 40962,
+// 51.2 and 45.6 at 163842.
 __device__ __forceinline__ int query_cell(const NListView& nl, d3 pi)
 {
     int c[3];
     cell_coords(nl, pi, c);
     const bool inside = c[0] >= 0 && c[0] < nl.shape[0] && c[1] >= 0 && c[1] < nl.shape[1] && c[2] >= 0 &&
                         c[2] < nl.shape[2];
-    return inside ? c[0] * nl.strides[0] + c[1] * nl.strides[1] + c[2] * nl.strides[2] : -1;
+    if (inside) return c[0] * nl.strides[0] + c[1] * nl.strides[1] + c[2] * nl.strides[2];
+    const long long w0 = nl.shape[0] + 4, w1 = nl.shape[1] + 4;    // cell_coords: -2 .. shape + 1
+    const long long id = c[0] + 2 + w0 * (c[1] + 2 + w1 * (c[2] + 2));
+    return id < 0x7fffff00ll ? -2 - (int)id : -1;
 }
 
 // Block-uniform: 2 to record (forced, or some vertex has moved skin / 2 or
@@ -541,35 +550,6 @@ __device__ __forceinline__ void record_neighbours(const MeshView& m, const NList
         pc.cnt[v] = (unsigned)word;
         pc.cell[v] = over == 0 ? cell : -1;
     }
-}
-
-// Replay of the recorded lists (false, and nothing visited, if v is not in
-// the cell they were recorded in).
-template <class F>
-__device__ __forceinline__ bool cached_neighbours(const MeshView& m, const NListView& nl, const PairCache& pc, int v,
-                                                  d3 pi, double dmax, int lane, F&& f)
-{
-    const int cell = pc.cell[v];
-    const unsigned word = pc.cnt[v];
-    if (cell < 0 || query_cell(nl, pi) != cell) return false;
-    const int k = (int)((word >> (4 * lane)) & 15u);
-    const int* e = pc.ent + ((size_t)v * kGroup + lane) * kPairCap;
-    int j[kPairCap];
-#pragma unroll
-    for (int i = 0; i < kPairCap; i++) j[i] = i < k ? e[i] : -1;
-    d3 pj[kPairCap];
-#pragma unroll
-    for (int i = 0; i < kPairCap; i++)
-        if (j[i] >= 0) pj[i] = load_p(m.x, j[i]);
-    const double dmax2 = dmax * dmax * (1.0 + 1e-15);
-#pragma unroll
-    for (int i = 0; i < kPairCap; i++) {
-        if (j[i] < 0) continue;
-        const d3 d = pi - pj[i];
-        const double sq = sqnorm(d);
-        if (sq <= dmax2 && sqrt(sq) < dmax) f(j[i], d);
-    }
-    return true;
 }
 
 // Exclusion masks of the stored stencil lists: bit i of vertex v is set if
@@ -1117,7 +1097,7 @@ __device__ __forceinline__ void rep_cached_body(const PassArgs& A, int lb)
     // this thread's vertex data, in flight while the mode is decided
     const int meta = mine ? m.meta[v] : 0;
     const d3 xv = mine ? load_p(m.x, v) : d3{0.0, 0.0, 0.0};
-    const int rec_cell = mine && pc.x_snap ? pc.cell[v] : -1;
+    const int rec_cell = mine && pc.x_snap ? pc.cell[v] : -1;    // -1: none
     const unsigned rec_word = mine && pc.x_snap ? pc.cnt[v] : 0u;
     const int mode = pc.x_snap ? pair_cache_mode(pc) : 0;    // block-uniform: 1 replay, 2 record, 0 full
     __shared__ int s_list[kVertsPerBlock];
@@ -1144,7 +1124,7 @@ __device__ __forceinline__ void rep_cached_body(const PassArgs& A, int lb)
         } else if (ring && mode == 1) {
             const int cell = rec_cell;
             const unsigned word = rec_word;
-            const bool replay = cell >= 0 && query_cell(A.nl, xv) == cell;
+            const bool replay = cell != -1 && query_cell(A.nl, xv) == cell;
             if (replay && word == 0u) {
                 done = true;    // nothing recorded: no pairs (the sums below would all be +0)
             } else if (replay) {

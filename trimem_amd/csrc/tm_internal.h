@@ -28,7 +28,7 @@ constexpr double kPairSkin = 0.2;  // skin = 0.2 lc1
 constexpr double kPairLimit = 0.25;
 struct PairCache {
     double* x_snap;         // [3N] positions at the recording; null: no cache
-    int* cell;              // [N] cell id at the recording, -1: replay not allowed
+    int* cell;              // [N] cell (query_cell) at the recording, -1: replay not allowed
     unsigned* cnt;          // [N] recorded candidates of each lane, 4 bits per lane
     int* ent;               // [8 kPairCap N] ids, lane-major per vertex
     double* disp_part;      // [disp_n] max |x - x_snap|^2 per pass-1 block (written by pass 1)
