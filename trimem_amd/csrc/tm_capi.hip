@@ -513,6 +513,7 @@ struct tm_nlist {
     // pair cache of the query (PairCache): recorded lists, valid for this
     // list and topology once a recording launch has been queued
     DevBuf<double> pc_x, pc_disp;
+    DevBuf<int> pc_fast;
     DevBuf<int> pc_cell, pc_ent;
     DevBuf<unsigned> pc_cnt;
     bool pc_ok = false;
@@ -681,6 +682,7 @@ void build_nlist(tm_nlist& L, tm_mesh& M)
         L.pc_ent.alloc((size_t)kPairLanes * kPairCap * n);
         const int nd = pass1_blocks(n);    // one displacement partial per pass-1 block
         L.pc_disp.alloc(nd);
+        L.pc_fast.alloc((size_t)kFastRow * nd);
         // cell -1: no replay; displacement bytes 0x7F (~1e306): a recording first
         launch_fill_ints(L.pc_cell.p, n, -1, reinterpret_cast<int*>(L.pc_disp.p), 2 * nd, 0x7F7F7F7F,
                          nullptr, 0, 0, g_rt.stream);
@@ -846,6 +848,7 @@ PassBuffers buffers(tm_energy& E, tm_mesh& M)
         b.pc = pair_cache_of(E, M);
         if (b.pc.x_snap) {
             b.pc.disp_part = L.pc_disp.p;
+            b.pc.fast = L.pc_fast.p;
             b.pc.disp_n = pass1_blocks(M.nv);
             b.pc.force = L.pc_ok ? 0 : 1;
         }
@@ -1652,6 +1655,7 @@ struct tm_replicas {
     // displacement check and of the cached query
     DevBuf<int> force_flags, d_block0_rc;
     DevBuf<double> disp_parts;
+    DevBuf<int> fast_parts;
     // parallel flip sweeps of the group: per-replica arguments and block
     // prefix tables (rebuilt by every sweep)
     DevBuf<PflipArgs> pf_args;
@@ -1728,6 +1732,7 @@ void refresh_replica_args(tm_replicas& S)
     S.total_rc = (b0c[S.R] + 7) / 8 * 8;    // a multiple of the 8 XCDs; padding blocks fall past the last replica's vertices
     S.d_block0_rc.alloc(S.R + 1);
     S.disp_parts.alloc(S.total_disp);
+    S.fast_parts.alloc((size_t)kFastRow * S.total_disp);
     S.force_flags.alloc(S.R);
     S.h_ones.assign(S.R, 1);
     for (int r = 0; r < S.R; r++) {
@@ -1742,6 +1747,7 @@ void refresh_replica_args(tm_replicas& S)
         b.pc = pair_cache_of(E, M);
         if (b.pc.x_snap) {
             b.pc.disp_part = S.disp_parts.p + b0d[r];
+            b.pc.fast = S.fast_parts.p + (size_t)kFastRow * b0d[r];
             b.pc.disp_n = b0d[r + 1] - b0d[r];
             b.pc.dforce = S.force_flags.p + r;
         }

@@ -496,18 +496,29 @@ __device__ __forceinline__ int query_cell(const NListView& nl, d3 pi)
     return id < 0x7fffff00ll ? -2 - (int)id : -1;
 }
 
-// Block-uniform: 2 to record (forced, or some vertex has moved skin / 2 or
-// more since the recording), 1 to replay.  Contains a barrier.
-__device__ __forceinline__ int pair_cache_mode(const PairCache& pc)
+// Build-time cells of the fast vertices, in LDS.
+struct FastCells {
+    int n;
+    int c[kFastMax][3];
+};
+
+// Block-uniform: 2 to record (forced, or too many vertices are fast), 1 to
+// replay; F then holds the fast vertices' cells.  Contains a barrier.
+__device__ __forceinline__ int pair_cache_mode(const PairCache& pc, const NListView& nl, FastCells& F)
 {
-    if (pc.force || (pc.dforce && *pc.dforce)) return 2;
     __shared__ int s_mode;
+    if (threadIdx.x == 0) F.n = 0;
+    if (pc.force || (pc.dforce && *pc.dforce)) {
+        __syncthreads();
+        return 2;
+    }
     if (threadIdx.x < 64) {
+        __builtin_amdgcn_wave_barrier();
         // one partial per pass-1 block: each lane has a batch of loads in
         // flight before it takes their maximum, instead of one round trip
         // per partial
         constexpr int kBatchLoads = 16;
-        double mx = 0.0;
+        bool over = false;
         for (int i0 = threadIdx.x; i0 < pc.disp_n; i0 += 64 * kBatchLoads) {
             double d[kBatchLoads];
 #pragma unroll
@@ -515,12 +526,29 @@ __device__ __forceinline__ int pair_cache_mode(const PairCache& pc)
                 const int i = i0 + 64 * u;
                 d[u] = i < pc.disp_n ? pc.disp_part[i] : 0.0;
             }
+            unsigned hit = 0;
 #pragma unroll
-            for (int u = 0; u < kBatchLoads; u++) mx = fmax(mx, d[u]);
+            for (int u = 0; u < kBatchLoads; u++) hit |= (d[u] < pc.limit2 ? 0u : 1u) << u;
+            while (hit) {
+                const int i = i0 + 64 * (__ffs(hit) - 1);
+                hit &= hit - 1u;
+                const int* f = pc.fast + (size_t)kFastRow * i;
+                const int n = f[0];
+                const int at = n > kFastSeg ? kFastMax : atomicAdd(&F.n, n);
+                if (at + n > kFastMax) {
+                    over = true;
+                    break;
+                }
+                for (int k = 0; k < n; k++) {
+                    const int id = f[1 + k], r = id % nl.strides[2];
+                    F.c[at + k][0] = r % nl.strides[1];
+                    F.c[at + k][1] = r / nl.strides[1];
+                    F.c[at + k][2] = id / nl.strides[2];
+                }
+            }
         }
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) mx = fmax(mx, __shfl_xor(mx, off, 64));
-        if (threadIdx.x == 0) s_mode = mx < pc.limit2 ? 1 : 2;
+        over = __any(over);
+        if (threadIdx.x == 0) s_mode = over ? 2 : 1;
     }
     __syncthreads();
     return s_mode;
@@ -773,8 +801,8 @@ __device__ __forceinline__ bool is_generic(int meta)
 // (kApart) the cached query runs after this kernel and sums column 5 of
 // the same 256-vertex blocks itself, in the same order; this kernel then
 // measures how far every vertex has moved since the cache's recording (the
-// largest squared displacement of the block, NaN counting as infinite), the
-// query's replay condition.  kFinal: nothing of the pass follows, and the last
+// largest squared displacement of the block, NaN counting as infinite) and
+// lists the cells of the fast ones, the query's replay condition.  kFinal: nothing of the pass follows, and the last
 // workgroup sums the partials (finalize_tail).
 template <class T, bool kApart = false, bool kFinal = !kApart>
 __device__ __forceinline__ void pass1_body(const PassArgs& A, int lb)
@@ -787,13 +815,14 @@ __device__ __forceinline__ void pass1_body(const PassArgs& A, int lb)
     const int vc = active ? v : m.nv - 1;    // lanes past the last vertex load a valid one
     const int meta = m.meta[vc];
     const double rv = (!kApart && A.rep_v && active) ? A.rep_v[v] : 0.0;
-    double disp = 0.0;
+    double disp = 0.0, own = 0.0;
     if (kApart && A.pc.x_snap && active) {
         const double* xs = A.pc.x_snap;
         const double dx = m.x[3 * v] - xs[3 * v], dy = m.x[3 * v + 1] - xs[3 * v + 1];
         const double dz = m.x[3 * v + 2] - xs[3 * v + 2];
         disp = dx * dx + dy * dy + dz * dz;
         if (!(disp == disp)) disp = INFINITY;
+        own = disp;
     }
     const int n = meta_valence(meta);
     const bool ring = active && !is_generic(meta);
@@ -844,8 +873,22 @@ __device__ __forceinline__ void pass1_body(const PassArgs& A, int lb)
         for (int w = 0; w < kWaves; w++) a += s_red[w * 6 + threadIdx.x];
         put(A.partials + (size_t)threadIdx.x * A.nblocks + lb, a);
     }
-    if (kApart && A.pc.x_snap && threadIdx.x == 63)
-        A.pc.disp_part[lb] = fmax(fmax(s_disp[0], s_disp[1]), fmax(s_disp[2], s_disp[3]));
+    if (kApart && A.pc.x_snap) {
+        const double mx = fmax(fmax(s_disp[0], s_disp[1]), fmax(s_disp[2], s_disp[3]));
+        if (threadIdx.x == 63) A.pc.disp_part[lb] = mx;
+        if (!(mx < A.pc.limit2)) {
+            __shared__ int s_fast;
+            if (threadIdx.x == 0) s_fast = 0;
+            __syncthreads();
+            int* row = A.pc.fast + (size_t)kFastRow * lb;
+            if (active && !(own < A.pc.limit2)) {
+                const int i = atomicAdd(&s_fast, 1);
+                if (i < kFastSeg) row[1 + i] = A.nl.vert_cell[v];
+            }
+            __syncthreads();
+            if (threadIdx.x == 0) row[0] = s_fast;
+        }
+    }
     if constexpr (kFinal)
         if (A.tail && last_block_of_many(A.count, lb, A.nblocks)) finalize_tail(A);
 }
@@ -946,6 +989,7 @@ __global__ void __launch_bounds__(kThreads) k_rep(PassArgs A)
 // Without cache buffers (a replica with a Verlet list in a cached group
 // launch) every ring vertex takes phase 2 without recording (mode 0).
 constexpr int kVertsPerBlock = kCachedVerts;
+constexpr int kWaveVerts = 16;
 
 // record_neighbours by one 64-lane wave instead of an 8-lane group, with
 // the same result bits.  The candidates are laid out as group_neighbours
@@ -959,7 +1003,7 @@ constexpr int kVertsPerBlock = kCachedVerts;
 // which records and adds it as RepTerms::add would.  Lanes 0-7 end with the
 // group's lane state; the caller reduces them with group_sum.
 __device__ __forceinline__ void wide_record(const MeshView& m, const NListView& nl, const PairCache& pc,
-                                            const EParams& p, int u, int n, d3 pu, RepTerms& tr)
+                                            const EParams& p, int u, int n, d3 pu, bool keep, RepTerms& tr)
 {
     const int L = threadIdx.x & 63;
     int rs[9], rl[9];
@@ -1016,7 +1060,7 @@ __device__ __forceinline__ void wide_record(const MeshView& m, const NListView& 
 #pragma unroll
     for (int k = 0; k < 9; k++) total += rl[k];
     const RingRegs R = load_ring(m, u, n);
-    const double dsk = p.rep_lc1 + pc.skin, dsk2 = dsk * dsk * (1.0 + 1e-15);
+    const double dsk = keep ? p.rep_lc1 + pc.skin : p.rep_lc1, dsk2 = dsk * dsk * (1.0 + 1e-15);
     const double dmax = p.rep_lc1, dmax2 = dmax * dmax * (1.0 + 1e-15);
     int* ent = pc.ent + ((size_t)u * kGroup + (L & 7)) * kPairCap;
     int rec = 0;
@@ -1061,7 +1105,7 @@ __device__ __forceinline__ void wide_record(const MeshView& m, const NListView& 
             const double fv = __shfl(val, src);
             const double gx = __shfl(gv.x, src), gy = __shfl(gv.y, src), gz = __shfl(gv.z, src);
             if (L == fo) {
-                if (rec < kPairCap) ent[rec] = fj;
+                if (keep && rec < kPairCap) ent[rec] = fj;
                 rec++;
                 if (ff & 2) {
                     tr.rep += fv;
@@ -1071,6 +1115,7 @@ __device__ __forceinline__ void wide_record(const MeshView& m, const NListView& 
             }
         }
     }
+    if (!keep) return;
     const int over = group_sum(rec > kPairCap ? 1 : 0);
     const int word = group_sum(min(rec, kPairCap) << (4 * (L & 7)));
     const int cell = query_cell(nl, pu);
@@ -1099,21 +1144,18 @@ __device__ __forceinline__ void rep_cached_body(const PassArgs& A, int lb)
     const d3 xv = mine ? load_p(m.x, v) : d3{0.0, 0.0, 0.0};
     const int rec_cell = mine && pc.x_snap ? pc.cell[v] : -1;    // -1: none
     const unsigned rec_word = mine && pc.x_snap ? pc.cnt[v] : 0u;
-    const int mode = pc.x_snap ? pair_cache_mode(pc) : 0;    // block-uniform: 1 replay, 2 record, 0 full
+    __shared__ FastCells s_fast;
+    const int mode = pc.x_snap ? pair_cache_mode(pc, A.nl, s_fast) : 0;    // block-uniform: 1 replay, 2 record, 0 full
     __shared__ int s_list[kVertsPerBlock];
     __shared__ double s_val[kVertsPerBlock];    // repulsion property per vertex (column 5 of pass 1)
     __shared__ int s_n;
-    __shared__ int s_rest[kVertsPerBlock];
-    __shared__ int s_nrest;
-    if (threadIdx.x == 0) {
-        s_n = 0;
-        s_nrest = 0;
-    }
+    if (threadIdx.x == 0) s_n = 0;
     __syncthreads();
     if (threadIdx.x < kVertsPerBlock) s_val[threadIdx.x] = 0.0;
     if (mine) {
         const bool ring = !is_generic(meta);
         bool done = !ring;
+        bool keep = true;    // its list may be replayed, or recorded
         double rep = 0.0;
         int cnt = 0;
         if (mode == 2) {
@@ -1122,9 +1164,20 @@ __device__ __forceinline__ void rep_cached_body(const PassArgs& A, int lb)
             pc.x_snap[3 * v + 2] = xv.z;
             if (!ring) pc.cell[v] = -1;
         } else if (ring && mode == 1) {
+            if (s_fast.n > 0) {
+                const double dx = xv.x - pc.x_snap[3 * v], dy = xv.y - pc.x_snap[3 * v + 1];
+                const double dz = xv.z - pc.x_snap[3 * v + 2];
+                keep = dx * dx + dy * dy + dz * dz < pc.limit2;
+                int c[3];
+                cell_coords(A.nl, xv, c);
+                for (int i = 0; i < s_fast.n; i++)
+                    if (abs(c[0] - s_fast.c[i][0]) <= 1 && abs(c[1] - s_fast.c[i][1]) <= 1 &&
+                        abs(c[2] - s_fast.c[i][2]) <= 1)
+                        keep = false;
+            }
             const int cell = rec_cell;
             const unsigned word = rec_word;
-            const bool replay = cell != -1 && query_cell(A.nl, xv) == cell;
+            const bool replay = keep && cell != -1 && query_cell(A.nl, xv) == cell;
             if (replay && word == 0u) {
                 done = true;    // nothing recorded: no pairs (the sums below would all be +0)
             } else if (replay) {
@@ -1164,48 +1217,38 @@ __device__ __forceinline__ void rep_cached_body(const PassArgs& A, int lb)
             A.pair_cnt[v] = cnt;
             s_val[threadIdx.x] = ring ? rep : A.gprops[6 * v + 5];
         } else {
-            s_list[atomicAdd(&s_n, 1)] = v;
+            s_list[atomicAdd(&s_n, 1)] = keep ? v : ~v;
         }
     }
     __syncthreads();
-    int n_full = s_n;
-    const int* list = s_list;
-    if (mode == 1 && n_full > 0) {
-        // a replay launch leaves few vertices per block to the full query,
-        // so its latency counts: each takes a whole wave (wide_record)
-        const int wv = threadIdx.x / 64;
-        for (int i = wv; i < n_full; i += 256 / 64) {
-            const int u = s_list[i];
-            const d3 xu = load_p(m.x, u);
-            if (A.nl.kind == 0) {
-                RepTerms tr;
-                wide_record(m, A.nl, pc, p, u, meta_valence(m.meta[u]), xu, tr);
-                tr.group_reduce();
-                if ((threadIdx.x & 63) == 0) {
-                    A.rep_v[u] = tr.rep;
-                    A.pair_cnt[u] = tr.cnt;
-                    s_val[u - base] = tr.rep;
-                    store_rep_g(A, u, tr);
-                }
-            } else if ((threadIdx.x & 63) == 0) {
-                s_rest[atomicAdd(&s_nrest, 1)] = u;
-            }
+    const int n_full = s_n;
+    // a replay launch leaves few vertices per block to the full query, so its
+    // latency counts: up to kWaveVerts take a whole wave each (wide_record)
+    const bool waves = mode == 1 && n_full <= kWaveVerts;
+    for (int i = threadIdx.x / 64; waves && i < n_full; i += 256 / 64) {
+        const int e = s_list[i], u = e < 0 ? ~e : e;
+        RepTerms tr;
+        wide_record(m, A.nl, pc, p, u, meta_valence(m.meta[u]), load_p(m.x, u), e >= 0, tr);
+        tr.group_reduce();
+        if ((threadIdx.x & 63) == 0) {
+            A.rep_v[u] = tr.rep;
+            A.pair_cnt[u] = tr.cnt;
+            s_val[u - base] = tr.rep;
+            store_rep_g(A, u, tr);
         }
-        __syncthreads();
-        n_full = s_nrest;
-        list = s_rest;
     }
     const int g = threadIdx.x / kGroup, lane = threadIdx.x % kGroup;
-    for (int i = g; i < n_full; i += 256 / kGroup) {
-        const int u = list[i];
+    for (int i = g; !waves && i < n_full; i += 256 / kGroup) {
+        const int e = s_list[i], u = e < 0 ? ~e : e;
         const d3 xu = load_p(m.x, u);
         const int n = meta_valence(m.meta[u]);
         RepTerms tr;
         auto add = [&](int, d3 d) { tr.add(d, p); };
         // a replay launch records the lists of the vertices that left
         // their recorded cell (in the cell they are in now), so each pays
-        // the full query once per cell it enters
-        if (mode != 0) record_neighbours<kBatch>(m, A.nl, pc, u, n, xu, p.rep_lc1, lane, add);
+        // the full query once per cell it enters; a vertex that is fast or has
+        // a fast candidate records nothing
+        if (mode != 0 && e >= 0) record_neighbours<kBatch>(m, A.nl, pc, u, n, xu, p.rep_lc1, lane, add);
         else group_neighbours<kBatch>(m, A.nl, u, n, xu, p.rep_lc1, lane, add);
         tr.group_reduce();
         if (lane == 0) {

@@ -11,31 +11,36 @@ namespace tmh {
 // to), and exclusion depends on the topology only.  A recording launch runs
 // the full query with radius lc1 + skin and keeps, per vertex and lane, the
 // non-excluded candidates it meets, in the lane's visit order; later
-// launches replay those lists with the exact lc1 test while every vertex has
-// moved less than skin / 2 since the recording (no other candidate can have
-// come within lc1) and the vertex is in the cell it was recorded in (the
-// full query would visit the same candidates in the same order).  Each lane
-// then adds the same terms in the same order as the full query: the results
-// are bit-identical.
+// launches replay a list with the exact lc1 test while neither the vertex nor
+// one of its candidates has moved so far that another candidate can have come
+// within lc1, and the vertex is in the cell it was recorded in (the full query
+// would visit the same candidates in the same order).  Each lane then adds the
+// same terms in the same order as the full query: the results are
+// bit-identical.
 constexpr int kPairLanes = 8;      // lanes per vertex of the query
 constexpr int kPairCap = 4;        // recorded candidates per lane (more: that vertex takes the full query)
 constexpr double kPairSkin = 0.2;  // skin = 0.2 lc1
-// Replay while every vertex has moved less than 0.25 skin from the snapshot
-// of the last recording of all lists.  A vertex that left the cell its list
-// was recorded in records it again there (the snapshot stays), so two lists
-// can be recorded at different times: a pair's distance then changed by at
-// most 4 x 0.25 skin since either list was recorded.
+// A vertex is slow while it has moved less than 0.25 skin from the snapshot of
+// the last recording of all lists, else fast.  Lists are replayed for slow
+// vertices with no fast one among their candidates.  A slow vertex that left the
+// cell its list was recorded in records it again there (the snapshot stays, and
+// again only while its candidates are slow), so two lists can be recorded at
+// different times: a pair's distance then changed by at most 4 x 0.25 skin since
+// either list was recorded.
 constexpr double kPairLimit = 0.25;
+// More fast vertices than this in one block, or in all, record all lists again.
+constexpr int kFastSeg = 32, kFastMax = 256, kFastRow = kFastSeg + 1;
 struct PairCache {
     double* x_snap;         // [3N] positions at the recording; null: no cache
     int* cell;              // [N] cell (query_cell) at the recording, -1: replay not allowed
     unsigned* cnt;          // [N] recorded candidates of each lane, 4 bits per lane
     int* ent;               // [8 kPairCap N] ids, lane-major per vertex
     double* disp_part;      // [disp_n] max |x - x_snap|^2 per pass-1 block (written by pass 1)
+    int* fast;              // [kFastRow disp_n] per block with fast vertices: their number and build-time cells
     int disp_n;
     int* dforce;            // replica groups: device flag, nonzero records (the reduction clears it)
     double skin;
-    double limit2;          // replay while max |x - x_snap|^2 < limit2
+    double limit2;          // fast: |x - x_snap|^2 >= limit2
     int force;              // single meshes: 1 records in this launch
 };
 constexpr int kCachedVerts = 256;    // vertices per block of the cached query
