@@ -976,14 +976,16 @@ __global__ void __launch_bounds__(kThreads) k_rep(PassArgs A)
 }
 
 // The repulsion query with the pair cache (PairCache), kVertsPerBlock
-// vertices per block of 256 threads.  Phase 1, one thread per vertex (the
-// first kVertsPerBlock threads): a vertex whose lists may be
-// replayed sums each lane's recorded pairs in that lane's order and combines
-// the eight lane sums in the order of group_sum ((l0+l1)+(l2+l3)) +
-// ((l4+l5)+(l6+l7)), so it gets the bits of the 8-lane query; the other ring
-// vertices (all of them in a recording launch) go to a block-local list.
-// Phase 2: the block's 32 lane groups run the full query (recording when the
-// mode says so) over that list.  Replays are the common case and want few,
+// vertices per block of 256 threads.  Phase 1, one thread per vertex: a vertex
+// whose lists may be replayed is done if nothing was recorded, else goes to a
+// block-local list; the other ring vertices (all of them in a recording launch)
+// go to a second one.  Phase 2: the block's 32 lane groups replay the first list,
+// lane l the pairs that lane l of the query recorded, in their order, and
+// group_sum over the lanes, which gives the bits of the 8-lane query.  A chain of
+// two loads per vertex, its entries as one vector, two vertices of a group in
+// flight: MEASURE_REPLAY
+// Phase 3: the lane groups run the full query (recording when the mode says so)
+// over the second list.  Replays are the common case and want few,
 // full blocks; a recording launch the device decides on (some vertex moved
 // too far) is slower than k_rep, as each group takes 8 vertices in turn.
 // Without cache buffers (a replica with a Verlet list in a cached group
@@ -1149,15 +1151,20 @@ __device__ __forceinline__ void rep_cached_body(const PassArgs& A, int lb)
     __shared__ int s_list[kVertsPerBlock];
     __shared__ double s_val[kVertsPerBlock];    // repulsion property per vertex (column 5 of pass 1)
     __shared__ int s_n;
-    if (threadIdx.x == 0) s_n = 0;
+    __shared__ int s_rep[kVertsPerBlock];
+    __shared__ unsigned s_word[kVertsPerBlock];
+    __shared__ int s_nrep;
+    if (threadIdx.x == 0) {
+        s_n = 0;
+        s_nrep = 0;
+    }
     __syncthreads();
     if (threadIdx.x < kVertsPerBlock) s_val[threadIdx.x] = 0.0;
     if (mine) {
         const bool ring = !is_generic(meta);
         bool done = !ring;
         bool keep = true;    // its list may be replayed, or recorded
-        double rep = 0.0;
-        int cnt = 0;
+        bool listed = false;
         if (mode == 2) {
             pc.x_snap[3 * v] = xv.x;
             pc.x_snap[3 * v + 1] = xv.y;
@@ -1179,48 +1186,75 @@ __device__ __forceinline__ void rep_cached_body(const PassArgs& A, int lb)
             const unsigned word = rec_word;
             const bool replay = keep && cell != -1 && query_cell(A.nl, xv) == cell;
             if (replay && word == 0u) {
-                done = true;    // nothing recorded: no pairs (the sums below would all be +0)
+                done = true;    // nothing recorded: no pairs (the sums over none are +0)
             } else if (replay) {
-                const double dmax = p.rep_lc1, dmax2 = dmax * dmax * (1.0 + 1e-15);
-                // lane l's terms, then lane pairs, as group_sum adds them
-                auto lane_terms = [&](int l) {
-                    RepTerms t;
-                    const int k = (int)((word >> (4 * l)) & 15u);
-                    const int* e = pc.ent + ((size_t)v * kGroup + l) * kPairCap;
-                    for (int i = 0; i < k; i++) {
-                        const d3 d = xv - load_p(m.x, e[i]);
-                        const double sq = sqnorm(d);
-                        if (sq <= dmax2 && sqrt(sq) < dmax) t.add(d, p);
-                    }
-                    return t;
-                };
-                double rh[kGroup / 2];
-                d3 gh[kGroup / 2];
-#pragma unroll
-                for (int h = 0; h < kGroup / 2; h++) {
-                    const RepTerms a = lane_terms(2 * h), b = lane_terms(2 * h + 1);
-                    rh[h] = a.rep + b.rep;
-                    gh[h] = a.g + b.g;
-                    cnt += a.cnt + b.cnt;
-                }
-                RepTerms t;
-                t.rep = (rh[0] + rh[1]) + (rh[2] + rh[3]);
-                t.g = (gh[0] + gh[1]) + (gh[2] + gh[3]);
-                t.cnt = cnt;
-                rep = t.rep;
-                store_rep_g(A, v, t);
-                done = true;
+                const int at = atomicAdd(&s_nrep, 1);
+                s_rep[at] = v;
+                s_word[at] = word;
+                listed = true;
             }
         }
         if (done) {
-            A.rep_v[v] = rep;
-            A.pair_cnt[v] = cnt;
-            s_val[threadIdx.x] = ring ? rep : A.gprops[6 * v + 5];
-        } else {
+            A.rep_v[v] = 0.0;
+            A.pair_cnt[v] = 0;
+            if (!ring) s_val[threadIdx.x] = A.gprops[6 * v + 5];
+        } else if (!listed) {
             s_list[atomicAdd(&s_n, 1)] = keep ? v : ~v;
         }
     }
     __syncthreads();
+    const int g = threadIdx.x / kGroup, lane = threadIdx.x % kGroup;
+    constexpr int kGroups = 256 / kGroup, kAhead = 2;
+    for (int i0 = g; i0 < s_nrep; i0 += kAhead * kGroups) {
+        static_assert(kPairCap == 8, "a lane's entries are two vectors, the second rarely used");
+        const double dmax = p.rep_lc1, dmax2 = dmax * dmax * (1.0 + 1e-15);
+        int u[kAhead], k[kAhead];
+        const int4* ent[kAhead];
+        int4 e[kAhead];
+        d3 xu[kAhead], pj[kAhead][4];
+        auto positions = [&](int4 id, int n, d3 (&out)[4]) {
+            if (n > 0) out[0] = load_p(m.x, id.x);
+            if (n > 1) out[1] = load_p(m.x, id.y);
+            if (n > 2) out[2] = load_p(m.x, id.z);
+            if (n > 3) out[3] = load_p(m.x, id.w);
+        };
+#pragma unroll
+        for (int a = 0; a < kAhead; a++) {
+            const int i = i0 + a * kGroups, ic = i < s_nrep ? i : i0;
+            u[a] = s_rep[ic];
+            k[a] = i < s_nrep ? (int)((s_word[ic] >> (4 * lane)) & 15u) : 0;
+            xu[a] = load_p(m.x, u[a]);
+            ent[a] = reinterpret_cast<const int4*>(pc.ent + ((size_t)u[a] * kGroup + lane) * kPairCap);
+            e[a] = k[a] > 0 ? *ent[a] : make_int4(0, 0, 0, 0);
+        }
+#pragma unroll
+        for (int a = 0; a < kAhead; a++) positions(e[a], k[a], pj[a]);
+#pragma unroll
+        for (int a = 0; a < kAhead; a++) {
+            RepTerms t;
+            auto add = [&](int n) {
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    if (q >= n) continue;
+                    const d3 d = xu[a] - pj[a][q];
+                    const double sq = sqnorm(d);
+                    if (sq <= dmax2 && sqrt(sq) < dmax) t.add(d, p);
+                }
+            };
+            add(k[a]);
+            if (k[a] > 4) {
+                positions(ent[a][1], k[a] - 4, pj[a]);
+                add(k[a] - 4);
+            }
+            t.group_reduce();
+            if (lane == 0 && i0 + a * kGroups < s_nrep) {
+                A.rep_v[u[a]] = t.rep;
+                A.pair_cnt[u[a]] = t.cnt;
+                s_val[u[a] - base] = t.rep;
+                store_rep_g(A, u[a], t);
+            }
+        }
+    }
     const int n_full = s_n;
     // a replay launch leaves few vertices per block to the full query, so its
     // latency counts: up to kWaveVerts take a whole wave each (wide_record)
@@ -1237,8 +1271,7 @@ __device__ __forceinline__ void rep_cached_body(const PassArgs& A, int lb)
             store_rep_g(A, u, tr);
         }
     }
-    const int g = threadIdx.x / kGroup, lane = threadIdx.x % kGroup;
-    for (int i = g; !waves && i < n_full; i += 256 / kGroup) {
+    for (int i = g; !waves && i < n_full; i += kGroups) {
         const int e = s_list[i], u = e < 0 ? ~e : e;
         const d3 xu = load_p(m.x, u);
         const int n = meta_valence(m.meta[u]);
