@@ -505,7 +505,7 @@ struct tm_nlist {
     int exclusion = 0;
     double rlist = 0.1;
     NListView v{};
-    DevBuf<int> cell_start, cell_verts, vert_cell, counts, fill, scan_tmp, adj_start, adj, adj_counts;
+    DevBuf<int> cell_start, cell_verts, vert_cell, counts, place, scan_tmp, adj_start, adj, adj_counts;
     DevBuf<int> cand_count, cand_start, cand;
     DevBuf<int2> vcand;
     DevBuf<unsigned long long> excl_mask;
@@ -521,7 +521,7 @@ struct tm_nlist {
     DevBuf<int> dm_counts, dm_off;
     DevBuf<double> dm_d;
     DevBuf<int> dm_i, dm_j;
-    DevBuf<double> box_part, pd_dist;
+    DevBuf<double> pd_dist;
     DevBuf<int> pd_j, pd_count;
     int nv = 0;
     NListView view() const { return v; }
@@ -554,18 +554,33 @@ void scan(const int* in, int* out, int n, DevBuf<int>& tmp)
 
 // CellList ctor (cell_list.h:43-87) and, for kind 1, VerletList ctor
 // (verlet_list.h:18-35), on the mesh's current device positions.
-void build_nlist(tm_nlist& L, tm_mesh& M)
+// the Verlet adjacency from the cells of its list
+void build_verlet(tm_nlist& L, tm_mesh& M)
 {
-    if (!(L.rlist > 0) || !std::isfinite(L.rlist)) throw TmError(TM_E_INVALID, "rlist must be positive");
     const int n = M.nv;
-    L.nv = n;
-    const int nbox = box_scratch_doubles();
-    L.box_part.alloc(nbox);
-    launch_box(M.x.p, n, L.box_part.p, g_rt.stream);
+    NListView& v = L.v;
+    L.adj_counts.alloc(n + 1);
+    L.adj_start.alloc(n + 1);
+    HIPCHECK(hipMemsetAsync(L.adj_counts.p, 0, sizeof(int) * (n + 1), g_rt.stream));
+    launch_verlet_count(M.view(), v, L.rlist, L.adj_counts.p, g_rt.stream);
     check_launch();
-    std::vector<double> part(nbox);
-    d2h(part.data(), L.box_part.p, sizeof(double) * nbox);
+    scan(L.adj_counts.p, L.adj_start.p, n + 1, L.scan_tmp);
+    int total = 0;
+    d2h(&total, L.adj_start.p + n, sizeof(int));
     sync();
+    L.adj.alloc(total);
+    launch_verlet_fill(M.view(), v, L.rlist, L.adj_start.p, L.adj.p, g_rt.stream);
+    check_launch();
+    v.kind = 1;
+    v.adj_start = L.adj_start.p;
+    v.adj = L.adj.p;
+}
+
+// The grid of a list from the box partials of its vertices; returns the number of
+// cells.
+long long nlist_grid(tm_nlist& L, int n, const double* part)
+{
+    const int nbox = box_scratch_doubles();
     double tight[6] = {DBL_MAX, DBL_MAX, DBL_MAX, -DBL_MAX, -DBL_MAX, -DBL_MAX};    // the vertices' own box
     for (int b = 0; b < nbox / 6; b++)
         for (int k = 0; k < 3; k++) {
@@ -614,83 +629,142 @@ void build_nlist(tm_nlist& L, tm_mesh& M)
     v.strides[0] = 1;
     v.strides[1] = v.shape[0];
     v.strides[2] = v.shape[0] * v.shape[1];
-    const int nc = (int)ncells;
-    L.counts.alloc(nc + 1);
-    L.cell_start.alloc(nc + 1);
-    L.fill.alloc(nc);
-    L.vert_cell.alloc(n);
-    L.cell_verts.alloc(n);
-    const bool cells = L.kind == 0 && n > 0;    // the per-cell candidate lists
-    if (cells) L.cand_count.alloc(n + 1);
-    launch_fill_ints(L.counts.p, nc + 1, 0, L.fill.p, nc, 0, cells ? L.cand_count.p + n : nullptr, cells ? 1 : 0, 0,
-                     g_rt.stream);
-    check_launch();
-    launch_cell_ids(M.x.p, n, v, L.vert_cell.p, L.counts.p, g_rt.stream);
-    check_launch();
-    scan(L.counts.p, L.cell_start.p, nc + 1, L.scan_tmp);
-    launch_cell_scatter(L.vert_cell.p, n, L.cell_start.p, L.fill.p, L.cell_verts.p, g_rt.stream);
-    check_launch();
-    launch_cell_sort_segments(L.vert_cell.p, n, L.cell_start.p, M.d_perm.p, L.cell_verts.p, g_rt.stream);
-    check_launch();
-    v.cell_start = L.cell_start.p;
-    v.cell_verts = L.cell_verts.p;
-    v.vert_cell = L.vert_cell.p;
-    v.perm = M.d_perm.p;
-    if (L.kind == 0 && n > 0) {
-        if ((long long)27 * n > INT_MAX) throw TmError(TM_E_UNSUPPORTED, "mesh too large for the candidate table");
-        L.cand_start.alloc(n + 1);
-        launch_cand_count(v, n, L.cand_count.p, g_rt.stream);
-        check_launch();
-        scan(L.cand_count.p, L.cand_start.p, n + 1, L.scan_tmp);
-        // a vertex is in the stencil lists of at most 27 cells: 27 N bounds
-        // the total without reading it back
-        L.cand.alloc((size_t)27 * n);
-        launch_cand_fill(v, n, L.cand_start.p, L.cand.p, g_rt.stream);
-        check_launch();
-        L.vcand.alloc(n);
-        launch_cand_vrange(v, n, L.cand_start.p, L.vcand.p, g_rt.stream);
-        check_launch();
-        v.vcand = L.vcand.p;
-        v.cand = L.cand.p;
-        v.cand_start = L.cand_start.p;
-    }
-    if (L.kind == 1) {
-        L.adj_counts.alloc(n + 1);
-        L.adj_start.alloc(n + 1);
-        HIPCHECK(hipMemsetAsync(L.adj_counts.p, 0, sizeof(int) * (n + 1), g_rt.stream));
-        launch_verlet_count(M.view(), v, L.rlist, L.adj_counts.p, g_rt.stream);
-        check_launch();
-        scan(L.adj_counts.p, L.adj_start.p, n + 1, L.scan_tmp);
-        int total = 0;
-        d2h(&total, L.adj_start.p + n, sizeof(int));
-        sync();
-        L.adj.alloc(total);
-        launch_verlet_fill(M.view(), v, L.rlist, L.adj_start.p, L.adj.p, g_rt.stream);
-        check_launch();
-        v.kind = 1;
-        v.adj_start = L.adj_start.p;
-        v.adj = L.adj.p;
-    }
     L.v = v;
-    if (L.kind == 0 && n > 0) {
-        L.excl_mask.alloc((size_t)2 * n);
-        L.mask_topo = ~0u;
-        ensure_masks(L, M);
-        L.pc_x.alloc((size_t)3 * n);
-        L.pc_cell.alloc(n);
-        L.pc_cnt.alloc(n);
-        L.pc_ent.alloc((size_t)kPairLanes * kPairCap * n);
-        const int nd = pass1_blocks(n);    // one displacement partial per pass-1 block
-        L.pc_disp.alloc(nd);
-        L.pc_fast.alloc((size_t)kFastRow * nd);
-        // cell -1: no replay; displacement bytes 0x7F (~1e306): a recording first
-        launch_fill_ints(L.pc_cell.p, n, -1, reinterpret_cast<int*>(L.pc_disp.p), 2 * nd, 0x7F7F7F7F,
-                         nullptr, 0, 0, g_rt.stream);
-        check_launch();
-        L.pc_ok = false;
+    return ncells;
+}
+
+// (Re)builds the lists of R meshes together: one round trip for all boxes, then
+// one launch of each kind for all.
+struct NlistJob {
+    tm_nlist* L;
+    tm_mesh* M;
+};
+struct NlistTables {    // a build's arguments, and on the device those of several lists
+    std::vector<NlistBuild> h;
+    std::vector<int> h_block0;
+    DevBuf<NlistBuild> builds;
+    DevBuf<int> block0;
+};
+void build_nlists(const std::vector<NlistJob>& jobs, NlistTables& T)
+{
+    const int R = (int)jobs.size();
+    if (R == 0) return;
+    std::vector<NlistBuild>& h = T.h;
+    std::vector<int>& block0 = T.h_block0;
+    h.assign(R, NlistBuild{});
+    block0.resize((size_t)kShapes * (R + 1));
+    NlistGroup g{h.data(), R, nullptr, nullptr, {}};
+    for (int r = 0; r < R; r++) {
+        tm_nlist& L = *jobs[r].L;
+        if (!(L.rlist > 0) || !std::isfinite(L.rlist)) throw TmError(TM_E_INVALID, "rlist must be positive");
+        L.nv = jobs[r].M->nv;
+        h[r].x = jobs[r].M->x.p;
+        h[r].n = L.nv;
     }
-    // no wait here: everything that reads the list is queued behind it on the
-    // library stream (the host already waited once, for the bounding box)
+    auto tabulate = [&]() {
+        for (int k = 0; k < kShapes; k++) {
+            int* b0 = block0.data() + (size_t)k * (R + 1);
+            b0[0] = 0;
+            for (int r = 0; r < R; r++) b0[r + 1] = b0[r] + nlist_blocks(h[r], k);
+            g.total[k] = b0[R];
+        }
+        if (R == 1) return;
+        T.builds.alloc(R);
+        T.block0.alloc(block0.size());
+        h2d(T.builds.p, h.data(), sizeof(NlistBuild) * R);
+        h2d(T.block0.p, block0.data(), sizeof(int) * block0.size());
+        g.d = T.builds.p;
+        g.block0 = T.block0.p;
+    };
+    {
+        const size_t nbox = box_scratch_doubles();
+        HostRing& ring = host_ring();
+        std::lock_guard<std::mutex> guard(ring.lock);
+        ring.buf.alloc(kRingPiece * kRingPieces);
+        const size_t at_once = kRingPiece * kRingPieces / (nbox * sizeof(double));
+        if ((size_t)R > at_once) throw TmError(TM_E_UNSUPPORTED, "too many lists in one build");
+        double* box = reinterpret_cast<double*>(ring.buf.p);
+        for (int r = 0; r < R; r++) h[r].box = box + nbox * r;
+        tabulate();
+        launch_nlist_box(g, g_rt.stream);
+        check_launch();
+        sync();
+        for (int r = 0; r < R; r++) {
+            const long long ncells = nlist_grid(*jobs[r].L, jobs[r].M->nv, h[r].box);
+            h[r].nc = (int)ncells;
+        }
+    }
+    for (int r = 0; r < R; r++) {
+        tm_nlist& L = *jobs[r].L;
+        tm_mesh& M = *jobs[r].M;
+        const int n = M.nv, nc = h[r].nc;
+        NlistBuild& b = h[r];
+        L.counts.alloc(nc + 1);
+        L.cell_start.alloc(nc + 1);
+        L.place.alloc(n);
+        L.vert_cell.alloc(n);
+        L.cell_verts.alloc(n);
+        L.scan_tmp.alloc(scan_block_sums_size(std::max(n, nc) + 1) + 1);
+        b.perm = M.d_perm.p;
+        b.m = M.view();
+        b.counts = L.counts.p;
+        b.cell_start = L.cell_start.p;
+        b.vert_cell = L.vert_cell.p;
+        b.place = L.place.p;
+        b.cell_verts = L.cell_verts.p;
+        b.sums = L.scan_tmp.p;
+        L.v.cell_start = L.cell_start.p;
+        L.v.cell_verts = L.cell_verts.p;
+        L.v.vert_cell = L.vert_cell.p;
+        L.v.perm = M.d_perm.p;
+        if (L.kind == 0 && n > 0) {
+            if ((long long)27 * n > INT_MAX) throw TmError(TM_E_UNSUPPORTED, "mesh too large for the candidate table");
+            L.cand_count.alloc(n + 1);
+            L.cand_start.alloc(n + 1);
+            // a vertex is in the stencil lists of at most 27 cells: 27 N bounds
+            // the total without reading it back
+            L.cand.alloc((size_t)27 * n);
+            L.vcand.alloc(n);
+            L.excl_mask.alloc((size_t)2 * n);
+            L.pc_x.alloc((size_t)3 * n);
+            L.pc_cell.alloc(n);
+            L.pc_cnt.alloc(n);
+            L.pc_ent.alloc((size_t)kPairLanes * kPairCap * n);
+            L.pc_disp.alloc(pass1_blocks(n));    // one displacement partial per pass-1 block
+            L.pc_fast.alloc((size_t)kFastRow * pass1_blocks(n));
+            b.cand_count = L.cand_count.p;
+            b.cand_start = L.cand_start.p;
+            b.cand = L.cand.p;
+            b.vcand = L.vcand.p;
+            b.mask = L.excl_mask.p;
+            b.pc_cell = L.pc_cell.p;
+            L.v.vcand = L.vcand.p;
+            L.v.cand = L.cand.p;
+            L.v.cand_start = L.cand_start.p;
+        }
+        b.nl = L.v;    // masks not set: they are what the build makes
+    }
+    tabulate();
+    launch_nlist_build(g, g_rt.stream);
+    check_launch();
+    for (int r = 0; r < R; r++) {
+        tm_nlist& L = *jobs[r].L;
+        tm_mesh& M = *jobs[r].M;
+        if (L.kind == 1) build_verlet(L, M);
+        if (L.kind == 0 && M.nv > 0) {
+            L.mask_topo = M.topo_version;
+            L.v.excl_mask = L.excl_mask.p;
+            L.pc_ok = false;
+        }
+    }
+    // no wait here: everything that reads the lists is queued behind them on the
+    // library stream (the host already waited once, for the bounding boxes)
+}
+
+void build_nlist(tm_nlist& L, tm_mesh& M)
+{
+    NlistTables one;
+    build_nlists({NlistJob{&L, &M}}, one);
 }
 
 void check_params(const tm_params& p)
@@ -797,7 +871,7 @@ void ensure_energy_buffers(tm_energy& E, const tm_mesh& M)
 // list is built into the energy manager's spare, whose buffers remain from
 // the rebuild before, and swapped in only when complete, so a failed build
 // leaves the current list in place.
-void rebuild_nlist(tm_energy& E, tm_mesh& M)
+tm_nlist& spare_nlist(tm_energy& E)
 {
     check_params(E.params);
     if (!E.spare) E.spare = new tm_nlist();
@@ -805,9 +879,17 @@ void rebuild_nlist(tm_energy& E, tm_mesh& M)
     L.kind = E.params.rep_nlist;
     L.exclusion = E.params.rep_exclusion;
     L.rlist = E.params.rep_rlist;
-    build_nlist(L, M);
+    return L;
+}
+void take_spare(tm_energy& E)
+{
     std::swap(E.nlist, E.spare);
     E.gen++;
+}
+void rebuild_nlist(tm_energy& E, tm_mesh& M)
+{
+    build_nlist(spare_nlist(E), M);
+    take_spare(E);
 }
 
 // The pair-cache buffers of the energy manager's cell list (x_snap null when
@@ -1653,6 +1735,7 @@ struct tm_replicas {
     // pair cache: per-replica recording flags (device; the reduction clears
     // them), displacement partials, and the prefix tables of the
     // displacement check and of the cached query
+    NlistTables nl_tables;    // of the group's list builds
     DevBuf<int> force_flags, d_block0_rc;
     DevBuf<double> disp_parts;
     DevBuf<int> fast_parts;
@@ -2145,12 +2228,13 @@ int tm_replicas_update_repulsion(tm_replicas* rs)
 {
     API_BEGIN
     tm_replicas& S = *rs;
+    std::vector<NlistJob> jobs(S.R);
     for (int r = 0; r < S.R; r++) {
-        tm_mesh& M = *S.meshes[r];
-        tm_energy& E = *S.ems[r];
-        upload_points(M);
-        rebuild_nlist(E, M);
+        upload_points(*S.meshes[r]);
+        jobs[r] = NlistJob{&spare_nlist(*S.ems[r]), S.meshes[r]};
     }
+    build_nlists(jobs, S.nl_tables);
+    for (tm_energy* E : S.ems) take_spare(*E);
     refresh_replica_args(S);
     API_END
 }

@@ -622,13 +622,14 @@ __device__ __forceinline__ bool mask_member(const int* tab, int j)
     return false;
 }
 
-__global__ void __launch_bounds__(256) k_excl_mask(MeshView m, NListView nl, unsigned long long* __restrict__ mask)
+__device__ __forceinline__ void excl_mask_body(const MeshView& m, const NListView& nl,
+                                               unsigned long long* __restrict__ mask, int lb)
 {
     constexpr int kGroups = 256 / kGroup;
     __shared__ int s_tab[kGroups][kMaskTab];
     __shared__ int s_cnt[kGroups];
     __shared__ int s_ovf[kGroups];
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    const int t = lb * 256 + threadIdx.x;
     const int gi = threadIdx.x / kGroup;
     const int v = t / kGroup, lane = t % kGroup;
     const bool active = v < m.nv;
@@ -696,10 +697,30 @@ __global__ void __launch_bounds__(256) k_excl_mask(MeshView m, NListView nl, uns
     }
 }
 
+__global__ void __launch_bounds__(256) k_excl_mask(MeshView m, NListView nl, unsigned long long* __restrict__ mask)
+{
+    excl_mask_body(m, nl, mask, blockIdx.x);
+}
+__global__ void __launch_bounds__(256) k_excl_mask_grouped(const NlistBuild* __restrict__ b,
+                                                           const int* __restrict__ block0, int R)
+{
+    const int r = find_replica(block0, R, blockIdx.x);
+    excl_mask_body(b[r].m, b[r].nl, b[r].mask, (int)blockIdx.x - block0[r]);
+}
+
 void launch_excl_mask(const MeshView& m, const NListView& nl, unsigned long long* mask, hipStream_t s)
 {
     if (m.nv <= 0) return;
     hipLaunchKernelGGL(k_excl_mask, dim3((m.nv * kGroup + 255) / 256), dim3(256), 0, s, m, nl, mask);
+}
+
+void launch_nlist_masks(const NlistGroup& g, hipStream_t s)
+{
+    if (g.total[kShapeMask] <= 0) return;
+    if (g.R == 1) launch_excl_mask(g.h[0].m, g.h[0].nl, g.h[0].mask, s);
+    else
+        hipLaunchKernelGGL(k_excl_mask_grouped, dim3(g.total[kShapeMask]), dim3(256), 0, s, g.d,
+                           g.block0 + kShapeMask * (g.R + 1), g.R);
 }
 
 // --------------------------------------------------------------- pass 1 ---

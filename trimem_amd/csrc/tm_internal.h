@@ -182,19 +182,41 @@ void launch_build_ring(const MeshView& m, int* ring, int* meta, int* overflow, h
 // neighbour lists (tm_nlist.hip)
 int box_scratch_doubles();
 void launch_fill_ints(int* a, int na, int va, int* b, int nb, int vb, int* c, int nc, int vc, hipStream_t s);
-void launch_box(const double* x, int n, double* part, hipStream_t s);
-void launch_cell_ids(const double* x, int n, const NListView& nl, int* vert_cell, int* counts, hipStream_t s);
 void launch_exclusive_scan(const int* in, int* out, int n, int* block_sums, hipStream_t s);
 int scan_block_sums_size(int n);
-void launch_cell_scatter(const int* vert_cell, int n, const int* cell_start, int* fill, int* cell_verts,
-                         hipStream_t s);
-void launch_cell_sort_segments(const int* vert_cell, int n, const int* cell_start, const int* perm, int* cell_verts,
-                               hipStream_t s);
-// per occupied cell, the vertices of its 27-cell stencil (count, then fill
-// after an exclusive scan of the counts)
-void launch_cand_count(const NListView& nl, int n, int* count, hipStream_t s);
-void launch_cand_fill(const NListView& nl, int n, const int* cand_start, int* cand, hipStream_t s);
-void launch_cand_vrange(const NListView& nl, int n, const int* cand_start, int2* vcand, hipStream_t s);
+// One list of a build.
+struct NlistBuild {
+    const double* x;
+    const int* perm;
+    int n, nc;                 // vertices, cells
+    double* box;               // [box_scratch_doubles] pinned
+    NListView nl;              // the grid, and the tables as they will be
+    MeshView m;
+    int *counts, *cell_start;  // [nc + 1]
+    int *vert_cell, *place, *cell_verts;    // [n]
+    int *cand_count, *cand_start;           // [n + 1]; a Verlet list: these and below null
+    int* cand;                 // [27 n]
+    int2* vcand;               // [n]
+    unsigned long long* mask;  // [2 n]
+    int* pc_cell;              // [n]
+    int* sums;                 // [scan_block_sums_size(max(n, nc) + 1)]
+};
+// Workgroups of a list in the launches of each shape.
+enum {
+    kShapeBox, kShapeVerts, kShapeCells, kShapeCand, kShapeVertsCand, kShapeVertsSort, kShapeMask, kShapes
+};
+int nlist_blocks(const NlistBuild& b, int shape);
+struct NlistGroup {
+    const NlistBuild* h;       // [R]
+    int R;
+    const NlistBuild* d;       // R > 1: the same in device memory
+    const int* block0;         // [kShapes][R + 1] prefix tables of nlist_blocks
+    int total[kShapes];
+};
+void launch_nlist_box(const NlistGroup& g, hipStream_t s);
+// everything after the host has set the grids
+void launch_nlist_build(const NlistGroup& g, hipStream_t s);
+void launch_nlist_masks(const NlistGroup& g, hipStream_t s);    // tm_energy.hip
 // exclusion masks of the stored stencil lists (tm_energy.hip); nl needs
 // vcand and cand, its excl_mask is ignored
 void launch_excl_mask(const MeshView& m, const NListView& nl, unsigned long long* mask, hipStream_t s);

@@ -9,7 +9,10 @@
 // FP64 from the reduced box), flat cell ids sum_k int((p_k - min_k) / r_k)
 // * stride_k (cell_list.h:70-79), then a counting sort: histogram, exclusive
 // scan, scatter, and a per-cell sort by vertex id so that the order inside a
-// cell is ascending like the reference's push_back order.  The reference keys
+// cell is ascending like the reference's push_back order.  Every kernel of the
+// build takes one list (its arguments by value) or many (a table of them and a
+// prefix table of workgroups): the lists of a replica group are built together,
+// with the launches and the one host round trip of a single list.  The reference keys
 // its cells in a map (cell_list.h:31), so only occupied cells cost memory;
 // here the table is dense over the occupied sub-grid, the global cells lo ..
 // hi that hold a vertex at build time, which is the mesh's own bounding box
@@ -32,22 +35,24 @@ namespace tmh {
 // ----------------------------------------------------------------- box ----
 // Bounding box of the vertices, as kBoxBlocks per-block partial minima and
 // maxima (part[6 b + k], min in k < 3, max in k >= 3; +DBL_MAX and -DBL_MAX
-// for a block without vertices).  The host, which reads the box back anyway
-// to size the grid, combines them (min and max are exact in any order) and
+// for a block without vertices).  They go to pinned host memory:
+// the host, which needs the box to size the grid, combines them (min and max are exact in any order) and
 // applies the reference's initial values (cell_list.h:46-47); a last-block
 // combine would need a device-scope fence in every block, which costs more
 // than the whole pass.
 constexpr int kBoxBlocks = 64;
-__global__ void __launch_bounds__(256) k_box(const double* __restrict__ x, int n, double* __restrict__ part)
+__device__ __forceinline__ void box_body(const NlistBuild& b, int lb)
 {
+    const double* __restrict__ x = b.x;
+    const int n = b.n;
     __shared__ double s[6][4];
     double mn[3] = {DBL_MAX, DBL_MAX, DBL_MAX};
     double mx[3] = {-DBL_MAX, -DBL_MAX, -DBL_MAX};
     // kBoxBatch points per thread and step, all their loads in flight before
     // the first comparison
     constexpr int kBoxBatch = 8;
-    const int stride = gridDim.x * blockDim.x;
-    for (int i0 = blockIdx.x * blockDim.x + threadIdx.x; i0 < n; i0 += kBoxBatch * stride) {
+    const int stride = kBoxBlocks * blockDim.x;
+    for (int i0 = lb * blockDim.x + threadIdx.x; i0 < n; i0 += kBoxBatch * stride) {
         double v[kBoxBatch][3];
 #pragma unroll
         for (int u = 0; u < kBoxBatch; u++) {
@@ -81,7 +86,7 @@ __global__ void __launch_bounds__(256) k_box(const double* __restrict__ x, int n
         int k = threadIdx.x;
         double r = s[k][0];
         for (int w = 1; w < 4; w++) r = k < 3 ? fmin(r, s[k][w]) : fmax(r, s[k][w]);
-        part[blockIdx.x * 6 + k] = r;
+        b.box[lb * 6 + k] = r;
     }
 }
 
@@ -104,10 +109,6 @@ void launch_fill_ints(int* a, int na, int va, int* b, int nb, int vb, int* c, in
     hipLaunchKernelGGL(k_fill_ints, dim3((n + 255) / 256), dim3(256), 0, s, a, na, va, b, nb, vb, c, nc, vc);
 }
 
-void launch_box(const double* x, int n, double* part, hipStream_t s)
-{
-    hipLaunchKernelGGL(k_box, dim3(kBoxBlocks), dim3(256), 0, s, x, n, part);
-}
 
 // ------------------------------------------------------------- binning ----
 // Build-time cell of vertex v in the occupied sub-grid.  The coordinate is
@@ -125,148 +126,124 @@ __device__ __forceinline__ int flat_cell(const NListView& nl, const double* x, i
     return id;
 }
 
-__global__ void k_cell_ids(const double* __restrict__ x, int n, NListView nl, int* __restrict__ vert_cell,
-                           int* __restrict__ counts)
+// all cells empty
+constexpr int kClearTile = 4096;
+__device__ __forceinline__ void clear_body(const NlistBuild& b, int lb)
 {
-    int v = blockIdx.x * blockDim.x + threadIdx.x;
-    if (v >= n) return;
-    int c = flat_cell(nl, x, v);
-    vert_cell[v] = c;
-    atomicAdd(&counts[c], 1);
+    const int end = min((lb + 1) * kClearTile, b.nc + 1);
+    for (int i = lb * kClearTile + threadIdx.x; i < end; i += 256) b.counts[i] = 0;
 }
 
-void launch_cell_ids(const double* x, int n, const NListView& nl, int* vert_cell, int* counts, hipStream_t s)
+// each vertex's cell and its place among the cell's vertices as they come (the
+// count that it found), which makes the scatter a plain store; the pair cache
+// starts with nothing to replay
+__device__ __forceinline__ void cells_body(const NlistBuild& b, int lb)
 {
-    hipLaunchKernelGGL(k_cell_ids, dim3((n + 255) / 256), dim3(256), 0, s, x, n, nl, vert_cell, counts);
+    const int v = lb * 256 + threadIdx.x;
+    if (v >= b.n) return;
+    const int c = flat_cell(b.nl, b.x, v);
+    b.vert_cell[v] = c;
+    b.place[v] = atomicAdd(&b.counts[c], 1);
+    if (!b.cand) return;
+    b.pc_cell[v] = -1;    // no replay
+    if (v == 0) b.cand_count[b.n] = 0;
 }
 
 // ------------------------------------------------ stencil candidate lists
-// The 27-cell stencil of cell (c0, c1, c2) as 9 rows of x-consecutive cells,
-// clipped to the grid like the query of cell_list.h:133-219; f(start, len)
-// gets each row's range in cell_verts.
-template <class F>
-__device__ __forceinline__ void for_stencil_rows(const NListView& nl, const int c[3], F&& f)
+// The 27-cell stencil of cell c as 9 rows of x-consecutive cells, clipped to the
+// grid like the query of cell_list.h:133-219: each row's range in cell_verts,
+// all loads in flight at once.
+struct StencilRows {
+    int start[9], len[9];
+};
+__device__ __forceinline__ StencilRows stencil_rows(const NListView& nl, int cell)
 {
-    const int i0 = max(c[0] - 1, 0), i1 = min(c[0] + 1, nl.shape[0] - 1);
-    if (i0 > i1) return;
-    for (int r = 0; r < 9; r++) {
-        const int kk = c[2] + r / 3 - 1, jj = c[1] + r % 3 - 1;
-        if (kk < 0 || kk >= nl.shape[2] || jj < 0 || jj >= nl.shape[1]) continue;
-        const int base = jj * nl.strides[1] + kk * nl.strides[2];
-        const int s0 = nl.cell_start[base + i0];
-        f(s0, nl.cell_start[base + i1 + 1] - s0);
+    const int c2 = cell / nl.strides[2], c1 = (cell - c2 * nl.strides[2]) / nl.strides[1];
+    const int c0 = cell - c2 * nl.strides[2] - c1 * nl.strides[1];
+    const int i0 = max(c0 - 1, 0), i1 = min(c0 + 1, nl.shape[0] - 1);
+    StencilRows r;
+#pragma unroll
+    for (int k = 0; k < 9; k++) {
+        const int kk = c2 + k / 3 - 1, jj = c1 + k % 3 - 1;
+        const bool in = kk >= 0 && kk < nl.shape[2] && jj >= 0 && jj < nl.shape[1];
+        const int base = in ? jj * nl.strides[1] + kk * nl.strides[2] : 0;
+        r.start[k] = in ? nl.cell_start[base + i0] : 0;
+        r.len[k] = in ? nl.cell_start[base + i1 + 1] : 0;
     }
+#pragma unroll
+    for (int k = 0; k < 9; k++) r.len[k] -= r.start[k];
+    return r;
 }
 
-__device__ __forceinline__ bool cand_leader(const NListView& nl, int slot, int c[3])
+// the counting sort's scatter; with it the stencil size of each occupied cell at
+// its first slot, 0 at the others
+__device__ __forceinline__ void scatter_body(const NlistBuild& b, int lb)
 {
-    const int cf = nl.vert_cell[nl.cell_verts[slot]];
-    if (nl.cell_start[cf] != slot) return false;
-    c[2] = cf / nl.strides[2];
-    c[1] = (cf - c[2] * nl.strides[2]) / nl.strides[1];
-    c[0] = cf - c[2] * nl.strides[2] - c[1] * nl.strides[1];
-    return true;
+    const int v = lb * 256 + threadIdx.x;
+    if (v >= b.n) return;
+    const int c = b.vert_cell[v], place = b.place[v], slot = b.nl.cell_start[c] + place;
+    b.cell_verts[slot] = v;
+    if (!b.cand) return;
+    int total = 0;
+    if (place == 0) {
+        const StencilRows r = stencil_rows(b.nl, c);
+#pragma unroll
+        for (int k = 0; k < 9; k++) total += r.len[k];
+    }
+    b.cand_count[slot] = total;
 }
 
-// count[slot] = stencil size for the first slot of each occupied cell, else 0
-__global__ void k_cand_count(NListView nl, int n, int* __restrict__ count)
+// The thread at the start of a cell's segment sorts it by user vertex id (cells
+// hold a handful of vertices), the order in which the reference fills its cells.
+__device__ __forceinline__ void sort_segment(const NlistBuild& b, int i)
 {
-    const int slot = blockIdx.x * blockDim.x + threadIdx.x;
-    if (slot >= n) return;
-    int c[3], total = 0;
-    if (cand_leader(nl, slot, c)) for_stencil_rows(nl, c, [&](int, int len) { total += len; });
-    count[slot] = total;
-}
-
-__global__ void k_cand_fill(NListView nl, int n, const int* __restrict__ cand_start, int* __restrict__ cand)
-{
-    const int slot = blockIdx.x * blockDim.x + threadIdx.x;
-    if (slot >= n) return;
-    int c[3];
-    if (!cand_leader(nl, slot, c)) return;
-    int o = cand_start[slot];
-    for_stencil_rows(nl, c, [&](int s0, int len) {
-        for (int q = 0; q < len; q++) cand[o++] = nl.cell_verts[s0 + q];
-    });
-}
-
-// vcand[v] = list range of the build-time cell of v
-__global__ void k_cand_vrange(NListView nl, int n, const int* __restrict__ cand_start, int2* __restrict__ vcand)
-{
-    const int v = blockIdx.x * blockDim.x + threadIdx.x;
-    if (v >= n) return;
-    const int s = nl.cell_start[nl.vert_cell[v]];
-    vcand[v] = make_int2(cand_start[s], cand_start[s + 1]);
-}
-
-void launch_cand_vrange(const NListView& nl, int n, const int* cand_start, int2* vcand, hipStream_t s)
-{
-    if (n <= 0) return;
-    hipLaunchKernelGGL(k_cand_vrange, dim3((n + 255) / 256), dim3(256), 0, s, nl, n, cand_start, vcand);
-}
-
-void launch_cand_count(const NListView& nl, int n, int* count, hipStream_t s)
-{
-    if (n <= 0) return;
-    hipLaunchKernelGGL(k_cand_count, dim3((n + 255) / 256), dim3(256), 0, s, nl, n, count);
-}
-
-void launch_cand_fill(const NListView& nl, int n, const int* cand_start, int* cand, hipStream_t s)
-{
-    if (n <= 0) return;
-    hipLaunchKernelGGL(k_cand_fill, dim3((n + 255) / 256), dim3(256), 0, s, nl, n, cand_start, cand);
-}
-
-__global__ void k_cell_scatter(const int* __restrict__ vert_cell, int n, const int* __restrict__ cell_start,
-                               int* __restrict__ fill, int* __restrict__ cell_verts)
-{
-    int v = blockIdx.x * blockDim.x + threadIdx.x;
-    if (v >= n) return;
-    int c = vert_cell[v];
-    int pos = atomicAdd(&fill[c], 1);
-    cell_verts[cell_start[c] + pos] = v;
-}
-
-void launch_cell_scatter(const int* vert_cell, int n, const int* cell_start, int* fill, int* cell_verts,
-                         hipStream_t s)
-{
-    hipLaunchKernelGGL(k_cell_scatter, dim3((n + 255) / 256), dim3(256), 0, s, vert_cell, n, cell_start, fill,
-                       cell_verts);
-}
-
-// The thread sitting at the start of a cell's segment sorts the segment by
-// user vertex id (cells hold a handful of vertices), the order in which the
-// reference fills its cells.
-__global__ void k_cell_sort_segments(const int* __restrict__ vert_cell, int n, const int* __restrict__ cell_start,
-                                     const int* __restrict__ perm, int* __restrict__ cell_verts)
-{
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    int c = vert_cell[cell_verts[i]];
-    if (cell_start[c] != i) return;
-    int e = cell_start[c + 1];
+    int* cell_verts = b.cell_verts;
+    const int c = b.vert_cell[cell_verts[i]];
+    if (b.nl.cell_start[c] != i) return;
+    const int e = b.nl.cell_start[c + 1];
     for (int a = i + 1; a < e; a++) {
-        int key = cell_verts[a];
-        int kp = perm[key];
-        int b = a - 1;
-        while (b >= i && perm[cell_verts[b]] > kp) {
-            cell_verts[b + 1] = cell_verts[b];
-            b--;
+        const int key = cell_verts[a], kp = b.perm[key];
+        int q = a - 1;
+        while (q >= i && b.perm[cell_verts[q]] > kp) {
+            cell_verts[q + 1] = cell_verts[q];
+            q--;
         }
-        cell_verts[b + 1] = key;
+        cell_verts[q + 1] = key;
     }
 }
-
-void launch_cell_sort_segments(const int* vert_cell, int n, const int* cell_start, const int* perm, int* cell_verts,
-                               hipStream_t s)
+__device__ __forceinline__ void sort_body(const NlistBuild& b, int lb)
 {
-    hipLaunchKernelGGL(k_cell_sort_segments, dim3((n + 255) / 256), dim3(256), 0, s, vert_cell, n, cell_start, perm,
-                       cell_verts);
+    const int i = lb * 256 + threadIdx.x;
+    if (i < b.n) sort_segment(b, i);
+}
+
+// The stencil lists: the vertices of a cell share its rows (place k takes row k,
+// k + the cell's vertices, ...), and each stores its vertex's range.  What bounds it
+// are the lines of the cell table that the rows' ends are on.
+__device__ __forceinline__ void fill_body(const NlistBuild& b, int lb)
+{
+    const int i = lb * 256 + threadIdx.x;
+    if (i >= b.n) return;
+    const int v = b.cell_verts[i], c = b.vert_cell[v];
+    const int s0 = b.nl.cell_start[c], verts = b.nl.cell_start[c + 1] - s0;
+    const StencilRows r = stencil_rows(b.nl, c);
+    const int first = b.cand_start[s0];
+    b.vcand[v] = make_int2(first, b.cand_start[s0 + 1]);
+    int o = first, turn = i - s0;
+#pragma unroll
+    for (int k = 0; k < 9; k++) {
+        if (turn == 0) {
+            for (int q = 0; q < r.len[k]; q++) b.cand[o + q] = b.cell_verts[r.start[k] + q];
+            turn = verts;
+        }
+        turn--;
+        o += r.len[k];
+    }
 }
 
 // ---------------------------------------------------- exclusive scan ------
-// Three phases: block-local scans of 4096 elements with block totals, a scan
-// of the totals by one block, and the add-back.
+// Block-local scans of 4096 elements with block totals, and the add-back of the
+// totals before each block.
 constexpr int kScanThreads = 1024;
 constexpr int kScanItems = 4;
 constexpr int kScanTile = kScanThreads * kScanItems;
@@ -299,23 +276,36 @@ __device__ __forceinline__ int block_exclusive_scan(int v, int* s_warp, int* tot
     return base + x - v;
 }
 
+__device__ __forceinline__ void scan_tile(const int* __restrict__ in, int* __restrict__ out, int n,
+                                          int* __restrict__ sums, int lb)
+{
+    __shared__ int s_warp[16];
+    static_assert(kScanItems == 4, "a thread's elements are one vector");
+    const int base = lb * kScanTile + threadIdx.x * kScanItems;
+    int4 v = make_int4(0, 0, 0, 0);
+    if (base + 3 < n) {
+        v = *reinterpret_cast<const int4*>(in + base);
+    } else {
+        if (base < n) v.x = in[base];
+        if (base + 1 < n) v.y = in[base + 1];
+        if (base + 2 < n) v.z = in[base + 2];
+    }
+    int total;
+    const int off = block_exclusive_scan(v.x + v.y + v.z + v.w, s_warp, &total);
+    const int4 o = make_int4(off, off + v.x, off + v.x + v.y, off + v.x + v.y + v.z);
+    if (base + 3 < n) {
+        *reinterpret_cast<int4*>(out + base) = o;
+    } else {
+        if (base < n) out[base] = o.x;
+        if (base + 1 < n) out[base + 1] = o.y;
+        if (base + 2 < n) out[base + 2] = o.z;
+    }
+    if (threadIdx.x == 0) sums[lb] = total;
+}
 __global__ void __launch_bounds__(kScanThreads) k_scan_tiles(const int* __restrict__ in, int* __restrict__ out,
                                                              int n, int* __restrict__ sums)
 {
-    __shared__ int s_warp[16];
-    const int base = blockIdx.x * kScanTile + threadIdx.x * kScanItems;
-    int loc[kScanItems];
-    int acc = 0;
-    for (int k = 0; k < kScanItems; k++) {
-        int v = (base + k < n) ? in[base + k] : 0;
-        loc[k] = acc;
-        acc += v;
-    }
-    int total;
-    int off = block_exclusive_scan(acc, s_warp, &total);
-    for (int k = 0; k < kScanItems; k++)
-        if (base + k < n) out[base + k] = off + loc[k];
-    if (threadIdx.x == 0) sums[blockIdx.x] = total;
+    scan_tile(in, out, n, sums, blockIdx.x);
 }
 
 __global__ void __launch_bounds__(kScanThreads) k_scan_sums(int* __restrict__ sums, int nb)
@@ -334,19 +324,148 @@ __global__ void __launch_bounds__(kScanThreads) k_scan_sums(int* __restrict__ su
     if (threadIdx.x == 0) sums[nb] = carry;
 }
 
-__global__ void k_scan_add(int* __restrict__ out, int n, const int* __restrict__ sums)
+// The add-back of tile lb.  Every workgroup adds up the totals before it for
+// itself (few, and read once each), which saves the launch that scans them;
+// kScanned: that launch has run (more than kSumTiles tiles).
+constexpr int kSumTiles = 2048;
+template <bool kScanned>
+__device__ __forceinline__ void scan_add(int* __restrict__ out, int n, const int* __restrict__ sums, int lb)
 {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) out[i] += sums[i / kScanTile];
+    __shared__ int s_part[kScanThreads / 64];
+    int before = 0;
+    if constexpr (kScanned) {
+        before = sums[lb];
+    } else {
+        for (int i = threadIdx.x; i < lb; i += kScanThreads) before += sums[i];
+        for (int off = 32; off > 0; off >>= 1) before += __shfl_xor(before, off, 64);
+        if ((threadIdx.x & 63) == 0) s_part[threadIdx.x >> 6] = before;
+        __syncthreads();
+        before = 0;
+        for (int w = 0; w < kScanThreads / 64; w++) before += s_part[w];
+    }
+    for (int k = 0; k < kScanItems; k++) {
+        const int i = lb * kScanTile + k * kScanThreads + threadIdx.x;
+        if (i < n) out[i] += before;
+    }
+}
+template <bool kScanned>
+__global__ void __launch_bounds__(kScanThreads) k_scan_add(int* __restrict__ out, int n, const int* __restrict__ sums)
+{
+    scan_add<kScanned>(out, n, sums, blockIdx.x);
 }
 
 void launch_exclusive_scan(const int* in, int* out, int n, int* block_sums, hipStream_t s)
 {
-    int nb = (n + kScanTile - 1) / kScanTile;
+    const int nb = (n + kScanTile - 1) / kScanTile;
     hipLaunchKernelGGL(k_scan_tiles, dim3(nb), dim3(kScanThreads), 0, s, in, out, n, block_sums);
-    hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(kScanThreads), 0, s, block_sums, nb);
-    hipLaunchKernelGGL(k_scan_add, dim3((n + 255) / 256), dim3(256), 0, s, out, n, block_sums);
+    if (nb > kSumTiles) {
+        hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(kScanThreads), 0, s, block_sums, nb);
+        hipLaunchKernelGGL(k_scan_add<true>, dim3(nb), dim3(kScanThreads), 0, s, out, n, block_sums);
+    } else {
+        hipLaunchKernelGGL(k_scan_add<false>, dim3(nb), dim3(kScanThreads), 0, s, out, n, block_sums);
+    }
 }
+
+// the build's two scans: the cells' counts, and the stencil sizes, whose add-back
+// launch also sorts the cells' segments
+__device__ __forceinline__ void cell_tiles_body(const NlistBuild& b, int lb)
+{
+    scan_tile(b.counts, b.cell_start, b.nc + 1, b.sums, lb);
+}
+__device__ __forceinline__ void cell_starts_body(const NlistBuild& b, int lb)
+{
+    scan_add<false>(b.cell_start, b.nc + 1, b.sums, lb);
+}
+__device__ __forceinline__ void cand_tiles_body(const NlistBuild& b, int lb)
+{
+    scan_tile(b.cand_count, b.cand_start, b.n + 1, b.sums, lb);
+}
+__device__ __forceinline__ void cand_starts_body(const NlistBuild& b, int lb)
+{
+    scan_add<false>(b.cand_start, b.n + 1, b.sums, lb);
+    for (int k = 0; k < kScanItems; k++) {
+        const int i = lb * kScanTile + k * kScanThreads + threadIdx.x;
+        if (i < b.n) sort_segment(b, i);
+    }
+}
+
+// ---------------------------------------------------------- the build ----
+#define TM_BUILD_KERNEL(name, threads)                                                                          \
+    __global__ void __launch_bounds__(threads) k_nl_##name(NlistBuild b) { name##_body(b, blockIdx.x); }        \
+    __global__ void __launch_bounds__(threads) k_nl_##name##_grouped(const NlistBuild* __restrict__ b,          \
+                                                                    const int* __restrict__ block0, int R)      \
+    {                                                                                                           \
+        const int r = find_replica(block0, R, blockIdx.x);                                                      \
+        name##_body(b[r], (int)blockIdx.x - block0[r]);                                                         \
+    }
+TM_BUILD_KERNEL(box, 256)
+TM_BUILD_KERNEL(clear, 256)
+TM_BUILD_KERNEL(cells, 256)
+TM_BUILD_KERNEL(cell_tiles, kScanThreads)
+TM_BUILD_KERNEL(cell_starts, kScanThreads)
+TM_BUILD_KERNEL(scatter, 256)
+TM_BUILD_KERNEL(sort, 256)
+TM_BUILD_KERNEL(cand_tiles, kScanThreads)
+TM_BUILD_KERNEL(cand_starts, kScanThreads)
+TM_BUILD_KERNEL(fill, 256)
+#undef TM_BUILD_KERNEL
+
+static int ceil_div(int a, int b) { return (a + b - 1) / b; }
+int nlist_blocks(const NlistBuild& b, int shape)
+{
+    switch (shape) {
+    case kShapeBox: return kBoxBlocks;
+    case kShapeVerts: return ceil_div(b.n, 256);
+    case kShapeCells: return ceil_div(b.nc + 1, kScanTile);
+    case kShapeCand: return b.cand ? ceil_div(b.n + 1, kScanTile) : 0;
+    case kShapeVertsCand: return b.cand ? ceil_div(b.n, 256) : 0;
+    case kShapeVertsSort: return b.cand ? 0 : ceil_div(b.n, 256);
+    default: return b.cand ? ceil_div(b.n * kPairLanes, 256) : 0;    // kShapeMask
+    }
+}
+static_assert(kClearTile == kScanTile, "kShapeCells");
+
+#define TM_BUILD_LAUNCH(name, shape, threads)                                                                   \
+    if (g.total[shape] > 0) {                                                                                   \
+        if (g.R == 1)                                                                                           \
+            hipLaunchKernelGGL(k_nl_##name, dim3(g.total[shape]), dim3(threads), 0, s, g.h[0]);                 \
+        else                                                                                                    \
+            hipLaunchKernelGGL(k_nl_##name##_grouped, dim3(g.total[shape]), dim3(threads), 0, s, g.d,           \
+                               g.block0 + shape * (g.R + 1), g.R);                                              \
+    }
+void launch_nlist_box(const NlistGroup& g, hipStream_t s) { TM_BUILD_LAUNCH(box, kShapeBox, 256) }
+void launch_nlist_build(const NlistGroup& g, hipStream_t s)
+{
+    TM_BUILD_LAUNCH(clear, kShapeCells, 256)
+    TM_BUILD_LAUNCH(cells, kShapeVerts, 256)
+    int tiles = 0;
+    for (int r = 0; r < g.R; r++) tiles = std::max(tiles, nlist_blocks(g.h[r], kShapeCells));
+    if (tiles > kSumTiles) {
+        for (int r = 0; r < g.R; r++)
+            launch_exclusive_scan(g.h[r].counts, g.h[r].cell_start, g.h[r].nc + 1, g.h[r].sums, s);
+    } else {
+        TM_BUILD_LAUNCH(cell_tiles, kShapeCells, kScanThreads)
+        TM_BUILD_LAUNCH(cell_starts, kShapeCells, kScanThreads)
+    }
+    TM_BUILD_LAUNCH(scatter, kShapeVerts, 256)
+    TM_BUILD_LAUNCH(sort, kShapeVertsSort, 256)
+    // (at most 2^31 / 27 vertices: 19419 tiles)
+    tiles = 0;
+    for (int r = 0; r < g.R; r++) tiles = std::max(tiles, nlist_blocks(g.h[r], kShapeCand));
+    if (tiles > kSumTiles) {
+        for (int r = 0; r < g.R; r++)
+            if (g.h[r].cand) {
+                launch_exclusive_scan(g.h[r].cand_count, g.h[r].cand_start, g.h[r].n + 1, g.h[r].sums, s);
+                hipLaunchKernelGGL(k_nl_sort, dim3(nlist_blocks(g.h[r], kShapeVerts)), dim3(256), 0, s, g.h[r]);
+            }
+    } else {
+        TM_BUILD_LAUNCH(cand_tiles, kShapeCand, kScanThreads)
+        TM_BUILD_LAUNCH(cand_starts, kShapeCand, kScanThreads)
+    }
+    TM_BUILD_LAUNCH(fill, kShapeVertsCand, 256)
+    launch_nlist_masks(g, s);
+}
+#undef TM_BUILD_LAUNCH
 
 // ------------------------------------------------------ distance matrix ---
 __device__ __forceinline__ double dist_ab(const double* x, int a, int b)
