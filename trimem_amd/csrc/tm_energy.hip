@@ -119,19 +119,6 @@ __device__ __forceinline__ d3 load_p(const double* __restrict__ x, int v)
     return d3{x[3 * v], x[3 * v + 1], x[3 * v + 2]};
 }
 
-// ------------------------------------------------------- block mapping ---
-// Workgroups are dispatched round-robin over the 8 XCDs (block b on XCD
-// b % 8), each with its own L2.  Launching a multiple of 8 blocks and giving
-// XCD x the logical blocks [x * G/8, (x+1) * G/8) makes each XCD work on one
-// contiguous range of (spatially ordered) vertices, so its L2 holds that
-// region and its halo instead of a slice of the whole mesh.
-constexpr int kXcds = 8;
-__device__ __forceinline__ int logical_block()
-{
-    const int chunk = gridDim.x / kXcds;
-    return (blockIdx.x % kXcds) * chunk + blockIdx.x / kXcds;
-}
-
 // ------------------------------------------------------------ reduction ---
 // Column k of block_sum6 alone, by the same operations in the same order (a
 // butterfly within each wave, then the waves in order), so its bits are those
@@ -575,7 +562,7 @@ __device__ __forceinline__ void record_neighbours(const MeshView& m, const NList
     const int word = group_sum(min(rec, kPairCap) << (4 * lane));
     const int cell = query_cell(nl, pi);
     if (lane == 0) {
-        pc.cnt[v] = (unsigned)word;
+        pc.cnt[v] = word;
         pc.cell[v] = over == 0 ? cell : -1;
     }
 }
@@ -699,19 +686,21 @@ __device__ __forceinline__ void excl_mask_body(const MeshView& m, const NListVie
 
 __global__ void __launch_bounds__(256) k_excl_mask(MeshView m, NListView nl, unsigned long long* __restrict__ mask)
 {
-    excl_mask_body(m, nl, mask, blockIdx.x);
+    excl_mask_body(m, nl, mask, logical_block());
 }
 __global__ void __launch_bounds__(256) k_excl_mask_grouped(const NlistBuild* __restrict__ b,
                                                            const int* __restrict__ block0, int R)
 {
-    const int r = find_replica(block0, R, blockIdx.x);
-    excl_mask_body(b[r].m, b[r].nl, b[r].mask, (int)blockIdx.x - block0[r]);
+    const int lb = logical_block();
+    if (lb >= block0[R]) return;
+    const int r = find_replica(block0, R, lb);
+    excl_mask_body(b[r].m, b[r].nl, b[r].mask, lb - block0[r]);
 }
 
 void launch_excl_mask(const MeshView& m, const NListView& nl, unsigned long long* mask, hipStream_t s)
 {
     if (m.nv <= 0) return;
-    hipLaunchKernelGGL(k_excl_mask, dim3((m.nv * kGroup + 255) / 256), dim3(256), 0, s, m, nl, mask);
+    hipLaunchKernelGGL(k_excl_mask, dim3(tuned_blocks(m.nv, 256)), dim3(256), 0, s, m, nl, mask);
 }
 
 void launch_nlist_masks(const NlistGroup& g, hipStream_t s)
@@ -719,7 +708,7 @@ void launch_nlist_masks(const NlistGroup& g, hipStream_t s)
     if (g.total[kShapeMask] <= 0) return;
     if (g.R == 1) launch_excl_mask(g.h[0].m, g.h[0].nl, g.h[0].mask, s);
     else
-        hipLaunchKernelGGL(k_excl_mask_grouped, dim3(g.total[kShapeMask]), dim3(256), 0, s, g.d,
+        hipLaunchKernelGGL(k_excl_mask_grouped, dim3((g.total[kShapeMask] + kXcds - 1) / kXcds * kXcds), dim3(256), 0, s, g.d,
                            g.block0 + kShapeMask * (g.R + 1), g.R);
 }
 
@@ -1004,7 +993,7 @@ __global__ void __launch_bounds__(kThreads) k_rep(PassArgs A)
 // lane l the pairs that lane l of the query recorded, in their order, and
 // group_sum over the lanes, which gives the bits of the 8-lane query.  A chain of
 // two loads per vertex, its entries as one vector, two vertices of a group in
-// flight: MEASURE_REPLAY
+// flight.
 // Phase 3: the lane groups run the full query (recording when the mode says so)
 // over the second list.  Replays are the common case and want few,
 // full blocks; a recording launch the device decides on (some vertex moved

@@ -62,6 +62,19 @@ struct PassBuffers {
     unsigned* count;    // [kLastCounters] zeros (tm_last.h)
     Globals* globals;
     Globals* host;      // pinned copy of globals the pass also writes; null: none
+// ------------------------------------------------------- block mapping ---
+// Workgroups are dispatched round-robin over the 8 XCDs (block b on XCD
+// b % 8), each with its own L2.  Launching a multiple of 8 blocks and giving
+// XCD x the logical blocks [x * G/8, (x+1) * G/8) makes each XCD work on one
+// contiguous range of (spatially ordered) vertices, so its L2 holds that
+// region and its halo instead of a slice of the whole mesh.
+constexpr int kXcds = 8;
+__device__ __forceinline__ int logical_block()
+{
+    const int chunk = gridDim.x / kXcds;
+    return (blockIdx.x % kXcds) * chunk + blockIdx.x / kXcds;
+}
+
     const int* list;    // boundary / degenerate vertices
     int nlist;
     PairCache pc;       // x_snap null: the query runs in full every time
@@ -203,7 +216,8 @@ struct NlistBuild {
 };
 // Workgroups of a list in the launches of each shape.
 enum {
-    kShapeBox, kShapeVerts, kShapeCells, kShapeCand, kShapeVertsCand, kShapeVertsSort, kShapeMask, kShapes
+    kShapeBox, kShapeVerts, kShapeCells, kShapeCand, kShapeStarts, kShapeFill, kShapeVertsSort, kShapeMask,
+    kShapes
 };
 int nlist_blocks(const NlistBuild& b, int shape);
 struct NlistGroup {

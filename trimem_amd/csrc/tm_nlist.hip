@@ -217,27 +217,32 @@ __device__ __forceinline__ void sort_body(const NlistBuild& b, int lb)
     if (i < b.n) sort_segment(b, i);
 }
 
-// The stencil lists: the vertices of a cell share its rows (place k takes row k,
-// k + the cell's vertices, ...), and each stores its vertex's range.  What bounds it
-// are the lines of the cell table that the rows' ends are on.
+// The stencil lists, eight lanes per slot: the slots of a cell take its candidates
+// in turns of eight, each lane its own from its row, and the first lane stores the
+// range of the slot's vertex.  A chain of five loads, whatever the list's length
+// (16.9 us at 163842 vertices, 5.5 at 2562; with one thread per slot copying whole
+// rows 22.5 and 15.1).
 __device__ __forceinline__ void fill_body(const NlistBuild& b, int lb)
 {
-    const int i = lb * 256 + threadIdx.x;
+    const int t = lb * 256 + threadIdx.x, i = t / 8, lane = t % 8;
     if (i >= b.n) return;
     const int v = b.cell_verts[i], c = b.vert_cell[v];
     const int s0 = b.nl.cell_start[c], verts = b.nl.cell_start[c + 1] - s0;
     const StencilRows r = stencil_rows(b.nl, c);
-    const int first = b.cand_start[s0];
-    b.vcand[v] = make_int2(first, b.cand_start[s0 + 1]);
-    int o = first, turn = i - s0;
+    const int first = b.cand_start[s0], total = b.cand_start[s0 + 1] - first;
+    if (lane == 0) b.vcand[v] = make_int2(first, first + total);
+    for (int k = 8 * (i - s0) + lane; k < total; k += 8 * verts) {
+        int q = k, at = 0;
+        bool found = false;
 #pragma unroll
-    for (int k = 0; k < 9; k++) {
-        if (turn == 0) {
-            for (int q = 0; q < r.len[k]; q++) b.cand[o + q] = b.cell_verts[r.start[k] + q];
-            turn = verts;
+        for (int w = 0; w < 9; w++) {
+            if (!found && q < r.len[w]) {
+                at = r.start[w] + q;
+                found = true;
+            }
+            if (!found) q -= r.len[w];
         }
-        turn--;
-        o += r.len[k];
+        b.cand[first + k] = b.cell_verts[at];
     }
 }
 
@@ -382,32 +387,49 @@ __device__ __forceinline__ void cand_tiles_body(const NlistBuild& b, int lb)
 }
 __device__ __forceinline__ void cand_starts_body(const NlistBuild& b, int lb)
 {
-    scan_add<false>(b.cand_start, b.n + 1, b.sums, lb);
-    for (int k = 0; k < kScanItems; k++) {
-        const int i = lb * kScanTile + k * kScanThreads + threadIdx.x;
-        if (i < b.n) sort_segment(b, i);
-    }
+    // a thread per slot, for the sort's sake (at 163842 vertices 28.8 us with
+    // the scan's tiles, 11.3 with these); few totals, so every
+    // workgroup adds up those before its tile
+    __shared__ int s_part[4];
+    const int i = lb * 256 + threadIdx.x;
+    int before = 0;
+    for (int k = threadIdx.x; k < lb * 256 / kScanTile; k += 256) before += b.sums[k];
+    for (int off = 32; off > 0; off >>= 1) before += __shfl_xor(before, off, 64);
+    if ((threadIdx.x & 63) == 0) s_part[threadIdx.x >> 6] = before;
+    __syncthreads();
+    before = s_part[0] + s_part[1] + s_part[2] + s_part[3];
+    if (i <= b.n) b.cand_start[i] += before;
+    if (i < b.n) sort_segment(b, i);
 }
 
 // ---------------------------------------------------------- the build ----
-#define TM_BUILD_KERNEL(name, threads)                                                                          \
-    __global__ void __launch_bounds__(threads) k_nl_##name(NlistBuild b) { name##_body(b, blockIdx.x); }        \
+// kNear: the kernels of vertices and slots, whose neighbours read the same lines
+// (logical_block); their grids are rounded up to it.
+template <bool kNear>
+__device__ __forceinline__ int build_block()
+{
+    return kNear ? logical_block() : (int)blockIdx.x;
+}
+#define TM_BUILD_KERNEL(name, threads, near)                                                                    \
+    __global__ void __launch_bounds__(threads) k_nl_##name(NlistBuild b) { name##_body(b, build_block<near>()); } \
     __global__ void __launch_bounds__(threads) k_nl_##name##_grouped(const NlistBuild* __restrict__ b,          \
                                                                     const int* __restrict__ block0, int R)      \
     {                                                                                                           \
-        const int r = find_replica(block0, R, blockIdx.x);                                                      \
-        name##_body(b[r], (int)blockIdx.x - block0[r]);                                                         \
+        const int lb = build_block<near>();                                                                     \
+        if (lb >= block0[R]) return;                                                                            \
+        const int r = find_replica(block0, R, lb);                                                              \
+        name##_body(b[r], lb - block0[r]);                                                                      \
     }
-TM_BUILD_KERNEL(box, 256)
-TM_BUILD_KERNEL(clear, 256)
-TM_BUILD_KERNEL(cells, 256)
-TM_BUILD_KERNEL(cell_tiles, kScanThreads)
-TM_BUILD_KERNEL(cell_starts, kScanThreads)
-TM_BUILD_KERNEL(scatter, 256)
-TM_BUILD_KERNEL(sort, 256)
-TM_BUILD_KERNEL(cand_tiles, kScanThreads)
-TM_BUILD_KERNEL(cand_starts, kScanThreads)
-TM_BUILD_KERNEL(fill, 256)
+TM_BUILD_KERNEL(box, 256, false)
+TM_BUILD_KERNEL(clear, 256, false)
+TM_BUILD_KERNEL(cells, 256, true)
+TM_BUILD_KERNEL(cell_tiles, kScanThreads, false)
+TM_BUILD_KERNEL(cell_starts, kScanThreads, false)
+TM_BUILD_KERNEL(scatter, 256, true)
+TM_BUILD_KERNEL(sort, 256, true)
+TM_BUILD_KERNEL(cand_tiles, kScanThreads, false)
+TM_BUILD_KERNEL(cand_starts, 256, true)
+TM_BUILD_KERNEL(fill, 256, true)
 #undef TM_BUILD_KERNEL
 
 static int ceil_div(int a, int b) { return (a + b - 1) / b; }
@@ -418,37 +440,39 @@ int nlist_blocks(const NlistBuild& b, int shape)
     case kShapeVerts: return ceil_div(b.n, 256);
     case kShapeCells: return ceil_div(b.nc + 1, kScanTile);
     case kShapeCand: return b.cand ? ceil_div(b.n + 1, kScanTile) : 0;
-    case kShapeVertsCand: return b.cand ? ceil_div(b.n, 256) : 0;
+    case kShapeStarts: return b.cand ? ceil_div(b.n + 1, 256) : 0;
+    case kShapeFill: return b.cand ? ceil_div(b.n, 32) : 0;
     case kShapeVertsSort: return b.cand ? 0 : ceil_div(b.n, 256);
     default: return b.cand ? ceil_div(b.n * kPairLanes, 256) : 0;    // kShapeMask
     }
 }
 static_assert(kClearTile == kScanTile, "kShapeCells");
 
-#define TM_BUILD_LAUNCH(name, shape, threads)                                                                   \
+#define TM_BUILD_LAUNCH(name, shape, threads, near)                                                             \
     if (g.total[shape] > 0) {                                                                                   \
+        const dim3 grid(near ? ceil_div(g.total[shape], kXcds) * kXcds : g.total[shape]);                       \
         if (g.R == 1)                                                                                           \
-            hipLaunchKernelGGL(k_nl_##name, dim3(g.total[shape]), dim3(threads), 0, s, g.h[0]);                 \
+            hipLaunchKernelGGL(k_nl_##name, grid, dim3(threads), 0, s, g.h[0]);                                 \
         else                                                                                                    \
-            hipLaunchKernelGGL(k_nl_##name##_grouped, dim3(g.total[shape]), dim3(threads), 0, s, g.d,           \
+            hipLaunchKernelGGL(k_nl_##name##_grouped, grid, dim3(threads), 0, s, g.d,                           \
                                g.block0 + shape * (g.R + 1), g.R);                                              \
     }
-void launch_nlist_box(const NlistGroup& g, hipStream_t s) { TM_BUILD_LAUNCH(box, kShapeBox, 256) }
+void launch_nlist_box(const NlistGroup& g, hipStream_t s) { TM_BUILD_LAUNCH(box, kShapeBox, 256, false) }
 void launch_nlist_build(const NlistGroup& g, hipStream_t s)
 {
-    TM_BUILD_LAUNCH(clear, kShapeCells, 256)
-    TM_BUILD_LAUNCH(cells, kShapeVerts, 256)
+    TM_BUILD_LAUNCH(clear, kShapeCells, 256, false)
+    TM_BUILD_LAUNCH(cells, kShapeVerts, 256, true)
     int tiles = 0;
     for (int r = 0; r < g.R; r++) tiles = std::max(tiles, nlist_blocks(g.h[r], kShapeCells));
     if (tiles > kSumTiles) {
         for (int r = 0; r < g.R; r++)
             launch_exclusive_scan(g.h[r].counts, g.h[r].cell_start, g.h[r].nc + 1, g.h[r].sums, s);
     } else {
-        TM_BUILD_LAUNCH(cell_tiles, kShapeCells, kScanThreads)
-        TM_BUILD_LAUNCH(cell_starts, kShapeCells, kScanThreads)
+        TM_BUILD_LAUNCH(cell_tiles, kShapeCells, kScanThreads, false)
+        TM_BUILD_LAUNCH(cell_starts, kShapeCells, kScanThreads, false)
     }
-    TM_BUILD_LAUNCH(scatter, kShapeVerts, 256)
-    TM_BUILD_LAUNCH(sort, kShapeVertsSort, 256)
+    TM_BUILD_LAUNCH(scatter, kShapeVerts, 256, true)
+    TM_BUILD_LAUNCH(sort, kShapeVertsSort, 256, true)
     // (at most 2^31 / 27 vertices: 19419 tiles)
     tiles = 0;
     for (int r = 0; r < g.R; r++) tiles = std::max(tiles, nlist_blocks(g.h[r], kShapeCand));
@@ -456,13 +480,14 @@ void launch_nlist_build(const NlistGroup& g, hipStream_t s)
         for (int r = 0; r < g.R; r++)
             if (g.h[r].cand) {
                 launch_exclusive_scan(g.h[r].cand_count, g.h[r].cand_start, g.h[r].n + 1, g.h[r].sums, s);
-                hipLaunchKernelGGL(k_nl_sort, dim3(nlist_blocks(g.h[r], kShapeVerts)), dim3(256), 0, s, g.h[r]);
+                hipLaunchKernelGGL(k_nl_sort, dim3(ceil_div(nlist_blocks(g.h[r], kShapeVerts), kXcds) * kXcds), dim3(256),
+                                   0, s, g.h[r]);
             }
     } else {
-        TM_BUILD_LAUNCH(cand_tiles, kShapeCand, kScanThreads)
-        TM_BUILD_LAUNCH(cand_starts, kShapeCand, kScanThreads)
+        TM_BUILD_LAUNCH(cand_tiles, kShapeCand, kScanThreads, false)
+        TM_BUILD_LAUNCH(cand_starts, kShapeStarts, 256, true)
     }
-    TM_BUILD_LAUNCH(fill, kShapeVertsCand, 256)
+    TM_BUILD_LAUNCH(fill, kShapeFill, 256, true)
     launch_nlist_masks(g, s);
 }
 #undef TM_BUILD_LAUNCH
