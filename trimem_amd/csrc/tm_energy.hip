@@ -541,11 +541,49 @@ __device__ __forceinline__ int pair_cache_mode(const PairCache& pc, const NListV
     return s_mode;
 }
 
+// Whether vertex v, recorded at pi in cell c, has a non-excluded candidate within
+// `radius` in the stencil of another cell that it reaches while it is slow (the
+// cells of pi -+ kPairLimit skin), by its lane group.
+__device__ __forceinline__ bool candidate_around(const MeshView& m, const NListView& nl, const PairCache& pc, int v,
+                                                 int n, d3 pi, double radius, int lane)
+{
+    const double reach = kPairLimit * pc.skin * (1.0 + 1e-12);
+    int c[3], lo[3], hi[3];
+    cell_coords(nl, pi, c);
+    cell_coords(nl, d3{pi.x - reach, pi.y - reach, pi.z - reach}, lo);
+    cell_coords(nl, d3{pi.x + reach, pi.y + reach, pi.z + reach}, hi);
+    if (lo[0] == hi[0] && lo[1] == hi[1] && lo[2] == hi[2]) return false;
+    const RingRegs R = load_ring(m, v, n);
+    const double r2 = radius * radius * (1.0 + 1e-15);
+    const int ny = hi[1] - lo[1] + 3, nz = hi[2] - lo[2] + 3;
+    int found = 0;
+    for (int i = lane; i < ny * nz && !found; i += kGroup) {
+        const int y = lo[1] - 1 + i % ny, z = lo[2] - 1 + i / ny;
+        if (y < 0 || y >= nl.shape[1] || z < 0 || z >= nl.shape[2]) continue;
+        const int base = y * nl.strides[1] + z * nl.strides[2];
+        const bool own = abs(y - c[1]) <= 1 && abs(z - c[2]) <= 1;    // its middle cells were searched
+        for (int side = 0; side < (own ? 2 : 1); side++) {
+            const int x0 = max(own && side == 1 ? c[0] + 2 : lo[0] - 1, 0);
+            const int x1 = min(own && side == 0 ? c[0] - 2 : hi[0] + 1, nl.shape[0] - 1);
+            if (x0 > x1) continue;
+            const int end = nl.cell_start[base + x1 + 1];
+            for (int q = nl.cell_start[base + x0]; q < end; q++) {
+                const int j = nl.cell_verts[q];
+                const d3 d = pi - load_p(m.x, j);
+                const double sq = sqnorm(d);
+                if (!(sq > r2) && !excluded_fast(m, R, v, j, nl.exclusion)) found = 1;
+            }
+        }
+    }
+    return group_sum(found) > 0;
+}
+
 // The full query with radius dmax + skin, keeping each lane's non-excluded
 // candidates in its visit order; f sees the pairs within dmax, in the order
 // and with the test of the plain query.  Lane 0 stores the counts and the
-// cell the lists are valid in (-1 when a lane overflows).
-template <int kBatch, class F>
+// cell the lists are valid in (-1 when a lane overflows).  kAround: look for
+// candidates that the vertex may reach too (pi is the snapshot's position).
+template <int kBatch, bool kAround = false, class F>
 __device__ __forceinline__ void record_neighbours(const MeshView& m, const NListView& nl, const PairCache& pc, int v,
                                                   int n, d3 pi, double dmax, int lane, F&& f)
 {
@@ -559,8 +597,9 @@ __device__ __forceinline__ void record_neighbours(const MeshView& m, const NList
         if (sq <= dmax2 && sqrt(sq) < dmax) f(j, d);
     });
     const int over = group_sum(rec > kPairCap ? 1 : 0);
-    const int word = group_sum(min(rec, kPairCap) << (4 * lane));
+    unsigned word = (unsigned)group_sum(min(rec, kPairCap) << (4 * lane));
     const int cell = query_cell(nl, pi);
+    if (kAround && word == 0u && !candidate_around(m, nl, pc, v, n, pi, dmax + pc.skin, lane)) word = kEmptyAround;
     if (lane == 0) {
         pc.cnt[v] = word;
         pc.cell[v] = over == 0 ? cell : -1;
@@ -1194,8 +1233,9 @@ __device__ __forceinline__ void rep_cached_body(const PassArgs& A, int lb)
             }
             const int cell = rec_cell;
             const unsigned word = rec_word;
-            const bool replay = keep && cell != -1 && query_cell(A.nl, xv) == cell;
-            if (replay && word == 0u) {
+            const bool around = keep && cell != -1 && word == kEmptyAround;
+            const bool replay = around || (keep && cell != -1 && query_cell(A.nl, xv) == cell);
+            if (around || (replay && word == 0u)) {
                 done = true;    // nothing recorded: no pairs (the sums over none are +0)
             } else if (replay) {
                 const int at = atomicAdd(&s_nrep, 1);
@@ -1333,7 +1373,7 @@ __global__ void __launch_bounds__(256) k_rep_cached_grouped(const PassArgs* __re
 // A recording launch the host asks for (new list or topology): the layout
 // of k_rep (32 vertices per block, one lane group each), recording every
 // ring vertex's lists and every vertex's position.
-template <int kBatch>
+template <int kBatch, bool kAround>
 __global__ void __launch_bounds__(256) k_rep_record(PassArgs A)
 {
     const MeshView& m = A.m;
@@ -1357,8 +1397,8 @@ __global__ void __launch_bounds__(256) k_rep_record(PassArgs A)
             if (!ring) pc.cell[v] = -1;
         }
         if (ring)
-            record_neighbours<kBatch>(m, A.nl, pc, v, meta_valence(meta), xv, p.rep_lc1, lane,
-                                      [&](int, d3 d) { tr.add(d, p); });
+            record_neighbours<kBatch, kAround>(m, A.nl, pc, v, meta_valence(meta), xv, p.rep_lc1, lane,
+                                               [&](int, d3 d) { tr.add(d, p); });
     }
     tr.group_reduce();
     const double rep = tr.rep;
@@ -1770,6 +1810,17 @@ void launch_pass1_body(const PassArgs& a, int mixed, const Tuning& t, hipStream_
     else launch_marked(k_pass1<double>, grid, block, s, marks, a);
 }
 
+template <bool kAround>
+static void record_dispatch(const Tuning& t, dim3 grid, dim3 block, const PassArgs& a, hipStream_t s)
+{
+    switch (t.rep_batch) {
+    case 1: hipLaunchKernelGGL((k_rep_record<1, kAround>), grid, block, 0, s, a); break;
+    case 2: hipLaunchKernelGGL((k_rep_record<2, kAround>), grid, block, 0, s, a); break;
+    case 8: hipLaunchKernelGGL((k_rep_record<8, kAround>), grid, block, 0, s, a); break;
+    default: hipLaunchKernelGGL((k_rep_record<4, kAround>), grid, block, 0, s, a); break;
+    }
+}
+
 void launch_rep(const PassArgs& a, const Tuning& t, hipStream_t s)
 {
     if (!a.rep_v || a.m.nv == 0) return;
@@ -1780,12 +1831,8 @@ void launch_rep(const PassArgs& a, const Tuning& t, hipStream_t s)
     const dim3 block(256);
     if (a.pc.force) {
         const dim3 grid(tuned_blocks(a.m.nv, 256));
-        switch (t.rep_batch) {
-        case 1: hipLaunchKernelGGL(k_rep_record<1>, grid, block, 0, s, a); break;
-        case 2: hipLaunchKernelGGL(k_rep_record<2>, grid, block, 0, s, a); break;
-        case 8: hipLaunchKernelGGL(k_rep_record<8>, grid, block, 0, s, a); break;
-        default: hipLaunchKernelGGL(k_rep_record<4>, grid, block, 0, s, a); break;
-        }
+        if (a.m.nv <= kAroundVerts) record_dispatch<true>(t, grid, block, a, s);
+        else record_dispatch<false>(t, grid, block, a, s);
         return;
     }
     const dim3 grid(nblocks(nblocks(a.m.nv, kVertsPerBlock), kXcds) * kXcds);

@@ -33,6 +33,17 @@ constexpr double kPairSkin = 0.2;  // skin = 0.2 lc1
 // different times: a pair's distance then changed by at most 4 x 0.25 skin since
 // either list was recorded.
 constexpr double kPairLimit = 0.25;
+// Recorded counts of a vertex without a non-excluded candidate within lc1 + skin
+// in the stencil of any cell that a slow vertex can be in: no pairs, whichever of
+// them it is in.
+constexpr unsigned kEmptyAround = 0xf0000000u;    // no count reaches 15
+// Looked for by recordings of meshes of at most this many vertices.  It costs the
+// recording a chain of loads and spares the replays that of the vertices that
+// change cells: at 2562 vertices a recording takes 15.3 us instead of 7.0, the
+// queries of a trajectory 9.9 instead of 13.9 each.  At 163842, where a recording
+// is bound by its loads, a step with its ten queries takes as long with it as
+// without.
+constexpr int kAroundVerts = 16384;
 // More fast vertices than this in one block, or in all, record all lists again.
 constexpr int kFastSeg = 32, kFastMax = 256, kFastRow = kFastSeg + 1;
 struct PairCache {
@@ -51,17 +62,6 @@ struct PairCache {
 constexpr int kCachedVerts = 256;    // vertices per block of the cached query
 constexpr int kPass1Verts = 256;     // vertices (one lane each) per block of pass 1
 
-// energy passes (tm_energy.hip)
-struct PassBuffers {
-    double* q;          // [N] curvature / area per vertex
-    double* gprops;     // [6N] properties of listed (boundary) vertices
-    int* pair_cnt;      // [N] repulsion pairs per vertex (k_rep)
-    double* rep_v;      // [N] repulsion property per vertex (k_rep)
-    double* rep_g;      // [3N] repulsion gradient, rows of vertices with pairs (k_rep)
-    double* partials;   // [6 * pass1 blocks]
-    unsigned* count;    // [kLastCounters] zeros (tm_last.h)
-    Globals* globals;
-    Globals* host;      // pinned copy of globals the pass also writes; null: none
 // ------------------------------------------------------- block mapping ---
 // Workgroups are dispatched round-robin over the 8 XCDs (block b on XCD
 // b % 8), each with its own L2.  Launching a multiple of 8 blocks and giving
@@ -75,6 +75,17 @@ __device__ __forceinline__ int logical_block()
     return (blockIdx.x % kXcds) * chunk + blockIdx.x / kXcds;
 }
 
+// energy passes (tm_energy.hip)
+struct PassBuffers {
+    double* q;          // [N] curvature / area per vertex
+    double* gprops;     // [6N] properties of listed (boundary) vertices
+    int* pair_cnt;      // [N] repulsion pairs per vertex (k_rep)
+    double* rep_v;      // [N] repulsion property per vertex (k_rep)
+    double* rep_g;      // [3N] repulsion gradient, rows of vertices with pairs (k_rep)
+    double* partials;   // [6 * pass1 blocks]
+    unsigned* count;    // [kLastCounters] zeros (tm_last.h)
+    Globals* globals;
+    Globals* host;      // pinned copy of globals the pass also writes; null: none
     const int* list;    // boundary / degenerate vertices
     int nlist;
     PairCache pc;       // x_snap null: the query runs in full every time
