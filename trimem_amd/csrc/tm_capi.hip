@@ -207,7 +207,14 @@ struct tm_mesh {
     // device state
     bool dev = false;
     DevBuf<double> x;
-    DevBuf<int> d_to, d_next, d_prev, d_face, d_vhe, d_fhe, ring, meta, flag;
+    DevBuf<int> d_to, d_next, d_prev, d_face, d_vhe, d_fhe, ring, meta;
+    // what the host waits for after a sweep
+    struct Report {
+        int overflow;         // a vertex has more neighbours than the ring table has columns
+        SerialState serial;
+        double parallel[8];
+    };
+    HostBuf<Report> report;
     // vertices evaluated by the half-edge walker: boundary, isolated or with
     // fewer than three neighbours (flips preserve this set on valid meshes)
     DevBuf<int> generic;
@@ -377,6 +384,15 @@ void reorder_vertices(tm_mesh& M)
     M.v_he.swap(vhe);
 }
 
+// the ring table of the current half-edge arrays; report->overflow is set when
+// this has run
+void queue_ring(tm_mesh& M)
+{
+    M.report.p->overflow = 0;
+    launch_build_ring(M.view(), M.ring.p, M.meta.p, &M.report.p->overflow, g_rt.stream);
+    check_launch();
+}
+
 void ensure_device(tm_mesh& M)
 {
     ensure_runtime();
@@ -394,7 +410,7 @@ void ensure_device(tm_mesh& M)
     M.d_iperm.alloc(M.nv);
     h2d(M.d_perm.p, M.perm.data(), sizeof(int) * M.nv);
     h2d(M.d_iperm.p, M.iperm.data(), sizeof(int) * M.nv);
-    M.flag.alloc(4);
+    M.report.alloc(1);
     h2d(M.d_to.p, M.he_to.data(), sizeof(int) * M.nh);
     h2d(M.d_next.p, M.he_next.data(), sizeof(int) * M.nh);
     h2d(M.d_prev.p, M.he_prev.data(), sizeof(int) * M.nh);
@@ -418,13 +434,9 @@ void ensure_device(tm_mesh& M)
     M.n_generic = (int)gl.size();
     M.generic.alloc(std::max<size_t>(gl.size(), 1));
     h2d(M.generic.p, gl.data(), sizeof(int) * gl.size());
-    HIPCHECK(hipMemsetAsync(M.flag.p, 0, sizeof(int) * 4, g_rt.stream));
-    launch_build_ring(M.view(), M.ring.p, M.meta.p, M.flag.p, g_rt.stream);
-    check_launch();
-    int ovf = 0;
-    d2h(&ovf, M.flag.p, sizeof(int));
+    queue_ring(M);
     sync();
-    if (ovf) throw TmError(TM_E_UNSUPPORTED, "vertex valence exceeds the ring-table width (32)");
+    if (M.report.p->overflow) throw TmError(TM_E_UNSUPPORTED, "vertex valence exceeds the ring-table width (32)");
     M.dev = true;
 }
 
@@ -1471,8 +1483,10 @@ static PflipArgs pflip_args(tm_energy& E, tm_mesh& M, const EParams& ep, uint64_
 // The serial sweep in windows of W proposals (launch_serial_windows).  The
 // number of windows a sweep needs depends on how many proposals each
 // commits, so they are launched in batches sized from the rate so far, with
-// the state read back between batches; surplus windows return at once.
-static void serial_windows(tm_energy& E, tm_mesh& M, int nflips, const int* proposals, const double* uniforms,
+// the state read back between batches; surplus windows return at once.  The ring
+// table is rebuilt behind each batch (the sweep does not read it), so that after
+// the last one the host has waited for everything.
+static SerialState serial_windows(tm_energy& E, tm_mesh& M, int nflips, const int* proposals, const double* uniforms,
                            int n_uniforms, uint64_t seed, int injected, int W)
 {
     const size_t w = (size_t)W;
@@ -1484,19 +1498,18 @@ static void serial_windows(tm_energy& E, tm_mesh& M, int nflips, const int* prop
     const NListView nl = E.nlist->view();
     launch_serial_begin(M.flip_view(), rows, E.globals.p, p, nflips, E.sf_state.p, E.sf_fstamp.p, g_rt.stream);
     int batch = std::max(1, std::min(1024, nflips / W + 1));
-    SerialState h{};
     for (;;) {
         launch_serial_windows(M.flip_view(), rows, nl, p, nflips, proposals, uniforms, n_uniforms, seed, injected, W,
                               E.sf_state.p, E.sf_rec.p, E.sf_fstamp.p, batch, g_rt.stream);
         check_launch();
-        d2h(&h, E.sf_state.p, sizeof(SerialState));
+        queue_ring(M);
+        d2h(&M.report.p->serial, E.sf_state.p, sizeof(SerialState));
         sync();
-        if (h.done) break;
+        const SerialState h = M.report.p->serial;
+        if (h.done) return h;
         const double per_window = std::max(1.0, (double)h.pos / std::max(h.window, 1));
         batch = std::min(4096, (int)std::ceil((nflips - h.pos) / per_window * 1.1) + 1);
     }
-    int res[3] = {h.acc, h.used, h.err};
-    h2d(E.flip_result.p, res, sizeof(res));
 }
 
 static int flip_impl(tm_energy* em, tm_mesh* mesh, int nflips, const int* proposals, const double* uniforms,
@@ -1513,23 +1526,24 @@ static int flip_impl(tm_energy* em, tm_mesh* mesh, int nflips, const int* propos
         if (n_uniforms > 0) h2d(em->uniforms.p, uniforms, sizeof(double) * n_uniforms);
     }
     const int W = em->tune.serial_window;
+    int res[3] = {0, 0, 0};
     if (W == 0) {
         launch_flip_serial(mesh->flip_view(), em->nlist->view(), eparams_of(*em), nflips,
                            injected ? em->proposals.p : nullptr, injected ? em->uniforms.p : nullptr, n_uniforms,
                            seed, injected, em->globals.p, em->flip_result.p, g_rt.stream);
         check_launch();
+        queue_ring(*mesh);
+        d2h(res, em->flip_result.p, sizeof(res));
+        sync();
     } else {
-        serial_windows(*em, *mesh, nflips, injected ? em->proposals.p : nullptr, injected ? em->uniforms.p : nullptr,
-                       n_uniforms, seed, injected, W);
+        const SerialState st =
+            serial_windows(*em, *mesh, nflips, injected ? em->proposals.p : nullptr,
+                           injected ? em->uniforms.p : nullptr, n_uniforms, seed, injected, W);
+        res[0] = st.acc;
+        res[1] = st.used;
+        res[2] = st.err;
     }
-    HIPCHECK(hipMemsetAsync(mesh->flag.p, 0, sizeof(int), g_rt.stream));
-    launch_build_ring(mesh->view(), mesh->ring.p, mesh->meta.p, mesh->flag.p, g_rt.stream);
-    check_launch();
-    int res[4] = {0, 0, 0, 0};
-    d2h(res, em->flip_result.p, sizeof(int) * 3);
-    int ovf = 0;
-    d2h(&ovf, mesh->flag.p, sizeof(int));
-    sync();
+    const int ovf = mesh->report.p->overflow;
     mesh->host_stale = true;
     if (res[0] > 0 || res[2] != 0 || ovf) mesh->topo_version++;   // only accepted flips change topology
     if (res[2] == 1) throw TmError(TM_E_INVALID, "flip proposal out of range");
@@ -1556,14 +1570,12 @@ int tm_flip_parallel(tm_energy* em, tm_mesh* mesh, double flip_ratio, uint64_t s
         launch_flip_parallel(pflip_args(*em, *mesh, eparams_of(*em), seed, nflips, batch), em->tune.pflip_window,
                              g_rt.stream);
     check_launch();
-    HIPCHECK(hipMemsetAsync(mesh->flag.p, 0, sizeof(int), g_rt.stream));
-    launch_build_ring(mesh->view(), mesh->ring.p, mesh->meta.p, mesh->flag.p, g_rt.stream);
-    check_launch();
-    double st[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    if (nflips > 0) d2h(st, em->pf_state.p, sizeof(st));
-    int ovf = 0;
-    d2h(&ovf, mesh->flag.p, sizeof(int));
+    queue_ring(*mesh);
+    double* st = mesh->report.p->parallel;
+    std::fill(st, st + 8, 0.0);
+    if (nflips > 0) d2h(st, em->pf_state.p, 8 * sizeof(double));
     sync();
+    const int ovf = mesh->report.p->overflow;
     mesh->host_stale = true;
     if (st[7] > 0 || ovf) mesh->topo_version++;
     if (nflips > 0) std::copy(st, st + 8, em->pf_last);
@@ -1743,6 +1755,7 @@ struct tm_replicas {
     // prefix tables (rebuilt by every sweep)
     DevBuf<PflipArgs> pf_args;
     DevBuf<int> pf_block0;
+    HostBuf<double> pf_report;    // [8 R] the sweeps' final states
     std::vector<int> h_ones;
     int total_disp = 0, total_rc = 0;    // displacement partials, cached-query blocks
     std::vector<unsigned> gens;    // each member's tm_energy::gen when the table was built
@@ -1997,25 +2010,24 @@ int tm_replicas_pflip(tm_replicas* rs, double flip_ratio, const uint64_t* seeds,
                        max_nv, max_nh, max_batch};
     launch_flip_parallel_grouped(g, g_rt.stream);
     check_launch();
-    std::vector<double> st(8 * (size_t)S.R, 0.0);
-    std::vector<int> ovf(S.R, 0);
+    S.pf_report.alloc(8 * (size_t)S.R);
+    std::fill(S.pf_report.p, S.pf_report.p + 8 * (size_t)S.R, 0.0);
     for (int r = 0; r < S.R; r++) {
         tm_mesh& M = *S.meshes[r];
-        HIPCHECK(hipMemsetAsync(M.flag.p, 0, sizeof(int), g_rt.stream));
-        launch_build_ring(M.view(), M.ring.p, M.meta.p, M.flag.p, g_rt.stream);
-        check_launch();
-        if (h[r].nflips > 0) d2h(&st[8 * (size_t)r], S.ems[r]->pf_state.p, 8 * sizeof(double));
-        d2h(&ovf[r], M.flag.p, sizeof(int));
+        queue_ring(M);
+        if (h[r].nflips > 0) d2h(S.pf_report.p + 8 * (size_t)r, S.ems[r]->pf_state.p, 8 * sizeof(double));
     }
     sync();
     bool overflow = false;
     for (int r = 0; r < S.R; r++) {
         tm_mesh& M = *S.meshes[r];
+        const double* st = S.pf_report.p + 8 * (size_t)r;
+        const int ovf = M.report.p->overflow;
         M.host_stale = true;
-        if (st[8 * (size_t)r + 7] > 0 || ovf[r]) M.topo_version++;
-        if (h[r].nflips > 0) std::copy(&st[8 * (size_t)r], &st[8 * (size_t)r] + 8, S.ems[r]->pf_last);
-        overflow = overflow || ovf[r];
-        if (accepted) accepted[r] = (int)st[8 * (size_t)r + 7];
+        if (st[7] > 0 || ovf) M.topo_version++;
+        if (h[r].nflips > 0) std::copy(st, st + 8, S.ems[r]->pf_last);
+        overflow = overflow || ovf;
+        if (accepted) accepted[r] = (int)st[7];
     }
     if (overflow) throw TmError(TM_E_UNSUPPORTED, "vertex valence exceeds the ring-table width (32)");
     API_END

@@ -44,7 +44,7 @@ __global__ void k_build_ring(MeshView m, int* __restrict__ ring, int* __restrict
         } while (h != h0 && n <= kMaxValence);
     }
     if (n > kMaxValence) {
-        atomicOr(overflow, 1);
+        *overflow = 1;    // pinned host memory
         n = kMaxValence;
         b = 0;    // route to the halfedge walker
     }

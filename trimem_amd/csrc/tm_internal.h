@@ -199,7 +199,7 @@ void launch_faces(const MeshView& m, const int* perm, int* out, int first, int n
 // w); host: pinned, 16-byte aligned
 void launch_take_points(const double* host, const int* at, double* x, int n, hipStream_t s);
 void launch_give_rows(const double* src, const int* idx, double* host, int first, int n, int w, hipStream_t s);
-// Rebuild ring table and meta from the halfedge arrays; sets *overflow to 1
+// Rebuild ring table and meta from the halfedge arrays; sets *overflow (pinned) to 1
 // if a vertex has more than kMaxValence neighbours.
 void launch_build_ring(const MeshView& m, int* ring, int* meta, int* overflow, hipStream_t s);
 
