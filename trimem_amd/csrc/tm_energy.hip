@@ -486,7 +486,7 @@ __device__ __forceinline__ int query_cell(const NListView& nl, d3 pi)
 // Build-time cells of the fast vertices, in LDS.
 struct FastCells {
     int n;
-    int c[kFastMax][3];
+    int4 c[kFastMax];
 };
 
 // Block-uniform: 2 to record (forced, or too many vertices are fast), 1 to
@@ -528,9 +528,7 @@ __device__ __forceinline__ int pair_cache_mode(const PairCache& pc, const NListV
                 }
                 for (int k = 0; k < n; k++) {
                     const int id = f[1 + k], r = id % nl.strides[2];
-                    F.c[at + k][0] = r % nl.strides[1];
-                    F.c[at + k][1] = r / nl.strides[1];
-                    F.c[at + k][2] = id / nl.strides[2];
+                    F.c[at + k] = make_int4(r % nl.strides[1], r / nl.strides[1], id / nl.strides[2], 0);
                 }
             }
         }
@@ -1226,10 +1224,17 @@ __device__ __forceinline__ void rep_cached_body(const PassArgs& A, int lb)
                 keep = dx * dx + dy * dy + dz * dz < pc.limit2;
                 int c[3];
                 cell_coords(A.nl, xv, c);
-                for (int i = 0; i < s_fast.n; i++)
-                    if (abs(c[0] - s_fast.c[i][0]) <= 1 && abs(c[1] - s_fast.c[i][1]) <= 1 &&
-                        abs(c[2] - s_fast.c[i][2]) <= 1)
-                        keep = false;
+                // (as vectors, several in flight: 16 us of a block's time with
+                // a hundred of them read one component after the other)
+                const int nfast = s_fast.n;
+                bool near = false;
+#pragma unroll 8
+                for (int i = 0; i < nfast; i++) {
+                    const int4 q = s_fast.c[i];
+                    near |= ((unsigned)(c[0] - q.x + 1) <= 2u) & ((unsigned)(c[1] - q.y + 1) <= 2u) &
+                            ((unsigned)(c[2] - q.z + 1) <= 2u);
+                }
+                keep = keep && !near;
             }
             const int cell = rec_cell;
             const unsigned word = rec_word;
