@@ -525,7 +525,7 @@ struct tm_nlist {
     // pair cache of the query (PairCache): recorded lists, valid for this
     // list and topology once a recording launch has been queued
     DevBuf<double> pc_x, pc_disp;
-    DevBuf<int> pc_fast;
+    DevBuf<int> pc_fast, pc_streak;
     DevBuf<int> pc_cell, pc_ent;
     DevBuf<unsigned> pc_cnt;
     bool pc_ok = false;
@@ -645,8 +645,9 @@ long long nlist_grid(tm_nlist& L, int n, const double* part)
     return ncells;
 }
 
-// (Re)builds the lists of R meshes together: one round trip for all boxes, then
-// one launch of each kind for all.
+// (Re)builds the lists of up to kBuildLists meshes together: one round trip for all
+// boxes (in the ring), then one launch of each kind for all.
+constexpr size_t kBuildLists = 1024;
 struct NlistJob {
     tm_nlist* L;
     tm_mesh* M;
@@ -693,8 +694,7 @@ void build_nlists(const std::vector<NlistJob>& jobs, NlistTables& T)
         HostRing& ring = host_ring();
         std::lock_guard<std::mutex> guard(ring.lock);
         ring.buf.alloc(kRingPiece * kRingPieces);
-        const size_t at_once = kRingPiece * kRingPieces / (nbox * sizeof(double));
-        if ((size_t)R > at_once) throw TmError(TM_E_UNSUPPORTED, "too many lists in one build");
+        if (nbox * sizeof(double) * R > kRingPiece * kRingPieces) throw TmError(TM_E_INVALID, "too many lists");
         double* box = reinterpret_cast<double*>(ring.buf.p);
         for (int r = 0; r < R; r++) h[r].box = box + nbox * r;
         tabulate();
@@ -740,6 +740,7 @@ void build_nlists(const std::vector<NlistJob>& jobs, NlistTables& T)
             L.excl_mask.alloc((size_t)2 * n);
             L.pc_x.alloc((size_t)3 * n);
             L.pc_cell.alloc(n);
+            L.pc_streak.alloc(2);
             L.pc_cnt.alloc(n);
             L.pc_ent.alloc((size_t)kPairLanes * kPairCap * n);
             L.pc_disp.alloc(pass1_blocks(n));    // one displacement partial per pass-1 block
@@ -750,6 +751,7 @@ void build_nlists(const std::vector<NlistJob>& jobs, NlistTables& T)
             b.vcand = L.vcand.p;
             b.mask = L.excl_mask.p;
             b.pc_cell = L.pc_cell.p;
+            b.pc_streak = L.pc_streak.p;
             L.v.vcand = L.vcand.p;
             L.v.cand = L.cand.p;
             L.v.cand_start = L.cand_start.p;
@@ -904,6 +906,12 @@ void rebuild_nlist(tm_energy& E, tm_mesh& M)
     take_spare(E);
 }
 
+// the list's count of evaluations in a row with fast vertices (null: none kept)
+int* streak_of(tm_energy* E)
+{
+    return E && E->tune.pair_cache && E->nlist && E->nlist->kind == 0 ? E->nlist->pc_streak.p : nullptr;
+}
+
 // The pair-cache buffers of the energy manager's cell list (x_snap null when
 // it has none: a Verlet list, or no repulsion); the caller adds the
 // displacement partials and the recording flag.
@@ -917,6 +925,7 @@ PairCache pair_cache_of(tm_energy& E, tm_mesh& M)
         pc.cell = L.pc_cell.p;
         pc.cnt = L.pc_cnt.p;
         pc.ent = L.pc_ent.p;
+        pc.streak = L.pc_streak.p;
         pc.skin = skin;
         pc.limit2 = (kPairLimit * skin) * (kPairLimit * skin);
     }
@@ -1699,7 +1708,7 @@ int tm_hmc_step(tm_hmc* hmc, const tm_hmc_params* prm, double temperature, const
         check_launch();
     }
     launch_hmc_accept(n3, hmc->kpart0.p, hmc->kpart1.p, hmc->x0.p, M.x.p, harmonic, globals, mass, temperature,
-                      uniform, seed, step, st, g_rt.stream);
+                      uniform, seed, step, st, streak_of(harmonic ? nullptr : hmc->em), g_rt.stream);
     check_launch();
     launch_hmc_restore(n3, M.x.p, hmc->x0.p, st, g_rt.stream);
     check_launch();
@@ -1933,7 +1942,7 @@ void replicas_hmc_step(tm_replicas& S)
         mode |= i < S.L ? kHmcDrift : kHmcLast;
         launch_hmc_leap_grouped(S.d_hmc.p, S.d_hblock0.p, S.R, S.hmc_total, mode, g_rt.stream);
     }
-    launch_hmc_accept_grouped(S.d_hmc.p, S.R, g_rt.stream);
+    launch_hmc_accept_grouped(S.d_hmc.p, S.d_args.p, S.R, g_rt.stream);
     launch_hmc_restore_grouped(S.d_hmc.p, S.d_hblock0.p, S.R, S.hmc_total, g_rt.stream);
 }
 
@@ -2240,12 +2249,16 @@ int tm_replicas_update_repulsion(tm_replicas* rs)
 {
     API_BEGIN
     tm_replicas& S = *rs;
-    std::vector<NlistJob> jobs(S.R);
+    std::vector<NlistJob> jobs;
     for (int r = 0; r < S.R; r++) {
         upload_points(*S.meshes[r]);
-        jobs[r] = NlistJob{&spare_nlist(*S.ems[r]), S.meshes[r]};
+        jobs.push_back(NlistJob{&spare_nlist(*S.ems[r]), S.meshes[r]});
+        if (jobs.size() == kBuildLists || r + 1 == S.R) {
+            build_nlists(jobs, S.nl_tables);
+            if (r + 1 < S.R) sync();    // the tables are used again
+            jobs.clear();
+        }
     }
-    build_nlists(jobs, S.nl_tables);
     for (tm_energy* E : S.ems) take_spare(*E);
     refresh_replica_args(S);
     API_END
@@ -2863,7 +2876,7 @@ int tm_hmc_step_surrogate(tm_hmc* hmc, tm_surrogate* sg, const tm_hmc_params* pr
     }
     run_pass1(E, M, E.precision, nullptr);    // exact E(xn)
     launch_hmc_accept(n3, hmc->kpart0.p, hmc->kpart1.p, hmc->x0.p, M.x.p, 0, E.globals.p, mass, temperature,
-                      uniform, seed, step, st, g_rt.stream);
+                      uniform, seed, step, st, nullptr, g_rt.stream);
     launch_hmc_restore(n3, M.x.p, hmc->x0.p, st, g_rt.stream);
     check_launch();
     M.device_ahead = true;

@@ -200,6 +200,7 @@ __device__ __forceinline__ void finalize_tail(const PassArgs& A)
 {
     __shared__ double s_sum[6];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int streak = A.pc.x_snap ? get(A.pc.streak + 1) : 0;
     const bool two = wave < 2;
     const double* c0 = A.partials + (size_t)wave * A.nblocks;
     const double* c1 = A.partials + (size_t)(wave + 4) * A.nblocks;
@@ -235,6 +236,7 @@ __device__ __forceinline__ void finalize_tail(const PassArgs& A)
         *A.globals = g;
         if (A.host) *A.host = g;
         if (A.pc.dforce) *A.pc.dforce = 0;    // replica groups: the query of this evaluation recorded
+        if (A.pc.x_snap) A.pc.streak[0] = streak;
     }
 }
 
@@ -489,7 +491,8 @@ struct FastCells {
     int4 c[kFastMax];
 };
 
-// Block-uniform: 2 to record (forced, or too many vertices are fast), 1 to
+// Block-uniform: 2 to record (forced, or too many vertices are fast or for too
+// long), 1 to
 // replay; F then holds the fast vertices' cells.  Contains a barrier.
 __device__ __forceinline__ int pair_cache_mode(const PairCache& pc, const NListView& nl, FastCells& F)
 {
@@ -505,6 +508,7 @@ __device__ __forceinline__ int pair_cache_mode(const PairCache& pc, const NListV
         // flight before it takes their maximum, instead of one round trip
         // per partial
         constexpr int kBatchLoads = 16;
+        const int streak = pc.streak[0];
         bool over = false;
         for (int i0 = threadIdx.x; i0 < pc.disp_n; i0 += 64 * kBatchLoads) {
             double d[kBatchLoads];
@@ -533,7 +537,7 @@ __device__ __forceinline__ int pair_cache_mode(const PairCache& pc, const NListV
             }
         }
         over = __any(over);
-        if (threadIdx.x == 0) s_mode = over ? 2 : 1;
+        if (threadIdx.x == 0) s_mode = over || (F.n > 0 && streak >= kPatience) ? 2 : 1;
     }
     __syncthreads();
     return s_mode;
@@ -1195,6 +1199,8 @@ __device__ __forceinline__ void rep_cached_body(const PassArgs& A, int lb)
     const unsigned rec_word = mine && pc.x_snap ? pc.cnt[v] : 0u;
     __shared__ FastCells s_fast;
     const int mode = pc.x_snap ? pair_cache_mode(pc, A.nl, s_fast) : 0;    // block-uniform: 1 replay, 2 record, 0 full
+    if (pc.x_snap && lb == 0 && threadIdx.x == 0)
+        put(pc.streak + 1, mode == 1 && s_fast.n > 0 ? pc.streak[0] + 1 : 0);
     __shared__ int s_list[kVertsPerBlock];
     __shared__ double s_val[kVertsPerBlock];    // repulsion property per vertex (column 5 of pass 1)
     __shared__ int s_n;
@@ -1392,6 +1398,7 @@ __global__ void __launch_bounds__(256) k_rep_record(PassArgs A)
     const bool active = v < m.nv;
     const int meta = active ? m.meta[v] : 0;
     const bool ring = active && !is_generic(meta);
+    if (t == 0) pc.streak[1] = 0;
     RepTerms tr;
     if (active) {
         const d3 xv = load_p(m.x, v);

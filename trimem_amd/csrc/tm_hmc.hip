@@ -116,7 +116,8 @@ __device__ __forceinline__ void leap_body(int n3, double* x, double* p, double* 
 // E(xn) from the last evaluation.
 __device__ __forceinline__ void accept_body(int nblk, const double* kpart0, const double* kpart1, int n3,
                                             const double* x0, const double* x, const Globals* globals, double mass,
-                                            double temperature, double uniform, uint64_t key, HmcState* st)
+                                            double temperature, double uniform, uint64_t key, HmcState* st,
+                                            int* streak)
 {
     __shared__ double s_w[kHmcThreads / 64];
     const bool harmonic = globals == nullptr;
@@ -153,6 +154,7 @@ __device__ __forceinline__ void accept_body(int nblk, const double* kpart0, cons
     if (!harmonic)
         for (int k = 0; k < 6; k++) st->props[k] = acc ? globals->props[k] : st->props0[k];
     st->n_accepted += (unsigned long long)acc;
+    if (acc && streak && *streak > 0) *streak = kPatience;    // the fast vertices stay: record
     st->n_steps += 1ull;
 }
 
@@ -181,9 +183,10 @@ __global__ void __launch_bounds__(kHmcThreads) k_hmc_accept(int nblk, const doub
                                                             int n3, const double* x0, const double* x,
                                                             const Globals* globals, double mass, double temperature,
                                                             double uniform, uint64_t seed, uint64_t step,
-                                                            HmcState* st)
+                                                            HmcState* st, int* streak)
 {
-    accept_body(nblk, kpart0, kpart1, n3, x0, x, globals, mass, temperature, uniform, hmc_key(seed, step), st);
+    accept_body(nblk, kpart0, kpart1, n3, x0, x, globals, mass, temperature, uniform, hmc_key(seed, step), st,
+                streak);
 }
 
 __global__ void __launch_bounds__(kHmcThreads) k_hmc_restore(int n3, double* x, const double* x0, const HmcState* st)
@@ -222,11 +225,12 @@ __global__ void __launch_bounds__(kHmcThreads) k_hmc_leap_grouped(const HmcArgs*
               blockIdx.x - block0[r]);
 }
 
-__global__ void __launch_bounds__(kHmcThreads) k_hmc_accept_grouped(const HmcArgs* __restrict__ H)
+__global__ void __launch_bounds__(kHmcThreads) k_hmc_accept_grouped(const HmcArgs* __restrict__ H,
+                                                                    const PassArgs* __restrict__ A)
 {
     const HmcArgs& h = H[blockIdx.x];
     accept_body(h.nblocks, h.kpart0, h.kpart1, h.n3, h.x0, h.x, h.globals, h.mass, h.temperature, -1.0,
-                hmc_key(h.seed, h.st->n_steps), h.st);
+                hmc_key(h.seed, h.st->n_steps), h.st, A[blockIdx.x].pc.x_snap ? A[blockIdx.x].pc.streak : nullptr);
 }
 
 __global__ void __launch_bounds__(kHmcThreads) k_hmc_restore_grouped(const HmcArgs* __restrict__ H,
@@ -284,10 +288,10 @@ void launch_hmc_leap(int n3, double* x, double* p, double* a, const double* g, d
 
 void launch_hmc_accept(int n3, const double* kpart0, const double* kpart1, const double* x0, const double* x,
                        int harmonic, const Globals* globals, double mass, double temperature, double uniform,
-                       uint64_t seed, uint64_t step, HmcState* st, hipStream_t s)
+                       uint64_t seed, uint64_t step, HmcState* st, int* streak, hipStream_t s)
 {
     hipLaunchKernelGGL(k_hmc_accept, dim3(1), dim3(kHmcThreads), 0, s, hmc_blocks(n3), kpart0, kpart1, n3, x0, x,
-                       harmonic ? nullptr : globals, mass, temperature, uniform, seed, step, st);
+                       harmonic ? nullptr : globals, mass, temperature, uniform, seed, step, st, streak);
 }
 
 void launch_hmc_restore(int n3, double* x, const double* x0, const HmcState* st, hipStream_t s)
@@ -306,9 +310,9 @@ void launch_hmc_leap_grouped(const HmcArgs* d, const int* d_block0, int R, int t
     hipLaunchKernelGGL(k_hmc_leap_grouped, dim3(total_blocks), dim3(kHmcThreads), 0, s, d, d_block0, R, mode);
 }
 
-void launch_hmc_accept_grouped(const HmcArgs* d, int R, hipStream_t s)
+void launch_hmc_accept_grouped(const HmcArgs* d, const PassArgs* a, int R, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_hmc_accept_grouped, dim3(R), dim3(kHmcThreads), 0, s, d);
+    hipLaunchKernelGGL(k_hmc_accept_grouped, dim3(R), dim3(kHmcThreads), 0, s, d, a);
 }
 
 void launch_hmc_restore_grouped(const HmcArgs* d, const int* d_block0, int R, int total_blocks, hipStream_t s)

@@ -44,7 +44,15 @@ constexpr unsigned kEmptyAround = 0xf0000000u;    // no count reaches 15
 // is bound by its loads, a step with its ten queries takes as long with it as
 // without.
 constexpr int kAroundVerts = 16384;
-// More fast vertices than this in one block, or in all, record all lists again.
+// Recording all lists again costs the query several times what the full queries
+// round a few fast vertices do, but those are paid on every evaluation.  A
+// trajectory that goes astray is rejected and takes its fast vertices back with it;
+// vertices that drift stay fast.  So all lists are recorded again when the end of a
+// trajectory with fast vertices is accepted, or after kPatience evaluations in a row
+// (HMC without rebuilds: 1963 steps/s at 40962 vertices and 1471 at 163842 while fast
+// vertices stayed until there were too many, 2470 and 1662 so).
+constexpr int kPatience = 12;
+// More fast vertices than this in one block, or in all, record at once.
 constexpr int kFastSeg = 32, kFastMax = 256, kFastRow = kFastSeg + 1;
 struct PairCache {
     double* x_snap;         // [3N] positions at the recording; null: no cache
@@ -55,6 +63,9 @@ struct PairCache {
     int* fast;              // [kFastRow disp_n] per block with fast vertices: their number and build-time cells
     int disp_n;
     int* dforce;            // replica groups: device flag, nonzero records (the reduction clears it)
+    // [0] evaluations in a row with fast vertices, [1] the same after this one: the
+    // query stores it, the sums' last step takes it over
+    int* streak;
     double skin;
     double limit2;          // fast: |x - x_snap|^2 >= limit2
     int force;              // single meshes: 1 records in this launch
@@ -223,6 +234,7 @@ struct NlistBuild {
     int2* vcand;               // [n]
     unsigned long long* mask;  // [2 n]
     int* pc_cell;              // [n]
+    int* pc_streak;            // [2]
     int* sums;                 // [scan_block_sums_size(max(n, nc) + 1)]
 };
 // Workgroups of a list in the launches of each shape.
@@ -361,7 +373,7 @@ void launch_hmc_leap(int n3, double* x, double* p, double* a, const double* g, d
                      int mode, const Globals* globals, HmcState* st, double* kpart, hipStream_t s);
 void launch_hmc_accept(int n3, const double* kpart0, const double* kpart1, const double* x0, const double* x,
                        int harmonic, const Globals* globals, double mass, double temperature, double uniform,
-                       uint64_t seed, uint64_t step, HmcState* st, hipStream_t s);
+                       uint64_t seed, uint64_t step, HmcState* st, int* streak, hipStream_t s);
 void launch_hmc_restore(int n3, double* x, const double* x0, const HmcState* st, hipStream_t s);
 
 // One replica of a grouped HMC step: device draws keyed by (seed, the
@@ -385,7 +397,7 @@ struct HmcArgs {
 void launch_hmc_begin_grouped(const HmcArgs* d, const int* d_block0, int R, int total_blocks, hipStream_t s);
 void launch_hmc_leap_grouped(const HmcArgs* d, const int* d_block0, int R, int total_blocks, int mode,
                              hipStream_t s);
-void launch_hmc_accept_grouped(const HmcArgs* d, int R, hipStream_t s);
+void launch_hmc_accept_grouped(const HmcArgs* d, const PassArgs* a, int R, hipStream_t s);
 void launch_hmc_restore_grouped(const HmcArgs* d, const int* d_block0, int R, int total_blocks, hipStream_t s);
 // Parallel-tempering exchange over a kappa_b ladder: ladder slots s and s+1
 // (s = parity, parity + 2, ...) swap their replicas with probability

@@ -146,7 +146,7 @@ __device__ __forceinline__ void cells_body(const NlistBuild& b, int lb)
     b.place[v] = atomicAdd(&b.counts[c], 1);
     if (!b.cand) return;
     b.pc_cell[v] = -1;    // no replay
-    if (v == 0) b.cand_count[b.n] = 0;
+    if (v == 0) b.cand_count[b.n] = b.pc_streak[0] = b.pc_streak[1] = 0;
 }
 
 // ------------------------------------------------ stencil candidate lists
