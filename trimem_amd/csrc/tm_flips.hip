@@ -1097,9 +1097,14 @@ __device__ __forceinline__ FlipEdge flip_edge_of(const int* m)    // words 13 ..
 }
 
 // The Metropolis test (flips.cpp:57-64) u <= min(1, exp(-de)) as de <= -log(u):
-// the logarithm is taken once per proposal, not in every step of a walk.
-// u = 0 always passes (-log(0) is infinite), a NaN never.
-__device__ __forceinline__ double minus_log(double u) { return -log(u); }
+// the logarithm is taken once per proposal, not in every step of a walk.  An
+// injected u may lie outside [0, 1]: u <= 0 passes whatever the (ordered) de, as
+// exp(-de) is never negative, u > 1 and NaN never pass.
+__device__ __forceinline__ double minus_log(double u)
+{
+    if (u <= 0.0) return INFINITY;
+    return u > 1.0 ? -INFINITY : -log(u);
+}
 
 // ================================================ windowed serial sweep ==
 // The serial sweep's decisions and topology from windows of W proposals
