@@ -1500,7 +1500,7 @@ static SerialState serial_windows(tm_energy& E, tm_mesh& M, int nflips, const in
 {
     const size_t w = (size_t)W;
     E.sf_state.alloc(1);
-    E.sf_rec.alloc(w * kFlipRecord);
+    E.sf_rec.alloc(w * kSerialRecord);
     E.sf_fstamp.alloc(M.nf);
     const FlipRows rows = M.flip_rows(false);
     const EParams p = eparams_of(E);

@@ -784,12 +784,7 @@ struct PatchShared {
     alignas(16) int nb[4][kRowW];    // the one-rings (kNoFace bits kept)
     int pre[4][9], st[4][9];    // candidate runs: inclusive prefix of their lengths, starts
     int list[4][kListMax];      // candidates inside the cutoff that a ring test has not excluded
-};
-
-struct NoClaim {
-    __device__ __forceinline__ void load(int, int) {}
-    __device__ __forceinline__ void issue(bool) {}
-    __device__ __forceinline__ void more(int, int, bool) {}
+    double term[4][2][8][4];    // eight slots' terms of a ring and side, on their way into a sum in order
 };
 
 struct PatchResult {
@@ -802,6 +797,18 @@ struct PatchResult {
     }
 };
 
+// A spoke a -> b with the two faces at it, (a, b, c) and (b, a, d), for the
+// halfedge functions: halfedge 0 is the spoke, 1 its twin, 2 and 4 their next ones.
+struct Hinge {
+    d3 p[4];
+    bool edge;    // the face of the twin is missing
+    __device__ __forceinline__ d3 P(int v) const { return p[v]; }
+    __device__ __forceinline__ int to(int h) const { return h == 0 ? 1 : (h == 1 ? 0 : (h == 2 ? 2 : 3)); }
+    __device__ __forceinline__ int from(int h) const { return to(h ^ 1); }
+    __device__ __forceinline__ int next(int h) const { return h == 0 ? 2 : 4; }
+    __device__ __forceinline__ bool edge_boundary(int) const { return edge; }
+};
+
 // vertex_properties (mesh_properties.cpp:12-49) summed over the four vertices
 // of interior edge e's flip patch (flip_utils.cpp:19-41), before and after the
 // flip, by one wave.  Lanes 16 g .. 16 g + 15 serve patch vertex g (ve[g]: to(2e),
@@ -810,16 +817,19 @@ struct PatchResult {
 // slots of the ring before the flip and lanes 8-15 those after it, which is
 // the same ring without the edge's other end (g 0, 2) or with the other
 // opposite vertex (g 1, 3) in front of the slot of `partner`; then all 16
-// test the repulsion candidates once, each against both rings.  Every
-// sum is a fixed butterfly, so the bits depend on the rows alone.  What bounds
+// test the repulsion candidates once, each against both rings.  What bounds
 // it is the chain of dependent loads: rows, positions and cell ranges,
-// candidate ids, candidate positions.  claim: PatchClaim claims every edge of
-// the patch meanwhile, NoClaim nothing.
-template <class Claim>
+// candidate ids, candidate positions.  side_work is done meanwhile: PatchClaim
+// claims every edge of the patch, and every sum is a fixed butterfly, whose bits
+// depend on the rows alone; WalkOrder (kWalk) finds where each vertex's circulator
+// starts, and every term and sum is computed as coop_patch computes it, in the
+// order of its walks, so every value has its bits.
+template <class SideWork>
 __device__ __forceinline__ PatchResult patch_eval(const FlipMeshView& fm, const NListView& nl, const EParams& p,
                                                   const FlipRows& rows, const int (&pv)[4], PatchShared& S,
-                                                  Claim& claim)
+                                                  SideWork& side_work)
 {
+    constexpr bool kWalk = SideWork::kWalk;
     const int lane = threadIdx.x & 63, g = lane >> 4, q = lane & 15;
     const int side = (lane >> 3) & 1, k8 = lane & 7;
     const int ve = g == 0 ? pv[0] : (g == 1 ? pv[1] : (g == 2 ? pv[2] : pv[3]));
@@ -831,7 +841,7 @@ __device__ __forceinline__ PatchResult patch_eval(const FlipMeshView& fm, const 
     // vertices' own positions
     const int* row = rows.nb + (size_t)kRowW * ve;
     int id = row[q];
-    claim.load(ve, q);
+    side_work.load(ve, q);
     const d3 xv{fm.x[3 * ve], fm.x[3 * ve + 1], fm.x[3 * ve + 2]};
     unsigned full = (unsigned)(__ballot(id >= 0) >> (16 * g)) & 0xffffu;
     int n0 = __ffs(~full) - 1;    // slots before the end mark
@@ -863,8 +873,8 @@ __device__ __forceinline__ PatchResult patch_eval(const FlipMeshView& fm, const 
     const int j0 = id & ~kNoFace, j2 = id2 & ~kNoFace;
     d3 xj{0, 0, 0};
     if (has) xj = d3{fm.x[3 * j0], fm.x[3 * j0 + 1], fm.x[3 * j0 + 2]};
-    claim.issue(has);
-    if (__ballot(has2)) claim.more(ve, 16 + q, has2);
+    side_work.issue(has);
+    if (__ballot(has2)) side_work.more(ve, 16 + q, has2);
     if (has) {
         S.nb[g][q] = id;
         S.pos[g][q][0] = xj.x;
@@ -922,43 +932,87 @@ __device__ __forceinline__ PatchResult patch_eval(const FlipMeshView& fm, const 
     };
     load_candidates(0);
 
-    // ring terms
+    // ring terms.  The walk starts at slot w0 of the stored ring and comes to the
+    // partner as its step rw; where it starts with the partner, it goes on from the
+    // slot after it once the two have lost each other, and still starts there when
+    // a vertex is added in front
     const int nS = side ? ((g & 1) ? n0 + 1 : n0 - 1) : n0;
+    int w0 = 0, rw = r;
+    if constexpr (kWalk) {
+        const unsigned a1 = (unsigned)(__ballot(has && j0 == side_work.from) >> (16 * g)) & 0xffffu;
+        const unsigned a2 = (unsigned)(__ballot(has2 && j2 == side_work.from) >> (16 * g)) & 0xffffu;
+        w0 = a1 ? __ffs(a1) - 1 : (a2 ? 16 + __ffs(a2) - 1 : 0);
+        rw = r >= w0 ? r - w0 : r - w0 + n0;
+    }
+    auto stored = [&](int s) { return w0 + s < n0 ? w0 + s : w0 + s - n0; };
     auto slot_of = [&](int s) {    // slot of the stored ring, or -1 for the vertex the flip adds
-        if (!side) return s;
-        if (g & 1) return s < r ? s : (s == r ? -1 : s - 1);
-        return s < r ? s : s + 1;
+        if (!side) return stored(s);
+        if (g & 1) {
+            const int at = kWalk && rw == 0 ? n0 : rw;
+            return s < at ? stored(s) : (s == at ? -1 : stored(s - 1));
+        }
+        return stored(s < rw ? s : s + 1);
     };
     auto at_slot = [&](int i) {
         const double* a = i < 0 ? S.pv[4 - g] : S.pos[g][i];    // g odd: 4 - g is the other opposite vertex
         return d3{a[0], a[1], a[2]};
     };
     double area = 0, vol = 0, curv = 0, teth = 0;
+    double walk = 0;    // kWalk: lane k8 < 4 of a side sums its k8-th quantity
     for (int c0 = 0; __ballot(c0 + k8 < nS); c0 += 8) {
         const int s = c0 + k8;
         const int i1 = s < nS ? slot_of(s) : 0, i2 = slot_of(s + 1 < nS ? s + 1 : 0);
         const bool nof = i1 >= 0 && (S.nb[g][i1] & kNoFace), nofn = i2 >= 0 && (S.nb[g][i2] & kNoFace);
         // a halfedge without a face contributes nothing
-        if (s < nS && !nof) {
-        const d3 ec = at_slot(i1) - xv, ep = at_slot(slot_of(s > 0 ? s - 1 : nS - 1)) - xv, en = at_slot(i2) - xv;
-        const d3 nc = cross(ec, ep), nn = cross(en, ec);
-        const double nl0 = norm(nc), el = norm(ec);
-        double da = 0.0;
-        if (!nofn) {
-            const double denom = nl0 * norm(nn);
-            if (denom != 0) da = om_angle(dot(nc, nn) / denom, dot(cross(nc, nn), ec));
-        }
-        const double fa = nl0 / 2;
-        curv += 0.5 * el * da;
-        area += fa;
-        vol += dot(xv, nc) / 6;
-        teth += p.bond_type == 0 ? bond_edge_value(el, p) : bond_area_value(fa, p);
+        const bool in = s < nS && !nof;
+        if constexpr (kWalk) {
+            double t[4] = {0, 0, 0, 0};
+            if (in) {
+                const Hinge hg{{xv, at_slot(i1), at_slot(slot_of(s > 0 ? s - 1 : nS - 1)), at_slot(i2)}, nofn};
+                const double el = mu_edge_length(hg, 0), da = om_dihedral_angle(hg, 0);
+                t[0] = mu_face_area(hg, 0);
+                t[1] = mu_face_volume(hg, 0);
+                t[2] = 0.5 * el * da;
+                t[3] = p.bond_type == 0 ? bond_edge_value(el, p) : bond_area_value(t[0], p);
+            }
+#pragma unroll
+            for (int c = 0; c < 4; c++) S.term[g][side][k8][c] = t[c];
+            wave_sync();
+            // (a zero leaves a sum as it is: none of them is ever -0)
+#pragma unroll
+            for (int i = 0; i < 8; i++) walk += S.term[g][side][i][k8 & 3];
+            wave_sync();
+        } else if (in) {
+            const d3 ec = at_slot(i1) - xv, ep = at_slot(slot_of(s > 0 ? s - 1 : nS - 1)) - xv, en = at_slot(i2) - xv;
+            const d3 nc = cross(ec, ep), nn = cross(en, ec);
+            const double nl0 = norm(nc), el = norm(ec);
+            double da = 0.0;
+            if (!nofn) {
+                const double denom = nl0 * norm(nn);
+                if (denom != 0) da = om_angle(dot(nc, nn) / denom, dot(cross(nc, nn), ec));
+            }
+            const double fa = nl0 / 2;
+            curv += 0.5 * el * da;
+            area += fa;
+            vol += dot(xv, nc) / 6;
+            teth += p.bond_type == 0 ? bond_edge_value(el, p) : bond_area_value(fa, p);
         }
     }
-    area = group_sum(area) / 3;
-    vol = group_sum(vol) / 3;
-    curv = group_sum(curv) / 2;
-    teth = group_sum(teth) / (p.bond_type == 0 ? 2 : 3);
+    if constexpr (kWalk) {
+        area = __shfl(walk, lane & ~7, 64);
+        vol = __shfl(walk, (lane & ~7) + 1, 64);
+        curv = __shfl(walk, (lane & ~7) + 2, 64);
+        teth = __shfl(walk, (lane & ~7) + 3, 64);
+    } else {
+        area = group_sum(area);
+        vol = group_sum(vol);
+        curv = group_sum(curv);
+        teth = group_sum(teth);
+    }
+    area /= 3;
+    vol /= 3;
+    curv /= 2;
+    teth /= (p.bond_type == 0 ? 2 : 3);
 
     // repulsion: each candidate inside the cutoff against the ring before the
     // flip and the one after it (mesh_repulsion.h:28-54; exclusion as in
@@ -1017,6 +1071,7 @@ __device__ __forceinline__ PatchResult patch_eval(const FlipMeshView& fm, const 
             }
             wave_sync();
             for (int i0 = 0; __ballot(i0 < listed); i0 += 16) {
+                double v0 = 0.0, v1 = 0.0;
                 if (i0 + q < listed) {
                     const int w = S.list[g][i0 + q], c = w & ~(3 << 30);
                     bool e0 = w & (1 << 30), e1 = w < 0;
@@ -1047,17 +1102,29 @@ __device__ __forceinline__ PatchResult patch_eval(const FlipMeshView& fm, const 
                     }
                     if (!(e0 && e1)) {
                         const double v = rep_value(norm(dc), p.rep_lc1, p.rep_r);
-                        if (!e0) rep0 += v;
-                        if (!e1) rep1 += v;
+                        if (!e0) v0 = v;
+                        if (!e1) v1 = v;
                     }
+                }
+                if constexpr (kWalk) {
+                    // in the candidates' order, which the list keeps
+                    for (int i = 0; i < 16 && __ballot(i0 + i < listed); i++) {
+                        rep0 += __shfl(v0, i, 16);
+                        rep1 += __shfl(v1, i, 16);
+                    }
+                } else {
+                    rep0 += v0;
+                    rep1 += v1;
                 }
             }
             t0 += kListMax;
             if (!__ballot(t0 < total)) break;
             load_candidates(t0);
         }
-        rep0 = row_sum(rep0);
-        rep1 = row_sum(rep1);
+        if constexpr (!kWalk) {
+            rep0 = row_sum(rep0);
+            rep1 = row_sum(rep1);
+        }
     }
     res.val[0] = area;
     res.val[1] = vol;
@@ -1067,33 +1134,45 @@ __device__ __forceinline__ PatchResult patch_eval(const FlipMeshView& fm, const 
     res.val[5] = side ? rep1 : rep0;
 #pragma unroll
     for (int k = 0; k < 6; k++) {
-        res.val[k] += __shfl_xor(res.val[k], 16, 64);
-        res.val[k] += __shfl_xor(res.val[k], 32, 64);
+        if constexpr (kWalk) {
+            // vertex by vertex, as the edge's halfedges then name them: from
+            // to(2e) on, which after the flip is the vertex that came second
+            const int first = (side_work.swapped ? 32 : 0) + 16 * side;
+            double sum = 0.0;
+#pragma unroll
+            for (int i = 0; i < 4; i++) sum += __shfl(res.val[k], ((first + 16 * i) & 48) + 8 * side, 64);
+            res.val[k] = sum;
+        } else {
+            res.val[k] += __shfl_xor(res.val[k], 16, 64);
+            res.val[k] += __shfl_xor(res.val[k], 32, 64);
+        }
     }
     return res;
 }
 
-// A proposal's record, one 128-byte line that its wave stores in one go: words
-// 0-11 the patch differences (after minus before), 12 its validity (1
-// flippable, 0 not, -1 index out of range), 13-25 the FlipEdge.  The readers
-// take lines with several lanes each: read by one thread each, a record would
-// be thirteen requests for the same line.
-__device__ __forceinline__ void put_record(int* rec, int lane, int valid, const double (&d)[6], const FlipEdge& f)
+// A proposal's record, which its wave stores in one go: kD doubles (of the
+// parallel sweep the patch differences, after minus before; of the serial sweep
+// the sums before the flip, then after it) in words 0 .. 2 kD - 1, then its validity
+// (1 flippable, 0 not, -1 index out of range) and the FlipEdge.  The readers take
+// records with several lanes each: read by one thread each, a record would be
+// a request for the same line per word pair.
+template <int kD>
+__device__ __forceinline__ void put_record(int* rec, int lane, int valid, const double (&d)[kD], const FlipEdge& f)
 {
     int w = 0;
 #pragma unroll
-    for (int c = 0; c < 6; c++)
+    for (int c = 0; c < kD; c++)
         if ((lane >> 1) == c) w = (lane & 1) ? __double2hiint(d[c]) : __double2loint(d[c]);
     const int rest[14] = {valid, f.e, f.pv[0], f.pv[1], f.pv[2], f.pv[3], f.a1, f.a2, f.b1, f.b2, f.fa, f.fb, f.ha,
                           f.hb};
 #pragma unroll
     for (int c = 0; c < 14; c++)
-        if (lane == 12 + c) w = rest[c];
-    if (lane < 26) put(rec + lane, w);
+        if (lane == 2 * kD + c) w = rest[c];
+    if (lane < 2 * kD + 14) put(rec + lane, w);
 }
-__device__ __forceinline__ FlipEdge flip_edge_of(const int* m)    // words 13 .. 25 of a record
+__device__ __forceinline__ FlipEdge flip_edge_of(const int* m)    // the words after a record's validity
 {
-    return FlipEdge{m[13], {m[14], m[15], m[16], m[17]}, m[18], m[19], m[20], m[21], m[22], m[23], m[24], m[25]};
+    return FlipEdge{m[0], {m[1], m[2], m[3], m[4]}, m[5], m[6], m[7], m[8], m[9], m[10], m[11], m[12]};
 }
 
 // The Metropolis test (flips.cpp:57-64) u <= min(1, exp(-de)) as de <= -log(u):
@@ -1107,30 +1186,109 @@ __device__ __forceinline__ double minus_log(double u)
 }
 
 // ================================================ windowed serial sweep ==
-// The serial sweep's decisions and topology from windows of W proposals
-// evaluated at once.  One launch per window: a wave per proposal evaluates
-// is_flip_ok and its patch before and after the flip on the topology at the
-// window start, and the last workgroup commits the window in order up to the
-// first proposal whose evaluation an earlier one has changed.
+// The serial sweep's decisions, topology and running properties, bit for bit,
+// from windows of W proposals evaluated at once.  One launch per window: a wave
+// per proposal evaluates is_flip_ok and its patch before and after the flip on
+// the topology at the window start, and the last workgroup commits the window in
+// order up to the first proposal whose evaluation an earlier one has changed.
 // What an earlier proposal j of the window changes for a later one k:
 //   * accepted: the one-rings of j's four patch vertices V(j).  k read the
 //     one-rings of its patch vertices P_k and, for exclusion level 2, the
 //     neighbour sets of their one-ring vertices N(P_k); so V(j) meeting P_k (or
 //     N(P_k)) makes k stale.
-//   * rejected (do_flip twice): nothing that an evaluation reads.  Every
-//     vertex keeps its neighbours in the same cyclic order; only ids move.
-// The commit tests all proposals up to the first stale one against the
-// current state at once and takes the first acceptance: a rejection leaves the
-// state, so every decision is that of the sequential walk.  The halfedge
-// arrays are then rewritten (do_flip or do_flip twice) by one thread per
+//   * rejected (do_flip twice): every vertex keeps its neighbours in the same
+//     cyclic order, but the edge's halfedges swap direction, so a later
+//     proposal of the same edge adds its patch vertices in another order, and
+//     an endpoint whose circulator started on the edge starts at the next
+//     spoke.  k is decided only while no accepted proposal has met P_k, so
+//     every earlier one that could have done this to it was rejected, if it was
+//     valid: WalkOrder works out the order from the window's proposals alone.
+// The commit tests all proposals up to the first stale one against the current
+// state at once and takes the first acceptance: a rejection leaves the state, so
+// every decision is that of the sequential walk to rounding.  One wave then runs
+// the one-workgroup sweep's rounding path (props -= old, += new; on rejection
+// -= new, += old) through these decisions, a component per lane, and every thread
+// takes its proposal's decision again, from the path's own states.  The window ends
+// after the first one that this changes.
+// The halfedge arrays are then rewritten (do_flip or do_flip twice) by one thread per
 // committed proposal.  Proposals that share a face must follow each other (a
 // stamp per face holds the window's first valid proposal on it): those
 // connected through shared faces get ascending ranks, and the ranks are
 // applied one after the other.
 // A window commits at least its first proposal, which cannot be stale.
-// At level 7 (491520 edges) a window of 256 takes 38 us; evaluating by ring
-// walks (30 us) and committing along the serial rounding path (51 us) were two
-// launches.
+// At level 7 (491520 edges) a window of 256 takes 44 us, 6.2 of them for the
+// rounding path and 1.3 for the decisions on it; evaluating by ring walks (30 us)
+// and committing (51 us) were two launches.
+
+// The proposals of its window before a wave's own, four per lane, and the spokes at
+// which the circulators of its patch vertices start when it is decided.
+struct WalkOrder {
+    static constexpr bool kWalk = true;
+    const FlipMeshView& fm;
+    const FlipRows& rows;
+    const int (&before)[kSerialWindowMax / 64];    // lane l: the edges of proposals l, l + 64, ..., -1: none
+    bool swapped;    // the edge's halfedges have swapped direction
+    int h = 0;       // lanes of a vertex: the halfedge at which its walk starts
+    int from = 0;    // its target
+    __device__ WalkOrder(const FlipMeshView& m, const FlipRows& r, const int (&b)[kSerialWindowMax / 64], int e)
+        : fm(m), rows(r), before(b)
+    {
+        int n = 0;
+#pragma unroll
+        for (int u = 0; u < kSerialWindowMax / 64; u++) n += __popcll(__ballot(before[u] == e));
+        swapped = n & 1;
+    }
+    __device__ __forceinline__ void load(int v, int) { h = fm.v_he[v]; }
+    __device__ __forceinline__ void more(int, int, bool) {}
+    __device__ __forceinline__ void issue(bool)
+    {
+        bool hit = false;
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+            const int e = __builtin_amdgcn_readlane(h, 16 * g) >> 1;
+#pragma unroll
+            for (int u = 0; u < kSerialWindowMax / 64; u++) hit |= before[u] == e;
+        }
+        if (__ballot(hit)) moved();
+        from = fm.he_to[h];
+    }
+    // each valid earlier proposal of the edge a walk starts on moves it to the
+    // next spoke, where a later one may move it again
+    __device__ __forceinline__ void moved()
+    {
+        const int lane = threadIdx.x & 63;
+        for (int g = 0; g < 4; g++) {
+            int at = __builtin_amdgcn_readlane(h, 16 * g);
+            for (int j = -1;;) {
+                int next = kSerialWindowMax;
+#pragma unroll
+                for (int u = kSerialWindowMax / 64 - 1; u >= 0; u--) {
+                    const unsigned long long b = __ballot(before[u] == at >> 1 && 64 * u + lane > j);
+                    if (b) next = 64 * u + __ffsll((long long)b) - 1;
+                }
+                if (next == kSerialWindowMax || !flippable(at >> 1)) break;
+                j = next;
+                at = fm.he_next[at ^ 1];
+            }
+            if (lane >> 4 == g) h = at;
+        }
+    }
+    // flip_ok of an edge, by the wave
+    __device__ __forceinline__ bool flippable(int e)
+    {
+        static_assert(kRowW == 32, "a lane per slot of two rows");
+        const FlipEdge f = load_flip_edge(fm, e);
+        if (f.fa < 0 || f.fb < 0) return false;
+        const int lane = threadIdx.x & 63;
+        const int id = rows.nb[(size_t)kRowW * (lane < 32 ? f.pv[1] : f.pv[3]) + (lane & 31)];
+        const unsigned long long b = __ballot(id >= 0);
+        const unsigned c = (unsigned)b, d = (unsigned)(b >> 32);
+        if (c == ~0u || d == ~0u || f.pv[1] == f.pv[3]) return false;
+        const int n = __ffs(~c) - 1;    // slots of the first row before its end mark
+        return !__ballot(lane < n && (id & ~kNoFace) == f.pv[3]);
+    }
+};
+
 __global__ void __launch_bounds__(256) k_sf_begin(FlipMeshView fm, FlipRows rows, const Globals* __restrict__ g0,
                                                   EParams p, int nflips, SerialState* __restrict__ st,
                                                   unsigned long long* __restrict__ fstamp)
@@ -1148,9 +1306,14 @@ __global__ void __launch_bounds__(256) k_sf_begin(FlipMeshView fm, FlipRows rows
     st->count = 0u;
 }
 
-constexpr int kRecInts = 26;    // the used words of a record
+constexpr int kRecInts = 38;    // the used words of a record
+constexpr int kRecValid = 24, kRecEdge = 25;
 struct SerialShared {
     alignas(16) int rec[kSerialWindowMax * kRecInts];
+    // the rounding path: properties after each proposal's flip, and their energies
+    double after[kSerialWindowMax][6];
+    double energy[kSerialWindowMax];
+    unsigned long long acc[kPatchWaves];    // the accepted proposals
     // one-rings of every proposal's patch, kRowPair slots each and -1 past the
     // end, as int4 chunks rotated by the proposal's number (bank conflicts)
     int4 ring[kSerialWindowMax][kRowPair];
@@ -1162,6 +1325,68 @@ struct SerialShared {
     int nflip, flip[kSerialWindowMax];
 };
 
+// a record's sums before the flip (0-5) and after it (6-11)
+__device__ __forceinline__ const double* sums_of(const int* m) { return reinterpret_cast<const double*>(m); }
+
+// One wave runs the serial sweep's rounding path from properties P through the
+// proposals [0, end) and some after them, lane c < 6 the component c (an invalid
+// proposal's sums are zeros); bit k of acc: proposal k is accepted.
+__device__ __forceinline__ void serial_path(SerialShared& S, const double (&P)[6], int end)
+{
+    const int c = threadIdx.x & 63;
+    if (c >= 6) return;
+    double x = c == 0 ? P[0] : (c == 1 ? P[1] : (c == 2 ? P[2] : (c == 3 ? P[3] : (c == 4 ? P[4] : P[5]))));
+    // kStep proposals in registers, the next ones' loads in flight, and nothing
+    // but the chain of additions where none is accepted: one wave alone issues an
+    // instruction at a time (256 proposals take 6.2 us; with bounds, register moves
+    // and the choice between two states in the loop 12.3)
+    constexpr int kStep = 16;
+    static_assert(kSerialWindowMax % (2 * kStep) == 0, "two steps per round");
+    struct Sums {
+        double o[kStep], n[kStep];
+    } a, b;
+    auto load = [&](int i0, Sums& s) {
+        const double* d = sums_of(S.rec + kRecInts * min(i0, kSerialWindowMax - kStep)) + c;
+#pragma unroll
+        for (int i = 0; i < kStep; i++) {
+            s.o[i] = d[kRecInts / 2 * i];
+            s.n[i] = d[kRecInts / 2 * i + 6];
+        }
+    };
+    auto run = [&](int i0, const Sums& s) {
+        double q[kStep];
+        const unsigned acc =
+            __builtin_amdgcn_readfirstlane((int)(unsigned)(S.acc[i0 >> 6] >> (i0 & 63))) & ((1u << kStep) - 1u);
+        if (acc == 0u) {
+#pragma unroll
+            for (int i = 0; i < kStep; i++) {
+                q[i] = x - s.o[i];
+                q[i] += s.n[i];
+                x = q[i] - s.n[i];
+                x += s.o[i];
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < kStep; i++) {
+                q[i] = x - s.o[i];
+                q[i] += s.n[i];
+                double r = q[i] - s.n[i];
+                r += s.o[i];
+                x = (acc >> i) & 1u ? q[i] : r;
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < kStep; i++) S.after[i0 + i][c] = q[i];
+    };
+    load(0, a);
+    for (int i0 = 0; i0 < end; i0 += 2 * kStep) {
+        load(i0 + kStep, b);
+        run(i0, a);
+        load(i0 + 2 * kStep, a);
+        run(i0 + kStep, b);
+    }
+}
+
 __device__ __forceinline__ void sf_commit(const FlipMeshView& fm, const FlipRows& rows, const EParams& p, int nflips,
                                           const double* __restrict__ uniforms, int n_uniforms, uint64_t seed,
                                           int injected, int W, int need_nb, SerialState* __restrict__ st,
@@ -1171,19 +1396,19 @@ __device__ __forceinline__ void sf_commit(const FlipMeshView& fm, const FlipRows
     const int pos0 = st->pos, used0 = st->used, wid = st->window + 1;
     const int cnt = min(W, nflips - pos0);
     {
-        // sixteen lanes per record
+        // thirty-two lanes per record
         const unsigned long long* src = reinterpret_cast<const unsigned long long*>(rec);
-        const int c = tid & 15, r0 = tid >> 4;
-        unsigned long long w[16];
+        const int c = tid & 31, r0 = tid >> 5;
+        unsigned long long w[32];
 #pragma unroll
-        for (int i = 0; i < 16; i++) {
-            const int r = r0 + 16 * i;
-            w[i] = r < cnt && c < kRecInts / 2 ? get(src + (size_t)(kFlipRecord / 2) * r + c) : 0ull;
+        for (int i = 0; i < 32; i++) {
+            const int r = r0 + 8 * i;
+            w[i] = r < cnt && c < kRecInts / 2 ? get(src + (size_t)(kSerialRecord / 2) * r + c) : 0ull;
         }
 #pragma unroll
-        for (int i = 0; i < 16; i++)
+        for (int i = 0; i < 32; i++)
             if (c < kRecInts / 2)
-                *reinterpret_cast<unsigned long long*>(S.rec + kRecInts * (r0 + 16 * i) + 2 * c) = w[i];
+                *reinterpret_cast<unsigned long long*>(S.rec + kRecInts * (r0 + 8 * i) + 2 * c) = w[i];
     }
     double P[6], e0 = st->e0;
 #pragma unroll
@@ -1194,23 +1419,24 @@ __device__ __forceinline__ void sf_commit(const FlipMeshView& fm, const FlipRows
     // thread k holds proposal k of the window
     const int k = tid;
     const int* m = S.rec + kRecInts * k;
-    const int v = k < cnt ? m[12] : -2;
-    const int pv0 = m[14], pv1 = m[15], pv2 = m[16], pv3 = m[17];
-    const bool inner = v >= 0 && m[22] >= 0 && m[23] >= 0;
+    const int v = k < cnt ? m[kRecValid] : -2;
+    const FlipEdge fe = flip_edge_of(m + kRecEdge);
+    const int pv0 = fe.pv[0], pv1 = fe.pv[1], pv2 = fe.pv[2], pv3 = fe.pv[3];
+    const bool inner = v >= 0 && fe.fa >= 0 && fe.fb >= 0;
     double dp[6];
 #pragma unroll
-    for (int c = 0; c < 6; c++) dp[c] = __hiloint2double(m[2 * c + 1], m[2 * c]);
+    for (int c = 0; c < 6; c++) dp[c] = sums_of(m)[6 + c] - sums_of(m)[c];
     // window positions of the first valid proposals on its faces, and the
     // rings that acceptances are checked against
     int l0 = k, l1 = k;
     bool wide = false;
     if (v == 1) {
-        const unsigned long long s0 = get(fstamp + m[22]), s1 = get(fstamp + m[23]);
+        const unsigned long long s0 = get(fstamp + fe.fa), s1 = get(fstamp + fe.fb);
         if (need_nb) {
             int4 w[8];
 #pragma unroll
             for (int g = 0; g < 4; g++) {
-                const int4* row = reinterpret_cast<const int4*>(rows.nb + (size_t)kRowW * m[14 + g]);
+                const int4* row = reinterpret_cast<const int4*>(rows.nb + (size_t)kRowW * fe.pv[g]);
                 w[2 * g] = row[0];
                 w[2 * g + 1] = row[1];
             }
@@ -1248,15 +1474,19 @@ __device__ __forceinline__ void sf_commit(const FlipMeshView& fm, const FlipRows
     // rejected and the sweep stops after it
     const int movf = injected ? max(n_uniforms - used0, 0) : INT_MAX;
     const bool ovf = v == 1 && mr == movf, can = v == 1 && mr < movf;
-    double nlu = 0.0;
-    if (can) nlu = minus_log(injected ? uniforms[used0 + mr] : rng_uniform(seed, (uint64_t)(used0 + mr)));
+    const double u =
+        !can ? __builtin_nan("") : (injected ? uniforms[used0 + mr] : rng_uniform(seed, (uint64_t)(used0 + mr)));
+    const double nlu = minus_log(u);
+    double P0[6], start0 = e0;
+#pragma unroll
+    for (int c = 0; c < 6; c++) P0[c] = P[c];
 
     // every thread carries the state; one barrier per step
     bool stale = false, accepted = false;
-    int pos = 0, err = 0, it = 0, nacc = 0;
+    int pos = 0, err = 0, it = 0;
     while (pos < cnt) {
         // the first proposal that is not to be decided now (1), finds the
-        // uniform stream empty (2) or is accepted (3)
+        // uniform stream empty (2) or is likely to be accepted (3)
         int what = 0;
         if (k >= pos && k < cnt) {
             if (stale || v < 0) what = 1;
@@ -1288,9 +1518,8 @@ __device__ __forceinline__ void sf_commit(const FlipMeshView& fm, const FlipRows
         if (what != 3) break;
         const int* f = S.rec + kRecInts * first;
 #pragma unroll
-        for (int c = 0; c < 6; c++) P[c] += __hiloint2double(f[2 * c + 1], f[2 * c]);
+        for (int c = 0; c < 6; c++) P[c] += sums_of(f)[6 + c] - sums_of(f)[c];
         e0 = energy_of(P, p);
-        nacc++;
         if (k == first) accepted = true;
         // later proposals whose patch meets the accepted patch are stale; at
         // exclusion level 2 its one-rings count too (adjacency is symmetric:
@@ -1310,13 +1539,72 @@ __device__ __forceinline__ void sf_commit(const FlipMeshView& fm, const FlipRows
             }
             if ((S.wide[first >> 6] >> (first & 63)) & 1ull)
                 for (int g = 0; g < 4; g++) {
-                    const int* row = rows.nb + (size_t)kRowW * f[14 + g];
+                    const int* row = rows.nb + (size_t)kRowW * f[kRecEdge + 1 + g];
                     for (int i = 0; i < kRowW && row[i] >= 0; i++) check(row[i] & ~kNoFace);
                 }
         }
 #pragma unroll
-        for (int g = 0; g < 4; g++) check(f[14 + g]);
+        for (int g = 0; g < 4; g++) check(f[kRecEdge + 1 + g]);
         stale = stale || (hit && inner);
+    }
+
+    // the same decisions from the rounding path
+    int nacc = 0;
+    {
+        const unsigned long long b = __ballot(accepted);
+        if ((tid & 63) == 0) S.acc[wave] = b;
+        __syncthreads();
+        if (wave == 0) serial_path(S, P0, pos);
+        __syncthreads();
+        const double en = k < pos ? energy_of(S.after[k], p) : 0.0;
+        S.energy[k] = en;
+        __syncthreads();
+        // the energy before this proposal: that of the acceptance before it
+        int last = -1;
+#pragma unroll
+        for (int w = 0; w < kPatchWaves; w++) {
+            unsigned long long a = S.acc[w];
+            if (64 * w + 63 >= k) a &= 64 * w < k ? (1ull << (k - 64 * w)) - 1ull : 0ull;
+            if (a) last = 64 * w + 63 - __clzll((long long)a);
+        }
+        const double de = en - (last < 0 ? start0 : S.energy[last]);
+        const double alpha = de < 0.0 ? 1.0 : exp(-de);
+        const bool take = k < pos && u <= alpha;
+        const unsigned long long m = __ballot(take != accepted);
+        int* slots = S.slots[it++ & 1];
+        if ((tid & 63) == 0) slots[wave] = m ? 64 * wave + __ffsll((long long)m) - 1 : INT_MAX;
+        __syncthreads();
+        int changed = INT_MAX;
+#pragma unroll
+        for (int i = 0; i < kPatchWaves; i++) changed = min(changed, slots[i]);
+        if (changed != INT_MAX) {
+            pos = changed + 1;
+            err = 0;
+            accepted = k < changed ? accepted : k == changed && !accepted;
+        }
+        // the state after the last committed proposal
+        if (pos > 0) {
+            const bool now = (((S.acc[(pos - 1) >> 6] >> ((pos - 1) & 63)) & 1ull) != 0ull) != (pos - 1 == changed);
+            const double* d = sums_of(S.rec + kRecInts * (pos - 1));
+#pragma unroll
+            for (int c = 0; c < 6; c++) {
+                const double q = S.after[pos - 1][c];
+                double r = q - d[6 + c];
+                r += d[c];
+                P[c] = now ? q : r;
+            }
+        }
+        e0 = start0;
+        int at = -1;
+#pragma unroll
+        for (int w = 0; w < kPatchWaves; w++) {
+            unsigned long long a = S.acc[w];
+            if (64 * w + 63 >= pos) a &= 64 * w < pos ? (1ull << (pos - 64 * w)) - 1ull : 0ull;
+            if (changed != INT_MAX && changed >> 6 == w) a ^= 1ull << (changed & 63);
+            nacc += __popcll(a);
+            if (a) at = 64 * w + 63 - __clzll((long long)a);
+        }
+        if (at >= 0) e0 = S.energy[at];
     }
 
     // ranks of the committed flips along shared faces: the labels become the
@@ -1354,7 +1642,7 @@ __device__ __forceinline__ void sf_commit(const FlipMeshView& fm, const FlipRows
     const int maxrank = S.maxrank;
     for (int i = 0; i <= maxrank; i++) {
         if (commit && rank == i) {
-            const FlipEdge f = i == 0 ? flip_edge_of(m) : load_flip_edge(fm, m[13]);
+            const FlipEdge f = i == 0 ? fe : load_flip_edge(fm, fe.e);
             if (accepted) store_flip(fm, f);
             else store_flip_twice(fm, f);
         }
@@ -1366,8 +1654,8 @@ __device__ __forceinline__ void sf_commit(const FlipMeshView& fm, const FlipRows
     // as the records have them)
     for (int t = tid; t < 4 * S.nflip; t += 256) {
         const int g = t & 3;
-        const int* f = S.rec + kRecInts * S.flip[t >> 2];
-        flip_row(rows, f[14 + g], g, g < 2 ? f[16] : f[14], g == 1 ? f[17] : f[15], f[13], make_int2(0, 0));
+        const int* f = S.rec + kRecInts * S.flip[t >> 2] + kRecEdge + 1;    // the patch vertices
+        flip_row(rows, f[g], g, g < 2 ? f[2] : f[0], g == 1 ? f[3] : f[1], f[-1], make_int2(0, 0));
     }
     // state; the uniforms used are the valid proposals before pos
     if (pos < cnt ? k == pos : tid == 0) {
@@ -1408,23 +1696,31 @@ __global__ void __launch_bounds__(256) k_sf_window(FlipMeshView fm, FlipRows row
         const int e = injected ? proposals[i] : rng_edge(seed, (uint64_t)i, ne);
         int valid = -1;
         FlipEdge f{};
-        double d[6] = {0, 0, 0, 0, 0, 0};
+        double d[12] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
         if (e >= 0 && e < ne) {
             f = load_flip_edge(fm, e);
             valid = 0;
             if (f.fa >= 0 && f.fb >= 0) {
-                NoClaim none;
-                const PatchResult r = patch_eval(fm, nl, p, rows, f.pv, S.patch[wave], none);
+                int before[kSerialWindowMax / 64];
+#pragma unroll
+                for (int u = 0; u < kSerialWindowMax / 64; u++) {
+                    const int j = 64 * u + lane;
+                    before[u] = -1;
+                    if (j < k) before[u] = injected ? proposals[i - k + j] : rng_edge(seed, (uint64_t)(i - k + j), ne);
+                }
+                WalkOrder order(fm, rows, before, e);
+                const PatchResult r = patch_eval(fm, nl, p, rows, f.pv, S.patch[wave], order);
                 if (r.ok) {
                     valid = 1;
                     const unsigned long long key =
                         ((unsigned long long)(unsigned)(st->window + 1) << 32) | (unsigned)(W - k);
                     if (lane < 2) atomicMax(&fstamp[lane ? f.fb : f.fa], key);
-                    r.difference(d);
+#pragma unroll
+                    for (int c = 0; c < 12; c++) d[c] = __shfl(r.val[c % 6], c < 6 ? 0 : 8, 64);
                 }
             }
         }
-        put_record(rec + (size_t)kFlipRecord * k, lane, valid, d, f);
+        put_record(rec + (size_t)kSerialRecord * k, lane, valid, d, f);
     }
     if (!last_block(&st->count, (unsigned)blocks)) return;
     sf_commit(fm, rows, p, nflips, uniforms, n_uniforms, seed, injected, W, need_nb, st, rec, fstamp, S.serial);
@@ -1503,6 +1799,7 @@ __device__ __forceinline__ int pflip_nprop(const PflipArgs& a, int round)
 // atomics go out behind the position loads, and what they replaced is looked
 // at after the evaluation.
 struct PatchClaim {
+    static constexpr bool kWalk = false;
     const PflipArgs& a;
     const unsigned long long key;
     const int round;
@@ -1648,7 +1945,7 @@ __device__ __forceinline__ void pflip_decide(const PflipArgs& a, int round, int 
                 m[2 * c] = (int)(unsigned)x;
                 m[2 * c + 1] = (int)(unsigned)(x >> 32);
             }
-            const FlipEdge f = flip_edge_of(m);
+            const FlipEdge f = flip_edge_of(m + 13);
             const int g = t & 3;
             const int2 ed = g == 1 ? make_int2(f.b2 >> 1, f.b1 >> 1) : make_int2(f.a2 >> 1, f.a1 >> 1);
             const int me = g == 0 ? f.pv[0] : (g == 1 ? f.pv[1] : (g == 2 ? f.pv[2] : f.pv[3]));

@@ -301,11 +301,12 @@ struct SerialState {
     double e0;
     unsigned count;    // workgroups of the window that have finished
 };
-constexpr int kFlipRecord = 32;    // ints per proposal record
+constexpr int kFlipRecord = 32;      // ints per proposal record of the parallel sweep
+constexpr int kSerialRecord = 40;    // ... and of the serial one
 // rows, face stamps and the starting state
 void launch_serial_begin(const FlipMeshView& fm, const FlipRows& rows, const Globals* g0, const EParams& p, int nflips,
                          SerialState* st, unsigned long long* fstamp, hipStream_t s);
-// rec: [kFlipRecord W], fstamp: [faces]
+// rec: [kSerialRecord W], fstamp: [faces]
 void launch_serial_windows(const FlipMeshView& fm, const FlipRows& rows, const NListView& nl, const EParams& p,
                            int nflips, const int* proposals, const double* uniforms, int n_uniforms, uint64_t seed,
                            int injected, int W, SerialState* st, int* rec, unsigned long long* fstamp,
