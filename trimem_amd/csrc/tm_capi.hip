@@ -24,6 +24,7 @@
 #include <numeric>
 #include <random>
 #include <stdexcept>
+#include <unordered_set>
 #include <string>
 #include <unordered_map>
 #include <vector>
@@ -854,11 +855,12 @@ EParams eparams_of(const tm_energy& E)
     return p;
 }
 
-// the counters of a properties pass, zero between launches
-void alloc_pass_count(DevBuf<unsigned>& c)
+// the counters of `passes` properties passes, zero between launches
+void alloc_pass_count(DevBuf<unsigned>& c, int passes = 1)
 {
-    c.alloc(kLastCounters);
-    launch_fill_ints(reinterpret_cast<int*>(c.p), kLastCounters, 0, nullptr, 0, 0, nullptr, 0, 0, g_rt.stream);
+    c.alloc((size_t)kLastCounters * passes);
+    launch_fill_ints(reinterpret_cast<int*>(c.p), kLastCounters * passes, 0, nullptr, 0, 0, nullptr, 0, 0,
+                     g_rt.stream);
     check_launch();
 }
 
@@ -1768,6 +1770,9 @@ struct tm_replicas {
     std::vector<int> h_ones;
     int total_disp = 0, total_rc = 0;    // displacement partials, cached-query blocks
     std::vector<unsigned> gens;    // each member's tm_energy::gen when the table was built
+    // zeros, the properties pass's counters of each member: a manager may be a
+    // member more than once
+    DevBuf<unsigned> pass_counts;
     GroupLaunch group() const
     {
         return GroupLaunch{d_args.p,  h_args.data(), R, d_block0.p, total_blocks, d_block0_rep.p, total_rep,
@@ -1812,6 +1817,22 @@ namespace {
 
 void set_group_shape(tm_replicas& S, const Tuning& t, bool force);
 
+// whether each member is the first, or the last, with its energy manager
+std::vector<char> first_members(const tm_replicas& S)
+{
+    std::vector<char> first(S.R);
+    std::unordered_set<const tm_energy*> seen;
+    for (int r = 0; r < S.R; r++) first[r] = seen.insert(S.ems[r]).second;
+    return first;
+}
+std::vector<char> last_members(const tm_replicas& S)
+{
+    std::vector<char> last(S.R);
+    std::unordered_set<const tm_energy*> seen;
+    for (int r = S.R; r-- > 0;) last[r] = seen.insert(S.ems[r]).second;
+    return last;
+}
+
 // Rebuild the device table of pass arguments from the replicas' current
 // buffers and neighbour lists.  With a ladder, each replica's kappa_b is that
 // of the slot it holds on the device.
@@ -1840,6 +1861,8 @@ void refresh_replica_args(tm_replicas& S)
     S.fast_parts.alloc((size_t)kFastRow * S.total_disp);
     S.force_flags.alloc(S.R);
     S.h_ones.assign(S.R, 1);
+    if (!S.pass_counts.p) alloc_pass_count(S.pass_counts, S.R);
+    const std::vector<char> first = first_members(S);
     for (int r = 0; r < S.R; r++) {
         tm_mesh& M = *S.meshes[r];
         tm_energy& E = *S.ems[r];
@@ -1849,7 +1872,9 @@ void refresh_replica_args(tm_replicas& S)
         EParams ep = eparams_of(E);
         if (S.has_ladder) ep.kappa_b = S.h_ladder[slot_of[r]];
         PassBuffers b = buffers(E, M);
-        b.pc = pair_cache_of(E, M);
+        b.count = S.pass_counts.p + (size_t)kLastCounters * r;
+        // one member keeps a list's recordings
+        b.pc = first[r] ? pair_cache_of(E, M) : PairCache{};
         if (b.pc.x_snap) {
             b.pc.disp_part = S.disp_parts.p + b0d[r];
             b.pc.fast = S.fast_parts.p + (size_t)kFastRow * b0d[r];
@@ -1976,6 +2001,61 @@ int tm_replicas_destroy(tm_replicas* rs)
     return TM_OK;
 }
 
+// One sweep of each of these members, whose meshes and managers are distinct, their
+// final states into pf_report; whether a valence became too large.
+static bool pflip_members(tm_replicas& S, const std::vector<int>& members, const std::vector<int>& slot_of,
+                          double flip_ratio, const uint64_t* seeds)
+{
+    const int R = (int)members.size();
+    std::vector<PflipArgs> h(R);
+    std::vector<int> b0(R + 1, 0);
+    int rounds = 0, max_nv = 0, max_nh = 0, max_batch = 0;
+    for (int i = 0; i < R; i++) {
+        const int r = members[i];
+        tm_mesh& M = *S.meshes[r];
+        tm_energy& E = *S.ems[r];
+        // as tm_flip_parallel: the FP64 properties at the current positions
+        // start each replica's Metropolis walk
+        upload_points(M);
+        run_pass1(E, M, 0, nullptr);
+        const int ne = M.nh / 2, nflips = (int)(ne * flip_ratio), batch = std::max(1, ne / 1024);
+        EParams ep = eparams_of(E);
+        if (S.has_ladder) ep.kappa_b = S.h_ladder[slot_of[r]];
+        h[i] = pflip_args(E, M, ep, seeds[r], nflips, batch);
+        if (nflips > 0) rounds = std::max(rounds, (nflips + batch - 1) / batch);
+        b0[i + 1] = b0[i] + pflip_round_blocks(batch);
+        max_nv = std::max(max_nv, M.nv);
+        max_nh = std::max(max_nh, M.nh);
+        max_batch = std::max(max_batch, batch);
+    }
+    S.pf_args.alloc(R);
+    S.pf_block0.alloc(R + 1);
+    h2d(S.pf_args.p, h.data(), sizeof(PflipArgs) * R);
+    h2d(S.pf_block0.p, b0.data(), sizeof(int) * (R + 1));
+    const PflipGroup g{S.pf_args.p, R, rounds, S.ems[0]->tune.pflip_window, S.pf_block0.p, b0[R],
+                       max_nv, max_nh, max_batch};
+    launch_flip_parallel_grouped(g, g_rt.stream);
+    check_launch();
+    for (int i = 0; i < R; i++) {
+        const int r = members[i];
+        queue_ring(*S.meshes[r]);
+        if (h[i].nflips > 0) d2h(S.pf_report.p + 8 * (size_t)r, S.ems[r]->pf_state.p, 8 * sizeof(double));
+    }
+    sync();
+    bool overflow = false;
+    for (int i = 0; i < R; i++) {
+        const int r = members[i];
+        tm_mesh& M = *S.meshes[r];
+        const double* st = S.pf_report.p + 8 * (size_t)r;
+        const int ovf = M.report.p->overflow;
+        M.host_stale = true;
+        if (st[7] > 0 || ovf) M.topo_version++;
+        if (h[i].nflips > 0) std::copy(st, st + 8, S.ems[r]->pf_last);
+        overflow = overflow || ovf;
+    }
+    return overflow;
+}
+
 int tm_replicas_pflip(tm_replicas* rs, double flip_ratio, const uint64_t* seeds, int* accepted)
 {
     API_BEGIN
@@ -1991,53 +2071,23 @@ int tm_replicas_pflip(tm_replicas* rs, double flip_ratio, const uint64_t* seeds,
         sync();
         for (int s = 0; s < S.R; s++) slot_of[owner[s]] = s;
     }
-    std::vector<PflipArgs> h(S.R);
-    std::vector<int> b0(S.R + 1, 0);
-    int rounds = 0, max_nv = 0, max_nh = 0, max_batch = 0;
-    for (int r = 0; r < S.R; r++) {
-        tm_mesh& M = *S.meshes[r];
-        tm_energy& E = *S.ems[r];
-        // as tm_flip_parallel: the FP64 properties at the current positions
-        // start each replica's Metropolis walk
-        upload_points(M);
-        run_pass1(E, M, 0, nullptr);
-        const int ne = M.nh / 2, nflips = (int)(ne * flip_ratio), batch = std::max(1, ne / 1024);
-        EParams ep = eparams_of(E);
-        if (S.has_ladder) ep.kappa_b = S.h_ladder[slot_of[r]];
-        h[r] = pflip_args(E, M, ep, seeds[r], nflips, batch);
-        if (nflips > 0) rounds = std::max(rounds, (nflips + batch - 1) / batch);
-        b0[r + 1] = b0[r] + pflip_round_blocks(batch);
-        max_nv = std::max(max_nv, M.nv);
-        max_nh = std::max(max_nh, M.nh);
-        max_batch = std::max(max_batch, batch);
-    }
-    S.pf_args.alloc(S.R);
-    S.pf_block0.alloc(S.R + 1);
-    h2d(S.pf_args.p, h.data(), sizeof(PflipArgs) * S.R);
-    h2d(S.pf_block0.p, b0.data(), sizeof(int) * (S.R + 1));
-    const PflipGroup g{S.pf_args.p, S.R, rounds, S.ems[0]->tune.pflip_window, S.pf_block0.p, b0[S.R],
-                       max_nv, max_nh, max_batch};
-    launch_flip_parallel_grouped(g, g_rt.stream);
-    check_launch();
     S.pf_report.alloc(8 * (size_t)S.R);
     std::fill(S.pf_report.p, S.pf_report.p + 8 * (size_t)S.R, 0.0);
-    for (int r = 0; r < S.R; r++) {
-        tm_mesh& M = *S.meshes[r];
-        queue_ring(M);
-        if (h[r].nflips > 0) d2h(S.pf_report.p + 8 * (size_t)r, S.ems[r]->pf_state.p, 8 * sizeof(double));
-    }
-    sync();
     bool overflow = false;
-    for (int r = 0; r < S.R; r++) {
-        tm_mesh& M = *S.meshes[r];
-        const double* st = S.pf_report.p + 8 * (size_t)r;
-        const int ovf = M.report.p->overflow;
-        M.host_stale = true;
-        if (st[7] > 0 || ovf) M.topo_version++;
-        if (h[r].nflips > 0) std::copy(st, st + 8, S.ems[r]->pf_last);
-        overflow = overflow || ovf;
-        if (accepted) accepted[r] = (int)st[7];
+    // members with a mesh or a manager in common sweep one after another
+    std::vector<int> todo(S.R), now, later;
+    std::iota(todo.begin(), todo.end(), 0);
+    for (; !todo.empty(); todo.swap(later)) {
+        now.clear();
+        later.clear();
+        std::unordered_set<const void*> taken;
+        for (int r : todo) {
+            const bool mesh = taken.insert(S.meshes[r]).second, em = taken.insert(S.ems[r]).second;
+            (mesh && em ? now : later).push_back(r);
+        }
+        overflow = pflip_members(S, now, slot_of, flip_ratio, seeds) || overflow;
     }
+    for (int r = 0; accepted && r < S.R; r++) accepted[r] = (int)S.pf_report.p[8 * (size_t)r + 7];
     if (overflow) throw TmError(TM_E_UNSUPPORTED, "vertex valence exceeds the ring-table width (32)");
     API_END
 }
@@ -2249,17 +2299,21 @@ int tm_replicas_update_repulsion(tm_replicas* rs)
 {
     API_BEGIN
     tm_replicas& S = *rs;
+    // each manager's list once, whatever the number of its memberships, on the
+    // mesh of the last of them
     std::vector<NlistJob> jobs;
+    const std::vector<char> last = last_members(S);
     for (int r = 0; r < S.R; r++) {
         upload_points(*S.meshes[r]);
-        jobs.push_back(NlistJob{&spare_nlist(*S.ems[r]), S.meshes[r]});
+        if (last[r]) jobs.push_back(NlistJob{&spare_nlist(*S.ems[r]), S.meshes[r]});
         if (jobs.size() == kBuildLists || r + 1 == S.R) {
             build_nlists(jobs, S.nl_tables);
             if (r + 1 < S.R) sync();    // the tables are used again
             jobs.clear();
         }
     }
-    for (tm_energy* E : S.ems) take_spare(*E);
+    for (int r = 0; r < S.R; r++)
+        if (last[r]) take_spare(*S.ems[r]);
     refresh_replica_args(S);
     API_END
 }
