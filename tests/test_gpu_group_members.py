@@ -1,6 +1,8 @@
 """GPU: the members of a replica group.  A mesh and its manager may be members more
-than once, and a mesh may be a member with several managers: each member's results
-are those of its mesh alone."""
+than once, a mesh may be a member with several managers, meshes without
+vertices may stand anywhere among the others, and one member's list may have so many
+cells that the scan of the tiles is a launch of its own: each member's results are
+those of its mesh alone."""
 import ctypes
 
 import numpy as np
@@ -9,7 +11,9 @@ import pytest
 from trimem_amd import capi
 from trimem_amd import meshes as M
 
+from test_gpu_nlist_build import to_core_params
 from test_gpu_replicas import core, params    # noqa: F401
+from oracle import oracle as O
 
 pytestmark = pytest.mark.gpu
 
@@ -20,10 +24,26 @@ def sphere(core, level, seed, **kw):    # noqa: F811
     return mesh, core.EnergyManager(mesh, params(core, lbar, **kw))
 
 
+def far_spheres(core, cells=204):    # noqa: F811
+    """Two small spheres in opposite corners of cells^3 cells: 2073 tiles of them."""
+    v, f, _ = M.jittered_icosphere(2, seed=3)
+    r = 0.45 / cells
+    x = np.concatenate([r * v + r, r * v + (1.0 - r)])
+    x -= x.min(axis=0)
+    faces = np.concatenate([f, f + len(v)]).astype(np.int32)
+    rl = x.max() / (cells + 0.5)
+    mesh = core.TriMesh(x, faces)
+    p = O.Params(rep_rlist=rl, rep_lc1=rl, rep_exclusion=1, bond_lc0=rl, bond_lc1=0.1 * rl)
+    return mesh, core.EnergyManager(mesh, to_core_params(core, p))
+
+
 def compare(core, group, singles):    # noqa: F811
     group.eval()
     g = group.globals()
     for i, (n, e) in enumerate(singles):
+        if n.n_vertices() == 0:
+            assert np.all(g[i, :6] == 0.0) and np.isnan(g[i, 6])    # (A / A0 - 1)^2 of 0 / 0
+            continue
         assert g[i, 6] == e.energy(n), i
         assert np.array_equal(group.gradient(i), e.gradient(n)), i
 
@@ -88,3 +108,20 @@ def test_sweeps_of_one_mesh_follow_each_other(core, same_manager):    # noqa: F8
     assert list(acc) == want and min(want) > 0
     assert np.array_equal(m.fv_indices(), n.fv_indices())
     assert np.array_equal(extra[0].fv_indices(), extra1[0].fv_indices())
+
+
+def test_members_without_vertices_and_with_many_cells(core):    # noqa: F811
+    def members():
+        def none():
+            mesh = core.TriMesh(np.zeros((0, 3)), np.zeros((0, 3), np.int32))
+            return mesh, core.EnergyManager(mesh, params(core, 1.0))
+        return [none(), sphere(core, 2, 1), none(), none(), far_spheres(core),
+                sphere(core, 3, 2, n_search="verlet-list"), none()]
+    a, b = members(), members()
+    group = core.Replicas([m for m, _ in a], [e for _, e in a])
+    compare(core, group, b)
+    group.update_repulsion()
+    for n, e in b:
+        e.update_repulsion(n)
+    compare(core, group, b)
+    compare(core, group, b)

@@ -1718,7 +1718,7 @@ PassArgs pass_args(const MeshView& m, const NListView& nl, const EParams& p, con
     a.nlist = b.nlist;
     a.nblocks = pass1_blocks(m.nv);
     a.count = b.count;
-    a.tail = a.nblocks <= kTailBlocks;
+    a.tail = a.nblocks > 0 && a.nblocks <= kTailBlocks;    // no vertices, no last workgroup
     a.pc = a.rep_v ? b.pc : PairCache{};
     a.theta = b.theta;
     return a;
