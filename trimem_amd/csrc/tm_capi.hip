@@ -2796,8 +2796,10 @@ int tm_surrogate_loss_grad(tm_surrogate* sg, double* loss, float* grad)
     check_launch();
     float l = 0.0f;
     d2h(&l, S.b.loss, sizeof(float));
-    if (grad) d2h(grad, S.grad.p, sizeof(float) * kSgParams);
+    std::vector<float> g(grad ? kSgParams : 0);    // a call that fails stores nothing
+    d2h(g.data(), S.grad.p, sizeof(float) * g.size());
     sg_check_err(S);    // waits
+    if (grad) std::copy(g.begin(), g.end(), grad);
     if (loss) *loss = l;
     API_END
 }
