@@ -2521,6 +2521,7 @@ struct tm_surrogate {
     bool fallback = false;
     int since_probe = 0;
     bool pending = false;        // the last guarded step was surrogate-driven, its outcome unread
+    unsigned twin_topo = ~0u;    // topology of the twin table
     unsigned checked_topo = ~0u; // topology whose features were last checked
     bool topo_ok = false;        // ... and whether the network can take it (closed, valences 3..10)
     long long n_sg = 0, n_exact = 0, n_switch = 0;
@@ -2625,6 +2626,18 @@ void sg_check_err(tm_surrogate& S)
     }
 }
 
+// the loss and its parameter gradient after a forward pass with a target; the twin
+// table follows the flips
+void sg_gradient(tm_surrogate& S)
+{
+    const tm_mesh& M = *S.mesh;
+    if (S.twin_topo != M.topo_version) {
+        sg_twin(M.view(), S.twin.p, g_rt.stream);
+        S.twin_topo = M.topo_version;
+    }
+    sg_backward(M.view(), S.b, S.geo, S.theta.p, S.pk, S.twin.p, S.grad.p, g_rt.stream);
+}
+
 // the exact gradient at the current positions (energy manager buffers)
 void sg_exact_gradient(tm_surrogate& S, double* vprops = nullptr)
 {
@@ -2652,7 +2665,6 @@ int tm_surrogate_create(tm_mesh* mesh, tm_energy* em, uint64_t seed, tm_surrogat
     S->nv = M.nv;
     sg_alloc(*S);
     HIPCHECK(hipMemsetAsync(S->err.p, 0, sizeof(int), g_rt.stream));
-    sg_twin(M.view(), S->twin.p, g_rt.stream);
     // mean edge length and raw features of the current state fix the
     // normalisation
     double lsum = 0.0;
@@ -2792,7 +2804,7 @@ int tm_surrogate_loss_grad(tm_surrogate* sg, double* loss, float* grad)
     sg_exact_gradient(S, mixed ? S.vprops.p : nullptr);
     sg_feature_pass(S, mixed);
     sg_forward(S.mesh->view(), S.b, S.geo, S.theta.p, S.pk, S.sigma_F, S.em->grad.p, nullptr, g_rt.stream);
-    sg_backward(S.mesh->view(), S.b, S.geo, S.theta.p, S.pk, S.twin.p, S.grad.p, g_rt.stream);
+    sg_gradient(S);
     check_launch();
     float l = 0.0f;
     d2h(&l, S.b.loss, sizeof(float));
@@ -2874,7 +2886,7 @@ int tm_surrogate_train(tm_surrogate* sg, int epochs, float lr, uint64_t seed, do
                                     g_rt.stream));
             sg_feature_pass(S);
             sg_forward(M.view(), S.b, S.geo, S.theta.p, S.pk, S.sigma_F, S.snap_g[k]->p, nullptr, g_rt.stream);
-            sg_backward(M.view(), S.b, S.geo, S.theta.p, S.pk, S.twin.p, S.grad.p, g_rt.stream);
+            sg_gradient(S);
             sg_adam(kSgParams, S.theta.p, S.grad.p, S.m1.p, S.m2.p, lr, ++S.adam_step, g_rt.stream);
             sg_pack(S.theta.p, S.pk, g_rt.stream);
             HIPCHECK(hipMemcpyAsync(S.losses.p + i, S.b.loss, sizeof(float), hipMemcpyDeviceToDevice, g_rt.stream));
