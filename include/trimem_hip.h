@@ -264,11 +264,10 @@ typedef struct tm_tuning {
     int rep_threads;     /* repulsion query: 64, 128, 256 or 512 threads per block */
     int rep_batch;       /* candidates in flight per lane: 1, 2, 4 or 8 */
     int pass2_threads;   /* gradient pass: 64, 128, 256 or 512 */
-    int rep_fused;       /* 1: the query shares the launch of the properties pass
-                            (256 threads, rep_threads unused), 0: its own launch */
+    int rep_fused;       /* 0 or 1, without effect: the query has its own launch */
     int pair_cache;      /* 1 (default): the cell-list query replays recorded
                             candidate lists while they are provably complete
-                            (single meshes; bit-identical), 0: full query */
+                            (bit-identical), 0: full query */
     int pflip_window;    /* 1..256 (default 256): proposals the parallel flip
                             sweep tests at once against the running state when
                             it looks for the next acceptance; every window
@@ -280,8 +279,7 @@ typedef struct tm_tuning {
 } tm_tuning;
 int tm_energy_set_tuning(tm_energy* em, const tm_tuning* t);
 int tm_energy_get_tuning(const tm_energy* em, tm_tuning* out);
-/* ms_rep / ms_pass2 (may be NULL): the winners' times per launch (ms_rep:
- * of the fused properties launch when rep_fused is chosen) */
+/* ms_rep / ms_pass2 (may be NULL): the winners' times per launch */
 int tm_energy_autotune(tm_energy* em, tm_mesh* mesh, tm_tuning* out, double* ms_rep, double* ms_pass2);
 
 /* ---- replica groups: batched meshes, parallel tempering, graph replay ----
@@ -304,7 +302,8 @@ int tm_replicas_eval(tm_replicas* rs, int flags);
  * replica r draws its proposals from seeds[r] and flips with the kappa_b of
  * the ladder slot it holds; each replica's flips and accepted count are
  * those of tm_flip_parallel(ems[r], meshes[r], flip_ratio, seeds[r], 0, .)
- * (round k of every replica runs in one launch per phase).  accepted:
+ * (round k of every replica runs in one launch; replicas with a mesh or an
+ * energy manager in common sweep one after another).  accepted:
  * int[n_replicas] or NULL.  flip_ratio > 1 -> TM_E_RANGE. */
 int tm_replicas_pflip(tm_replicas* rs, double flip_ratio, const uint64_t* seeds, int* accepted);
 /* out[7 r + k]: the six global properties (area, volume, curvature,

@@ -565,8 +565,6 @@ void scan(const int* in, int* out, int n, DevBuf<int>& tmp)
     check_launch();
 }
 
-// CellList ctor (cell_list.h:43-87) and, for kind 1, VerletList ctor
-// (verlet_list.h:18-35), on the mesh's current device positions.
 // the Verlet adjacency from the cells of its list
 void build_verlet(tm_nlist& L, tm_mesh& M)
 {
@@ -646,8 +644,10 @@ long long nlist_grid(tm_nlist& L, int n, const double* part)
     return ncells;
 }
 
-// (Re)builds the lists of up to kBuildLists meshes together: one round trip for all
-// boxes (in the ring), then one launch of each kind for all.
+// CellList ctor (cell_list.h:43-87) and, for kind 1, VerletList ctor
+// (verlet_list.h:18-35), on the meshes' current device positions, of up to
+// kBuildLists distinct lists together: one round trip for all boxes (in the ring),
+// then one launch of each kind for all.
 constexpr size_t kBuildLists = 1024;
 struct NlistJob {
     tm_nlist* L;

@@ -470,9 +470,9 @@ __device__ __forceinline__ void store_rep_g(const PassArgs& A, int v, const RepT
 // sphere's outermost vertices move and their stencils still reach into the
 // grid.  (-1, no replay, only where the ids would not fit.)  While those
 // vertices had no cell and took the full query on every evaluation, the launch
-// waited for them: an evaluation of a sphere moved by 0.5% of an edge since the
-// list was built took 31.8 us at 642 vertices, now 27.6; 36.5 and 32.7 at 40962,
-// 51.2 and 45.6 at 163842.
+// waited for them: the same positions, 0.5% of an edge from those of the list,
+// evaluated again and again took 31.8 us at 642 vertices, now 27.6; 36.5 and 32.7
+// at 40962, 51.2 and 45.6 at 163842.
 __device__ __forceinline__ int query_cell(const NListView& nl, d3 pi)
 {
     int c[3];
@@ -492,8 +492,7 @@ struct FastCells {
 };
 
 // Block-uniform: 2 to record (forced, or too many vertices are fast or for too
-// long), 1 to
-// replay; F then holds the fast vertices' cells.  Contains a barrier.
+// long), 1 to replay; F then holds the fast vertices' cells.  Contains a barrier.
 __device__ __forceinline__ int pair_cache_mode(const PairCache& pc, const NListView& nl, FastCells& F)
 {
     __shared__ int s_mode;
@@ -1370,8 +1369,8 @@ __global__ void __launch_bounds__(256) k_rep_cached(PassArgs A)
     rep_cached_body<kBatch>(A, logical_block());
 }
 
-// replica groups: block0 gives each replica pass1_blocks / 8 blocks (its
-// pass-1 partial rows, 32 vertices each, in blocks of 256 vertices)
+// replica groups: block0 gives each replica its pass1_blocks, a workgroup for each
+// pass-1 block of 256 vertices
 template <int kBatch>
 __global__ void __launch_bounds__(256) k_rep_cached_grouped(const PassArgs* __restrict__ A,
                                                             const int* __restrict__ block0, int R)

@@ -147,13 +147,12 @@ PassArgs pass_args(const MeshView& m, const NListView& nl, const EParams& p, con
 // Launch shapes that do not change any result bit: the repulsion query and
 // pass 2 write per-vertex values only, and each lane visits its candidates in
 // the same order whatever the batch.  (Pass 1's blocks fix the order of the
-// global sums and stay at 256 threads; fused, the query's blocks cover the
-// same 32 vertices as pass-1 blocks and sum their column the same way.)
+// global sums and stay at 256 threads.)
 struct Tuning {
     int rep_threads = 256;    // 64, 128, 256 or 512
     int rep_batch = 2;        // candidates in flight per lane: 1, 2, 4 or 8
     int p2_threads = 256;     // 64, 128, 256 or 512
-    int rep_fused = 0;        // 1: the query shares the pass-1 launch (256 threads), 0: its own launch
+    int rep_fused = 0;        // taken and kept; the query has its own launch either way
     int pair_cache = 1;       // 1: replay recorded candidate lists (single meshes, cell list)
     int pflip_window = 256;   // proposals the pflip Metropolis scan tests at once (1..256)
     int serial_window = 256;  // proposals per window of the serial sweep (1..256), 0: one workgroup

@@ -35,11 +35,9 @@ namespace tmh {
 // ----------------------------------------------------------------- box ----
 // Bounding box of the vertices, as kBoxBlocks per-block partial minima and
 // maxima (part[6 b + k], min in k < 3, max in k >= 3; +DBL_MAX and -DBL_MAX
-// for a block without vertices).  They go to pinned host memory:
-// the host, which needs the box to size the grid, combines them (min and max are exact in any order) and
-// applies the reference's initial values (cell_list.h:46-47); a last-block
-// combine would need a device-scope fence in every block, which costs more
-// than the whole pass.
+// for a block without vertices).  They go to pinned host memory: the host needs
+// the box anyway, to size the grid, so it combines them (min and max are exact in
+// any order) and applies the reference's initial values (cell_list.h:46-47).
 constexpr int kBoxBlocks = 64;
 __device__ __forceinline__ void box_body(const NlistBuild& b, int lb)
 {
