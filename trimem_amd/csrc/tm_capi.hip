@@ -74,10 +74,14 @@ constexpr int kNoAllocScratchDoubles = kNoAllocCounterBytes / sizeof(double) + k
 static __device__ __align__(256) double scratch[kNoAllocScratchDoubles];
 constexpr int kMaxDevices = 64;
 
+constexpr size_t kRingPiece = 512 << 10;    // HostRing
+constexpr int kRingPieces = 8;
+
 struct Runtime {
     bool init = false;
     int device = 0;
     hipStream_t stream = nullptr;
+    hipEvent_t arrived[kRingPieces] = {};    // HostRing's: events of the stream's device, whichever thread is first
     void* scratch[kMaxDevices] = {};    // device address of `scratch` on each device
     hipEvent_t pass1_marks[2] = {};     // tm_mark_pass1: taken by the next properties pass
 };
@@ -92,6 +96,7 @@ void ensure_runtime()
         throw TmError(TM_E_DEVICE, "device index out of range");
     HIPCHECK(hipSetDevice(g_rt.device));
     HIPCHECK(hipStreamCreateWithFlags(&g_rt.stream, hipStreamNonBlocking));
+    for (hipEvent_t& e : g_rt.arrived) HIPCHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     // the scratch array's address on this device, with the device current
     void* sp = nullptr;
     HIPCHECK(hipGetSymbolAddress(&sp, HIP_SYMBOL(scratch)));
@@ -154,12 +159,9 @@ struct HostBuf {
 // piece has been copied.  A gradient of 163842 vertices takes 250 us with 8 pieces
 // of 512 KB, 266 with 4, 283 and 304 with 8 and 4 of 256 KB (a wait per piece),
 // 299 with 2 of 2 MB (no overlap); one copy into pageable memory took 404.
-constexpr size_t kRingPiece = 512 << 10;
-constexpr int kRingPieces = 8;
 struct HostRing {
     std::mutex lock;
     HostBuf<char> buf;
-    hipEvent_t arrived[kRingPieces] = {};
 };
 HostRing& host_ring()
 {
@@ -174,18 +176,16 @@ void to_host(void* dst, size_t rows, size_t row_bytes, F&& piece)
     HostRing& R = host_ring();
     std::lock_guard<std::mutex> guard(R.lock);
     R.buf.alloc(kRingPiece * kRingPieces);
-    for (hipEvent_t& e : R.arrived)
-        if (!e) HIPCHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     const size_t per = kRingPiece / row_bytes, pieces = (rows + per - 1) / per;
     auto slot = [&](size_t k) { return R.buf.p + (k % kRingPieces) * kRingPiece; };
     auto start = [&](size_t k) {
         piece(slot(k), (int)(k * per), (int)std::min(per, rows - k * per));
         check_launch();
-        if (pieces > 1) HIPCHECK(hipEventRecord(R.arrived[k % kRingPieces], g_rt.stream));
+        if (pieces > 1) HIPCHECK(hipEventRecord(g_rt.arrived[k % kRingPieces], g_rt.stream));
     };
     for (size_t k = 0; k < std::min<size_t>(pieces, kRingPieces); k++) start(k);
     for (size_t k = 0; k < pieces; k++) {
-        if (pieces > 1) HIPCHECK(hipEventSynchronize(R.arrived[k % kRingPieces]));
+        if (pieces > 1) HIPCHECK(hipEventSynchronize(g_rt.arrived[k % kRingPieces]));
         else sync();
         std::memcpy((char*)dst + k * per * row_bytes, slot(k), std::min(per, rows - k * per) * row_bytes);
         if (k + kRingPieces < pieces) start(k + kRingPieces);
@@ -409,6 +409,7 @@ void ensure_device(tm_mesh& M)
     M.meta.alloc(M.nv);
     M.d_perm.alloc(M.nv);
     M.d_iperm.alloc(M.nv);
+    M.stage.alloc((size_t)M.nv * 3);
     h2d(M.d_perm.p, M.perm.data(), sizeof(int) * M.nv);
     h2d(M.d_iperm.p, M.iperm.data(), sizeof(int) * M.nv);
     M.report.alloc(1);
@@ -451,7 +452,6 @@ constexpr int kTakeVerts = 65536;
 // three doubles per vertex from host memory, in internal order
 void upload_rows(tm_mesh& M, const double* host, double* dst)
 {
-    M.stage.alloc((size_t)3 * M.nv);
     h2d(M.stage.p, host, sizeof(double) * 3 * M.nv);
     launch_gather_rows(M.stage.p, M.d_perm.p, dst, M.nv, 3, g_rt.stream);
 }
