@@ -492,23 +492,20 @@ struct FastCells {
 };
 
 // Block-uniform: 2 to record (forced, or too many vertices are fast or for too
-// long), 1 to replay; F then holds the fast vertices' cells.  Contains a barrier.
+// long), 1 to replay; F (F.n 0 on entry) then holds the fast vertices' cells.
+// Contains a barrier.
 __device__ __forceinline__ int pair_cache_mode(const PairCache& pc, const NListView& nl, FastCells& F)
 {
     __shared__ int s_mode;
-    if (threadIdx.x == 0) F.n = 0;
     if (pc.force || (pc.dforce && *pc.dforce)) {
         __syncthreads();
         return 2;
     }
     if (threadIdx.x < 64) {
-        __builtin_amdgcn_wave_barrier();
         // one partial per pass-1 block: each lane has a batch of loads in
-        // flight before it takes their maximum, instead of one round trip
-        // per partial
+        // flight before it compares them, instead of one round trip per partial
         constexpr int kBatchLoads = 16;
-        const int streak = pc.streak[0];
-        bool over = false;
+        bool some = false, over = false;
         for (int i0 = threadIdx.x; i0 < pc.disp_n; i0 += 64 * kBatchLoads) {
             double d[kBatchLoads];
 #pragma unroll
@@ -516,6 +513,11 @@ __device__ __forceinline__ int pair_cache_mode(const PairCache& pc, const NListV
                 const int i = i0 + 64 * u;
                 d[u] = i < pc.disp_n ? pc.disp_part[i] : 0.0;
             }
+            bool any = false;
+#pragma unroll
+            for (int u = 0; u < kBatchLoads; u++) any |= !(d[u] < pc.limit2);
+            if (__builtin_expect(!__any(any), 1)) continue;
+            some = true;
             unsigned hit = 0;
 #pragma unroll
             for (int u = 0; u < kBatchLoads; u++) hit |= (d[u] < pc.limit2 ? 0u : 1u) << u;
@@ -535,8 +537,9 @@ __device__ __forceinline__ int pair_cache_mode(const PairCache& pc, const NListV
                 }
             }
         }
-        over = __any(over);
-        if (threadIdx.x == 0) s_mode = over || (F.n > 0 && streak >= kPatience) ? 2 : 1;
+        int mode = 1;
+        if (__builtin_expect(some, 0)) mode = __any(over) || pc.streak[0] >= kPatience ? 2 : 1;
+        if (threadIdx.x == 0) s_mode = mode;
     }
     __syncthreads();
     return s_mode;
@@ -1197,21 +1200,19 @@ __device__ __forceinline__ void rep_cached_body(const PassArgs& A, int lb)
     const int rec_cell = mine && pc.x_snap ? pc.cell[v] : -1;    // -1: none
     const unsigned rec_word = mine && pc.x_snap ? pc.cnt[v] : 0u;
     __shared__ FastCells s_fast;
-    const int mode = pc.x_snap ? pair_cache_mode(pc, A.nl, s_fast) : 0;    // block-uniform: 1 replay, 2 record, 0 full
-    if (pc.x_snap && lb == 0 && threadIdx.x == 0)
-        put(pc.streak + 1, mode == 1 && s_fast.n > 0 ? pc.streak[0] + 1 : 0);
     __shared__ int s_list[kVertsPerBlock];
     __shared__ double s_val[kVertsPerBlock];    // repulsion property per vertex (column 5 of pass 1)
     __shared__ int s_n;
     __shared__ int s_rep[kVertsPerBlock];
     __shared__ unsigned s_word[kVertsPerBlock];
     __shared__ int s_nrep;
-    if (threadIdx.x == 0) {
-        s_n = 0;
-        s_nrep = 0;
-    }
-    __syncthreads();
-    if (threadIdx.x < kVertsPerBlock) s_val[threadIdx.x] = 0.0;
+    if (threadIdx.x == 0) s_n = s_nrep = s_fast.n = 0;
+    s_val[threadIdx.x] = 0.0;
+    if (!pc.x_snap) __syncthreads();
+    const int mode = pc.x_snap ? pair_cache_mode(pc, A.nl, s_fast) : 0;    // block-uniform: 1 replay, 2 record, 0 full
+    if (pc.x_snap && lb == 0 && threadIdx.x == 0)
+        put(pc.streak + 1, mode == 1 && s_fast.n > 0 ? pc.streak[0] + 1 : 0);
+    const int nfast = s_fast.n;
     if (mine) {
         const bool ring = !is_generic(meta);
         bool done = !ring;
@@ -1223,7 +1224,7 @@ __device__ __forceinline__ void rep_cached_body(const PassArgs& A, int lb)
             pc.x_snap[3 * v + 2] = xv.z;
             if (!ring) pc.cell[v] = -1;
         } else if (ring && mode == 1) {
-            if (s_fast.n > 0) {
+            if (nfast > 0) {
                 const double dx = xv.x - pc.x_snap[3 * v], dy = xv.y - pc.x_snap[3 * v + 1];
                 const double dz = xv.z - pc.x_snap[3 * v + 2];
                 keep = dx * dx + dy * dy + dz * dz < pc.limit2;
@@ -1231,7 +1232,6 @@ __device__ __forceinline__ void rep_cached_body(const PassArgs& A, int lb)
                 cell_coords(A.nl, xv, c);
                 // (as vectors, several in flight: 16 us of a block's time with
                 // a hundred of them read one component after the other)
-                const int nfast = s_fast.n;
                 bool near = false;
 #pragma unroll 8
                 for (int i = 0; i < nfast; i++) {
@@ -1265,7 +1265,9 @@ __device__ __forceinline__ void rep_cached_body(const PassArgs& A, int lb)
     __syncthreads();
     const int g = threadIdx.x / kGroup, lane = threadIdx.x % kGroup;
     constexpr int kGroups = 256 / kGroup, kAhead = 2;
-    for (int i0 = g; i0 < s_nrep; i0 += kAhead * kGroups) {
+    // (the phases that most launches on a sphere skip lie behind the rest: their
+    // code in the way cost 0.3 us)
+    for (int i0 = g; __builtin_expect(i0 < s_nrep, 0); i0 += kAhead * kGroups) {
         static_assert(kPairCap == 8, "a lane's entries are two vectors, the second rarely used");
         const double dmax = p.rep_lc1, dmax2 = dmax * dmax * (1.0 + 1e-15);
         int u[kAhead], k[kAhead];
@@ -1331,7 +1333,7 @@ __device__ __forceinline__ void rep_cached_body(const PassArgs& A, int lb)
             store_rep_g(A, u, tr);
         }
     }
-    for (int i = g; !waves && i < n_full; i += kGroups) {
+    for (int i = g; __builtin_expect(!waves && i < n_full, 0); i += kGroups) {
         const int e = s_list[i], u = e < 0 ? ~e : e;
         const d3 xu = load_p(m.x, u);
         const int n = meta_valence(m.meta[u]);
