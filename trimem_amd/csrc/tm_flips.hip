@@ -1176,9 +1176,10 @@ __device__ __forceinline__ FlipEdge flip_edge_of(const int* m)    // the words a
 }
 
 // The Metropolis test (flips.cpp:57-64) u <= min(1, exp(-de)) as de <= -log(u):
-// the logarithm is taken once per proposal, not in every step of a walk.  An
-// injected u may lie outside [0, 1]: u <= 0 passes whatever the (ordered) de, as
-// exp(-de) is never negative, u > 1 and NaN never pass.
+// the logarithm is taken once per proposal, not in every step of a walk.  The same
+// test but for the rounding of its two sides: the serial sweep only looks ahead
+// with it.  An injected u may lie outside [0, 1]: u <= 0 passes whatever the
+// (ordered) de, as exp(-de) is never negative, u > 1 and NaN never pass.
 __device__ __forceinline__ double minus_log(double u)
 {
     if (u <= 0.0) return INFINITY;
